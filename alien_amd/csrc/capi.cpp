@@ -49,6 +49,19 @@ void copyOut(const std::vector<alien_cell_to>& c, const std::vector<alien_partic
     if (!p.empty()) std::memcpy(parts, p.data(), p.size() * sizeof(alien_particle_to));
 }
 
+// a resident world as transfer objects (the counts are written before the buffers are checked)
+void readWorld(WorldSet& set, int w, alien_cell_to* cells, uint64_t cellCap, uint64_t* numCells, alien_particle_to* parts,
+               uint64_t partCap, uint64_t* numParts) {
+    const uint64_t n = uint64_t(set.numCells(w));
+    const WorldSet::ParticleRead particles = set.beginParticles(w);
+    if (numCells) *numCells = n;
+    if (numParts) *numParts = particles.count;
+    if (n > cellCap || particles.count > partCap)
+        throw Error(ALIEN_E_CAPACITY, "output buffer too small (counts were written)");
+    set.readParticles(particles, parts);
+    set.readCells(w, cells);
+}
+
 constexpr int kStripCapMax = alien::kStripMax;
 
 double nowSeconds() {
@@ -212,12 +225,7 @@ int alien_get_data(alien_world* w, alien_cell_to* cells, uint64_t cellCap, uint6
                    alien_particle_to* particles, uint64_t particleCap, uint64_t* numParticles) {
     return guarded([&] {
         requireHealthy(w);
-        WorldImage img;
-        w->set->extract(0, img);
-        std::vector<alien_cell_to> c;
-        std::vector<alien_particle_to> p;
-        img.toTO(c, p);
-        copyOut(c, p, cells, cellCap, numCells, particles, particleCap, numParticles);
+        readWorld(*w->set, 0, cells, cellCap, numCells, particles, particleCap, numParticles);
     });
 }
 
@@ -455,12 +463,7 @@ int alien_batch_get_data(alien_batch* b, int32_t world, alien_cell_to* cells, ui
         require(b != nullptr, "null batch");
         b->flush();
         require(world >= 0 && world < b->resident, "world index out of range");
-        WorldImage img;
-        b->set->extract(world, img);
-        std::vector<alien_cell_to> c;
-        std::vector<alien_particle_to> p;
-        img.toTO(c, p);
-        copyOut(c, p, cells, cellCap, numCells, particles, particleCap, numParticles);
+        readWorld(*b->set, world, cells, cellCap, numCells, particles, particleCap, numParticles);
     });
 }
 
@@ -790,11 +793,11 @@ struct alien_server {
             std::string snapErr;
             try {
                 for (auto& f : finished) {
-                    WorldImage img;
-                    set->extract(f.second, img);
-                    std::vector<alien_cell_to> c;
-                    std::vector<alien_particle_to> p;
-                    img.toTO(c, p);
+                    const WorldSet::ParticleRead particles = set->beginParticles(f.second);
+                    std::vector<alien_particle_to> p(particles.count);
+                    set->readParticles(particles, p.data());
+                    std::vector<alien_cell_to> c(size_t(set->numCells(f.second)));
+                    set->readCells(f.second, c.data());
                     snaps.push_back({f.first, {std::move(c), std::move(p)}});
                     set->setActive(f.second, false);
                 }

@@ -165,6 +165,12 @@ struct __align__(16) StagedParticle {
 // part of the world's state in between: get_data, statistics and rebuilt sets include it)
 constexpr uint32_t kStagedPending = 0x100u;
 
+// pass-through fields of a cell that no kernel of the step reads (genomeComplexity as its bits)
+struct CellExtra {
+    uint32_t mutationId, genomeComplexity;
+    uint8_t cellFunction, ancestorMutationId, selected, pad;
+};
+
 struct Ctx {
     int numWorlds;
     int cellCap;  // total cells (= sum of numCells)

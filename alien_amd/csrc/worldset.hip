@@ -251,6 +251,9 @@ WorldImage WorldImage::fromTO(const alien_world_desc& desc, const alien_params& 
         h.ancestorMutationId[sl] = c.ancestorMutationId;
         h.selected[sl] = c.selected;
         h.genomeComplexity[sl] = c.genomeComplexity;
+        uint32_t genome = 0;
+        std::memcpy(&genome, &c.genomeComplexity, sizeof(genome));
+        h.hasExtra = h.hasExtra || (c.mutationId | genome | c.cellFunction | c.ancestorMutationId | c.selected) != 0u;
     }
     img.ppos.resize(np);
     img.pvel.resize(np);
@@ -275,6 +278,7 @@ WorldImage WorldImage::fromTO(const alien_world_desc& desc, const alien_params& 
         img.pid[i] = p.id;
         h.particleId[i] = p.id;
         h.particleSelected[i] = p.selected;
+        h.hasSelected = h.hasSelected || p.selected != 0;
     }
     img.numParticles = np;
     // Living states need tracking on the device only if some cell is not trivially Ready: a state
@@ -414,7 +418,9 @@ WorldSet::WorldSet() {
     check_hip(hipEventCreateWithFlags(&side_.mapped, hipEventDisableTiming), "hipEventCreate");
     check_hip(hipEventCreateWithFlags(&side_.join, hipEventDisableTiming), "hipEventCreate");
     check_hip(hipEventCreateWithFlags(&liveReady_, hipEventDisableTiming), "hipEventCreate");
-    check_hip(hipHostMalloc(reinterpret_cast<void**>(&liveHost_), sizeof(int), hipHostMallocDefault), "hipHostMalloc");
+    check_hip(hipHostMalloc(reinterpret_cast<void**>(&liveHost_), 64 + sizeof(DevCounters), hipHostMallocDefault),
+              "hipHostMalloc");
+    hostWord_ = reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(liveHost_) + 64);
 }
 
 WorldSet::~WorldSet() {
@@ -638,6 +644,23 @@ void WorldSet::build(const std::vector<Source>& sources) {
     stiff_ = static_cast<float*>(A(sizeof(float) * NC));
     cid_ = static_cast<unsigned long long*>(A(sizeof(unsigned long long) * NC));
     ageBase_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
+    bool anyExtra = false;
+    for (const auto& h : hosts) anyExtra = anyExtra || h.hasExtra;
+    extra_ = anyExtra ? static_cast<CellExtra*>(A(sizeof(CellExtra) * NC)) : nullptr;
+    selected_.assign(hosts.size(), nullptr);
+    for (size_t w = 0; w < hosts.size(); ++w)
+        if (hosts[w].hasSelected) {
+            selected_[w] = static_cast<uint8_t*>(A(hosts[w].particleSelected.size()));
+            check_hip(hipMemcpy(selected_[w], hosts[w].particleSelected.data(), hosts[w].particleSelected.size(),
+                                hipMemcpyHostToDevice),
+                      "H2D");
+        }
+    dWords_ = static_cast<unsigned long long*>(A(sizeof(unsigned long long) * 2));
+    rankOfSlot_ = nullptr;
+    rankState_.assign(hosts.size(), 0);
+    idBits_.assign(hosts.size(), 0);
+    scratch_ = nullptr;
+    scratchBytes_ = 0;
     staged_ = partStage_ > 0 ? static_cast<StagedParticle*>(A(sizeof(StagedParticle) * NC)) : nullptr;
     splitStaged_ = splitStage_ > 0 ? static_cast<StagedParticle*>(A(sizeof(StagedParticle) * size_t(splitStage_))) : nullptr;
     living_[0] = static_cast<uint8_t*>(A(NC));
@@ -765,6 +788,21 @@ void WorldSet::build(const std::vector<Source>& sources) {
             pendingCopies.push_back({wi, int(ow.partOff), o.splitStaged_, np});
         }
     }
+    if (extra_)
+        for (size_t wi = 0; wi < hosts.size(); ++wi) {
+            const HostWorld& h = hosts[wi];
+            std::vector<CellExtra> x(static_cast<size_t>(h.numCells));
+            for (size_t k = 0; k < x.size(); ++k) {
+                std::memcpy(&x[k].genomeComplexity, &h.genomeComplexity[k], sizeof(uint32_t));
+                x[k].mutationId = h.mutationId[k];
+                x[k].cellFunction = h.cellFunction[k];
+                x[k].ancestorMutationId = h.ancestorMutationId[k];
+                x[k].selected = h.selected[k];
+            }
+            if (!x.empty())
+                check_hip(hipMemcpy(extra_ + worlds[wi].cellOff, x.data(), sizeof(CellExtra) * x.size(), hipMemcpyHostToDevice),
+                          "H2D");
+        }
     check_hip(hipStreamSynchronize(stream_), "hipStreamSynchronize");
 
     hosts_ = std::move(hosts);
@@ -1212,23 +1250,147 @@ int WorldSet::numParticles(int w) {
     return c.numParticles;
 }
 
-int WorldSet::liveParticles(int w) {
+DevCounters WorldSet::counters(int w) {
+    DevCounters* c = reinterpret_cast<DevCounters*>(hostWord_);
+    check_hip(hipMemcpyAsync(c, dCtr_ + w, sizeof(*c), hipMemcpyDeviceToHost, stream_), "D2H");
     synchronize();
-    const int np = numParticles(w);
-    std::vector<uint8_t> f(static_cast<size_t>(std::max(np, 0)));
-    if (np > 0)
-        check_hip(hipMemcpy(f.data(), buf_[parity_].pflags + worlds_.at(w).partOff, size_t(np), hipMemcpyDeviceToHost),
-                  "D2H");
-    int live = 0;
-    for (uint8_t x : f) live += (x & kParticleDead) ? 0 : 1;
-    if (splitStage_ > 0 && np > 0) {  // and the split halves waiting for the next map
-        std::vector<StagedParticle> rec(static_cast<size_t>(np));
-        check_hip(hipMemcpy(rec.data(), splitStaged_ + worlds_.at(w).partOff, sizeof(StagedParticle) * size_t(np),
-                            hipMemcpyDeviceToHost),
-                  "D2H");
-        for (const StagedParticle& r : rec) live += (r.color & kStagedPending) ? 1 : 0;
+    return *c;
+}
+
+unsigned long long WorldSet::readWord(int k) {
+    check_hip(hipMemcpyAsync(hostWord_, dWords_ + k, sizeof(*hostWord_), hipMemcpyDeviceToHost, stream_), "D2H");
+    synchronize();
+    return *hostWord_;
+}
+
+void* WorldSet::scratch(size_t bytes) {
+    if (bytes <= sizeof(int4) * size_t(candCap_)) return cand_;
+    if (bytes > scratchBytes_) {
+        if (scratch_) release(scratch_);
+        scratch_ = nullptr;
+        scratchBytes_ = 0;
+        scratch_ = alloc(bytes);
+        scratchBytes_ = bytes;
     }
-    return live;
+    return scratch_;
+}
+
+PackParticles WorldSet::packParticles(int w, int np) const {
+    const HotBuffers& S = buf_[parity_];
+    const int off = worlds_.at(w).partOff;
+    PackParticles a{};
+    a.np = np;
+    a.entries = splitStage_ > 0 ? 2 * np : np;
+    a.ppos = S.ppos + off;
+    a.pvel = S.pvel + off;
+    a.pen = S.pen + off;
+    a.pslot = S.pslot + off;
+    a.pflags = S.pflags + off;
+    a.pid = S.pid + off;
+    a.halves = splitStage_ > 0 ? splitStaged_ + off : nullptr;
+    a.selected = selected_.at(w);
+    return a;
+}
+
+int WorldSet::liveParticles(int w) {
+    const int np = counters(w).numParticles;
+    if (np <= 0) return 0;
+    const PackParticles a = packParticles(w, np);
+    uint32_t* tiles = static_cast<uint32_t*>(scratch(sizeof(uint32_t) * (size_t(a.entries) / kPartTile + 1)));
+    launch_part_keys(a, tiles, nullptr, dWords_, stream_);
+    check_hip(hipGetLastError(), "particle count");
+    return int(readWord(0));
+}
+
+WorldSet::ParticleRead WorldSet::beginParticles(int w) {
+    ParticleRead r;
+    const int np = counters(w).numParticles;
+    if (np <= 0) return r;
+    r.from = packParticles(w, np);
+    const size_t n = size_t(r.from.entries), sortBytes = SortBuffers::bytes(n);
+    char* p = static_cast<char*>(scratch(sortBytes + sizeof(uint32_t) * (n / kPartTile + 1)));
+    r.sort = SortBuffers::at(p, n);
+    launch_part_keys(r.from, reinterpret_cast<uint32_t*>(p + sortBytes), &r.sort, dWords_, stream_);
+    check_hip(hipGetLastError(), "particle keys");
+    r.count = size_t(readWord(0));
+    if (r.count > 1) r.differing = readWord(1);
+    return r;
+}
+
+void WorldSet::readParticles(const ParticleRead& r, alien_particle_to* out) {
+    if (r.count == 0) return;
+    const int at = launch_radix_sort(r.sort, int(r.count), r.differing, stream_);
+    check_hip(hipGetLastError(), "particle sort");
+    read_records(r.count, sizeof(alien_particle_to), out, stream_, [&](size_t first, size_t count, void* to) {
+        launch_pack_particles(r.from, r.sort.vals[at], int(first), int(count), to, stream_);
+    });
+}
+
+// The ids of a set's cells never change, and a cell keeps its slot: the slots' ranks by id are taken
+// once.  Cells with equal ids come in index order, which does change: such a world is sorted per call.
+void WorldSet::ensureRanks(int w) {
+    if (rankState_.at(w)) return;
+    const DevWorld& dw = worlds_.at(w);
+    const int n = dw.numCells;
+    if (!rankOfSlot_) rankOfSlot_ = static_cast<int*>(alloc(sizeof(int) * size_t(cellCap_)));
+    const SortBuffers b = SortBuffers::at(scratch(SortBuffers::bytes(size_t(n))), size_t(n));
+    launch_fill_u32(reinterpret_cast<uint32_t*>(dWords_), 0u, 4, stream_);
+    launch_cell_keys(cid_ + dw.cellOff, nullptr, n, b, dWords_, stream_);
+    check_hip(hipGetLastError(), "cell keys");
+    idBits_[w] = readWord(0);
+    const int at = launch_radix_sort(b, n, idBits_[w], stream_);
+    launch_cell_ranks(b.keys[at], b.vals[at], n, rankOfSlot_ + dw.cellOff, dWords_ + 1, stream_);
+    check_hip(hipGetLastError(), "cell ranks");
+    rankState_[w] = readWord(1) ? 2 : 1;
+}
+
+void WorldSet::readCells(int w, alien_cell_to* out) {
+    const DevWorld& dw = worlds_.at(w);
+    const int n = dw.numCells;
+    if (n == 0) return;
+    ensureRanks(w);
+    const HotBuffers& S = buf_[parity_];
+    const int off = dw.cellOff;
+    PackCells a{};
+    a.slot = S.slot + off;
+    a.flags = S.flags + off;
+    a.pos = S.pos + off;
+    a.vel = S.vel + off;
+    a.btgt = S.btgt + off;
+    a.brest = S.brest + off;
+    a.bang = S.bang + off;
+    a.plane = size_t(cellCap_);
+    a.cid = cid_ + off;
+    a.energy = energy_ + off;
+    a.stiff = stiff_ + off;
+    a.ageBase = ageBase_ + off;
+    a.creature = creature_ + off;
+    a.steps = uint32_t(hosts_.at(w).stepsSinceSet);
+    a.stepped = hosts_.at(w).stepsSinceSet > 0;
+    // (a world without tracked living states has every cell Ready without a count)
+    a.living = livingWork_.at(w) ? living_[parity_] + off : nullptr;
+    a.activation = livingWork_.at(w) ? activation_ + off : nullptr;
+    a.extra = extra_ ? extra_ + off : nullptr;
+    const bool equal = rankState_.at(w) == 2;
+    const size_t sortBytes = equal ? SortBuffers::bytes(size_t(n)) : 0;
+    char* p = static_cast<char*>(scratch(sortBytes + 2 * sizeof(int) * size_t(n)));
+    int* rankOf = reinterpret_cast<int*>(p + sortBytes);
+    if (equal) {
+        const SortBuffers b = SortBuffers::at(p, size_t(n));
+        launch_cell_keys(a.cid, a.slot, n, b, dWords_, stream_);
+        const int at = launch_radix_sort(b, n, idBits_[w], stream_);
+        launch_cell_ranks(b.keys[at], b.vals[at], n, rankOf, nullptr, stream_);
+        a.order = b.vals[at];
+    } else {
+        int* order = rankOf + n;
+        launch_cell_order(a.slot, rankOfSlot_ + off, n, order, rankOf, stream_);
+        a.order = order;
+    }
+    a.rankOf = rankOf;
+    check_hip(hipGetLastError(), "cell order");
+    read_records(size_t(n), sizeof(alien_cell_to), out, stream_, [&](size_t first, size_t count, void* to) {
+        launch_pack_cells(a, int(first), int(count), to, stream_);
+    });
 }
 
 uint64_t WorldSet::timestep(int w) {
@@ -1695,33 +1857,26 @@ alien_totals WorldSet::totals(int wi) {
 alien_statistics WorldSet::statistics(int wi) {
     const DevWorld& w = worlds_.at(wi);
     alien_statistics st{};
-    st.timestep = timestep(wi);
+    const DevCounters ctr = counters(wi);
+    st.timestep = ctr.timestep;
     int cellBlocks = 0;
-    const int blocks = statistics_blocks(w.numCells, w.partCap, cellBlocks);
+    // (the particle slots beyond the live range would only add zeros)
+    const int blocks = statistics_blocks(w.numCells, std::min(ctr.numParticles, w.partCap), cellBlocks);
     if (blocks == 0) return st;
+    // the blocks' partials go to pinned memory, or through the scratch when they are too many for it
+    const size_t enBytes = sizeof(double) * size_t(blocks) * kColors, bytes = enBytes + sizeof(int) * size_t(blocks) * kColors;
+    PinnedBuffer pinned;
+    const bool fits = bytes <= PinnedBuffer::kBytes;
+    std::vector<char> host(fits ? 0 : bytes);
+    char* p = static_cast<char*>(fits ? pinned.data() : scratch(bytes));
+    launch_statistics(makeCtx(parity_), wi, cellBlocks, blocks, reinterpret_cast<int*>(p + enBytes),
+                      reinterpret_cast<double*>(p), stream_);
+    check_hip(hipGetLastError(), "statistics");
     synchronize();
-    int* cnt = nullptr;
-    double* en = nullptr;
-    check_hip(hipMalloc(&cnt, sizeof(int) * size_t(blocks) * kColors), "hipMalloc");
-    if (hipMalloc(&en, sizeof(double) * size_t(blocks) * kColors) != hipSuccess) {
-        (void)hipFree(cnt);
-        throw Error(ALIEN_E_OOM, "hipMalloc failed (statistics)");
-    }
-    std::vector<int> hc(size_t(blocks) * kColors);
-    std::vector<double> he(size_t(blocks) * kColors);
-    try {
-        launch_statistics(makeCtx(parity_), wi, cellBlocks, blocks, cnt, en, stream_);
-        check_hip(hipGetLastError(), "statistics");
-        synchronize();
-        check_hip(hipMemcpy(hc.data(), cnt, sizeof(int) * hc.size(), hipMemcpyDeviceToHost), "D2H");
-        check_hip(hipMemcpy(he.data(), en, sizeof(double) * he.size(), hipMemcpyDeviceToHost), "D2H");
-    } catch (...) {
-        (void)hipFree(cnt);
-        (void)hipFree(en);
-        throw;
-    }
-    (void)hipFree(cnt);
-    (void)hipFree(en);
+    if (!fits) check_hip(hipMemcpy(host.data(), p, bytes, hipMemcpyDeviceToHost), "D2H");
+    const char* from = fits ? p : host.data();
+    const double* he = reinterpret_cast<const double*>(from);
+    const int* hc = reinterpret_cast<const int*>(from + enBytes);
     for (int b = 0; b < blocks; ++b)
         for (int k = 0; k < kColors; ++k) {
             (b < cellBlocks ? st.numCells : st.numParticles)[k] += hc[size_t(b) * kColors + k];

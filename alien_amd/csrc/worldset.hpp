@@ -19,6 +19,7 @@
 #include "../../include/alien_hip.h"
 #include "engine_types.hpp"
 #include "kernels.hpp"
+#include "readback.hpp"
 
 namespace alien {
 
@@ -67,6 +68,8 @@ struct HostWorld {
     std::vector<float> genomeComplexity;
     std::vector<uint64_t> particleId;
     std::vector<uint8_t> particleSelected;
+    bool hasExtra = false;     // some cell has a non-zero CellExtra field
+    bool hasSelected = false;  // some particle is selected
 };
 
 // complete state of one world in the device layout, staged in host memory
@@ -130,6 +133,18 @@ public:
     // advance every world by n timesteps
     void step(uint64_t n);
     void extract(int w, WorldImage& out);
+    // The world as transfer objects in ascending id order, packed on the device (k_readback.hip):
+    // first the living particles (their count, and their records to `out`; both calls without anything
+    // in between, they share the scratch), then the cells.
+    struct ParticleRead {
+        size_t count = 0;
+        PackParticles from{};
+        SortBuffers sort{};
+        unsigned long long differing = 0;
+    };
+    ParticleRead beginParticles(int w);
+    void readParticles(const ParticleRead& r, alien_particle_to* out);
+    void readCells(int w, alien_cell_to* out);
     alien_totals totals(int w);
     alien_statistics statistics(int w);  // per-colour counts and energies, reduced on the device
     // the same result without allocating device memory (the library's per-device scratch array);
@@ -190,12 +205,20 @@ private:
     // moves the particles to arrays with the given capacities per world (and a staging area)
     void growParticles(const std::vector<int64_t>& caps);
     void release(void* p);  // frees one allocation of alloc()
+    // device scratch between steps: the fusion candidate list, or (beyond its size) an allocation that
+    // grows with the largest request
+    void* scratch(size_t bytes);
+    PackParticles packParticles(int w, int np) const;
+    DevCounters counters(int w);
+    unsigned long long readWord(int k);  // dWords_[k] once the stream has drained
+    void ensureRanks(int w);  // ranks of the world's slots by cell id, once per set
     void updateRadiation();  // shape_.hasRadiation from the active worlds' parameters
     void anchorAges(int w);  // worlds_[w].ageTs from its timestep and steps simulated
 
     hipStream_t stream_ = nullptr;
     SideStream side_;  // particle kernels beside the neighbour pass
     int* liveHost_ = nullptr;        // pinned: live particles as read by checkParticlesAsync
+    unsigned long long* hostWord_ = nullptr;  // pinned, behind it: words and counters read back
     hipEvent_t liveReady_ = nullptr;  // recorded after that read
     bool livePending_ = false;
     std::vector<HostWorld> hosts_;
@@ -224,6 +247,14 @@ private:
     int splitStage_ = 0;                     // first split staging slot (0: none)
     StagedParticle* splitStaged_ = nullptr;  // [splitStage_] with a split staging area
     int numCellBlocks_ = 0;
+    CellExtra* extra_ = nullptr;  // [cellCap] by slot, if some world has any
+    std::vector<uint8_t*> selected_;  // per world: selection by particle slot, if some particle is selected
+    unsigned long long* dWords_ = nullptr;  // [2] results of the read-back kernels
+    int* rankOfSlot_ = nullptr;  // [cellCap] read-back order of the worlds' slots (ensureRanks)
+    std::vector<uint8_t> rankState_;  // per world: 0 not ranked yet, 1 ranked, 2 equal ids (ranked per call)
+    std::vector<unsigned long long> idBits_;  // per world: bits in which the cell ids differ
+    void* scratch_ = nullptr;
+    size_t scratchBytes_ = 0;
     uint8_t* living_[2] = {nullptr, nullptr};  // living states by slot, alternating with the parity
     uint32_t* activation_ = nullptr;
     uint32_t* creature_ = nullptr;

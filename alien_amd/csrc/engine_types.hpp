@@ -41,6 +41,8 @@ constexpr uint32_t kMaxConnShift = 4;          // bits 4..7
 constexpr uint32_t kColorShift = 8;            // bits 8..15
 constexpr uint32_t kBarrierBit = 1u << 16;
 constexpr uint32_t kDetachedBit = 1u << 17;
+// stage byte of a cell (Ctx::stage)
+constexpr uint8_t kStagedCell = 1, kDropBonds = 2, kMarkedCell = 4;
 // particle flags byte
 constexpr uint8_t kParticleColorMask = 0x7F;
 constexpr uint8_t kParticleDead = 0x80;
@@ -239,8 +241,10 @@ struct Ctx {
     uint32_t* mflags;
     int* newidx;   // [cellCap] A index -> new index
     int* psorted;  // [partCap]
-    uint8_t* stagedMark;  // [cellCap] end-of-step cell is staged (bonded or barrier at the neighbour pass);
-                          // written for the cells of bond-work worlds
+    // [cellCap] kStagedCell: the end-of-step cell is staged (bonded or barrier at the neighbour pass);
+    // kDropBonds: it loses all its bonds at the end of the step; kMarkedCell: it or a bond partner
+    // does.  The neighbour pass writes the byte of every cell of the bond-work worlds.
+    uint8_t* stage;
     float2* own;    // [cellCap]
     float2* shift;  // [cellCap] Verlet displacement of a staged cell, applied after the second force pass
     float* bstiff;  // [cellCap] stiffness of a bonded cell in end-of-step order (written by the neighbour pass)
@@ -248,8 +252,6 @@ struct Ctx {
     float2* out1;  // [kMaxBonds][cellCap]
     float2* out2;
     uint32_t* valid;  // [cellCap]
-    uint8_t* delFlag;
-    uint8_t* mark;
     unsigned long long* claim;  // [cellCap]
     int4* cand;                 // [candCap] (a, b, world, live)
     int candCap;
@@ -259,7 +261,6 @@ struct Ctx {
     int* cclaim;      // [cellCap]
     const int2* cellBlocks;  // per block: (world, first global cell index)
     const int2* bondBlocks;  // the same over the worlds with bond work
-    const int2* binBlocks;   // per block: (world, first global bin index) over cell bins
     const int2* pbinBlocks;  // per block: (world, first global bin index) over particle bins
     // per block of partBlockParticles live particles: (world, first global particle index), over
     // the active worlds' live ranges; written by the host when the tables are built and by the
@@ -269,7 +270,7 @@ struct Ctx {
     int partBlockParticles;
     const int2* tileBlocks;  // per block: (world, tile index), -1 for padding blocks
     const int2* livingBlocks;  // per block: (world, first global cell index) over livingWork worlds
-    int numCellBlocks, cellBlockCells;  // entries of cellBlocks, cells per entry
+    int blockThreads;  // cells, bins or living cells per entry of the block tables above
 };
 
 }  // namespace alien

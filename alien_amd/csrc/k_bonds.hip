@@ -8,164 +8,184 @@
 // CellConnectionProcessor (source/EngineGpuKernels/CellConnectionProcessor.cuh): fusion pairs
 // claim their cells and bond neighbours and apply only when every claim holds (R5); bond deletion
 // works from per-cell flags (R6).
-#include "kernels_common.hpp"
+//
+// The phase is a chain of launches, each of which needs all cells of the one before it.  Short ones
+// cost their latency, not their work (18,000 cells: 2 to 12 us each), so what is independent shares a
+// launch: the living states, and on workgroups of their own the stages of the particles' chain
+// (particle_steps.hpp).  A step of 18,000 bonded cells with 700 particles took 126 us in 22 launches and
+// takes 90 us in 11; 10,700 cells at ALIEN's default parameters 176 us in 27 and 124 us in 12; 840,000
+// bonded cells without particles 336 us and 331 us.
 #include "kernels.hpp"
+#include "particle_steps.hpp"
 
 namespace alien {
 
 // The kernels below run one thread per cell of the worlds that can have bonded or barrier cells
 // (bond block table) and act on the staged cells: those the neighbour pass found bonded or barrier
-// (stagedMark), which is the set CellProcessor's bonded-cell passes cover.  Cells bonded by this
-// step's fusion are not among them.
-__device__ __forceinline__ bool staged_cell(const Ctx& c, int& x, int& wi) {
-    const int2 blk = c.bondBlocks[blockIdx.x];
+// (stage), which is the set CellProcessor's bonded-cell passes cover.  Cells bonded by this step's
+// fusion are not among them.
+__device__ __forceinline__ bool staged_cell(const Ctx& c, int block, int& x, int& wi, uint8_t& stage) {
+    const int2 blk = c.bondBlocks[block];
     wi = blk.x;
     x = blk.y + int(threadIdx.x);
     const DevWorld& w = c.worlds[wi];
-    return x < w.cellOff + w.numCells && c.stagedMark[x] != 0;
-}
-
-// bond targets of the staged cells from start-of-step to end-of-step indices
-__global__ void k_remap(Ctx c) {
-    const int cap = c.cellCap;
-    int x, wi;
-    if (!staged_cell(c, x, wi)) return;
-    {
-        const DevWorld& w = c.worlds[wi];
-        const int nc = flags_num_conn(c.B.flags[x]);
-        // all targets first, then all lookups, then the stores (so that the loads overlap)
-        int t[kMaxBonds], ni[kMaxBonds];
-#pragma unroll
-        for (int b = 0; b < kMaxBonds; ++b) t[b] = b < nc ? c.B.btgt[b * cap + x] : 0;
-#pragma unroll
-        for (int b = 0; b < kMaxBonds; ++b) ni[b] = b < nc ? c.newidx[w.cellOff + t[b]] : 0;
-#pragma unroll
-        for (int b = 0; b < kMaxBonds; ++b)
-            if (b < nc) c.B.btgt[b * cap + x] = ni[b] - w.cellOff;
-    }
+    stage = 0;
+    if (x >= w.cellOff + w.numCells) return false;
+    stage = c.stage[x];
+    return stage != 0;
 }
 
 // bond vector from x to o.  In the second pass the cells stand at pos + shift; the vector is taken
 // as the start-of-pass difference plus the difference of the shifts, which keeps the FP32 result
 // close to the exact one (rounding pos + shift first would cost up to ulp(world size)).
-__device__ __forceinline__ f2 bond_vector(const Ctx& c, int o, f2 px, f2 sx, int pass, float Wf, float Hf) {
+template <int kPass>
+__device__ __forceinline__ f2 bond_vector(const Ctx& c, int o, f2 px, f2 sx, float Wf, float Hf) {
     const f2 d = torus_delta(to_f2(c.B.pos[o]), px, Wf, Hf);
-    if (pass == 0) return d;
+    if constexpr (kPass == 0) return d;
     return add(d, sub(to_f2(c.shift[o]), sx));
 }
 
-// connection forces of the staged cells: own force plus per-bond angle forces for the partners;
-// pass 1 also runs checkConnections (CellProcessor.cuh:493-523) on the moved positions.  The
-// partners' data of all the cell's bonds is loaded up front, so the loads are in flight together
-// (lanes skip the slots beyond their cell's bonds: 7 % faster than loading all six).
-// (at most 80 VGPRs, six waves per SIMD: the partner loads are latency-bound)
-__global__ void __attribute__((amdgpu_waves_per_eu(6))) k_conn_own(Ctx c, int pass) {
+// Connection forces of a staged cell: own force plus per-bond angle forces for the partners; pass 1
+// also runs checkConnections (CellProcessor.cuh:493-523) on the moved positions.  The partners' data of
+// all the cell's bonds is loaded up front, so the loads are in flight together (lanes skip the slots
+// beyond their cell's bonds: 7 % faster than loading all six).
+// Pass 0 finds the bond targets in start-of-step indices, as the neighbour pass left them, and
+// renumbers them to the end-of-step order: it takes its own list from B (which it rewrites) and its
+// partners' lists from A, so that no thread reads a list another rewrites.
+template <int kPass> __device__ __forceinline__ void conn_own(const Ctx& c, int block) {
     const int cap = c.cellCap;
     int x, wi;
-    if (!staged_cell(c, x, wi)) return;
-    {
-        const DevWorld& w = c.worlds[wi];
-        const DevParams& P = c.params[wi];
-        const uint32_t fx = c.B.flags[x];
-        const int nc = flags_num_conn(fx);
-        if (nc == 0 || flags_barrier(fx)) {
-            c.valid[x] = 0u;
-            if (pass == 1) c.stretched[x] = 0;  // checkConnections skips barrier cells
-            return;
+    uint8_t stage;
+    if (!staged_cell(c, block, x, wi, stage)) return;
+    const DevWorld& w = c.worlds[wi];
+    const DevParams& P = c.params[wi];
+    const uint32_t fx = c.B.flags[x];
+    const int nc = flags_num_conn(fx);
+    // the partners' indices in the arrays their bond lists are read from (pass 0: A, pass 1: B), and
+    // in B
+    const HotBuffers& L = kPass == 0 ? c.A : c.B;
+    int tl[kMaxBonds], tg[kMaxBonds];
+#pragma unroll
+    for (int b = 0; b < kMaxBonds; ++b) tl[b] = b < nc ? w.cellOff + c.B.btgt[b * cap + x] : x;
+#pragma unroll
+    for (int b = 0; b < kMaxBonds; ++b) tg[b] = kPass == 0 && b < nc ? c.newidx[tl[b]] : tl[b];
+    if constexpr (kPass == 0) {
+#pragma unroll
+        for (int b = 0; b < kMaxBonds; ++b)
+            if (b < nc) c.B.btgt[b * cap + x] = tg[b] - w.cellOff;
+    }
+    if (nc == 0 || flags_barrier(fx)) {
+        c.valid[x] = 0u;
+        if (kPass == 1) c.stretched[x] = 0;  // checkConnections skips barrier cells
+        return;
+    }
+    const float Wf = float(w.W), Hf = float(w.H);
+    const bool considerAngles = (c.ctr[wi].timestep % 3ull) == 0ull;
+    const f2 px = to_f2(c.B.pos[x]);
+    const f2 shx = kPass == 0 ? f2{0.0f, 0.0f} : to_f2(c.shift[x]);
+    const float sx = c.bstiff[x];
+    const float kx2 = sx * sx;
+    f2 disp[kMaxBonds];
+    float kc2[kMaxBonds], rest[kMaxBonds];
+#pragma unroll
+    for (int b = 0; b < kMaxBonds; ++b) {
+        const int o = tg[b];
+        kc2[b] = 0.0f;
+        rest[b] = 0.0f;
+        disp[b] = f2{0.0f, 0.0f};
+        if (b < nc) {
+            const float so = c.bstiff[o];
+            kc2[b] = so * so;
+            rest[b] = c.B.brest[b * cap + x];
+            disp[b] = bond_vector<kPass>(c, o, px, shx, Wf, Hf);
         }
-        const float Wf = float(w.W), Hf = float(w.H);
-        const bool considerAngles = (c.ctr[wi].timestep % 3ull) == 0ull;
-        const f2 px = to_f2(c.B.pos[x]);
-        const f2 shx = pass == 0 ? f2{0.0f, 0.0f} : to_f2(c.shift[x]);
-        const float sx = c.bstiff[x];
-        const float kx2 = sx * sx;
-        int tg[kMaxBonds];
-        f2 disp[kMaxBonds];
-        float kc2[kMaxBonds], rest[kMaxBonds];
+    }
+    // the bond before the first is the last one
+    f2 prevDisp = disp[0];
+    int lastTarget = tl[0];
 #pragma unroll
-        for (int b = 0; b < kMaxBonds; ++b) tg[b] = b < nc ? w.cellOff + c.B.btgt[b * cap + x] : x;
-#pragma unroll
-        for (int b = 0; b < kMaxBonds; ++b) {
-            const int o = tg[b];
-            kc2[b] = 0.0f;
-            rest[b] = 0.0f;
-            disp[b] = f2{0.0f, 0.0f};
-            if (b < nc) {
-                const float so = c.bstiff[o];
-                kc2[b] = so * so;
-                rest[b] = c.B.brest[b * cap + x];
-                disp[b] = bond_vector(c, o, px, shx, pass, Wf, Hf);
-            }
+    for (int b = 1; b < kMaxBonds; ++b)
+        if (b == nc - 1) {
+            prevDisp = disp[b];
+            lastTarget = tl[b];
         }
-        // the bond before the first is the last one
-        f2 prevDisp = disp[0];
-        int lastTarget = tg[0];
+    f2 force = {0.0f, 0.0f};
+    uint32_t v = 0u;
+    bool tooLong = false;
+    const float maxBind = P.maxBindingDistance[flags_color(fx) % kColors];
 #pragma unroll
-        for (int b = 1; b < kMaxBonds; ++b)
-            if (b == nc - 1) {
-                prevDisp = disp[b];
-                lastTarget = tg[b];
-            }
-        f2 force = {0.0f, 0.0f};
-        uint32_t v = 0u;
-        bool tooLong = false;
-        const float maxBind = P.maxBindingDistance[flags_color(fx) % kColors];
+    for (int b = 0; b < kMaxBonds; ++b) {
+        if (b >= nc) break;
+        const int o = tl[b];
+        const f2 d = disp[b];
+        const float ad = len2(d);
+        if (kPass == 1 && ad > maxBind) tooLong = true;  // checkConnections on new positions
+        const float dev = ad - rest[b];
+        force = add(force, dvd(mul(mul(unit(d), dev), kx2 + kc2[b]), 6.0f));
+        bool skipped = false;  // a bond whose actual angle is negative keeps the previous vector
+        if (considerAngles && (nc > 2 || (nc == 2 && b == 0))) {
+            const int lc = b == 0 ? lastTarget : tl[b > 0 ? b - 1 : 0];
+            const uint32_t fo = L.flags[o];
+            const int no = flags_num_conn(fo);
+            // (the partner's list: its loads in flight together)
+            int lt[kMaxBonds];
 #pragma unroll
-        for (int b = 0; b < kMaxBonds; ++b) {
-            if (b >= nc) break;
-            const int o = tg[b];
-            const f2 d = disp[b];
-            const float ad = len2(d);
-            if (pass == 1 && ad > maxBind) tooLong = true;  // checkConnections on new positions
-            const float dev = ad - rest[b];
-            force = add(force, dvd(mul(mul(unit(d), dev), kx2 + kc2[b]), 6.0f));
-            bool skipped = false;  // a bond whose actual angle is negative keeps the previous vector
-            if (considerAngles && (nc > 2 || (nc == 2 && b == 0))) {
-                const int lc = b == 0 ? lastTarget : tg[b > 0 ? b - 1 : 0];
-                const uint32_t fo = c.B.flags[o];
-                const int no = flags_num_conn(fo);
-                bool tri = false;
-                for (int j = 0; j < no; ++j)
-                    if (w.cellOff + c.B.btgt[j * cap + o] == lc) {
-                        tri = true;
-                        break;
+            for (int j = 0; j < kMaxBonds; ++j) lt[j] = j < no ? L.btgt[j * cap + o] : -1;
+            bool tri = false;
+#pragma unroll
+            for (int j = 0; j < kMaxBonds; ++j) tri = tri || lt[j] == lc - w.cellOff;
+            if (!tri) {
+                const float angle = angle_of(d);
+                const float prevAngle = angle_of(prevDisp);
+                const float act = sub_angle(angle, prevAngle);
+                if (act < 0.0f) {
+                    skipped = true;
+                } else {
+                    const float ref = c.B.bang[b * cap + x];
+                    const float strength = fabsf(ref - act) / 2000.0f * kx2;
+                    f2 f1 = mul(dvd(unit(d), fmaxf(len2(d), P.minDistance)), strength);
+                    rot_cw(f1);
+                    f2 fb = mul(dvd(unit(prevDisp), fmaxf(len2(prevDisp), P.minDistance)), strength);
+                    rot_ccw(fb);
+                    if (ref < act) {
+                        f1 = mul(f1, -1.0f);
+                        fb = mul(fb, -1.0f);
                     }
-                if (!tri) {
-                    const float angle = angle_of(d);
-                    const float prevAngle = angle_of(prevDisp);
-                    const float act = sub_angle(angle, prevAngle);
-                    if (act < 0.0f) {
-                        skipped = true;
-                    } else {
-                        const float ref = c.B.bang[b * cap + x];
-                        const float strength = fabsf(ref - act) / 2000.0f * kx2;
-                        f2 f1 = mul(dvd(unit(d), fmaxf(len2(d), P.minDistance)), strength);
-                        rot_cw(f1);
-                        f2 fb = mul(dvd(unit(prevDisp), fmaxf(len2(prevDisp), P.minDistance)), strength);
-                        rot_ccw(fb);
-                        if (ref < act) {
-                            f1 = mul(f1, -1.0f);
-                            fb = mul(fb, -1.0f);
-                        }
-                        if (!flags_barrier(fo)) {
-                            c.out1[b * cap + x] = to_float2(f1);
-                            v |= 1u << b;
-                        }
-                        if (!flags_barrier(c.B.flags[lc])) {
-                            c.out2[b * cap + x] = to_float2(fb);
-                            v |= 1u << (6 + b);
-                        }
-                        force = sub(force, add(f1, fb));
+                    if (!flags_barrier(fo)) {
+                        c.out1[b * cap + x] = to_float2(f1);
+                        v |= 1u << b;
                     }
+                    if (!flags_barrier(L.flags[lc])) {
+                        c.out2[b * cap + x] = to_float2(fb);
+                        v |= 1u << (6 + b);
+                    }
+                    force = sub(force, add(f1, fb));
                 }
             }
-            if (!skipped) prevDisp = d;
         }
-        c.own[x] = to_float2(force);
-        c.valid[x] = v;
-        if (tooLong) c.delFlag[x] = 1;
-        if (pass == 1) c.stretched[x] = tooLong ? 1 : 0;
+        if (!skipped) prevDisp = d;
     }
+    c.own[x] = to_float2(force);
+    c.valid[x] = v;
+    if (tooLong) c.stage[x] = uint8_t(stage | kDropBonds);
+    if (kPass == 1) c.stretched[x] = tooLong ? 1 : 0;
+}
+
+// (at most 80 VGPRs, six waves per SIMD: the partner loads are latency-bound)
+__global__ void __attribute__((amdgpu_waves_per_eu(6))) k_conn_first(Ctx c, int partBlocks) {
+    const int b = int(blockIdx.x);
+    if (b < partBlocks)
+        part_move(c, {b, partBlocks});
+    else
+        conn_own<0>(c, b - partBlocks);
+}
+
+__global__ void __attribute__((amdgpu_waves_per_eu(6))) k_conn_second(Ctx c, int partBlocks) {
+    const int b = int(blockIdx.x);
+    if (b < partBlocks)
+        part_apply(c, {b, partBlocks});
+    else
+        conn_own<1>(c, b - partBlocks);
 }
 
 // own force plus the angle forces the partners wrote for this cell, in its bond order (R7); the
@@ -187,12 +207,12 @@ __device__ __forceinline__ f2 gather_conn(const Ctx& c, const DevWorld& w, int x
         if (vp == 0u) continue;  // the partner wrote no angle force this pass (2 of 3 steps)
         const int p = pt[q];
         const int np = flags_num_conn(c.B.flags[p]);
+        int lt[kMaxBonds];
+#pragma unroll
+        for (int kk = 0; kk < kMaxBonds; ++kk) lt[kk] = kk < np ? c.B.btgt[kk * cap + p] : -1;
         int b = -1;
-        for (int kk = 0; kk < np; ++kk)
-            if (c.B.btgt[kk * cap + p] == xl) {
-                b = kk;
-                break;
-            }
+#pragma unroll
+        for (int kk = kMaxBonds - 1; kk >= 0; --kk) b = lt[kk] == xl ? kk : b;
         if (b < 0) continue;
         if (vp & (1u << b)) acc = add(acc, to_f2(c.out1[b * cap + p]));
         const int b2 = (b + 1) % np;
@@ -203,53 +223,53 @@ __device__ __forceinline__ f2 gather_conn(const Ctx& c, const DevWorld& w, int x
 
 // Verlet position step (CellProcessor.cuh:525-544): the displacement is stored and applied after
 // the second force pass
-__global__ void k_conn_verlet_pos(Ctx c) {
+__device__ __forceinline__ void conn_pos(const Ctx& c, int block) {
     int x, wi;
-    if (!staged_cell(c, x, wi)) return;
-    {
-        const DevWorld& w = c.worlds[wi];
-        const DevParams& P = c.params[wi];
-        const uint32_t fx = c.B.flags[x];
-        const float dt = P.dt;
-        const f2 v = to_f2(c.B.vel[x]);
-        if (flags_barrier(fx)) {
-            c.shift[x] = to_float2(mul(v, dt));
-            return;
-        }
-        const f2 s1 = gather_conn(c, w, x, flags_num_conn(fx));
-        c.shift[x] = to_float2(add(mul(v, dt), mul(mul(mul(s1, dt), dt), 0.5f)));  // x/2 == x*0.5 exactly
-        c.s2[x] = to_float2(s1);
-    }
-}
-
-// Verlet velocity step, friction and decay flag (CellProcessor.cuh:546-559, 707-723, 786-790); the
-// moved position is written here, and its bin recorded for the next step's map
-__global__ void k_conn_verlet_vel(Ctx c) {
-    int x, wi;
-    const bool st = staged_cell(c, x, wi);
+    uint8_t stage;
+    if (!staged_cell(c, block, x, wi, stage)) return;
     const DevWorld& w = c.worlds[wi];
     const DevParams& P = c.params[wi];
-    const float dt = P.dt, friction = P.friction, maxEnergy = P.maxBindingEnergy;
-    // on an inner-friction step the velocity is left before friction for k_inner_friction
+    const uint32_t fx = c.B.flags[x];
+    const float dt = P.dt;
+    const f2 v = to_f2(c.B.vel[x]);
+    if (flags_barrier(fx)) {
+        c.shift[x] = to_float2(mul(v, dt));
+        return;
+    }
+    const f2 s1 = gather_conn(c, w, x, flags_num_conn(fx));
+    c.shift[x] = to_float2(add(mul(v, dt), mul(mul(mul(s1, dt), dt), 0.5f)));  // x/2 == x*0.5 exactly
+    c.s2[x] = to_float2(s1);
+}
+
+__global__ void k_conn_pos(Ctx c, int partBlocks) {
+    const int b = int(blockIdx.x);
+    if (b < partBlocks)
+        part_target(c, {b, partBlocks});
+    else
+        conn_pos(c, b - partBlocks);
+}
+
+// Verlet velocity step and friction (CellProcessor.cuh:546-559, 707-723); the moved position is
+// written here, and its bin recorded for the next step's map
+__device__ __forceinline__ void conn_vel(const Ctx& c, int block) {
+    int x, wi;
+    uint8_t stage;
+    if (!staged_cell(c, block, x, wi, stage)) return;
+    const DevWorld& w = c.worlds[wi];
+    const DevParams& P = c.params[wi];
+    const float dt = P.dt, friction = P.friction;
+    // on an inner-friction step the velocity is left before friction for the next launch
     const bool inner = P.innerFriction > 0.0f && (c.ctr[wi].timestep % 3ull) == 0ull;
     // every load before the first store, so that they are in flight together
-    uint32_t fx = 0u;
-    f2 p = {0.0f, 0.0f}, sh = {0.0f, 0.0f}, v0 = {0.0f, 0.0f}, s2 = {0.0f, 0.0f}, s1 = {0.0f, 0.0f};
-    float energy = 0.0f;
-    if (st) {
-        fx = c.B.flags[x];
-        p = to_f2(c.B.pos[x]);
-        sh = to_f2(c.shift[x]);
-        v0 = to_f2(c.B.vel[x]);
-        s2 = to_f2(c.s2[x]);
-        energy = c.energy[w.cellOff + c.B.slot[x]];
-        if (!flags_barrier(fx)) s1 = gather_conn(c, w, x, flags_num_conn(fx));
-    }
-    if (!st) return;
+    const uint32_t fx = c.B.flags[x];
+    const f2 p = to_f2(c.B.pos[x]), sh = to_f2(c.shift[x]), v0 = to_f2(c.B.vel[x]), s2 = to_f2(c.s2[x]);
+    // (the map gives the cell's start-of-step index at its end-of-step index)
+    const f2 pOld = to_f2(c.A.pos[c.sorted[x]]);
+    f2 s1 = {0.0f, 0.0f};
+    if (!flags_barrier(fx)) s1 = gather_conn(c, w, x, flags_num_conn(fx));
     const f2 p2 = torus_pos(add(p, sh), w.W, w.H);
     c.B.pos[x] = to_float2(p2);
-    // (the map gives the cell's start-of-step index at its end-of-step index)
-    bin_next(c, w, x, p2, cell_bin_of(w, to_f2(c.A.pos[c.sorted[x]])));
+    bin_next(c, w, x, p2, cell_bin_of(w, pOld));
     if (flags_barrier(fx)) return;
     const f2 acc = mul(add(s1, s2), 0.5f);
     f2 v = add(v0, mul(acc, dt));
@@ -259,23 +279,14 @@ __global__ void k_conn_verlet_vel(Ctx c) {
         v = mul(v, 1.0f - friction);
     }
     c.B.vel[x] = to_float2(v);
-    if (energy > maxEnergy) c.delFlag[x] = 1;
 }
 
 // applyInnerFriction (CellProcessor.cuh:678-705) every third step, then applyFriction (:707-723).
 // Jacobi (rule R11): each bond is relaxed twice for the cell, once for its own visit and once for
 // the partner's visit of the bond, toward the partner's start-of-pass velocity, in bond order;
 // barrier partners are skipped.
-__global__ void k_inner_friction(Ctx c) {
-    const int cap = c.cellCap;
-    int x, wi;
-    if (!staged_cell(c, x, wi)) return;
-    const DevParams& P = c.params[wi];
-    if (!(P.innerFriction > 0.0f) || (c.ctr[wi].timestep % 3ull) != 0ull) return;
-    const uint32_t fx = c.B.flags[x];
-    if (flags_barrier(fx)) return;
-    const DevWorld& w = c.worlds[wi];
-    const int nc = flags_num_conn(fx);
+__device__ __forceinline__ void inner_friction(const Ctx& c, const DevWorld& w, const DevParams& P, int x, int nc,
+                                               const int t[kMaxBonds]) {
     const float f = P.innerFriction;
     f2 vp[kMaxBonds];
     bool use[kMaxBonds];
@@ -284,9 +295,8 @@ __global__ void k_inner_friction(Ctx c) {
         use[b] = false;
         vp[b] = f2{0.0f, 0.0f};
         if (b < nc) {
-            const int p = w.cellOff + c.B.btgt[b * cap + x];
-            use[b] = !flags_barrier(c.B.flags[p]);
-            if (use[b]) vp[b] = to_f2(c.s2[p]);
+            use[b] = !flags_barrier(c.B.flags[t[b]]);
+            if (use[b]) vp[b] = to_f2(c.s2[t[b]]);
         }
     }
     f2 v = to_f2(c.s2[x]);
@@ -301,6 +311,44 @@ __global__ void k_inner_friction(Ctx c) {
     c.B.vel[x] = to_float2(v);
 }
 
+// CellProcessor.cuh:786-790: a cell with more energy than cellMaxBindingEnergy loses its bonds
+__device__ __forceinline__ bool above_max_energy(const Ctx& c, const DevWorld& w, const DevParams& P, int x) {
+    return !flags_barrier(c.B.flags[x]) && c.energy[w.cellOff + c.B.slot[x]] > P.maxBindingEnergy;
+}
+
+// Inner friction, and the marks of the structural operations: whether the cell or a bond partner loses
+// its bonds (R6), from the kDropBonds bits of the passes before and, with a finite maximum, from the
+// energies as absorption left them.  A cell sets its own bits here while its partners read its byte:
+// they take kDropBonds from the passes before or test the same energy, and get the same answer either way.
+__device__ __forceinline__ void friction_and_marks(const Ctx& c, int block) {
+    const int cap = c.cellCap;
+    int x, wi;
+    uint8_t stage;
+    if (!staged_cell(c, block, x, wi, stage)) return;
+    const DevWorld& w = c.worlds[wi];
+    const DevParams& P = c.params[wi];
+    const uint32_t fx = c.B.flags[x];
+    const int nc = flags_num_conn(fx);
+    int t[kMaxBonds];
+#pragma unroll
+    for (int b = 0; b < kMaxBonds; ++b) t[b] = b < nc ? w.cellOff + c.B.btgt[b * cap + x] : x;
+    uint32_t m = 0u;
+#pragma unroll
+    for (int b = 0; b < kMaxBonds; ++b)
+        if (b < nc) m |= c.stage[t[b]];
+    bool own = (stage & kDropBonds) != 0;
+    bool any = own || (m & kDropBonds) != 0u;
+    if (P.maxBindingEnergy < __builtin_huge_valf()) {
+        if (above_max_energy(c, w, P, x)) own = any = true;
+#pragma unroll
+        for (int b = 0; b < kMaxBonds; ++b)
+            if (b < nc && above_max_energy(c, w, P, t[b])) any = true;
+    }
+    if (any) c.stage[x] = uint8_t(kStagedCell | (own ? kDropBonds : 0) | kMarkedCell);
+    if (!(P.innerFriction > 0.0f) || (c.ctr[wi].timestep % 3ull) != 0ull || flags_barrier(fx)) return;
+    inner_friction(c, w, P, x, nc, t);
+}
+
 // ---------------------------------------------------------------------------------------------
 // living states of the worlds that track them (rule R17, cellDeathConsequences None), one thread
 // per end-of-step cell.  The three phases alternate between the two state buffers (living at the
@@ -308,8 +356,8 @@ __global__ void k_inner_friction(Ctx c) {
 // ---------------------------------------------------------------------------------------------
 constexpr uint8_t kReady = 0, kUnderConstruction = 1, kActivating = 2, kDetaching = 3, kReviving = 4, kDying = 5;
 
-__device__ __forceinline__ bool living_cell(const Ctx& c, int& x, int& wi) {
-    const int2 blk = c.livingBlocks[blockIdx.x];
+__device__ __forceinline__ bool living_cell(const Ctx& c, int block, int& x, int& wi) {
+    const int2 blk = c.livingBlocks[block];
     wi = blk.x;
     x = blk.y + int(threadIdx.x);
     const DevWorld& w = c.worlds[wi];
@@ -318,10 +366,10 @@ __device__ __forceinline__ bool living_cell(const Ctx& c, int& x, int& wi) {
 
 // checkConnections' Detaching marks on the partners of cells with an overstretched bond
 // (CellProcessor.cuh:515-520), then aging (:561-594)
-__global__ void k_living_mark_age(Ctx c) {
+__device__ __forceinline__ void living_mark_age(const Ctx& c, int block) {
     const int cap = c.cellCap;
     int x, wi;
-    if (!living_cell(c, x, wi)) return;
+    if (!living_cell(c, block, x, wi)) return;
     const DevWorld& w = c.worlds[wi];
     const uint32_t fx = c.B.flags[x];
     const int sl = w.cellOff + c.B.slot[x];
@@ -339,10 +387,10 @@ __global__ void k_living_mark_age(Ctx c) {
 }
 
 // the state transitions (CellProcessor.cuh:596-676) from the states after the marks
-__global__ void k_living_transition(Ctx c) {
+__device__ __forceinline__ void living_transition(const Ctx& c, int block) {
     const int cap = c.cellCap;
     int x, wi;
-    if (!living_cell(c, x, wi)) return;
+    if (!living_cell(c, block, x, wi)) return;
     const DevWorld& w = c.worlds[wi];
     const uint32_t fx = c.B.flags[x];
     const int sl = w.cellOff + c.B.slot[x];
@@ -369,10 +417,10 @@ __device__ __forceinline__ bool below_min_energy(const Ctx& c, const DevWorld& w
     return !flags_barrier(f) && c.energy[sl] < P.minEnergy[flags_color(f)];
 }
 
-__global__ void k_living_decay(Ctx c) {
+__device__ __forceinline__ void living_decay(const Ctx& c, int block) {
     const int cap = c.cellCap;
     int x, wi;
-    if (!living_cell(c, x, wi)) return;
+    if (!living_cell(c, block, x, wi)) return;
     const DevWorld& w = c.worlds[wi];
     const DevParams& P = c.params[wi];
     const uint32_t fx = c.B.flags[x];
@@ -398,7 +446,7 @@ __global__ void k_living_decay(Ctx c) {
 // kernels above need no partner, and one pass per cell gives their end-of-step state.
 __global__ void k_living_unbonded(Ctx c) {
     int x, wi;
-    if (!living_cell(c, x, wi)) return;
+    if (!living_cell(c, int(blockIdx.x), x, wi)) return;
     const DevWorld& w = c.worlds[wi];
     const DevParams& P = c.params[wi];
     const uint32_t fx = c.B.flags[x];
@@ -413,43 +461,27 @@ __global__ void k_living_unbonded(Ctx c) {
     c.livingNext[sl] = st;
 }
 
-void launch_living_transitions(const Ctx& c, const LaunchShape& sh, hipStream_t s, Recorder* rec) {
-    if (!sh.livingBlocks) return;
-    if (rec) rec->mark("living_mark_age");
-    hipLaunchKernelGGL(k_living_mark_age, dim3(sh.livingBlocks), dim3(sh.cellThreads), 0, s, c);
-    if (rec) rec->mark("living_transition");
-    hipLaunchKernelGGL(k_living_transition, dim3(sh.livingBlocks), dim3(sh.cellThreads), 0, s, c);
+// the velocity step, the marks and ages of the living states (from this step's overstretched bonds),
+// and the absorptions
+__global__ void k_conn_vel(Ctx c, int partBlocks, int bondBlocks) {
+    int b = int(blockIdx.x);
+    if (b < partBlocks) return part_absorb(c, {b, partBlocks});
+    b -= partBlocks;
+    if (b < bondBlocks) return conn_vel(c, b);
+    living_mark_age(c, b - bondBlocks);
 }
 
-void launch_living_decay(const Ctx& c, const LaunchShape& sh, hipStream_t s, Recorder* rec) {
-    if (!sh.livingBlocks) return;
-    if (rec) rec->mark("living_decay");
-    hipLaunchKernelGGL(k_living_decay, dim3(sh.livingBlocks), dim3(sh.cellThreads), 0, s, c);
+__global__ void k_marks(Ctx c, int bondBlocks) {
+    const int b = int(blockIdx.x);
+    if (b < bondBlocks)
+        friction_and_marks(c, b);
+    else
+        living_transition(c, b - bondBlocks);
 }
 
 // ---------------------------------------------------------------------------------------------
 // structural operations (CellConnectionProcessor.cuh), R5/R6
 // ---------------------------------------------------------------------------------------------
-__global__ void k_mark(Ctx c) {
-    const int cap = c.cellCap;
-    int x, wi;
-    if (!staged_cell(c, x, wi)) return;
-    {
-        // the cell or a bond partner flagged for deletion; the targets first, then their flags, so
-        // that the loads of all bonds are in flight together
-        const DevWorld& w = c.worlds[wi];
-        const int nc = flags_num_conn(c.B.flags[x]);
-        int t[kMaxBonds];
-#pragma unroll
-        for (int b = 0; b < kMaxBonds; ++b) t[b] = b < nc ? c.B.btgt[b * cap + x] : 0;
-        uint32_t m = c.delFlag[x];
-#pragma unroll
-        for (int b = 0; b < kMaxBonds; ++b)
-            if (b < nc) m |= c.delFlag[w.cellOff + t[b]];
-        c.mark[x] = m ? 1 : 0;
-    }
-}
-
 template <class F> __device__ __forceinline__ void for_claim_set(const Ctx& c, const DevWorld& w, int a, int b, F&& f) {
     const int cap = c.cellCap;
     f(a);
@@ -464,18 +496,27 @@ __device__ __forceinline__ unsigned long long claim_key(const DevWorld& w, int a
     return (static_cast<unsigned long long>(uint32_t(a - w.cellOff)) << 32) | uint32_t(b - w.cellOff);
 }
 
-__global__ void k_fuse_claim(Ctx c) {
+__device__ __forceinline__ void fuse_claim(const Ctx& c, Span at) {
     const int n = min(c.sc->candidates, c.candCap);
-    for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < n; q += gridDim.x * blockDim.x) {
+    for (int q = at.block * blockDim.x + threadIdx.x; q < n; q += at.blocks * blockDim.x) {
         int4 cd = c.cand[q];
         const DevWorld& w = c.worlds[cd.z];
-        if (c.mark[cd.x] || c.mark[cd.y]) {
+        if ((c.stage[cd.x] | c.stage[cd.y]) & kMarkedCell) {
             c.cand[q].w = 0;
             continue;
         }
         unsigned long long key = claim_key(w, cd.x, cd.y);
         for_claim_set(c, w, cd.x, cd.y, [&](int x) { atomicMin(&c.claim[x], key); });
     }
+}
+
+// the fusion claims, and the living states' decay (which reads the bond lists before fusions change them)
+__global__ void k_fuse_claim(Ctx c, int candBlocks) {
+    const int b = int(blockIdx.x);
+    if (b < candBlocks)
+        fuse_claim(c, {b, candBlocks});
+    else
+        living_decay(c, b - candBlocks);
 }
 
 // tryAddConnectionOneWay (CellConnectionProcessor.cuh:274-427) without angle alignment
@@ -608,9 +649,9 @@ __global__ void k_fuse_apply(Ctx c) {
     }
 }
 
-__global__ void k_fuse_reset(Ctx c) {
+__device__ __forceinline__ void fuse_reset(const Ctx& c, Span at) {
     const int n = min(c.sc->candidates, c.candCap);
-    for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < n; q += gridDim.x * blockDim.x) {
+    for (int q = at.block * blockDim.x + threadIdx.x; q < n; q += at.blocks * blockDim.x) {
         int4 cd = c.cand[q];
         if (!cd.w) continue;
         const DevWorld& w = c.worlds[cd.z];
@@ -641,64 +682,62 @@ __device__ void delete_one_way(const Ctx& c, int c1, int targetLocal) {
     }
 }
 
-__global__ void k_delete(Ctx c) {
+__device__ __forceinline__ void delete_bonds(const Ctx& c, int block) {
     const int cap = c.cellCap;
     int x, wi;
-    if (!staged_cell(c, x, wi)) return;
-    {
-        if (!c.mark[x]) return;
-        const DevWorld& w = c.worlds[wi];
-        const int nc = flags_num_conn(c.B.flags[x]);
-        int snap[kMaxBonds];
-        for (int b = 0; b < nc; ++b) snap[b] = c.B.btgt[b * cap + x];
-        const bool self = c.delFlag[x] != 0;
-        for (int b = 0; b < nc; ++b)
-            if (self || c.delFlag[w.cellOff + snap[b]]) delete_one_way(c, x, snap[b]);
-    }
+    uint8_t stage;
+    if (!staged_cell(c, block, x, wi, stage) || !(stage & kMarkedCell)) return;
+    const DevWorld& w = c.worlds[wi];
+    const int nc = flags_num_conn(c.B.flags[x]);
+    int snap[kMaxBonds];
+    for (int b = 0; b < nc; ++b) snap[b] = c.B.btgt[b * cap + x];
+    for (int b = 0; b < nc; ++b)
+        if ((stage | c.stage[w.cellOff + snap[b]]) & kDropBonds) delete_one_way(c, x, snap[b]);
 }
 
-// last kernel of the step: clears the flags of the staged cells and advances every world's
-// timestep (SimulationCudaFacade.cu:140-143)
-__global__ void k_clear_flags(Ctx c) {
-    if (blockIdx.x == 0)
+// Last launch of the step: frees the claims of this step's candidates, drops the bonds of the marked
+// cells (a pair with a marked cell claimed nothing, so the two touch different cells) and advances
+// every world's timestep (SimulationCudaFacade.cu:140-143).
+__global__ void k_fuse_end(Ctx c, int candBlocks) {
+    const int b = int(blockIdx.x);
+    if (b == 0)
         for (int wi = threadIdx.x; wi < c.numWorlds; wi += blockDim.x) c.ctr[wi].timestep += 1ull;
-    int x, wi;
-    if (!staged_cell(c, x, wi)) return;
-    c.mark[x] = 0;
-    c.delFlag[x] = 0;
+    if (b < candBlocks)
+        fuse_reset(c, {b, candBlocks});
+    else
+        delete_bonds(c, b - candBlocks);
 }
 
+// The phase after the neighbour pass in sets with bond work (SimulationKernelsLauncher.cu:38-91), with
+// the particles' chain from the movement on: their bin sort ran with the neighbour pass.  Energies
+// change in the absorptions only; before them the neighbour pass read them for fusion candidates, after
+// them the marks and the decay do.
 void launch_bonds(const Ctx& c, const LaunchShape& sh, hipStream_t s, Recorder* rec) {
-    const dim3 sg(sh.bondBlocks), cg(sh.candGrid);
-#define L(name, kernel, grid, threads, ...)                           \
-    do {                                                              \
-        if (rec) rec->mark(name);                                     \
-        hipLaunchKernelGGL(kernel, grid, threads, 0, s, __VA_ARGS__); \
+    const int parts = sh.hasParticles && sh.partBlocks ? sh.partGrid : 0;
+    const int bonds = sh.bondBlocks, living = sh.livingBlocks, cand = sh.candGrid;
+    const dim3 t(sh.cellThreads);
+#define L(name, kernel, grid, ...)                                         \
+    do {                                                                   \
+        if (rec) rec->mark(name);                                          \
+        hipLaunchKernelGGL(kernel, dim3(grid), t, 0, s, __VA_ARGS__);      \
     } while (0)
-    // no world can have a bonded or barrier cell this step (none has one and none can fuse): no
-    // cell is staged, and the scan at the start of the step advanced the timesteps
-    if (!sh.hasBondWork || sh.bondBlocks == 0) {
-        if (sh.livingBlocks) L("living_unbonded", k_living_unbonded, dim3(sh.livingBlocks), dim3(sh.cellThreads), c);
-        return;
-    }
-    const dim3 b(sh.cellThreads), cb(256);
-    L("remap", k_remap, sg, b, c);
-    L("conn_own", k_conn_own, sg, b, c, 0);
-    L("conn_verlet_pos", k_conn_verlet_pos, sg, b, c);
-    L("conn_own", k_conn_own, sg, b, c, 1);
-    L("conn_verlet_vel", k_conn_verlet_vel, sg, b, c);
-    // SimulationKernelsLauncher.cu:52-71: aging and living states, inner friction, friction and decay
-    launch_living_transitions(c, sh, s, rec);
-    if (sh.hasInnerFriction) L("inner_friction", k_inner_friction, sg, b, c);
-    launch_living_decay(c, sh, s, rec);
-    L("mark", k_mark, sg, b, c);
-    L("fuse_claim", k_fuse_claim, cg, cb, c);
-    L("fuse_apply", k_fuse_apply, cg, cb, c);
-    L("fuse_reset", k_fuse_reset, cg, cb, c);
-    L("delete", k_delete, sg, b, c);
-    L("clear_flags", k_clear_flags, sg, b, c);
+    L("conn_first", k_conn_first, parts + bonds, c, parts);
+    L("conn_pos", k_conn_pos, parts + bonds, c, parts);
+    L("conn_second", k_conn_second, parts + bonds, c, parts);
+    L("conn_vel", k_conn_vel, parts + bonds + living, c, parts, bonds);
+    L("marks", k_marks, bonds + living, c, bonds);
+    L("fuse_claim", k_fuse_claim, cand + living, c, cand);
+    L("fuse_apply", k_fuse_apply, cand, c);
+    L("fuse_end", k_fuse_end, cand + bonds, c, cand);
 #undef L
 }
 
-}  // namespace alien
+// a set without bond work has no staged cell, and the scan at the start of the step advanced the
+// timesteps
+void launch_living_unbonded(const Ctx& c, const LaunchShape& sh, hipStream_t s, Recorder* rec) {
+    if (!sh.livingBlocks) return;
+    if (rec) rec->mark("living_unbonded");
+    hipLaunchKernelGGL(k_living_unbonded, dim3(sh.livingBlocks), dim3(sh.cellThreads), 0, s, c);
+}
 
+}  // namespace alien

@@ -20,8 +20,8 @@
 // threshold of the correctly rounded square root.
 #include <type_traits>
 
-#include "kernels_common.hpp"
 #include "kernels.hpp"
+#include "particle_steps.hpp"
 
 namespace alien {
 
@@ -334,9 +334,10 @@ __device__ __forceinline__ void cell_finish(const Ctx& c, const DevWorld& w, con
     // would change nothing)
     // (the per-colour threshold is read from memory: indexing the register copy of the
     // parameters by a run-time colour would place the whole copy in scratch memory)
+    uint8_t stage = bari || nci != 0 ? kStagedCell : 0;
     if (P.decayProb > 0.0f && nci > 0 && !bari && lensq(F) > c.params[wi].maxForceSq[flags_color(fi)]) {
         const unsigned long long id = c.cid[w.cellOff + slot];
-        if (uniform_draw(w.seed, c.ctr[wi].timestep, id, kStreamForceDecay) < P.decayProb) c.delFlag[k] = 1;
+        if (uniform_draw(w.seed, c.ctr[wi].timestep, id, kStreamForceDecay) < P.decayProb) stage |= kDropBonds;
     }
     f2 v = vi;
     if (!bari) {  // applyForces
@@ -359,7 +360,7 @@ __device__ __forceinline__ void cell_finish(const Ctx& c, const DevWorld& w, con
         c.B.pos[k] = to_float2(pc);
         c.B.vel[k] = to_float2(v);
     }
-    if (w.bondWork) c.stagedMark[k] = uint8_t(bari || nci != 0);
+    if (w.bondWork) c.stage[k] = stage;
 }
 
 // One cell, neighbours visited one after another (forEachNb calls visit(o) in stencil order).
@@ -919,9 +920,14 @@ __device__ __forceinline__ bool chunk_rows(const Ctx& c, const DevWorld& w, cons
 // needs ~146 and would spill more than it gains.
 template <bool kFluid>
 __global__ void __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(kFluid ? 4 : 1)))
-k_neighbor_rows(Ctx c) {
+k_neighbor_rows(Ctx c, int sortBlocks) {
     __shared__ RowShared<kFluid ? 1 : kSubMax> S;
-    const int2 tb = c.tileBlocks[blockIdx.x];
+    // (the particles' bin sort, on workgroups of its own, in sets with bond work)
+    if (int(blockIdx.x) < sortBlocks) {
+        part_binsort(c, {int(blockIdx.x), sortBlocks});
+        return;
+    }
+    const int2 tb = c.tileBlocks[int(blockIdx.x) - sortBlocks];
     if (tb.x < 0) return;
     const int wi = tb.x;
     // the world and its parameters are read once, before any store: read through references,
@@ -1014,11 +1020,18 @@ __device__ __forceinline__ Nb map_nb(const Ctx& c, int m) {
 }
 
 // (at most 80 VGPRs: six waves per SIMD)
+template <bool kPartSort>
 __global__ void __launch_bounds__(64 * kCellWaves) __attribute__((amdgpu_waves_per_eu(6)))
-k_neighbor_cells(Ctx c, int tableBlocks) {
+k_neighbor_cells(Ctx c, int sortBlocks, int tableBlocks) {
     __shared__ CellShared SS[kCellWaves];
+    // (the particles' bin sort, on workgroups of its own, in sets with bond work)
+    if (kPartSort && int(blockIdx.x) < sortBlocks) {
+        part_binsort(c, {int(blockIdx.x), sortBlocks});
+        return;
+    }
+    const int block = kPartSort ? int(blockIdx.x) - sortBlocks : int(blockIdx.x);
     const int per = (tableBlocks + kXcdCount - 1) / kXcdCount;
-    const int e = int(blockIdx.x % kXcdCount) * per + int(blockIdx.x / kXcdCount);
+    const int e = (block % kXcdCount) * per + block / kXcdCount;
     if (e >= tableBlocks) return;
     const int2 blk = c.cellBlocks[e];
     const int wi = blk.x;
@@ -1281,13 +1294,22 @@ int neighbor_blocks_per_cu() {
     return e == hipSuccess ? std::max(1, n) : 1;
 }
 
-void launch_neighbor(const Ctx& c, const LaunchShape& sh, hipStream_t s, bool fluid, bool collision) {
-    if (fluid && sh.cellBlocks) {
-        const int grid = (sh.cellBlocks + kXcdCount - 1) / kXcdCount * kXcdCount;
-        hipLaunchKernelGGL(k_neighbor_cells, dim3(grid), dim3(sh.cellThreads), 0, s, c, sh.cellBlocks);
+void launch_neighbor(const Ctx& c, const LaunchShape& sh, hipStream_t s, bool withPartSort) {
+    // (the bin sort goes with the first launch)
+    int sort = withPartSort && sh.hasParticles && sh.partBlocks ? sh.pbinBlocks : 0;
+    const bool fluid = sh.hasFluid && sh.cellBlocks, collision = sh.hasCollision && sh.tileBlocks;
+    if (fluid || (sort && !collision)) {
+        const int grid = fluid ? (sh.cellBlocks + kXcdCount - 1) / kXcdCount * kXcdCount : 0;
+        if (sort)
+            hipLaunchKernelGGL(k_neighbor_cells<true>, dim3(sort + grid), dim3(sh.cellThreads), 0, s, c, sort, sh.cellBlocks);
+        else
+            hipLaunchKernelGGL(k_neighbor_cells<false>, dim3(grid), dim3(sh.cellThreads), 0, s, c, 0, sh.cellBlocks);
+        sort = 0;
     }
-    if (collision && sh.tileBlocks)
-        hipLaunchKernelGGL(k_neighbor_rows<false>, dim3(sh.tileBlocks), dim3(kRowThreads), 0, s, c);
+    if (collision) {
+        sort *= sh.binThreads / kRowThreads;
+        hipLaunchKernelGGL(k_neighbor_rows<false>, dim3(sort + sh.tileBlocks), dim3(kRowThreads), 0, s, c, sort);
+    }
 }
 
 }  // namespace alien

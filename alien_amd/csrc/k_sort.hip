@@ -8,8 +8,8 @@
 // cells that stay) plus the list of cells that moved in, one exclusive scan gives the offsets, and
 // the scatter places every cell at its rank among the bin's cells by previous index (R1), so the
 // map order is the logical order of the step.  Particles: counted with atomics, scattered, then sorted inside their bins.
-#include "kernels_common.hpp"
 #include "kernels.hpp"
+#include "particle_steps.hpp"
 
 namespace alien {
 
@@ -33,7 +33,7 @@ __global__ void k_cell_bin(Ctx c) {
 }
 
 __global__ void k_part_bin(Ctx c) {
-    for_live_particles(c, [&](int, const DevWorld& w, int i) {
+    for_live_particles(c, {int(blockIdx.x), int(gridDim.x)}, [&](int, const DevWorld& w, int i) {
         if (c.A.pflags[i] & kParticleDead)
             c.pbinOf[i] = -1;
         else
@@ -245,14 +245,14 @@ __global__ void __launch_bounds__(kMapScanThreads) k_map_scan(Ctx c, int tiles, 
 // list, then the store).
 constexpr int kScatterRuns = 4;
 
-__global__ void k_cell_scatter(Ctx c, int tableBlocks) {
+__device__ __forceinline__ void cell_scatter(const Ctx& c, int block, int tableBlocks) {
     const int lane = int(threadIdx.x) & 63;
     const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
     int i[kScatterRuns], bo[kScatterRuns], wi[kScatterRuns], cellOff[kScatterRuns], binOff[kScatterRuns];
     bool active[kScatterRuns];
 #pragma unroll
     for (int q = 0; q < kScatterRuns; ++q) {
-        const int e = int(blockIdx.x) * kScatterRuns + q;
+        const int e = block * kScatterRuns + q;
         const int2 blk = e < tableBlocks ? c.cellBlocks[e] : make_int2(0, 0);
         const DevWorld& w = c.worlds[blk.x];
         wi[q] = blk.x;
@@ -323,182 +323,20 @@ __global__ void k_cell_scatter(Ctx c, int tableBlocks) {
             c.mdens[dest] = c.A.dens[iq];
             c.mflags[dest] = c.A.flags[iq];
         }
+        if (c.partStage > 0) part_scatter_staged(c, c.worlds[wi[q]], iq);
     }
 }
 
-// particle i (A index or staging slot) of bin gb to its place in the map (the order inside the bin
-// is fixed by the bin sort)
-__device__ __forceinline__ void scatter_particle(const Ctx& c, const DevWorld& w, int gb, int i) {
-    const int rel = int(c.start[gb] - c.start[w.pbinOff]) + int(atomicSub(&c.count[gb], 1u)) - 1;
-    if (rel < w.partCap)
-        c.psorted[w.partOff + rel] = i;
+// One launch scatters the cells and, on workgroups of their own (first, so that they start with the
+// cells), the live particles; a cell's thread also takes the particle it emitted this step.  Both need
+// only the scan.  (As launches of their own on a second stream the two particle scatters cost 20 us of
+// the particle chain of a radiating world of 1M cells, which is longer than its fluid pass.)
+__global__ void k_scatter(Ctx c, int partBlocks, int tableBlocks) {
+    const int b = int(blockIdx.x);
+    if (b < partBlocks)
+        part_scatter(c, {b, partBlocks});
     else
-        atomicOr(&c.sc->errors, 4);  // (the host keeps room for a step's emissions: not reached)
-}
-
-__global__ void k_part_scatter(Ctx c) {
-    for_live_particles(c, [&](int, const DevWorld& w, int i) {
-        const int gb = c.pbinOf[i];
-        if (gb >= 0) scatter_particle(c, w, gb, i);
-        // the particle split off particle i at the end of the last step (cleared once read)
-        if (c.splitStage > 0) {
-            const int st = c.splitStage + i;
-            const int g2 = c.pbinOf[st];
-            if (g2 >= 0) {
-                c.pbinOf[st] = -1;
-                scatter_particle(c, w, g2, st);
-            }
-        }
-    });
-}
-
-// the particles cell radiation emitted this step, from their staging slots (cleared once read); one
-// workgroup per cell block
-__global__ void k_part_scatter_staged(Ctx c) {
-    const int2 blk = c.cellBlocks[blockIdx.x];
-    const DevWorld& w = c.worlds[blk.x];
-    const int i = blk.y + int(threadIdx.x);
-    if (i >= w.cellOff + w.numCells) return;
-    const int st = c.partStage + i;
-    const int gb = c.pbinOf[st];
-    if (gb < 0) return;
-    c.pbinOf[st] = -1;
-    scatter_particle(c, w, gb, st);
-}
-
-// sort the entries of one bin ascending (R1 stable order), small bins in registers
-template <bool kWriteInverse>
-__device__ __forceinline__ void sort_bin(int* arr, int s, int e, int* inverse) {
-    const int n = e - s;
-    if (n <= 0) return;
-    if (n == 1) {
-        if (kWriteInverse) inverse[arr[s]] = s;
-        return;
-    }
-    if (n <= 16) {
-        int v[16];
-#pragma unroll
-        for (int k = 0; k < 16; ++k)
-            if (k < n) v[k] = arr[s + k];
-        for (int k = 1; k < n; ++k) {
-            int x = v[k];
-            int j = k - 1;
-            while (j >= 0 && v[j] > x) {
-                v[j + 1] = v[j];
-                --j;
-            }
-            v[j + 1] = x;
-        }
-#pragma unroll
-        for (int k = 0; k < 16; ++k)
-            if (k < n) {
-                arr[s + k] = v[k];
-                if (kWriteInverse) inverse[v[k]] = s + k;
-            }
-        return;
-    }
-    for (int k = s + 1; k < e; ++k) {
-        int x = arr[k];
-        int j = k - 1;
-        while (j >= s && arr[j] > x) {
-            arr[j + 1] = arr[j];
-            --j;
-        }
-        arr[j + 1] = x;
-    }
-    if (kWriteInverse)
-        for (int k = s; k < e; ++k) inverse[arr[k]] = k;
-}
-
-// introspection only: cell map in logical order
-__global__ void k_cell_binsort(Ctx c) {
-    int2 blk = c.binBlocks[blockIdx.x];
-    const DevWorld w = c.worlds[blk.x];
-    int gb = blk.y + int(threadIdx.x);
-    if (gb >= w.binOff + w.nbx * w.nby) return;
-    int s, e;
-    cell_bin_range(c, w, gb - w.binOff, s, e);
-    sort_bin<true>(c.sorted, s, e, c.newidx);
-}
-
-// Particle map in logical order (the particles cell radiation emitted this step, from their staging
-// slots, sort behind every live particle's index); also publishes the new number of live
-// particles per world and the table of live particle blocks.
-__global__ void k_part_binsort(Ctx c) {
-    if (blockIdx.x == 0) {
-        for (int wi = threadIdx.x; wi < c.numWorlds; wi += blockDim.x) {
-            const DevWorld& w = c.worlds[wi];
-            const int live = min(int(c.start[w.pbinOff + w.pnbx * w.pnby] - c.start[w.pbinOff]), w.partCap);
-            c.ctr[wi].numParticles = live;
-            if (live > 0) atomicAdd(&c.sc->liveParticles, live);
-        }
-        __syncthreads();
-        // the table of live particle blocks, world by world
-        const int ppb = c.partBlockParticles;
-        int base = 0;
-        for (int wi = 0; wi < c.numWorlds; ++wi) {
-            const DevWorld& w = c.worlds[wi];
-            if (!w.active) continue;
-            const int nb = (c.ctr[wi].numParticles + ppb - 1) / ppb;
-            for (int j = int(threadIdx.x); j < nb; j += int(blockDim.x)) c.partBlocks[base + j] = make_int2(wi, w.partOff + j * ppb);
-            base += nb;
-        }
-        if (threadIdx.x == 0) *c.numPartBlocks = base;
-    }
-    int2 blk = c.pbinBlocks[blockIdx.x];
-    const DevWorld w = c.worlds[blk.x];
-    int gb = blk.y + int(threadIdx.x);
-    if (gb >= w.pbinOff + w.pnbx * w.pnby) return;
-    int s, e;
-    part_bin_range(c, w, gb - w.pbinOff, s, e);
-    sort_bin<false>(c.psorted, s, e, nullptr);
-}
-
-// The movement of the particles in map order (RadiationProcessor.cuh:61-70: position += velocity *
-// dt on the torus) into the end-of-step arrays, one thread per particle of the new live ranges; a
-// particle emitted this step comes from its staging record.
-__global__ void k_part_move(Ctx c) {
-    // (the start-of-step and end-of-step arrays are distinct)
-    const float2* __restrict__ appos = c.A.ppos;
-    const float2* __restrict__ apvel = c.A.pvel;
-    const float* __restrict__ apen = c.A.pen;
-    const int* __restrict__ aplast = c.A.plast;
-    const int* __restrict__ apslot = c.A.pslot;
-    const uint8_t* __restrict__ apflags = c.A.pflags;
-    const unsigned long long* __restrict__ apid = c.A.pid;
-    float2* __restrict__ bppos = c.B.ppos;
-    float2* __restrict__ bpvel = c.B.pvel;
-    float* __restrict__ bpen = c.B.pen;
-    int* __restrict__ bplast = c.B.plast;
-    int* __restrict__ bpslot = c.B.pslot;
-    uint8_t* __restrict__ bpflags = c.B.pflags;
-    unsigned long long* __restrict__ bpid = c.B.pid;
-    for_live_particles(c, [&](int wi, const DevWorld& w, int k) {
-        const float dt = c.params[wi].dt;
-        const int src = c.psorted[k];
-        const bool rad = c.partStage > 0 && src >= c.partStage;
-        if (rad || (c.splitStage > 0 && src >= c.splitStage)) {
-            const StagedParticle r = rad ? c.staged[src - c.partStage] : c.splitStaged[src - c.splitStage];
-            if (!rad) c.splitStaged[src - c.splitStage].color = r.color & ~kStagedPending;  // (in the arrays now)
-            const f2 v = to_f2(r.vel);
-            bppos[k] = to_float2(torus_pos(add(to_f2(r.pos), mul(v, dt)), w.W, w.H));
-            bpvel[k] = r.vel;
-            bpen[k] = r.energy;
-            bplast[k] = kNone;
-            bpslot[k] = kNone;
-            bpflags[k] = uint8_t(r.color & kParticleColorMask);
-            bpid[k] = r.id;
-            return;
-        }
-        const f2 v = to_f2(apvel[src]);
-        bppos[k] = to_float2(torus_pos(add(to_f2(appos[src]), mul(v, dt)), w.W, w.H));
-        bpvel[k] = to_float2(v);
-        bpen[k] = apen[src];
-        bplast[k] = aplast[src];
-        bpslot[k] = apslot[src];
-        bpflags[k] = apflags[src];
-        bpid[k] = apid[src];
-    });
+        cell_scatter(c, b - partBlocks, tableBlocks);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -528,27 +366,10 @@ void launch_map_scan(const Ctx& c, hipStream_t s, StepCounters* open, bool advan
 
 int map_scan_tiles(int numBins) { return (numBins + kMapScanTile - 1) / kMapScanTile; }
 
-void launch_cell_scatter(const Ctx& c, const LaunchShape& sh, hipStream_t s) {
-    if (sh.cellBlocks)
-        hipLaunchKernelGGL(k_cell_scatter, dim3((sh.cellBlocks + kScatterRuns - 1) / kScatterRuns), dim3(sh.cellThreads),
-                           0, s, c, sh.cellBlocks);
-}
-
-void launch_part_scatter(const Ctx& c, const LaunchShape& sh, hipStream_t s) {
-    if (sh.partBlocks) hipLaunchKernelGGL(k_part_scatter, dim3(sh.partGrid), dim3(sh.partThreads), 0, s, c);
-}
-
-void launch_part_sort(const Ctx& c, const LaunchShape& sh, hipStream_t s) {
-    if (!sh.hasParticles) return;
-    if (sh.partBlocks) hipLaunchKernelGGL(k_part_scatter, dim3(sh.partGrid), dim3(sh.partThreads), 0, s, c);
-    if (c.partStage > 0 && sh.cellBlocks)
-        hipLaunchKernelGGL(k_part_scatter_staged, dim3(sh.cellBlocks), dim3(sh.cellThreads), 0, s, c);
-    if (sh.pbinBlocks) hipLaunchKernelGGL(k_part_binsort, dim3(sh.pbinBlocks), dim3(sh.binThreads), 0, s, c);
-    if (sh.partBlocks) hipLaunchKernelGGL(k_part_move, dim3(sh.partGrid), dim3(sh.partThreads), 0, s, c);
-}
-
-void launch_cell_binsort(const Ctx& c, const LaunchShape& sh, hipStream_t s) {
-    if (sh.binBlocks) hipLaunchKernelGGL(k_cell_binsort, dim3(sh.binBlocks), dim3(sh.binThreads), 0, s, c);
+void launch_scatter(const Ctx& c, const LaunchShape& sh, hipStream_t s) {
+    const int parts = sh.hasParticles && sh.partBlocks ? sh.partGrid : 0;
+    const int cells = (sh.cellBlocks + kScatterRuns - 1) / kScatterRuns;
+    if (parts + cells) hipLaunchKernelGGL(k_scatter, dim3(parts + cells), dim3(sh.cellThreads), 0, s, c, parts, sh.cellBlocks);
 }
 
 }  // namespace alien

@@ -13,7 +13,7 @@ namespace alien {
 struct LaunchShape {
     int cellBlocks = 0, cellThreads = 256;
     int partBlocks = 0, partThreads = 256;
-    int binBlocks = 0, pbinBlocks = 0, binThreads = 256;
+    int pbinBlocks = 0, binThreads = 256;
     int tileBlocks = 0;    // neighbour-pass workgroups (including XCD padding)
     int partGrid = 64;     // grid-stride particle kernels
     int bondBlocks = 0;    // bond kernels: cell blocks of the worlds that can have bonded cells
@@ -27,7 +27,6 @@ struct LaunchShape {
     bool hasRadiation = false;  // some active world radiates (DevParams::radiates)
     bool hasSplitting = false;  // some active world's particles can split (DevParams::splits)
     int livingBlocks = 0;           // cell blocks of the worlds whose living states live on the device
-    bool hasInnerFriction = false;  // some active world with bond work has innerFriction > 0
 };
 
 // Optional per-launch hook: mark(name) is called right before each kernel launch and
@@ -44,13 +43,12 @@ int map_scan_tiles(int numBins);
 void launch_seed_bins(const Ctx& c, const LaunchShape& sh, hipStream_t s);
 // workgroups of the row-streaming (collision) neighbour pass one CU keeps resident
 int neighbor_blocks_per_cu();
-// A second stream of the same priority and two events: the particle kernels run on it beside the
-// neighbour pass (sort, movement, targets and fusion claims always; fusions and absorptions too
-// when no world has bond work, so that nothing in the pass reads the energies they change),
-// joined before the kernels after the pass.
+// A second stream of the same priority and two events: in sets without bond work the particles' chain
+// runs on it beside the neighbour pass (which then reads none of the energies it changes), joined
+// before the kernels after the pass.
 struct SideStream {
     hipStream_t stream = nullptr;
-    hipEvent_t fork = nullptr, mapped = nullptr, join = nullptr;  // after the scan, the scatter, the particles
+    hipEvent_t fork = nullptr, join = nullptr;  // after the scatter, after the particles
 };
 // rec != nullptr (per-kernel timing) launches everything on s, one kernel after another
 void launch_step(const Ctx& c, const LaunchShape& sh, hipStream_t s, Recorder* rec = nullptr,

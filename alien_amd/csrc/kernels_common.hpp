@@ -133,11 +133,17 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t& t
     return res;
 }
 
+// Several kernels run the cells' and the particles' work of a phase in one launch, each part on its
+// own workgroups: a workgroup's place among those of its part
+struct Span {
+    int block, blocks;
+};
+
 // grid-stride iteration over the blocks of live particles (the table the particle bin sort writes
 // for the live ranges it publishes)
-template <class F> __device__ __forceinline__ void for_live_particles(const Ctx& c, F&& f) {
+template <class F> __device__ __forceinline__ void for_live_particles(const Ctx& c, Span at, F&& f) {
     const int n = *c.numPartBlocks;
-    for (int e = blockIdx.x; e < n; e += gridDim.x) {
+    for (int e = at.block; e < n; e += at.blocks) {
         const int2 blk = c.partBlocks[e];
         const int live = c.ctr[blk.x].numParticles;
         const DevWorld& w = c.worlds[blk.x];

@@ -12,16 +12,19 @@
 namespace alien {
 
 void launch_map_scan(const Ctx& c, hipStream_t s, StepCounters* open, bool advanceTimestep);
-void launch_cell_scatter(const Ctx& c, const LaunchShape& sh, hipStream_t s);
-void launch_part_sort(const Ctx& c, const LaunchShape& sh, hipStream_t s);
-void launch_part_scatter(const Ctx& c, const LaunchShape& sh, hipStream_t s);
-void launch_cell_binsort(const Ctx& c, const LaunchShape& sh, hipStream_t s);
-void launch_neighbor(const Ctx& c, const LaunchShape& sh, hipStream_t s, bool fluid, bool collision);
-void launch_particles_pre(const Ctx& c, const LaunchShape& sh, hipStream_t s, Recorder* rec);
-void launch_particles_post(const Ctx& c, const LaunchShape& sh, hipStream_t s, Recorder* rec);
+void launch_scatter(const Ctx& c, const LaunchShape& sh, hipStream_t s);
+void launch_neighbor(const Ctx& c, const LaunchShape& sh, hipStream_t s, bool withPartSort);
+void launch_particles(const Ctx& c, const LaunchShape& sh, hipStream_t s, Recorder* rec);
 void launch_bonds(const Ctx& c, const LaunchShape& sh, hipStream_t s, Recorder* rec);
+void launch_living_unbonded(const Ctx& c, const LaunchShape& sh, hipStream_t s, Recorder* rec);
 void launch_radiation(const Ctx& c, const LaunchShape& sh, hipStream_t s, Recorder* rec);
 
+// Sets with bond work run on one stream: their phases after the neighbour pass are a chain of short
+// launches, and each carries a stage of the particles' chain on workgroups of its own.  A captured
+// graph with a fork in it is dispatched node by node (4 to 10 us between two kernels in a trace, where
+// a graph without forks shows none).  Without bond work there is one long launch, the neighbour pass,
+// and the particles' chain runs beside it on the second stream: absorption adds to cell energies,
+// which only fusion candidates and bonds read.
 void launch_step(const Ctx& c, const LaunchShape& sh, hipStream_t s, Recorder* rec, const SideStream* side) {
     // cell radiation comes first: the particles it emits enter this step's particle map
     launch_radiation(c, sh, s, rec);
@@ -29,38 +32,23 @@ void launch_step(const Ctx& c, const LaunchShape& sh, hipStream_t s, Recorder* r
     // it
     if (rec) rec->mark("map_scan");
     launch_map_scan(c, s, c.sc, !sh.hasBondWork);
-    // The particle kernels run beside the cell scatter and the neighbour pass: their sort and
-    // movement need only the scan (the particle bins' offsets), their targets and fusion claims
-    // also the cell map.
-    const bool fork = side && !rec && sh.hasParticles && sh.partBlocks;
-    // Absorption adds to cell energies, which the neighbour pass reads for fusion and the bond
-    // kernels for bond decay: without bond work (no bonded, barrier or bondable cell) neither
-    // reads them, and the fusions and absorptions run beside the neighbour pass as well.
-    const bool allBeside = fork && !sh.hasBondWork;
-    if (fork) {
-        (void)hipEventRecord(side->fork, s);
-        if (rec) rec->mark("cell_scatter");
-        launch_cell_scatter(c, sh, s);
-        (void)hipEventRecord(side->mapped, s);
-        launch_neighbor(c, sh, s, sh.hasFluid, sh.hasCollision);
-        (void)hipStreamWaitEvent(side->stream, side->fork, 0);
-        launch_part_sort(c, sh, side->stream);
-        (void)hipStreamWaitEvent(side->stream, side->mapped, 0);
-        launch_particles_pre(c, sh, side->stream, rec);
-        if (allBeside) launch_particles_post(c, sh, side->stream, rec);
-        (void)hipEventRecord(side->join, side->stream);
-        (void)hipStreamWaitEvent(s, side->join, 0);
+    if (rec) rec->mark("cell_scatter");
+    launch_scatter(c, sh, s);
+    const bool fork = side && !rec && !sh.hasBondWork && sh.hasParticles && sh.partBlocks;
+    if (fork) (void)hipEventRecord(side->fork, s);
+    if (rec) rec->mark("neighbor");
+    launch_neighbor(c, sh, s, sh.hasBondWork);
+    if (sh.hasBondWork) {
+        launch_bonds(c, sh, s, rec);
     } else {
-        if (rec) rec->mark("cell_scatter");
-        launch_cell_scatter(c, sh, s);
-        if (rec && sh.hasParticles) rec->mark("part_sort");
-        launch_part_sort(c, sh, s);
-        launch_particles_pre(c, sh, s, rec);
-        if (rec) rec->mark("neighbor");
-        launch_neighbor(c, sh, s, sh.hasFluid, sh.hasCollision);
+        if (fork) (void)hipStreamWaitEvent(side->stream, side->fork, 0);
+        launch_particles(c, sh, fork ? side->stream : s, rec);
+        if (fork) {
+            (void)hipEventRecord(side->join, side->stream);
+            (void)hipStreamWaitEvent(s, side->join, 0);
+        }
+        launch_living_unbonded(c, sh, s, rec);
     }
-    if (!allBeside) launch_particles_post(c, sh, s, rec);
-    launch_bonds(c, sh, s, rec);
     if (rec) rec->mark(nullptr);
 }
 
@@ -68,9 +56,7 @@ void launch_step(const Ctx& c, const LaunchShape& sh, hipStream_t s, Recorder* r
 // for the next step.
 void launch_debug_map(const Ctx& c, const LaunchShape& sh, hipStream_t s) {
     launch_map_scan(c, s, nullptr, false);
-    launch_cell_scatter(c, sh, s);
-    launch_part_scatter(c, sh, s);
-    launch_cell_binsort(c, sh, s);
+    launch_scatter(c, sh, s);
     launch_seed_bins(c, sh, s);
 }
 

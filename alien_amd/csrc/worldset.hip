@@ -415,7 +415,6 @@ WorldSet::WorldSet() {
     check_hip(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking), "hipStreamCreate");
     check_hip(hipStreamCreateWithFlags(&side_.stream, hipStreamNonBlocking), "hipStreamCreate");
     check_hip(hipEventCreateWithFlags(&side_.fork, hipEventDisableTiming), "hipEventCreate");
-    check_hip(hipEventCreateWithFlags(&side_.mapped, hipEventDisableTiming), "hipEventCreate");
     check_hip(hipEventCreateWithFlags(&side_.join, hipEventDisableTiming), "hipEventCreate");
     check_hip(hipEventCreateWithFlags(&liveReady_, hipEventDisableTiming), "hipEventCreate");
     check_hip(hipHostMalloc(reinterpret_cast<void**>(&liveHost_), 64 + sizeof(DevCounters), hipHostMallocDefault),
@@ -433,7 +432,6 @@ WorldSet::~WorldSet() {
     if (liveReady_) (void)hipEventDestroy(liveReady_);
     if (liveHost_) (void)hipHostFree(liveHost_);
     if (side_.fork) (void)hipEventDestroy(side_.fork);
-    if (side_.mapped) (void)hipEventDestroy(side_.mapped);
     if (side_.join) (void)hipEventDestroy(side_.join);
     if (side_.stream) (void)hipStreamDestroy(side_.stream);
     if (stream_) (void)hipStreamDestroy(stream_);
@@ -689,7 +687,7 @@ void WorldSet::build(const std::vector<Source>& sources) {
     mflags_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
     newidx_ = static_cast<int*>(A(sizeof(int) * NC));
     psorted_ = static_cast<int*>(A(sizeof(int) * NP));
-    stagedMark_ = static_cast<uint8_t*>(A(NC));
+    stage_ = static_cast<uint8_t*>(A(NC));
     own_ = static_cast<float2*>(A(sizeof(float2) * NC));
     shift_ = static_cast<float2*>(A(sizeof(float2) * NC));
     bstiff_ = static_cast<float*>(A(sizeof(float) * NC));
@@ -697,8 +695,6 @@ void WorldSet::build(const std::vector<Source>& sources) {
     out1_ = static_cast<float2*>(A(sizeof(float2) * kMaxBonds * size_t(NC)));
     out2_ = static_cast<float2*>(A(sizeof(float2) * kMaxBonds * size_t(NC)));
     valid_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
-    delFlag_ = static_cast<uint8_t*>(A(NC));
-    mark_ = static_cast<uint8_t*>(A(NC));
     claim_ = static_cast<unsigned long long*>(A(sizeof(unsigned long long) * NC));
     cand_ = static_cast<int4*>(A(sizeof(int4) * size_t(candCap_)));
     want_ = static_cast<int*>(A(sizeof(int) * NP));
@@ -846,8 +842,6 @@ void WorldSet::build(const std::vector<Source>& sources) {
     launch_fill_u32(reinterpret_cast<uint32_t*>(mapStatus_), 0u, 2 * size_t(map_scan_tiles(NB)), stream_);
     launch_fill_u32(mapEpochTicket_, 0u, 2, stream_);
     launch_fill_u32(reinterpret_cast<uint32_t*>(claim_), 0xffffffffu, size_t(NC) * 2, stream_);
-    launch_fill_u32(reinterpret_cast<uint32_t*>(delFlag_), 0u, (size_t(NC) + 3) / 4, stream_);
-    launch_fill_u32(reinterpret_cast<uint32_t*>(mark_), 0u, (size_t(NC) + 3) / 4, stream_);
     launch_fill_u32(reinterpret_cast<uint32_t*>(buf_[1].pflags), 0u, (size_t(NP) + 3) / 4, stream_);
     if (partStage_ > 0)  // no particle waits in a staging slot
         launch_fill_u32(reinterpret_cast<uint32_t*>(pbinOf_ + partStage_), 0xffffffffu, size_t(NC), stream_);
@@ -970,7 +964,7 @@ void WorldSet::buildTables() {
     if (stream_) synchronize();  // (the tables and the live counts read below are in use until then)
     for (auto& a : tableAllocs_) (void)hipFree(a.p);
     tableAllocs_.clear();
-    std::vector<int2> cells, bonds, bins, pbins, parts, living;
+    std::vector<int2> cells, bonds, pbins, parts, living;
     const int ct = shape_.cellThreads, pt = shape_.partThreads, bt = shape_.binThreads;
     for (int wi = 0; wi < int(worlds_.size()); ++wi) {
         if (!active_[wi]) continue;
@@ -980,7 +974,6 @@ void WorldSet::buildTables() {
             for (int s = 0; s < w.numCells; s += ct) bonds.push_back(make_int2(wi, w.cellOff + s));
         if (livingWork_[wi])
             for (int s = 0; s < w.numCells; s += ct) living.push_back(make_int2(wi, w.cellOff + s));
-        for (int s = 0; s < w.nbx * w.nby; s += bt) bins.push_back(make_int2(wi, w.binOff + s));
         for (int s = 0; s < w.pnbx * w.pnby; s += bt) pbins.push_back(make_int2(wi, w.pbinOff + s));
     }
     auto up = [&](const std::vector<int2>& v) -> int2* {
@@ -1035,7 +1028,6 @@ void WorldSet::buildTables() {
     shape_.partGrid = int(std::max<int64_t>(64, std::min<int64_t>(65536, (live + pt - 1) / pt + (radCells / 8 + pt - 1) / pt)));
     cellBlocks_ = up(cells);
     bondBlocks_ = up(bonds);
-    binBlocks_ = up(bins);
     pbinBlocks_ = up(pbins);
     tileBlocks_ = up(tileTable);
     livingBlocks_ = up(living);
@@ -1045,13 +1037,10 @@ void WorldSet::buildTables() {
     // the bond kernels run when an active world can have a bonded or barrier cell
     shape_.hasBondWork = !bonds.empty();
     shape_.partBlocks = int(partCapBlocks);
-    shape_.binBlocks = int(bins.size());
     shape_.pbinBlocks = int(pbins.size());
     shape_.tileBlocks = int(tileTable.size());
-    numCellBlocks_ = int(cells.size());
     shape_.hasFluid = shape_.hasCollision = false;
     for (const DevParams& p : params_) (p.motion == 0 ? shape_.hasFluid : shape_.hasCollision) = true;
-    updateInnerFriction();
     updateRadiation();
     invalidateGraphs();
 }
@@ -1082,15 +1071,6 @@ int stageLayout(int64_t caps, int cells, bool radiation, bool splitting, int& sp
     if (end >= (int64_t(1) << 31) - 1)
         throw Error(ALIEN_E_CAPACITY, "the particle slots and staging slots of the world set exceed 32-bit indices");
     return int(end);
-}
-
-// the inner-friction kernel runs when an active world with bond work has innerFriction > 0
-void WorldSet::updateInnerFriction() {
-    bool any = false;
-    for (size_t i = 0; i < worlds_.size(); ++i)
-        any = any || (active_[i] && bondWork_[i] && params_[i].innerFriction > 0.0f);
-    if (any != shape_.hasInnerFriction) invalidateGraphs();
-    shape_.hasInnerFriction = any;
 }
 
 void WorldSet::setBlockSize(int threads) {
@@ -1214,7 +1194,7 @@ Ctx WorldSet::makeCtx(int parity) const {
     c.mflags = mflags_;
     c.newidx = newidx_;
     c.psorted = psorted_;
-    c.stagedMark = stagedMark_;
+    c.stage = stage_;
     c.own = own_;
     c.shift = shift_;
     c.bstiff = bstiff_;
@@ -1222,8 +1202,6 @@ Ctx WorldSet::makeCtx(int parity) const {
     c.out1 = out1_;
     c.out2 = out2_;
     c.valid = valid_;
-    c.delFlag = delFlag_;
-    c.mark = mark_;
     c.claim = claim_;
     c.cand = cand_;
     c.candCap = candCap_;
@@ -1233,14 +1211,12 @@ Ctx WorldSet::makeCtx(int parity) const {
     c.cclaim = cclaim_;
     c.cellBlocks = cellBlocks_;
     c.bondBlocks = bondBlocks_;
-    c.binBlocks = binBlocks_;
     c.pbinBlocks = pbinBlocks_;
     c.partBlocks = partBlocks_;
     c.tileBlocks = tileBlocks_;
     c.numPartBlocks = numPartBlocks_;
     c.partBlockParticles = shape_.partThreads;
-    c.numCellBlocks = numCellBlocks_;
-    c.cellBlockCells = shape_.cellThreads;
+    c.blockThreads = shape_.cellThreads;
     return c;
 }
 
@@ -1443,7 +1419,6 @@ void WorldSet::setParams(int w, const alien_params& p) {
     } else if (fluid != shape_.hasFluid || collision != shape_.hasCollision) {
         invalidateGraphs();
     }
-    updateInnerFriction();
     updateRadiation();  // (the room for emitted particles is made before the next step)
 }
 

@@ -246,7 +246,6 @@ private:
     StagedParticle* staged_ = nullptr;  // [cellCap] with a staging area
     int splitStage_ = 0;                     // first split staging slot (0: none)
     StagedParticle* splitStaged_ = nullptr;  // [splitStage_] with a split staging area
-    int numCellBlocks_ = 0;
     CellExtra* extra_ = nullptr;  // [cellCap] by slot, if some world has any
     std::vector<uint8_t*> selected_;  // per world: selection by particle slot, if some particle is selected
     unsigned long long* dWords_ = nullptr;  // [2] results of the read-back kernels
@@ -276,15 +275,14 @@ private:
     float2 *mpos_ = nullptr, *mvel_ = nullptr;
     float* mdens_ = nullptr;
     uint32_t* mflags_ = nullptr;
-    uint8_t* stagedMark_ = nullptr;
+    uint8_t* stage_ = nullptr;
     float2 *own_ = nullptr, *shift_ = nullptr, *s2_ = nullptr, *out1_ = nullptr, *out2_ = nullptr;
     float* bstiff_ = nullptr;
     uint32_t* valid_ = nullptr;
-    uint8_t *delFlag_ = nullptr, *mark_ = nullptr;
     unsigned long long* claim_ = nullptr;
     int4* cand_ = nullptr;
     int *want_ = nullptr, *fclaim_ = nullptr, *absorbCell_ = nullptr, *cclaim_ = nullptr;
-    int2 *cellBlocks_ = nullptr, *bondBlocks_ = nullptr, *binBlocks_ = nullptr, *pbinBlocks_ = nullptr;
+    int2 *cellBlocks_ = nullptr, *bondBlocks_ = nullptr, *pbinBlocks_ = nullptr;
     int2* partBlocks_ = nullptr;
     int2* tileBlocks_ = nullptr;
     int* numPartBlocks_ = nullptr;  // (device) entries of partBlocks_
@@ -295,7 +293,6 @@ private:
     int stripCap_ = kStripMax;
     int chunkRows_ = 0;
     void adaptGrids();
-    void updateInnerFriction();
     std::vector<Arr> tableAllocs_;
 
     hipGraphExec_t graph_[2] = {nullptr, nullptr};  // one step from parity 0 / 1

@@ -496,12 +496,20 @@ __device__ __forceinline__ unsigned long long claim_key(const DevWorld& w, int a
     return (static_cast<unsigned long long>(uint32_t(a - w.cellOff)) << 32) | uint32_t(b - w.cellOff);
 }
 
+// A cell that loses its bonds this step, or has a partner that does, fuses with none.  Unbonded cells
+// have no marks: of the reasons to lose bonds, too much energy applies to them as well.
+__device__ __forceinline__ bool fusion_barred(const Ctx& c, const DevWorld& w, const DevParams& P, int x) {
+    const uint8_t stage = c.stage[x];
+    if (stage != 0) return (stage & kMarkedCell) != 0;
+    return P.maxBindingEnergy < __builtin_huge_valf() && above_max_energy(c, w, P, x);
+}
+
 __device__ __forceinline__ void fuse_claim(const Ctx& c, Span at) {
     const int n = min(c.sc->candidates, c.candCap);
     for (int q = at.block * blockDim.x + threadIdx.x; q < n; q += at.blocks * blockDim.x) {
         int4 cd = c.cand[q];
         const DevWorld& w = c.worlds[cd.z];
-        if ((c.stage[cd.x] | c.stage[cd.y]) & kMarkedCell) {
+        if (fusion_barred(c, w, c.params[cd.z], cd.x) || fusion_barred(c, w, c.params[cd.z], cd.y)) {
             c.cand[q].w = 0;
             continue;
         }

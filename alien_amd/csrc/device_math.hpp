@@ -24,13 +24,41 @@ struct f2 {
 __device__ __forceinline__ f2 add(f2 a, f2 b) { return {a.x + b.x, a.y + b.y}; }
 __device__ __forceinline__ f2 sub(f2 a, f2 b) { return {a.x - b.x, a.y - b.y}; }
 __device__ __forceinline__ f2 mul(f2 a, float m) { return {a.x * m, a.y * m}; }
-__device__ __forceinline__ f2 dvd(f2 a, float m) { return {a.x / m, a.y / m}; }
 __device__ __forceinline__ f2 neg(f2 a) { return {-a.x, -a.y}; }
 __device__ __forceinline__ f2 to_f2(float2 v) { return {v.x, v.y}; }
 __device__ __forceinline__ float2 to_float2(f2 v) { return make_float2(v.x, v.y); }
 
 __device__ __forceinline__ float dot2(f2 a, f2 b) { return a.x * b.x + a.y * b.y; }
 __device__ __forceinline__ float lensq(f2 v) { return v.x * v.x + v.y * v.y; }
+
+// Correctly rounded reciprocal, square root and division by a small constant in fewer operations than
+// the compiler's sequences, which also cover the ends of the exponent range (reciprocal 3 instead of
+// 11, square root 5 instead of 17, division 3 instead of 11): one correction step with fused
+// multiply-adds from the hardware's 1-ulp approximation (Markstein, "Computation of elementary
+// functions on the IBM RISC System/6000 processor", IBM J. Res. Dev. 34, 1990).  On gfx950 the results
+// equal the IEEE operation for all 2^23 significands at every exponent from -90 to 90 (checked for each;
+// division by 5 and 6); outside of mid_range, zero, infinity and NaN included, callers take the IEEE
+// operation itself.
+constexpr float kMidLow = 0x1p-80f, kMidHigh = 0x1p80f;
+__device__ __forceinline__ bool mid_range(float x) {
+    const float a = fabsf(x);
+    return __builtin_amdgcn_fmed3f(a, kMidLow, kMidHigh) == a;
+}
+__device__ __forceinline__ float mid_rcp(float x) {
+    const float r = __builtin_amdgcn_rcpf(x);
+    return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
+}
+__device__ __forceinline__ float mid_sqrt(float x) {
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float s = x * y;
+    return __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * y, s);
+}
+template <int kDivisor> __device__ __forceinline__ float mid_div(float a) {
+    constexpr float inv = 1.0f / float(kDivisor);
+    const float q = a * inv;
+    return __builtin_fmaf(__builtin_fmaf(-q, float(kDivisor), a), inv, q);
+}
+__device__ __forceinline__ f2 dvd(f2 a, float m) { return {a.x / m, a.y / m}; }
 __device__ __forceinline__ float len2(f2 v) { return __builtin_sqrtf(v.x * v.x + v.y * v.y); }
 
 // unit vector with the (1,0) fallback below 1e-5 (Math.cuh:246-261), as the product with the
@@ -78,15 +106,22 @@ __device__ __forceinline__ f2 stencil_delta(f2 a, f2 b, float W, float H, bool s
     return {a.x - b.x, a.y - b.y};
 }
 
-// BaseMap::correctPosition(float2&) (Map.cuh:20-26)
-__device__ __forceinline__ f2 torus_pos(f2 p, int W, int H) {
-    int ix = floor_int(p.x), iy = floor_int(p.y);
-    float fx = p.x - static_cast<float>(ix);
-    float fy = p.y - static_cast<float>(iy);
-    ix = wrap_int(ix, W);
-    iy = wrap_int(iy, H);
-    return {static_cast<float>(ix) + fx, static_cast<float>(iy) + fy};
+// BaseMap::correctPosition(float2&) (Map.cuh:20-26): the integer part wrapped onto the torus.  Within
+// one period either way the wrap is two selects; anything further (or not a number that fits an int)
+// takes the general wrap.
+__device__ __forceinline__ float torus_pos1(float p, int size) {
+    const float fl = __builtin_floorf(p);
+    int i = static_cast<int>(fl);
+    i = i < 0 ? i + size : i;
+    i = i >= size ? i - size : i;
+    float r = static_cast<float>(i) + (p - fl);
+    if (uint32_t(i) >= uint32_t(size)) {
+        const int k = floor_int(p);
+        r = static_cast<float>(wrap_int(k, size)) + (p - static_cast<float>(k));
+    }
+    return r;
 }
+__device__ __forceinline__ f2 torus_pos(f2 p, int W, int H) { return {torus_pos1(p.x, W), torus_pos1(p.y, H)}; }
 
 // arcsine: argument reduction asin(a) = pi/2 - 2 asin(sqrt((1-a)/2)) above 1/2, odd polynomial
 // x + x^3 P(x^2) below (coefficients least-squares fitted for this library; |err| < 1.7e-7 rad)
@@ -233,7 +268,7 @@ __device__ __forceinline__ float sph_w(float q) {
         r = kTwoThirds - q * q + 0.5f * q * q * q;
     else if (q < 2.0f) {
         r = 2.0f - q;
-        r = r * r * r / 6.0f;
+        r = mid_div<6>(r * r * r);  // (2 - q is 0 or at least 2^-23)
     } else
         r = 0.0f;
     r *= kKernelNorm;

@@ -139,7 +139,7 @@ struct StepCounters {
 struct HotBuffers {
     float2* pos;
     float2* vel;
-    float* dens;
+    float* dens;  // 1 / density of a fluid cell (set to 1 when a world changes its parameters, motion included)
     uint32_t* flags;
     int* slot;    // local cold slot of the cell (stable identity)
     int* btgt;    // [kMaxBonds][cellCap] local logical index of the bond partner
@@ -237,7 +237,6 @@ struct Ctx {
     // range (the fluid pass reads the state through `sorted`)
     float2* mpos;
     float2* mvel;
-    float* mdens;  // fluid: 1 / density
     uint32_t* mflags;
     int* newidx;   // [cellCap] A index -> new index
     int* psorted;  // [partCap]
@@ -268,6 +267,8 @@ struct Ctx {
     int2* partBlocks;
     int* numPartBlocks;
     int partBlockParticles;
+    const int2* fluidBlocks;  // per workgroup of the fluid pass: (world, its first wave)
+    const int2* edgeBlocks;  // per workgroup: (world, its first wave's edge unit and half), see k_fluid.hip
     const int2* tileBlocks;  // per block: (world, tile index), -1 for padding blocks
     const int2* livingBlocks;  // per block: (world, first global cell index) over livingWork worlds
     int blockThreads;  // cells, bins or living cells per entry of the block tables above

@@ -269,7 +269,7 @@ __device__ __forceinline__ void conn_vel(const Ctx& c, int block) {
     if (!flags_barrier(fx)) s1 = gather_conn(c, w, x, flags_num_conn(fx));
     const f2 p2 = torus_pos(add(p, sh), w.W, w.H);
     c.B.pos[x] = to_float2(p2);
-    bin_next(c, w, x, p2, cell_bin_of(w, pOld));
+    bin_next(c, w, x, p2, cell_bin_of(w, pOld) - w.binOff);
     if (flags_barrier(fx)) return;
     const f2 acc = mul(add(s1, s2), 0.5f);
     f2 v = add(v0, mul(acc, dt));
@@ -304,7 +304,7 @@ __device__ __forceinline__ void inner_friction(const Ctx& c, const DevWorld& w, 
 #pragma unroll
         for (int b = 0; b < kMaxBonds; ++b)
             if (b < nc && use[b]) {
-                const f2 avg = dvd(add(v, vp[b]), 2.0f);
+                const f2 avg = mul(add(v, vp[b]), 0.5f);
                 v = add(mul(v, 1.0f - f), mul(avg, f));
             }
     v = mul(v, 1.0f - P.friction);

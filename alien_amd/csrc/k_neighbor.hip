@@ -1,9 +1,4 @@
-// k_neighbor.hip — the neighbour pass of the physics timestep.
-//
-// ALIEN: calcCollisions_reconnectCells_correctOverlap / calcFluidForces_reconnectCells_correctOverlap
-// (source/EngineGpuKernels/CellProcessor.cuh:122-365), then checkForces/applyForces (:367-406); for
-// cells without bonds also the Verlet updates and friction of the same step (:525-559, :707-723),
-// which reduce to local operations when the connection forces are zero.
+// k_neighbor.hip — the collision neighbour pass, and the launch of both passes.
 //
 // One wave owns a strip of bin columns and walks it row by row (see "Row streaming" below).  Per
 // row it (1) tests the 3x3 bin stencil of every cell with the neighbour predicate on squared
@@ -11,377 +6,14 @@
 // pairs of the row one pair per lane, and (3) lets every cell add its pairs' terms in visiting
 // order, which gives the float sums of a sequential stencil walk bit for bit.  A cell with more
 // than 64 stencil candidates, or a strip whose rows do not fit LDS, walks its stencil
-// sequentially instead (same order, same results).  The kernel is instantiated per motion mode; a
-// workgroup of a world in the other mode exits at once.
-//
-// Divisions by per-world constants (1/h, 1/h^2, 1/h^3), by a cell's density, by |d| and by the
-// collision and viscosity denominators are products with the correctly rounded reciprocal (R16
-// of the oracle), and the length comparisons |v| > c are tests of |v|^2 against the exact
-// threshold of the correctly rounded square root.
+// sequentially instead (same order, same results).  A workgroup of a fluid world exits at once.
 #include <type_traits>
 
 #include "kernels.hpp"
+#include "neighbor_device.hpp"
 #include "particle_steps.hpp"
 
 namespace alien {
-
-struct Nb {
-    f2 pos, vel;
-    float dens;  // fluid: 1 / density; collision: density
-    uint32_t flags;
-    int aidx;  // index in the start-of-step arrays (A)
-    int lidx;  // index in the end-of-step arrays (B), the logical index of this step
-};
-
-__device__ __forceinline__ void push_candidate(const Ctx& c, int a, int b, int w) {
-    int q = atomicAdd(&c.sc->candidates, 1);
-    if (q < c.candCap)
-        c.cand[q] = make_int4(a, b, w, 1);
-    else
-        atomicOr(&c.sc->errors, 1);
-}
-
-// what a neighbour pair contributes
-constexpr uint32_t kPairBarrier = 1u;  // fluid: a barrier neighbour (A index, distance)
-constexpr uint32_t kPairSelf = 2u;     // fluid: the cell itself (density term only)
-constexpr uint32_t kPairOverlap = 4u;  // overlap correction
-constexpr uint32_t kPairForce = 8u;    // force terms
-constexpr int kPairTerms = 7;
-
-// neighbour predicate (fluid: CellProcessor.cuh:137-143; collision: Map.cuh:189 with
-// CellProcessor.cuh:290-296): |d| <= R tested as |d|^2 <= reachSq, which is exactly equivalent.
-// Cells are never detached here (detached cells come from cell functions), so the detached rule
-// never applies.
-template <bool kFluid>
-__device__ __forceinline__ bool is_neighbor(const Nb& s, const Nb& o, float Wf, float Hf, float reachSq) {
-    if constexpr (kFluid)
-        return lensq(torus_delta(s.pos, o.pos, Wf, Hf)) <= reachSq;
-    else
-        return o.aidx != s.aidx && lensq(sub(o.pos, s.pos)) <= reachSq;
-}
-
-// The contribution of neighbour o to cell s, for a pair that passed is_neighbor.  The logical
-// indices of the two cells are needed only for a fusion candidate: lidxOf() returns them as
-// (s, o) when asked.
-template <bool kFluid, class LidxOf>
-__device__ __forceinline__ uint32_t pair_term(const Ctx& c, const DevWorld& w, const DevParams& P, int wi, const Nb& s,
-                                              const Nb& o, bool bonded, float* t, bool seam, LidxOf&& lidxOf) {
-    const float Wf = float(w.W), Hf = float(w.H);
-    const float cmd = P.minDistance;
-    const bool bari = flags_barrier(s.flags);
-    const f2 pd = stencil_delta(s.pos, o.pos, Wf, Hf, seam);
-    const float d = len2(pd);
-    uint32_t f = 0u;
-    if constexpr (kFluid) {
-        // CellProcessor.cuh:144-231
-        if (flags_barrier(o.flags)) {
-            t[0] = __int_as_float(o.aidx);
-            t[1] = d;
-            return kPairBarrier;
-        }
-        t[0] = sph_w(d * P.invH) * P.invH2;
-        if (o.aidx == s.aidx) return kPairSelf;
-        if (!bari && d < cmd) {
-            const f2 D = dvd(mul(pd, cmd), 5.0f);
-            t[1] = D.x;
-            t[2] = D.y;
-            f |= kPairOverlap;
-        }
-        if (bonded) return f;
-        const f2 vd = sub(s.vel, o.vel);
-        const float factor = s.dens + o.dens;  // 1/density_i + 1/density_j
-        if (fabsf(d) > kNearZero) {
-            const float kd = sph_dw(d * P.invH) * P.invH3;
-            const f2 Fp = mul(mul(mul(pd, 1.0f / (-d)), factor), kd);
-            const f2 Fv = mul(mul(mul(mul(vd, o.dens), d), kd), 1.0f / (d * d + 0.25f));
-            t[3] = Fp.x;
-            t[4] = Fp.y;
-            t[5] = Fv.x;
-            t[6] = Fv.y;
-            f |= kPairForce;
-        }
-        if (flags_num_conn(s.flags) < flags_max_conn(s.flags) && flags_num_conn(o.flags) < flags_max_conn(o.flags) &&
-            !bari && lensq(vd) > P.fusionBelowSq) {
-            const int2 L = lidxOf();
-            if (L.x < L.y) {
-                const float ei = c.energy[w.cellOff + c.A.slot[s.aidx]];
-                const float ej = c.energy[w.cellOff + c.A.slot[o.aidx]];
-                if (ei <= P.maxBindingEnergy && ej <= P.maxBindingEnergy) push_candidate(c, L.x, L.y, wi);
-            }
-        }
-    } else {
-        // CellProcessor.cuh:297-361.  f(j,i) mirrors f(i,j): unit(-d) = -unit(d) and
-        // (-dv).(-d) = dv.d exactly, so only the barrier factor and the branch differ.
-        if (!bari && d < cmd) {
-            const f2 D = dvd(mul(pd, cmd), 5.0f);
-            t[0] = D.x;
-            t[1] = D.y;
-            f |= kPairOverlap;
-        }
-        if (bonded) return f;
-        const f2 vd = sub(s.vel, o.vel);
-        const float dvp = dot2(vd, pd);
-        const bool appr = dot2(pd, vd) < 0.0f;
-        const bool barj = flags_barrier(o.flags);
-        const bool fastI = appr && lensq(s.vel) > P.fastSq;
-        const bool fastJ = appr && lensq(o.vel) > P.fastSq;
-        f2 fastT = {0.0f, 0.0f}, repT = {0.0f, 0.0f};
-        if (fastI || fastJ) fastT = mul(mul(pd, dvp), 1.0f / (-2.0f * (d * d + 0.25f)));
-        if (!(fastI && fastJ)) repT = mul(mul(unit(pd), P.collisionDistance - d), P.repulsion);
-        const f2 fij = mul(fastI ? fastT : repT, bari ? 2.0f : 1.0f);
-        // -f(j,i); unit() of a (near) zero vector is (1,0) in both directions, so there the
-        // repulsion is not mirrored
-        const f2 fjRep = mul(repT, barj ? 2.0f : 1.0f);
-        const f2 nfji = fastJ ? mul(fastT, barj ? 2.0f : 1.0f) : (d > kNearZero ? fjRep : neg(fjRep));
-        t[2] = fij.x;
-        t[3] = fij.y;
-        t[4] = nfji.x;
-        t[5] = nfji.y;
-        f |= kPairForce;
-        if (flags_num_conn(s.flags) < flags_max_conn(s.flags) && flags_num_conn(o.flags) < flags_max_conn(o.flags) &&
-            appr && !bari && !barj && lensq(vd) > P.fusionBelowSq) {
-            const int2 L = lidxOf();
-            if (L.x < L.y) {
-                const float ei = c.energy[w.cellOff + c.A.slot[s.aidx]];
-                const float ej = c.energy[w.cellOff + c.A.slot[o.aidx]];
-                if (ei <= P.maxBindingEnergy && ej <= P.maxBindingEnergy) push_candidate(c, L.x, L.y, wi);
-            }
-        }
-    }
-    return f;
-}
-
-// per-cell sums of the pass, added in visiting order.  Of the barrier neighbours only the first
-// ten count, and of those the first nearest one (CellProcessor.cuh:234-246); it is tracked as the
-// barriers arrive.
-struct Acc {
-    f2 F, pc, D, Fp, Fv;
-    float rho;
-    int numBarrier;
-    int cb;  // nearest barrier (A index), -1 if none
-    float cbDist;
-};
-
-__device__ __forceinline__ void acc_init(Acc& a, const Nb& s) {
-    a.F = {0.0f, 0.0f};
-    a.pc = s.pos;
-    a.D = {0.0f, 0.0f};
-    a.Fp = {0.0f, 0.0f};
-    a.Fv = {0.0f, 0.0f};
-    a.rho = 0.0f;
-    a.numBarrier = 0;
-    a.cb = -1;
-    a.cbDist = 0.0f;
-}
-
-template <bool kFluid>
-__device__ __forceinline__ void acc_add(Acc& a, uint32_t f, const float* t) {
-    if constexpr (kFluid) {
-        if (f & kPairBarrier) {
-            if (a.numBarrier < 10 && (a.cb < 0 || t[1] < a.cbDist)) {
-                a.cb = __float_as_int(t[0]);
-                a.cbDist = t[1];
-            }
-            ++a.numBarrier;
-            return;
-        }
-        a.rho = a.rho + t[0];
-        if (f & kPairSelf) return;
-        if (f & kPairOverlap) a.D = add(a.D, f2{t[1], t[2]});
-        if (f & kPairForce) {
-            a.Fp = add(a.Fp, f2{t[3], t[4]});
-            a.Fv = add(a.Fv, f2{t[5], t[6]});
-        }
-    } else {
-        if (f & kPairOverlap) a.pc = add(a.pc, f2{t[0], t[1]});
-        if (f & kPairForce) {
-            a.F = add(a.F, f2{t[2], t[3]});
-            a.F = add(a.F, f2{t[4], t[5]});
-        }
-    }
-}
-
-// acc_add without branches, for terms zeroed before pair_term wrote them (lanes with !on add
-// nothing).  Adding a zero term leaves a sum that started at +0 unchanged bit for bit (such a sum
-// is never -0), so the flags select only what is not a plain zero: a barrier neighbour's data, and
-// the collision position sum, which starts at the cell's position.
-template <bool kFluid>
-__device__ __forceinline__ void acc_add_sel(Acc& a, bool on, uint32_t f, const float* t) {
-    if constexpr (kFluid) {
-        const bool bar = on && (f & kPairBarrier) != 0u;
-        const bool sum = on && !bar;
-        const bool near = bar && a.numBarrier < 10 && (a.cb < 0 || t[1] < a.cbDist);
-        a.cb = near ? __float_as_int(t[0]) : a.cb;
-        a.cbDist = near ? t[1] : a.cbDist;
-        a.numBarrier += bar ? 1 : 0;
-        a.rho = sum ? a.rho + t[0] : a.rho;
-        a.D.x = sum ? a.D.x + t[1] : a.D.x;
-        a.D.y = sum ? a.D.y + t[2] : a.D.y;
-        a.Fp.x = on ? a.Fp.x + t[3] : a.Fp.x;
-        a.Fp.y = on ? a.Fp.y + t[4] : a.Fp.y;
-        a.Fv.x = on ? a.Fv.x + t[5] : a.Fv.x;
-        a.Fv.y = on ? a.Fv.y + t[6] : a.Fv.y;
-    } else {
-        const bool ov = on && (f & kPairOverlap) != 0u;
-        a.pc.x = ov ? a.pc.x + t[0] : a.pc.x;
-        a.pc.y = ov ? a.pc.y + t[1] : a.pc.y;
-        f2 F = add(a.F, f2{t[2], t[3]});
-        F = add(F, f2{t[4], t[5]});
-        a.F.x = on ? F.x : a.F.x;
-        a.F.y = on ? F.y : a.F.y;
-    }
-}
-
-__device__ __forceinline__ void load_bonds(const Ctx& c, const Nb& s, int bt[kMaxBonds]) {
-    const int nci = flags_num_conn(s.flags);
-#pragma unroll
-    for (int b = 0; b < kMaxBonds; ++b) bt[b] = b < nci ? c.A.btgt[b * c.cellCap + s.aidx] : -1;
-}
-
-__device__ __forceinline__ bool is_bonded(const int bt[kMaxBonds], int jLocal) {
-    bool bonded = false;
-#pragma unroll
-    for (int b = 0; b < kMaxBonds; ++b) bonded = bonded || (bt[b] == jLocal);
-    return bonded;
-}
-
-// Barrier reflection, applyForces, and the end-of-step writes of one cell.  A bonded or barrier
-// cell is marked staged for the bond kernels of the step.
-template <bool kFluid>
-__device__ __forceinline__ void cell_finish(const Ctx& c, const DevWorld& w, const DevParams& P, int wi, const Nb& s,
-                                            int slot, const int bt[kMaxBonds], Acc& a, int gbOld = -1) {
-    const int cap = c.cellCap;
-    const float Wf = float(w.W), Hf = float(w.H);
-    const int i = s.aidx, k = s.lidx;
-    const f2 pi = s.pos, vi = s.vel;
-    const uint32_t fi = s.flags;
-    const int nci = flags_num_conn(fi);
-    const bool bari = flags_barrier(fi);
-    f2 F = a.F, pc = a.pc;
-    if constexpr (kFluid) {
-        if (a.cb >= 0) {  // barrier reflection, CellProcessor.cuh:234-274
-            const int cb = a.cb;
-            const float cbDist = a.cbDist;
-            const f2 pb = to_f2(c.A.pos[cb]);
-            const f2 vb = to_f2(c.A.vel[cb]);
-            const int nb = flags_num_conn(c.A.flags[cb]);
-            f2 rr = {0.0f, 0.0f};
-            if (nb <= 1) {
-                rr = torus_delta(pi, pb, Wf, Hf);
-            } else {
-                const float angleToCell = angle_of(torus_delta(pi, pb, Wf, Hf));
-                for (int q = 0; q < nb; ++q) {
-                    const f2 o1 = to_f2(c.A.pos[w.cellOff + c.A.btgt[q * cap + cb]]);
-                    const f2 o2 = to_f2(c.A.pos[w.cellOff + c.A.btgt[((q + 1) % nb) * cap + cb]]);
-                    const float a1 = angle_of(torus_delta(o1, pb, Wf, Hf));
-                    const float a2 = angle_of(torus_delta(o2, pb, Wf, Hf));
-                    if (angle_between(a1, a2, angleToCell)) {
-                        rr = sub(o2, o1);
-                        rot_ccw(rr);
-                        break;
-                    }
-                }
-            }
-            const f2 vr = sub(vi, vb);
-            const float dd = dot2(vr, rr);
-            if (dd < 0.0f) {
-                const float trs = fmaxf(0.05f, lensq(rr));
-                const float td = fmaxf(0.05f, cbDist);
-                F = add(F, dvd(sub(add(sub(vr, dvd(mul(mul(rr, 2.0f), dd), trs)), vb), vi), td));
-            }
-        }
-        F = add(F, add(mul(a.Fp, P.pressure), mul(a.Fv, P.viscosity)));
-        pc = add(pi, a.D);
-    }
-
-    // the cell in the end-of-step order; bond targets stay in start-of-step indices until the
-    // staged cells are renumbered (k_remap)
-    c.B.flags[k] = fi;
-    c.B.slot[k] = slot;
-    c.B.dens[k] = kFluid ? a.rho : s.dens;
-    if constexpr (kFluid) {
-        // (unrolled: a loop to nci would index bt at run time and place it in scratch memory)
-#pragma unroll
-        for (int b = 0; b < kMaxBonds; ++b)
-            if (b < nci) {
-                c.B.btgt[b * cap + k] = bt[b];
-                c.B.brest[b * cap + k] = c.A.brest[b * cap + i];
-                c.B.bang[b * cap + k] = c.A.bang[b * cap + i];
-            }
-        if (nci > 0) c.bstiff[k] = c.stiff[w.cellOff + slot];
-    } else {
-        // (collision worlds are mostly bonded cells: their bond data is loaded before any of it
-        // is stored, so that the loads are in flight together)
-        float brest[kMaxBonds], bang[kMaxBonds];
-#pragma unroll
-        for (int b = 0; b < kMaxBonds; ++b) {
-            brest[b] = b < nci ? c.A.brest[b * cap + i] : 0.0f;
-            bang[b] = b < nci ? c.A.bang[b * cap + i] : 0.0f;
-        }
-        const float stiff = nci > 0 ? c.stiff[w.cellOff + slot] : 0.0f;
-#pragma unroll
-        for (int b = 0; b < kMaxBonds; ++b)
-            if (b < nci) {
-                c.B.btgt[b * cap + k] = bt[b];
-                c.B.brest[b * cap + k] = brest[b];
-                c.B.bang[b * cap + k] = bang[b];
-            }
-        if (nci > 0) c.bstiff[k] = stiff;
-    }
-    if (nci > 0) c.newidx[i] = k;
-    // checkForces (CellProcessor.cuh:367-386): a bonded cell whose force is above cellMaxForce loses
-    // all its bonds with probability cellMaxForceDecayProb (deleting the bonds of an unbonded cell
-    // would change nothing)
-    // (the per-colour threshold is read from memory: indexing the register copy of the
-    // parameters by a run-time colour would place the whole copy in scratch memory)
-    uint8_t stage = bari || nci != 0 ? kStagedCell : 0;
-    if (P.decayProb > 0.0f && nci > 0 && !bari && lensq(F) > c.params[wi].maxForceSq[flags_color(fi)]) {
-        const unsigned long long id = c.cid[w.cellOff + slot];
-        if (uniform_draw(w.seed, c.ctr[wi].timestep, id, kStreamForceDecay) < P.decayProb) stage |= kDropBonds;
-    }
-    f2 v = vi;
-    if (!bari) {  // applyForces
-        v = add(v, F);
-        if (lensq(v) > P.maxVelSq) v = mul(unit(v), P.maxVelocity);
-    }
-    if (!bari && nci == 0) {
-        // no bonds: both connection-force passes yield zero, so the Verlet position and velocity
-        // updates and friction of this step are applied here with the same operations
-        const f2 zero = {0.0f, 0.0f};
-        const float dt = P.dt;
-        const f2 p2 = torus_pos(add(pc, add(mul(v, dt), mul(mul(mul(zero, dt), dt), 0.5f))), w.W, w.H);
-        const f2 acc = mul(add(zero, zero), 0.5f);
-        v = add(v, mul(acc, dt));
-        v = mul(v, 1.0f - P.friction);
-        c.B.pos[k] = to_float2(p2);
-        c.B.vel[k] = to_float2(v);
-        bin_next(c, w, k, p2, gbOld >= 0 ? gbOld : cell_bin_of(w, pi));
-    } else {
-        c.B.pos[k] = to_float2(pc);
-        c.B.vel[k] = to_float2(v);
-    }
-    if (w.bondWork) c.stage[k] = stage;
-}
-
-// One cell, neighbours visited one after another (forEachNb calls visit(o) in stencil order).
-template <bool kFluid, class ForEach>
-__device__ __forceinline__ void cell_direct(const Ctx& c, const DevWorld& w, const DevParams& P, int wi, const Nb& s,
-                                            ForEach&& forEachNb) {
-    const float Wf = float(w.W), Hf = float(w.H);
-    int bt[kMaxBonds];
-    load_bonds(c, s, bt);
-    Acc a;
-    acc_init(a, s);
-    forEachNb([&](const Nb& o) {
-        if (!is_neighbor<kFluid>(s, o, Wf, Hf, P.reachSq)) return;
-        float t[kPairTerms];
-        const uint32_t f = pair_term<kFluid>(c, w, P, wi, s, o, is_bonded(bt, o.aidx - w.cellOff), t, true,
-                                             [&] { return make_int2(s.lidx, o.lidx); });
-        acc_add<kFluid>(a, f, t);
-    });
-    cell_finish<kFluid>(c, w, P, wi, s, c.A.slot[s.aidx], bt, a);
-}
-
 
 // ---------------------------------------------------------------------------------------------
 // Row streaming.  A workgroup (one wave) owns a strip of up to kStripMax bin columns and a chunk of
@@ -419,7 +51,6 @@ struct RowShared {
     // repeated after the end so that a stencil range of up to 64 entries reads without wrapping
     float2 pos[kPool + kPosMirror];
     float2 vel[kPool];
-    float dens[kPool];  // fluid: 1 / density; collision: density
     uint16_t flags[kPool];  // the bits the pass reads of an entry's flags (flags16)
     int aidx[kPool];
     uint8_t sbin[kPool];  // bin slot: bin row * HX + halo column
@@ -445,7 +76,6 @@ struct RowFlight {
     uint32_t s0[kSlots], s1[kSlots];
     int aidx[2];
     float2 pos[2], vel[2];
-    float dens[2];
     uint32_t flags[2];
     int total;
 };
@@ -486,7 +116,7 @@ __device__ __forceinline__ Nb row_nb(const RS& S, const StripGeom& g, int r, int
     Nb o;
     o.pos = to_f2(S.pos[pp]);
     o.vel = to_f2(S.vel[pp]);
-    o.dens = S.dens[pp];
+    o.dens = 0.0f;
     o.flags = flags32(S.flags[pp]);
     o.aidx = S.aidx[pp];
     o.lidx = kLidx ? row_lidx<kSub>(S, g, r, pp) : -1;
@@ -498,7 +128,7 @@ __device__ __forceinline__ Nb global_nb(const Ctx& c, int a, int l) {
     Nb o;
     o.pos = to_f2(c.A.pos[a]);
     o.vel = to_f2(c.A.vel[a]);
-    o.dens = kFluid ? 1.0f / c.A.dens[a] : c.A.dens[a];
+    o.dens = kFluid ? c.A.dens[a] : 0.0f;
     o.flags = c.A.flags[a];
     o.aidx = a;
     o.lidx = l;
@@ -565,7 +195,6 @@ __device__ __forceinline__ void row_issue_entries(const Ctx& c, const StripGeom&
             F.aidx[q] = c.sorted[m];
             F.pos[q] = c.mpos[m];
             F.vel[q] = c.mvel[m];
-            F.dens[q] = c.mdens[m];
             F.flags[q] = c.mflags[m];
         }
     }
@@ -590,7 +219,6 @@ __device__ __forceinline__ void row_commit(const StripGeom& g, RS& S, const RowF
             S.pos[pp] = F.pos[q];
             if (pp < kPosMirror) S.pos[kPool + pp] = F.pos[q];
             S.vel[pp] = F.vel[q];
-            S.dens[pp] = F.dens[q];
             S.flags[pp] = flags16(F.flags[q]);
             S.aidx[pp] = a;
             S.sbin[pp] = uint8_t(j);
@@ -915,11 +543,10 @@ __device__ __forceinline__ bool chunk_rows(const Ctx& c, const DevWorld& w, cons
 
 // A collision world staged two bin rows at a time (sparse rows) runs a chunk whose two-row stages
 // do not fit as single bin rows over the same bins.
-// The fluid kernel is held to 128 VGPRs, four waves per SIMD (its 10.2 KB of LDS allow 16
-// workgroups per CU); it ran 4 % faster than at 135 VGPRs and three waves.  The collision kernel
-// needs ~146 and would spill more than it gains.
+// (four waves per SIMD, 128 VGPRs without scratch: at 133 VGPRs and three waves the eight-world batch ran
+// 13 % slower)
 template <bool kFluid>
-__global__ void __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(kFluid ? 4 : 1)))
+__global__ void __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
 k_neighbor_rows(Ctx c, int sortBlocks) {
     __shared__ RowShared<kFluid ? 1 : kSubMax> S;
     // (the particles' bin sort, on workgroups of its own, in sets with bond work)
@@ -963,347 +590,20 @@ k_neighbor_rows(Ctx c, int sortBlocks) {
     }
 }
 
-// ---------------------------------------------------------------------------------------------
-// Cell-parallel fluid pass.  The map is in logical order (cells by bin, inside a bin by previous
-// index), so the three stencil bins of a cell in one bin row are one contiguous range of the map,
-// and a wave of 64 consecutive map positions reads its candidates through it (the ranges of
-// neighbouring lanes overlap and stay in the caches; the start-of-step state is nearly in map
-// order, so the reads through the map are nearly sequential).  Per wave: every lane tests its
-// candidates into a mask in visiting order; the wave's neighbour pairs are listed back to back in
-// LDS and evaluated one pair per lane; every lane then adds its own pairs' terms in visiting order
-// (the float sums of a sequential stencil walk, bit for bit) and finishes its cell.  A cell in the
-// first or last bin column (its stencil wraps around the torus there), one with more than 64
-// candidates, and every cell of a grid narrower than three bins walks its stencil alone
-// (cell_direct, same order and results).  Workgroups of 1..4 waves (the cell block size), each
-// wave on its own with its own LDS (wave-level synchronisation only); block b
-// runs table entry (b mod 8) * ceil(T / 8) + b / 8, so each XCD sweeps one contiguous band of the
-// map and the stencil rows its waves share stay in its L2.
-// ---------------------------------------------------------------------------------------------
-constexpr int kCellWaves = 4;  // waves per workgroup at most (256-thread groups: 64- and 128-thread
-                               // groups ran 2.3x and 1.4x slower, 512-thread ones 9 % slower)
-constexpr int kCellRec = 256;  // pair records of one wave at a time
-
-constexpr int kCellStage = 192;  // staged candidate positions per stencil row (three per lane)
-
-struct CellShared {
-    // the wave's own cells (the self side of its pairs)
-    float2 pos[64];
-    float2 vel[64];
-    float dens[64];
-    uint32_t flags[64];
-    int aidx[64];
-    union {
-        // while candidates are tested: positions of the union of the lanes' ranges, per stencil
-        // row, and one entry past the end (read by the second test of an iteration that passes a
-        // list's end; its result is trimmed)
-        float2 cpos[3 * kCellStage + 1];
-        struct {
-            // pair records: neighbour map position, owner lane | bonded << 7
-            int rnb[kCellRec];
-            uint8_t rown[kCellRec];
-            // results of the pairs evaluated in one round: terms and the term flags
-            float res[kPairTerms + 1][64];
-        } pr;
-    } u;
-};
-
-// the cell at map position m (fluid: 1 / density) as a neighbour
-__device__ __forceinline__ Nb map_nb(const Ctx& c, int m) {
-    Nb o;
-    o.aidx = c.sorted[m];
-    o.pos = to_f2(c.A.pos[o.aidx]);
-    o.vel = to_f2(c.A.vel[o.aidx]);
-    o.dens = 1.0f / c.A.dens[o.aidx];
-    o.flags = c.A.flags[o.aidx];
-    o.lidx = m;
-    return o;
-}
-
-// (at most 80 VGPRs: six waves per SIMD)
-template <bool kPartSort>
-__global__ void __launch_bounds__(64 * kCellWaves) __attribute__((amdgpu_waves_per_eu(6)))
-k_neighbor_cells(Ctx c, int sortBlocks, int tableBlocks) {
-    __shared__ CellShared SS[kCellWaves];
-    // (the particles' bin sort, on workgroups of its own, in sets with bond work)
-    if (kPartSort && int(blockIdx.x) < sortBlocks) {
-        part_binsort(c, {int(blockIdx.x), sortBlocks});
-        return;
-    }
-    const int block = kPartSort ? int(blockIdx.x) - sortBlocks : int(blockIdx.x);
-    const int per = (tableBlocks + kXcdCount - 1) / kXcdCount;
-    const int e = (block % kXcdCount) * per + block / kXcdCount;
-    if (e >= tableBlocks) return;
-    const int2 blk = c.cellBlocks[e];
-    const int wi = blk.x;
-    const DevWorld w = c.worlds[wi];
-    const DevParams P = c.params[wi];
-    if (P.motion != 0) return;
-    const int lane = int(threadIdx.x) & 63, wave = int(threadIdx.x) >> 6;
-    CellShared& S = SS[wave];
-    const int m = blk.y + int(threadIdx.x);
-    const int mEnd = w.cellOff + w.numCells;
-    if (__builtin_amdgcn_readfirstlane(blk.y + wave * 64) >= mEnd) return;  // the whole wave is past the world
-    const bool active = m < mEnd;
-    const float Wf = float(w.W), Hf = float(w.H);
-    const float w0 = sph_w(0.0f) * P.invH2;  // a cell's own density term
-    const uint32_t base = c.start[w.binOff];
-    auto S0 = [&](int b) { return w.cellOff + int(c.start[w.binOff + b] - base); };
-
-    Nb self;
-    self.pos = {0.0f, 0.0f};
-    self.vel = {0.0f, 0.0f};
-    self.dens = 0.0f;
-    self.flags = 0u;
-    self.aidx = 0;
-    self.lidx = m;
-    int bx = 0, by = 0;
-    if (active) {
-        self = map_nb(c, m);
-        cell_bin_xy(w, self.pos, bx, by);
-    }
-    S.pos[lane] = to_float2(self.pos);
-    S.vel[lane] = to_float2(self.vel);
-    S.dens[lane] = self.dens;
-    S.flags[lane] = self.flags;
-    S.aidx[lane] = self.aidx;
-    // stencil rows above, own, below: one map range each (bins bx-1 .. bx+1)
-    int lo[3] = {0, 0, 0}, ns[3] = {0, 0, 0};
-    bool direct = active && (bx == 0 || bx == w.nbx - 1);
-    if (active && !direct) {
-#pragma unroll
-        for (int r = 0; r < 3; ++r) {
-            const int rb = wrap_small(by + r - 1, w.nby) * w.nbx;
-            lo[r] = S0(rb + bx - 1);
-            ns[r] = S0(rb + bx + 2) - lo[r];
-        }
-        if (ns[0] + ns[1] + ns[2] > 64) direct = true;
-    }
-    if (direct) ns[0] = ns[1] = ns[2] = 0;
-    // away from the seam rows (and in grids of at least eight bins each way) the plain difference
-    // equals the torus difference bit for bit: two stencil neighbours lie less than three bin
-    // edges apart, less than half the world
-    const bool seam = __any(active && (by == 0 || by == w.nby - 1)) || w.nbx < 8 || w.nby < 8;
-    unsigned long long mask = 0ull, bmask = 0ull;
-    int selfIdx = -1;  // pairs before the cell's own density term
-    // The union of the lanes' ranges of each stencil row is staged in LDS (all its loads in flight
-    // together) when it fits; a wave whose cells span two bin rows tests from global memory.
-    const bool tests = active && !direct;
-    // The staged range of each stencil row, [u0, u0 + un): from the first testing lane's range start
-    // to the last one's end (in one bin row both grow with the lane), used when every testing
-    // lane's range lies inside (a wave across two bin rows fails that).
-    int u0[3], un[3];
-    const unsigned long long testers = __ballot(tests);
-    bool staged = testers != 0ull;
-    if (staged) {
-        const int first = __builtin_ctzll(testers), last = 63 - __builtin_clzll(testers);
-        bool inside = true;
-#pragma unroll
-        for (int r = 0; r < 3; ++r) {
-            u0[r] = __builtin_amdgcn_readlane(lo[r], first);
-            un[r] = __builtin_amdgcn_readlane(lo[r] + ns[r], last) - u0[r];
-            inside = inside && (!tests || (lo[r] >= u0[r] && lo[r] + ns[r] <= u0[r] + un[r]));
-            staged = staged && un[r] >= 0 && un[r] <= kCellStage;
-        }
-        staged = staged && __all(inside);
-    }
-    if (!staged) u0[0] = u0[1] = u0[2] = un[0] = un[1] = un[2] = 0;
-    if (staged) {
-        int a[3][3];
-#pragma unroll
-        for (int r = 0; r < 3; ++r)
-#pragma unroll
-            for (int q = 0; q < 3; ++q) a[r][q] = lane + 64 * q < un[r] ? c.sorted[u0[r] + lane + 64 * q] : -1;
-        float2 v[3][3];
-#pragma unroll
-        for (int r = 0; r < 3; ++r)
-#pragma unroll
-            for (int q = 0; q < 3; ++q) v[r][q] = a[r][q] >= 0 ? c.A.pos[a[r][q]] : float2{0.0f, 0.0f};
-#pragma unroll
-        for (int r = 0; r < 3; ++r)
-#pragma unroll
-            for (int q = 0; q < 3; ++q) S.u.cpos[r * kCellStage + lane + 64 * q] = v[r][q];
-    }
-    __syncwarp();
-    if (tests) {
-        // the three ranges as one list in visiting order: candidate t lies in row 0 below n0, in
-        // row 1 below n01, else in row 2 (the wave runs its longest list, not its longest row)
-        const int n0 = ns[0], n01 = ns[0] + ns[1], nt = n01 + ns[2];
-        // candidate t lies at t plus its row's offset: in the staged rows (read as one array of
-        // three rows) or in the map
-        const int so0 = lo[0] - u0[0], so1 = kCellStage + lo[1] - u0[1] - n0, so2 = 2 * kCellStage + lo[2] - u0[2] - n01;
-        const int go0 = lo[0], go1 = lo[1] - n0, go2 = lo[2] - n01;
-        const int sd1 = so1 - so0, sd2 = so2 - so1, gd1 = go1 - go0, gd2 = go2 - go1;
-        auto test = [&](auto seamTag, auto stagedTag) {
-            constexpr bool kSeam = decltype(seamTag)::value;
-            constexpr bool kStaged = decltype(stagedTag)::value;
-            auto cand = [&](int t) -> f2 {
-                if constexpr (kStaged) {
-                    // (t <= nt: at most one entry past the last row's range, inside cpos; the
-                    // offsets in bytes, so that a row select is not scaled per candidate)
-                    int xb = 8 * t + 8 * so0;
-                    xb += t >= n0 ? 8 * sd1 : 0;
-                    xb += t >= n01 ? 8 * sd2 : 0;
-                    return to_f2(*reinterpret_cast<const float2*>(reinterpret_cast<const char*>(S.u.cpos) + xb));
-                } else {
-                    int x = t + go0;
-                    x += t >= n0 ? gd1 : 0;
-                    x += t >= n01 ? gd2 : 0;
-                    return to_f2(c.A.pos[c.sorted[min(x, mEnd - 1)]]);
-                }
-            };
-            // two candidates per iteration (the second may pass the list's end: trimmed below),
-            // their bits set in the half of the mask that holds t (a uniform loop bound per half:
-            // a wave's lists rarely pass 32 candidates)
-            auto half = [&](int t0, int t1, uint32_t& m32) {
-                for (int t = t0; t < t1; t += 2) {
-                    const f2 p0 = cand(t), p1 = cand(t + 1);
-                    const float d0 = lensq(kSeam ? torus_delta(self.pos, p0, Wf, Hf) : sub(self.pos, p0));
-                    const float d1 = lensq(kSeam ? torus_delta(self.pos, p1, Wf, Hf) : sub(self.pos, p1));
-                    const uint32_t bit = 1u << (t & 31);
-                    m32 |= (d0 <= P.reachSq ? bit : 0u) | (d1 <= P.reachSq ? bit << 1 : 0u);
-                }
-            };
-            uint32_t lo32 = 0u, hi32 = 0u;
-            half(0, min(nt, 32), lo32);
-            half(32, nt, hi32);
-            mask = (static_cast<unsigned long long>(hi32) << 32) | lo32;
-            mask &= nt >= 64 ? ~0ull : (1ull << nt) - 1ull;
-        };
-        if (staged) {
-            if (seam)
-                test(std::true_type{}, std::true_type{});
-            else
-                test(std::false_type{}, std::true_type{});
-        } else {
-            if (seam)
-                test(std::true_type{}, std::false_type{});
-            else
-                test(std::false_type{}, std::false_type{});
-        }
-        // a barrier cell meets itself as a barrier neighbour; any other cell adds its own density
-        // term at its place in the visiting order, without a pair
-        const int selfFlat = ns[0] + (m - lo[1]);
-        if (!flags_barrier(self.flags)) {
-            mask &= ~(1ull << selfFlat);
-            selfIdx = __builtin_popcountll(mask & ((1ull << selfFlat) - 1ull));
-        }
-        if (flags_num_conn(self.flags) > 0) {
-            // (the bond targets are loaded here and again at the end rather than held through the
-            // pair work: few cells of a fluid world have bonds, and the loads hit the cache)
-            int bt[kMaxBonds];
-            load_bonds(c, self, bt);
-            unsigned long long mm = mask;
-            while (mm) {
-                const int ci = __builtin_ctzll(mm);
-                mm &= mm - 1ull;
-                const int r = ci < ns[0] ? 0 : (ci < ns[0] + ns[1] ? 1 : 2);
-                const int rest = ci - (r == 0 ? 0 : (r == 1 ? ns[0] : ns[0] + ns[1]));
-                const int jm = (r == 0 ? lo[0] : (r == 1 ? lo[1] : lo[2])) + rest;
-                if (is_bonded(bt, c.sorted[jm] - w.cellOff)) bmask |= 1ull << ci;
-            }
-        }
-    }
-    const int count = __builtin_popcountll(mask);
-    const int inc = int(wave_inclusive_scan(uint32_t(count)));
-    const int numPairs = wave_last(inc);
-    const int pbase = inc - count;
-    __syncwarp();  // (the pair records reuse the staged positions' LDS)
-
-    Acc a;
-    acc_init(a, self);
-    for (int R0 = 0; R0 < numPairs; R0 += kCellRec) {
-        const int rend = min(numPairs, R0 + kCellRec);
-        // owners list their pairs of this window, in visiting order
-        if (count > 0 && pbase < rend && pbase + count > R0) {
-            unsigned long long mm = mask;
-            for (int p = pbase; mm; ++p) {
-                const int ci = __builtin_ctzll(mm);
-                mm &= mm - 1ull;
-                if (p < R0 || p >= rend) continue;
-                const int r = ci < ns[0] ? 0 : (ci < ns[0] + ns[1] ? 1 : 2);
-                const int rest = ci - (r == 0 ? 0 : (r == 1 ? ns[0] : ns[0] + ns[1]));
-                S.u.pr.rnb[p - R0] = (r == 0 ? lo[0] : (r == 1 ? lo[1] : lo[2])) + rest;
-                S.u.pr.rown[p - R0] = uint8_t(lane | int((bmask >> ci) & 1ull) << 7);
-            }
-        }
-        __syncwarp();
-        for (int off = R0; off < rend; off += 64) {
-            // pair terms, one pair per lane
-            const int p = off + lane;
-            float tm[kPairTerms];
-#pragma unroll
-            for (int v = 0; v < kPairTerms; ++v) tm[v] = 0.0f;
-            uint32_t f = 0u;
-            if (p < rend) {
-                const int jm = S.u.pr.rnb[p - R0];
-                const int ow = S.u.pr.rown[p - R0];
-                const int ol = ow & 63;
-                Nb s;
-                s.pos = to_f2(S.pos[ol]);
-                s.vel = to_f2(S.vel[ol]);
-                s.dens = S.dens[ol];
-                s.flags = S.flags[ol];
-                s.aidx = S.aidx[ol];
-                s.lidx = blk.y + wave * 64 + ol;
-                const Nb o = map_nb(c, jm);
-                f = pair_term<true>(c, w, P, wi, s, o, (ow >> 7) != 0, tm, seam,
-                                    [&] { return make_int2(s.lidx, o.lidx); });
-            }
-#pragma unroll
-            for (int v = 0; v < kPairTerms; ++v) S.u.pr.res[v][lane] = tm[v];
-            S.u.pr.res[kPairTerms][lane] = __uint_as_float(f);
-            __syncwarp();
-            // every owner adds its pairs of this round in visiting order
-            const int jlo = max(pbase, off), jhi = min(pbase + count, min(off + 64, rend));
-            for (int j = jlo; j < jhi; ++j) {
-                const int q = j - off;
-                float tt[kPairTerms];
-#pragma unroll
-                for (int v = 0; v < kPairTerms; ++v) tt[v] = S.u.pr.res[v][q];
-                const uint32_t ff = __float_as_uint(S.u.pr.res[kPairTerms][q]);
-                if (j - pbase == selfIdx) a.rho = a.rho + w0;
-                acc_add<true>(a, ff, tt);
-            }
-            __syncwarp();
-        }
-    }
-    if (!active) return;
-    if (direct) {
-        atomicAdd(&c.sc->directCells, 1ull);
-        cell_direct<true>(c, w, P, wi, self, [&](auto&& visit) {
-            for (int dy = -1; dy <= 1; ++dy) {
-                const int rb = wrap_small(by + dy, w.nby) * w.nbx;
-                for (int dx = -1; dx <= 1; ++dx) {
-                    const int b = rb + wrap_small(bx + dx, w.nbx);
-                    const int s1 = S0(b + 1);
-                    for (int j = S0(b); j < s1; ++j) visit(map_nb(c, j));
-                }
-            }
-        });
-        return;
-    }
-    if (selfIdx == count) a.rho = a.rho + w0;  // the own term after all pairs
-    int bt[kMaxBonds];
-    load_bonds(c, self, bt);
-    cell_finish<true>(c, w, P, wi, self, c.A.slot[self.aidx], bt, a, w.binOff + by * w.nbx + bx);
-}
-
 int neighbor_blocks_per_cu() {
     int n = 0;
     const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_neighbor_rows<false>, kRowThreads, 0);
     return e == hipSuccess ? std::max(1, n) : 1;
 }
 
+void launch_fluid(const Ctx& c, const LaunchShape& sh, hipStream_t s, int sortBlocks);
+
 void launch_neighbor(const Ctx& c, const LaunchShape& sh, hipStream_t s, bool withPartSort) {
     // (the bin sort goes with the first launch)
     int sort = withPartSort && sh.hasParticles && sh.partBlocks ? sh.pbinBlocks : 0;
-    const bool fluid = sh.hasFluid && sh.cellBlocks, collision = sh.hasCollision && sh.tileBlocks;
-    if (fluid || (sort && !collision)) {
-        const int grid = fluid ? (sh.cellBlocks + kXcdCount - 1) / kXcdCount * kXcdCount : 0;
-        if (sort)
-            hipLaunchKernelGGL(k_neighbor_cells<true>, dim3(sort + grid), dim3(sh.cellThreads), 0, s, c, sort, sh.cellBlocks);
-        else
-            hipLaunchKernelGGL(k_neighbor_cells<false>, dim3(grid), dim3(sh.cellThreads), 0, s, c, 0, sh.cellBlocks);
+    const bool collision = sh.hasCollision && sh.tileBlocks;
+    if (sh.fluidBlocks || (sort && !collision)) {
+        launch_fluid(c, sh, s, sort);
         sort = 0;
     }
     if (collision) {

@@ -320,7 +320,6 @@ __device__ __forceinline__ void cell_scatter(const Ctx& c, int block, int tableB
         if (c.params[wi[q]].motion != 0) {
             c.mpos[dest] = c.A.pos[iq];
             c.mvel[dest] = c.A.vel[iq];
-            c.mdens[dest] = c.A.dens[iq];
             c.mflags[dest] = c.A.flags[iq];
         }
         if (c.partStage > 0) part_scatter_staged(c, c.worlds[wi[q]], iq);

@@ -14,6 +14,7 @@ struct LaunchShape {
     int cellBlocks = 0, cellThreads = 256;
     int partBlocks = 0, partThreads = 256;
     int pbinBlocks = 0, binThreads = 256;
+    int fluidBlocks = 0, edgeBlocks = 0;  // workgroups of the fluid pass: inner cells, edge columns
     int tileBlocks = 0;    // neighbour-pass workgroups (including XCD padding)
     int partGrid = 64;     // grid-stride particle kernels
     int bondBlocks = 0;    // bond kernels: cell blocks of the worlds that can have bonded cells

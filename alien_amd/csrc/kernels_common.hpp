@@ -3,6 +3,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "device_math.hpp"
 #include "engine_types.hpp"
 
@@ -47,10 +49,11 @@ __device__ __forceinline__ void part_bin_range(const Ctx& c, const DevWorld& w, 
     e = w.partOff + min(int(c.start[w.pbinOff + b + 1] - base), w.partCap);
 }
 
-// cell bin of a position (global bin index), and its bin coordinates
+// bin coordinates of a position (on the torus up to rounding; anything else takes the general wrap),
+// and its global bin index
 __device__ __forceinline__ void cell_bin_xy(const DevWorld& w, f2 p, int& bx, int& by) {
-    int sx, sy;
-    slot_of(p, w.W, w.H, sx, sy);
+    int sx = static_cast<int>(__builtin_floorf(p.x)), sy = static_cast<int>(__builtin_floorf(p.y));
+    if (uint32_t(sx) >= uint32_t(w.W) || uint32_t(sy) >= uint32_t(w.H)) slot_of(p, w.W, w.H, sx, sy);
     bx = min(bin_coord(w, sx), w.nbx - 1);
     by = min(bin_coord(w, sy), w.nby - 1);
 }
@@ -69,18 +72,32 @@ __device__ __forceinline__ int cell_bin_of(const DevWorld& w, f2 p) {
 // so its order does not matter).
 __device__ __forceinline__ void push_mover(int* head, int* next, int gb, int k) { next[k] = atomicExch(&head[gb], k); }
 
-// next-step bin of the cell at end-of-step index k: end-of-step position pNew; gbOld, its bin in
-// this step's map (the bin of its start-of-step position)
-__device__ __forceinline__ void bin_next(const Ctx& c, const DevWorld& w, int k, f2 pNew, int gbOld) {
-    const int gb = cell_bin_of(w, pNew);
-    if (gb == gbOld) {
-        c.binOf[k] = gb;
+// base[i] through a 32-bit byte offset, which a 64-bit address of a signed index costs four operations
+// more than (a set's cells times 8 bytes, and a world's bins times 4, stay below 2^32)
+template <class T> __device__ __forceinline__ T* at32(T* base, uint32_t i) {
+    using Byte = typename std::conditional<std::is_const<T>::value, const char, char>::type;
+    return reinterpret_cast<T*>(reinterpret_cast<Byte*>(base) + uint32_t(i * uint32_t(sizeof(T))));
+}
+template <class T> __device__ __forceinline__ T ld32(const T* base, uint32_t i) { return *at32(base, i); }
+template <class T> __device__ __forceinline__ void st32(T* base, uint32_t i, T v) { *at32(base, i) = v; }
+static_assert(uint64_t(kMaxSetCells) * 8 < (uint64_t(1) << 32), "32-bit byte offsets");
+
+// next-step bin of the cell at end-of-step index k: end-of-step position pNew; bOld, its bin in this
+// step's map (the bin of its start-of-step position, counted from the world's first)
+__device__ __forceinline__ void bin_next(const Ctx& c, const DevWorld& w, int k, f2 pNew, int bOld) {
+    int bx, by;
+    cell_bin_xy(w, pNew, bx, by);
+    const int b = by * w.nbx + bx;
+    const int gb = w.binOff + b;
+    if (b == bOld) {
+        st32(c.binOf, k, gb);
         return;
     }
-    c.binOf[k] = int(uint32_t(gb) | kMoverBit);
-    push_mover(c.moverHeadNext, c.moverNext, gb, k);
-    atomicAdd(&c.deltaNext[gb], 1);
-    atomicSub(&c.deltaNext[gbOld], 1);
+    st32(c.binOf, k, int(uint32_t(gb) | kMoverBit));
+    st32(c.moverNext, k, atomicExch(at32(c.moverHeadNext + w.binOff, b), k));
+    int* delta = c.deltaNext + w.binOff;
+    atomicAdd(at32(delta, b), 1);
+    atomicSub(at32(delta, bOld), 1);
 }
 
 __device__ __forceinline__ void pbin_for_next_step(const Ctx& c, const DevWorld& w, int k, f2 p, uint32_t* hist) {

@@ -683,7 +683,6 @@ void WorldSet::build(const std::vector<Source>& sources) {
     sorted_ = static_cast<int*>(A(sizeof(int) * NC));
     mpos_ = static_cast<float2*>(A(sizeof(float2) * NC));
     mvel_ = static_cast<float2*>(A(sizeof(float2) * NC));
-    mdens_ = static_cast<float*>(A(sizeof(float) * NC));
     mflags_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
     newidx_ = static_cast<int*>(A(sizeof(int) * NC));
     psorted_ = static_cast<int*>(A(sizeof(int) * NP));
@@ -964,7 +963,7 @@ void WorldSet::buildTables() {
     if (stream_) synchronize();  // (the tables and the live counts read below are in use until then)
     for (auto& a : tableAllocs_) (void)hipFree(a.p);
     tableAllocs_.clear();
-    std::vector<int2> cells, bonds, pbins, parts, living;
+    std::vector<int2> cells, bonds, pbins, parts, living, edges, fluids;
     const int ct = shape_.cellThreads, pt = shape_.partThreads, bt = shape_.binThreads;
     for (int wi = 0; wi < int(worlds_.size()); ++wi) {
         if (!active_[wi]) continue;
@@ -974,6 +973,10 @@ void WorldSet::buildTables() {
             for (int s = 0; s < w.numCells; s += ct) bonds.push_back(make_int2(wi, w.cellOff + s));
         if (livingWork_[wi])
             for (int s = 0; s < w.numCells; s += ct) living.push_back(make_int2(wi, w.cellOff + s));
+        if (params_[wi].motion == 0 && w.numCells > 0) {  // waves of the fluid pass, see k_fluid.hip
+            for (int s = 0; s < 2 * (w.nby + 1); s += ct / 64) edges.push_back(make_int2(wi, s));
+            for (int s = 0; s < (w.numCells + 63) / 64 + 2; s += ct / 64) fluids.push_back(make_int2(wi, s));
+        }
         for (int s = 0; s < w.pnbx * w.pnby; s += bt) pbins.push_back(make_int2(wi, w.pbinOff + s));
     }
     auto up = [&](const std::vector<int2>& v) -> int2* {
@@ -1031,6 +1034,10 @@ void WorldSet::buildTables() {
     pbinBlocks_ = up(pbins);
     tileBlocks_ = up(tileTable);
     livingBlocks_ = up(living);
+    edgeBlocks_ = up(edges);
+    shape_.edgeBlocks = int(edges.size());
+    fluidBlocks_ = up(fluids);
+    shape_.fluidBlocks = int(fluids.size());
     shape_.livingBlocks = int(living.size());
     shape_.cellBlocks = int(cells.size());
     shape_.bondBlocks = int(bonds.size());
@@ -1190,7 +1197,6 @@ Ctx WorldSet::makeCtx(int parity) const {
     c.sorted = sorted_;
     c.mpos = mpos_;
     c.mvel = mvel_;
-    c.mdens = mdens_;
     c.mflags = mflags_;
     c.newidx = newidx_;
     c.psorted = psorted_;
@@ -1214,6 +1220,8 @@ Ctx WorldSet::makeCtx(int parity) const {
     c.pbinBlocks = pbinBlocks_;
     c.partBlocks = partBlocks_;
     c.tileBlocks = tileBlocks_;
+    c.edgeBlocks = edgeBlocks_;
+    c.fluidBlocks = fluidBlocks_;
     c.numPartBlocks = numPartBlocks_;
     c.partBlockParticles = shape_.partThreads;
     c.blockThreads = shape_.cellThreads;

@@ -273,7 +273,6 @@ private:
     uint32_t* mapEpochTicket_ = nullptr;  // [2]: epoch, ticket
     int *sorted_ = nullptr, *newidx_ = nullptr, *psorted_ = nullptr;
     float2 *mpos_ = nullptr, *mvel_ = nullptr;
-    float* mdens_ = nullptr;
     uint32_t* mflags_ = nullptr;
     uint8_t* stage_ = nullptr;
     float2 *own_ = nullptr, *shift_ = nullptr, *s2_ = nullptr, *out1_ = nullptr, *out2_ = nullptr;
@@ -285,6 +284,7 @@ private:
     int2 *cellBlocks_ = nullptr, *bondBlocks_ = nullptr, *pbinBlocks_ = nullptr;
     int2* partBlocks_ = nullptr;
     int2* tileBlocks_ = nullptr;
+    int2 *edgeBlocks_ = nullptr, *fluidBlocks_ = nullptr;
     int* numPartBlocks_ = nullptr;  // (device) entries of partBlocks_
     std::vector<uint8_t> bondWork_;  // per world: a bonded or barrier cell exists or can appear by fusion
     std::vector<uint8_t> active_;    // per world: included in the launch tables

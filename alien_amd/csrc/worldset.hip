@@ -453,7 +453,10 @@ void WorldSet::freeAll() {
     deviceBytes_ = 0;
 }
 
+// A graph is destroyed when no launch of it is in flight: the particles' kernels go in the middle of a
+// call, with up to 32 steps queued.
 void WorldSet::invalidateGraphs() {
+    if (graph_[0] || graph_[1] || graphMulti_[0] || graphMulti_[1]) (void)hipStreamSynchronize(stream_);
     for (auto* set : {graph_, graphMulti_})
         for (int p = 0; p < 2; ++p)
             if (set[p]) {

@@ -25,7 +25,14 @@ constexpr int kRowPool = 256;  // entries of three consecutive staged rows
 constexpr int kStripMax = 64;
 constexpr int kChunkMax = 8;  // bin rows per neighbour-pass chunk
 constexpr int kClaimFree = 0x7fffffff;
-constexpr uint32_t kMoverBit = 0x80000000u;  // binOf mark of a cell that changed bins
+// binOf: the cell's next bin, counted from its world's first (below 2^28: bins are at least two units wide
+// and worlds span at most 2^30 square units), and in the bits above it how the cell came there: 0 it stayed,
+// 1 to 9 from the bin around in that direction, kFarCode from further
+constexpr int kMoveShift = 28;
+constexpr uint32_t kBinMask = (1u << kMoveShift) - 1u, kFarCode = 15u, kFarMove = kFarCode << kMoveShift;
+constexpr int kGroupBins = 256;    // bins per wave of the cells' map; a world's bins are padded to a multiple
+constexpr int kBinOfPad = 576;     // entries of binOf that may be read (and not used) past the last cell
+constexpr int kSuperGroups = 256;  // groups per sum of groups
 constexpr int kXcdCount = 8;  // XCDs of an MI355X: workgroup b of a launch runs on XCD b % 8
 // Size limits of one world set.  Cell indices, bin offsets and the bond planes ([kMaxBonds][cap],
 // addressed as b * cap + x) are 32-bit ints in the kernels, so a set holds at most
@@ -173,6 +180,16 @@ struct CellExtra {
     uint8_t cellFunction, ancestorMutationId, selected, pad;
 };
 
+// Cells that the map cannot find near their new bin (k_sort.hip): all of them in one list, and a
+// list per bin.
+struct FarCells {
+    int* head;   // [numCellBins] one of the bin's, kNone without any; Ctx::moverNext goes on
+    int* count;  // [numCellBins]
+    int* group;  // [numCellBins / kGroupBins] number in the group's bins
+    int* total;  // entries in the list
+    int2* list;  // [cellCap] (A index, global bin); one array for both steps: read before it is written
+};
+
 struct Ctx {
     int numWorlds;
     int cellCap;  // total cells (= sum of numCells)
@@ -207,26 +224,27 @@ struct Ctx {
     uint32_t* activation;     // cold [cellCap]: activationTime (worlds with livingWork)
     uint32_t* creature;       // cold [cellCap]: creatureId (worlds with livingWork)
     uint8_t* stretched;       // [cellCap] end-of-step staged cell had a bond beyond cellMaxBindingDistance
-    int* binOf;     // [cellCap] global bin of A-cell i, | kMoverBit if it changed bins
+    int* binOf;     // [cellCap] next bin of A-cell i, and how it came there (kBinMask, kMoveShift)
     int* pbinOf;    // [partCap] global bin of A-particle i, -1 if dead
-    // Bin sizes.  Cell bins: written by the map count at the start of every step (the cells that
-    // land in the bin); particle bins: counted with atomics by the kernels that produce the
-    // end-of-step particle positions (and by seeding), brought back to zero by the particle scatter.
+    // Particles per bin: counted with atomics by the kernels that produce the end-of-step particle
+    // positions (and by seeding), brought back to zero by the particle scatter.
     uint32_t* count;      // [numBins] start-of-step state
     uint32_t* countNext;  // [numBins] end-of-step state (next step's `count`)
-    int numCellBins;
-    uint32_t* start;      // [numBins + 1] exclusive scan of this step's map
-    const uint32_t* startPrev;  // [numBins + 1] the last step's map (all zero after seeding)
-    // Cells that change bins ("movers"; after seeding every cell) are listed per new cell bin:
-    // moverHead[bin] is one of them (A index), moverNext[i] the next (kNone ends a list).
-    // moverHeadNext: the lists of the next step (built during this step).
-    int* moverHead;
-    int* moverHeadNext;
-    int* moverNext;  // [cellCap]
-    // per cell bin: movers in minus movers out (cell-bin size = last size + delta)
-    int* delta;
-    int* deltaNext;
-    // one-pass map scan: per tile of bins a status word (flag, launch epoch, sum), the launch epoch
+    int numCellBins;      // cell bins of all worlds, each world's padded to a multiple of kGroupBins
+    int cellCount;        // cells of all worlds
+    const int* groupWorld;  // [numCellBins / kGroupBins] the bins' world
+    // Cells that groups of kGroupBins cell bins, and kSuperGroups of those, gained (or lost) since the
+    // last map; ...Next: for the next step (built during this step)
+    int* groupSum;
+    int* groupSumNext;
+    int* superSum;
+    int* superSumNext;
+    uint32_t* start;      // [numBins + 1] offsets of this step's map (relative to the world's first bin's)
+    const uint32_t* startPrev;  // [numBins + 1] the last step's map
+    // far cells of this step's map, and of the next (entered during this step)
+    FarCells far, farNext;
+    int* moverNext;  // [cellCap] the bin's next far cell (kNone ends a list)
+    // one-pass scan of the particle bins: per tile of bins a status word (flag, launch epoch, sum), the launch epoch
     // and the tile ticket
     unsigned long long* mapStatus;
     uint32_t* mapEpoch;

@@ -2,12 +2,22 @@
 //
 // Replaces ALIEN's CellMap / ParticleMap (source/EngineGpuKernels/Map.cuh:71-280), which insert
 // pointers into a dense world-size grid with atomicCAS chains (cell map) or last-writer-wins
-// stores (particle map).  Here every bin of every world is one counter and one offset.  Cells:
-// the kernels that produce the end-of-step positions record each cell's next bin; at the start of
-// the next step the map count gives every bin its size from the same bin of the last map (the
-// cells that stay) plus the list of cells that moved in, one exclusive scan gives the offsets, and
-// the scatter places every cell at its rank among the bin's cells by previous index (R1), so the
-// map order is the logical order of the step.  Particles: counted with atomics, scattered, then sorted inside their bins.
+// stores (particle map).  Here every bin of every world is one offset.  The cells' map holds them by
+// bin and inside a bin by previous index (R1), so the map order is the logical order of the step.  The
+// kernels that produce the end-of-step positions record each cell's next bin and the direction it went
+// (binOf); the next map finds a bin's cells where they can be: almost all are still in the bin, and a
+// cell that moved comes from one of the eight bins around.  So a wave that builds the map of consecutive
+// bins reads what was recorded for the cells of three stretches of the last map — its own bins, the row
+// above, the row below — and needs no lists.  Where the bins start follows from where they started in the
+// last map and from the cells that changed groups of 256 bins since (groupSum: their numbers, added up by
+// the kernels that record the bins, one atomic per wave and group).  The map takes one launch.
+// (Recording every mover in a list of its new bin and counting it out of the old one cost three
+// device-scope atomics each, which the memory side executes: 40 of 143 us of the fluid pass with 4M
+// cells; clearing those lists and a scan over all bins with tiles that wait for the tiles before them,
+// 34 us more.  Steps then and now: 256k cells 26.5 and 22.1 us, 4M 168 and 139 us, 4M in bodies with
+// bonds 314 and 300 us.  A launch of its own that counts the groups took 18 us at 4M.)
+// Only cells that moved further, or across the torus' edge, or that are in no map yet are entered in a
+// list per bin ("far").  Particles: counted with atomics, scattered, then sorted inside their bins.
 #include "kernels.hpp"
 #include "particle_steps.hpp"
 
@@ -20,16 +30,29 @@ __global__ void k_fill_u32(uint32_t* p, uint32_t v, size_t n) {
 }
 
 // bins of the current state, used after data is set and after introspection: the current state
-// is in no map order yet, so every cell is a mover of the coming step
+// is in no map order yet (every bin of the last map is empty), so every cell is a far one of the
+// coming step
 __global__ void k_cell_bin(Ctx c) {
     int2 blk = c.cellBlocks[blockIdx.x];
     const DevWorld w = c.worlds[blk.x];
     int i = blk.y + int(threadIdx.x);
     if (i >= w.cellOff + w.numCells) return;
-    const int gb = cell_bin_of(w, to_f2(c.A.pos[i]));
-    c.binOf[i] = int(uint32_t(gb) | kMoverBit);
-    push_mover(c.moverHead, c.moverNext, gb, i);
-    atomicAdd(&c.delta[gb], 1);
+    int bx, by;
+    cell_bin_xy(w, to_f2(c.A.pos[i]), bx, by);
+    const int gb = w.binOff + by * w.nbx + bx;
+    c.binOf[i] = int(uint32_t(gb - w.binOff) | kFarMove);
+    c.far.list[i] = make_int2(i, gb);
+    list_far(c.far, c.moverNext, gb, i);
+}
+
+// (the groups gain their far cells)
+__global__ void k_seed_sums(Ctx c) {
+    const int g = int(blockIdx.x) * int(blockDim.x) + int(threadIdx.x);
+    const bool in = g < c.numCellBins / kGroupBins;
+    const int n = in ? c.far.group[g] : 0;
+    if (in) c.groupSum[g] = n;
+    const int sum = wave_last(int(wave_inclusive_scan(uint32_t(n))));  // (of one sum of groups)
+    if (in && g % 64 == 0) atomicAdd(&c.superSum[g / kSuperGroups], sum);
 }
 
 __global__ void k_part_bin(Ctx c) {
@@ -49,69 +72,79 @@ __global__ void k_part_bin(Ctx c) {
     });
 }
 
-constexpr int kScanItems = 8;  // consecutive bins per group of the map scan
+// The bins whose cells can be in bins [b0, b0 + nb) of a world without having moved far: three stretches
+// of bins, above, around and below, disjoint and in order (in narrow worlds they join).
+struct Reach {
+    int lo[3], hi[3];
+};
+__device__ __forceinline__ Reach reach_of(const DevWorld& w, int b0, int nb) {
+    const int n = w.nbx * w.nby;
+    Reach r;
+    r.lo[0] = max(b0 - w.nbx - 1, 0);
+    r.hi[0] = max(min(b0 + nb - w.nbx + 1, b0 - 1), r.lo[0]);
+    r.lo[1] = max(b0 - 1, 0);
+    r.hi[1] = min(b0 + nb + 1, n);
+    r.hi[2] = min(b0 + nb + w.nbx + 1, n);
+    r.lo[2] = min(max(b0 + w.nbx - 1, b0 + nb + 1), r.hi[2]);
+    return r;
+}
+// the same as places in the last map, counted from the world's first cell
+struct Places {
+    int s[3], e[3];
+};
+__device__ __forceinline__ Places places_of(const Reach& r, const uint32_t* prev) {
+    const int base = int(prev[0]);
+    Places p;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        p.s[k] = int(prev[r.lo[k]]) - base;
+        p.e[k] = int(prev[r.hi[k]]) - base;
+    }
+    return p;
+}
 
-// bin sizes base..base+7: a cell bin's size is its size in the last map plus its delta, a particle
-// bin's its count (the cell bins come first; `count` is read for particle bins only)
-__device__ __forceinline__ void load8(const uint32_t* count, const uint32_t* startPrev, const int* delta, int nCell,
-                                      size_t base, int n, uint32_t v[8]) {
-    if (base >= size_t(nCell) && base + 8 <= size_t(n)) {
-        const uint4 a = *reinterpret_cast<const uint4*>(count + base);
-        const uint4 b = *reinterpret_cast<const uint4*>(count + base + 4);
-        v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
-    } else if (base + 8 > size_t(nCell)) {
+__device__ __forceinline__ int world_of(const Ctx& c, int gb) { return c.numWorlds == 1 ? 0 : c.groupWorld[gb / kGroupBins]; }
+__device__ __forceinline__ uint32_t move_of(int x) { return uint32_t(x) >> kMoveShift; }
+// the recorded bin, counted from bin b0
+__device__ __forceinline__ uint32_t bin_from(int x, int b0) { return (uint32_t(x) & kBinMask) - uint32_t(b0); }
+
+// what cells [i0, end) of a world recorded, 64 per round, with all the loads in flight.  The first rounds
+// load without a look at the end (the array goes on beyond it, kBinOfPad).
+template <int kRounds>
+__device__ __forceinline__ void load_rounds(const int* binOf, int i0, int end, int lane, int (&x)[kRounds]) {
+    static_assert(64 * kRounds <= kBinOfPad, "loads beyond the end");
+    const int* at = binOf + i0;
 #pragma unroll
-        for (int k = 0; k < 8; ++k) v[k] = base + k >= size_t(nCell) && base + k < size_t(n) ? count[base + k] : 0u;
-    }
-    if (base >= size_t(nCell)) return;
-    uint32_t sp[9];
-    int dl[8];
-    if (base + 8 <= size_t(nCell)) {
-        const uint4 a = *reinterpret_cast<const uint4*>(startPrev + base);
-        const uint4 b = *reinterpret_cast<const uint4*>(startPrev + base + 4);
-        sp[0] = a.x, sp[1] = a.y, sp[2] = a.z, sp[3] = a.w, sp[4] = b.x, sp[5] = b.y, sp[6] = b.z, sp[7] = b.w;
-        sp[8] = startPrev[base + 8];
-        const int4 c0 = *reinterpret_cast<const int4*>(delta + base);
-        const int4 c1 = *reinterpret_cast<const int4*>(delta + base + 4);
-        dl[0] = c0.x, dl[1] = c0.y, dl[2] = c0.z, dl[3] = c0.w, dl[4] = c1.x, dl[5] = c1.y, dl[6] = c1.z, dl[7] = c1.w;
-    } else {
-        // (the end of the last cell bin is the start of the particle bins)
-#pragma unroll
-        for (int k = 0; k < 9; ++k) sp[k] = base + k <= size_t(nCell) ? startPrev[base + k] : 0u;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) dl[k] = base + k < size_t(nCell) ? delta[base + k] : 0;
-    }
-#pragma unroll
-    for (int k = 0; k < 8; ++k)
-        if (base + k < size_t(nCell)) v[k] = uint32_t(int(sp[k + 1] - sp[k]) + dl[k]);
+    for (int q = 0; q < kRounds; ++q)
+        if (q < kRounds - 1 || i0 + 64 * q < end) x[q] = at[lane + 64 * q];
 }
 
 // ---------------------------------------------------------------------------------------------
-// Offsets of a step's map in one pass over the bins.  Every workgroup takes the next tile of 8192
-// bins (tickets in the order the workgroups start), sums its bin sizes and publishes the sum, then
-// finds the sum of all bins before it by looking back over what the tiles before it published
-// (decoupled look-back: a tile publishes its own sum before it looks back, and every tile before
-// it holds an earlier ticket and has started, so each wait ends).  With that it writes the offsets
-// of its bins.  It also empties the next step's deltas and mover lists of its cell bins (their
-// last readers ran a step ago), and the first tile opens the step: clears the per-step list
-// counters and advances the worlds' timesteps if asked (a step without bond work has no later
-// reader of them).  `count` stays: the particle scatter counts its particle bins down to zero,
-// which leaves them cleared for the step after next (the two histograms alternate).
+// Offsets of the particle bins in one pass: a workgroup takes the next tile of bins (tickets in the order
+// the workgroups start), sums its bins up and publishes the sum, then finds the sum of all bins before
+// it by looking back over what the tiles before it published (decoupled look-back: a tile publishes its
+// own sum before it looks back, and every tile before it holds an earlier ticket and has started, so each
+// wait ends).  `count` stays: the particle scatter counts its bins down to zero, which leaves them
+// cleared for the step after next (the two histograms alternate).
 // ---------------------------------------------------------------------------------------------
-constexpr int kMapScanThreads = 1024;
-constexpr int kScanGroups = 1;  // groups of kScanItems consecutive bins per thread (2 measured slower)
-constexpr int kMapScanTile = kMapScanThreads * kScanGroups * kScanItems;
+constexpr int kScanItems = 8;  // consecutive particle bins per thread
+constexpr int kMapThreads = 256;
+constexpr int kPartScanTile = kMapThreads * kScanItems;
 // tile status word: flag (bits 62-63: 1 the tile's sum, 2 the sum up to and including the tile),
 // launch epoch (bits 32-61), value (bits 0-31)
 constexpr unsigned long long kTileSum = 1ull << 62, kTileInclusive = 2ull << 62;
 constexpr uint32_t kEpochMask = 0x3fffffffu;
 constexpr int kLookBackSpins = 1 << 22;  // far beyond any wait for a running tile
 
+// Workgroup b runs on XCD b % 8: of `blocks` (a multiple of 8) each XCD gets one contiguous run, so the
+// rows that neighbouring waves share stay in its L2
+__device__ __forceinline__ int xcd_run(int b, int blocks) { return (b % kXcdCount) * (blocks / kXcdCount) + b / kXcdCount; }
+
 __device__ __forceinline__ bool tile_status_ready(unsigned long long w, uint32_t epoch) {
     return (w >> 62) != 0ull && uint32_t((w >> 32) & kEpochMask) == epoch;
 }
 
-__global__ void __launch_bounds__(kMapScanThreads) k_map_scan(Ctx c, int tiles, StepCounters* open, int advance) {
+__device__ __forceinline__ void part_scan(const Ctx& c, int tiles) {
     __shared__ int sTile;
     __shared__ uint32_t sEpoch, sPrefix;
     const int tid = int(threadIdx.x), lane = tid & 63;
@@ -129,16 +162,20 @@ __global__ void __launch_bounds__(kMapScanThreads) k_map_scan(Ctx c, int tiles, 
     const int tile = sTile;
     const uint32_t epoch = sEpoch;
     const unsigned long long ep = (unsigned long long)epoch << 32;
-    const int n = c.numBins, nCell = c.numCellBins;
-    const size_t base0 = size_t(tile) * kMapScanTile + size_t(tid) * (kScanGroups * kScanItems);
-    uint32_t v[kScanGroups][kScanItems];
+    const uint32_t n = uint32_t(c.numBins);
+    const uint32_t base = uint32_t(c.numCellBins) + uint32_t(tile) * uint32_t(kPartScanTile) + uint32_t(tid * kScanItems);
+    uint32_t v[kScanItems];
+    if (base + 8 <= n) {
+        const uint4 a = *reinterpret_cast<const uint4*>(c.count + base);
+        const uint4 b = *reinterpret_cast<const uint4*>(c.count + base + 4);
+        v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+    } else {
 #pragma unroll
-    for (int g = 0; g < kScanGroups; ++g) load8(c.count, c.startPrev, c.delta, nCell, base0 + g * kScanItems, n, v[g]);
+        for (int k = 0; k < kScanItems; ++k) v[k] = base + k < n ? c.count[base + k] : 0u;
+    }
     uint32_t s = 0;
 #pragma unroll
-    for (int g = 0; g < kScanGroups; ++g)
-#pragma unroll
-        for (int k = 0; k < kScanItems; ++k) s += v[g][k];
+    for (int k = 0; k < kScanItems; ++k) s += v[k];
     uint32_t total;
     const uint32_t off = block_exclusive_scan(s, total);
     if (tid == 0)
@@ -179,53 +216,25 @@ __global__ void __launch_bounds__(kMapScanThreads) k_map_scan(Ctx c, int tiles, 
         }
         if (lane == 0) sPrefix = prefix;
     }
-    // the next step's deltas and mover lists start empty
-#pragma unroll
-    for (int g = 0; g < kScanGroups; ++g) {
-        const size_t base = base0 + g * kScanItems;
-        if (base + 8 <= size_t(nCell)) {
-            *reinterpret_cast<int4*>(c.deltaNext + base) = make_int4(0, 0, 0, 0);
-            *reinterpret_cast<int4*>(c.deltaNext + base + 4) = make_int4(0, 0, 0, 0);
-            *reinterpret_cast<int4*>(c.moverHeadNext + base) = make_int4(kNone, kNone, kNone, kNone);
-            *reinterpret_cast<int4*>(c.moverHeadNext + base + 4) = make_int4(kNone, kNone, kNone, kNone);
-        } else {
-#pragma unroll
-            for (int k = 0; k < 8; ++k)
-                if (base + k < size_t(nCell)) {
-                    c.deltaNext[base + k] = 0;
-                    c.moverHeadNext[base + k] = kNone;
-                }
-        }
-    }
-    if (tile == 0) {
-        if (open && tid == 0) {
-            open->candidates = 0;
-            open->liveParticles = 0;
-        }
-        if (advance)
-            for (int wi = tid; wi < c.numWorlds; wi += kMapScanThreads) c.ctr[wi].timestep += 1ull;
-    }
     __syncthreads();
-    uint32_t o = sPrefix + off;
+    // (a particle bin's offset counts from its world's first; the first bin's is also the end of the
+    // last cell bin)
+    uint32_t o = uint32_t(c.cellCount) + sPrefix + off;
+    uint32_t st8[kScanItems];
 #pragma unroll
-    for (int g = 0; g < kScanGroups; ++g) {
-        const size_t base = base0 + g * kScanItems;
-        uint32_t st8[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            st8[k] = o;
-            o += v[g][k];
-        }
-        if (base + 8 <= size_t(n)) {
-            *reinterpret_cast<uint4*>(c.start + base) = make_uint4(st8[0], st8[1], st8[2], st8[3]);
-            *reinterpret_cast<uint4*>(c.start + base + 4) = make_uint4(st8[4], st8[5], st8[6], st8[7]);
-        } else {
-#pragma unroll
-            for (int k = 0; k < 8; ++k)
-                if (base + k < size_t(n)) c.start[base + k] = st8[k];
-        }
-        if (base <= size_t(n - 1) && size_t(n - 1) < base + 8) c.start[n] = o;
+    for (int k = 0; k < kScanItems; ++k) {
+        st8[k] = o;
+        o += v[k];
     }
+    if (base + 8 <= n) {
+        *reinterpret_cast<uint4*>(c.start + base) = make_uint4(st8[0], st8[1], st8[2], st8[3]);
+        *reinterpret_cast<uint4*>(c.start + base + 4) = make_uint4(st8[4], st8[5], st8[6], st8[7]);
+    } else {
+#pragma unroll
+        for (int k = 0; k < kScanItems; ++k)
+            if (base + k < n) c.start[base + k] = st8[k];
+    }
+    if (base < n && n <= base + kScanItems) c.start[n] = o;
     // the last ticket: every ticket is gone; reset the ticket and advance the epoch for the next
     // launch
     if (tile == tiles - 1 && tid == 0) {
@@ -234,111 +243,354 @@ __global__ void __launch_bounds__(kMapScanThreads) k_map_scan(Ctx c, int tiles, 
     }
 }
 
-// Map scatter: cell i (A index, i.e. its place in the last map) goes to its bin at its rank by A
-// index among the bin's cells (R1).  The bin's stayers hold their places of the last map's bin in
-// order, so a stayer's rank among them is its place in that bin minus the movers that left the bin
-// before it (marked lanes of the wave, and cells of the bin in earlier waves), and a mover from a
-// lower place precedes them all, one from a higher place follows them all; every cell then adds
-// the bin's movers with a smaller A index.  A workgroup places the cells of kScatterRuns entries of
-// the cell block table, one cell of each per thread, with the loads of each phase issued for all
-// of them together (the pass is a chain of dependent loads: bin, then the bin's offsets and mover
-// list, then the store).
-constexpr int kScatterRuns = 4;
-
-__device__ __forceinline__ void cell_scatter(const Ctx& c, int block, int tableBlocks) {
-    const int lane = int(threadIdx.x) & 63;
-    const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    int i[kScatterRuns], bo[kScatterRuns], wi[kScatterRuns], cellOff[kScatterRuns], binOff[kScatterRuns];
-    bool active[kScatterRuns];
-#pragma unroll
-    for (int q = 0; q < kScatterRuns; ++q) {
-        const int e = block * kScatterRuns + q;
-        const int2 blk = e < tableBlocks ? c.cellBlocks[e] : make_int2(0, 0);
-        const DevWorld& w = c.worlds[blk.x];
-        wi[q] = blk.x;
-        cellOff[q] = w.cellOff;
-        binOff[q] = w.binOff;
-        i[q] = blk.y + int(threadIdx.x);
-        active[q] = e < tableBlocks && i[q] < w.cellOff + w.numCells;
-        bo[q] = active[q] ? c.binOf[i[q]] : 0;
-    }
-    int gb[kScatterRuns], s[kScatterRuns], e[kScatterRuns], head[kScatterRuns], dest0[kScatterRuns];
-    unsigned long long movers[kScatterRuns];
-#pragma unroll
-    for (int q = 0; q < kScatterRuns; ++q) {
-        const bool mover = (uint32_t(bo[q]) & kMoverBit) != 0u;
-        movers[q] = __ballot(active[q] && mover);
-        gb[q] = int(uint32_t(bo[q]) & ~kMoverBit);
-        const uint32_t spBase = c.startPrev[binOff[q]], stBase = c.start[binOff[q]];
-        const int g = active[q] ? gb[q] : binOff[q];
-        s[q] = cellOff[q] + int(c.startPrev[g] - spBase);
-        e[q] = cellOff[q] + int(c.startPrev[g + 1] - spBase);
-        head[q] = active[q] ? c.moverHead[g] : kNone;
-        dest0[q] = cellOff[q] + int(c.start[g] - stBase);
-    }
-    int rank[kScatterRuns];
-#pragma unroll
-    for (int q = 0; q < kScatterRuns; ++q) {
-        rank[q] = 0;
-        if (!active[q]) continue;
-        const int iq = i[q], i0 = iq - lane;  // the wave's first cell
-        if ((uint32_t(bo[q]) & kMoverBit) == 0u) {
-            // a stayer: s <= i < e
-            const int from = max(s[q], i0) - i0;
-            const unsigned long long fromMask = from >= 64 ? 0ull : ~((1ull << from) - 1ull);
-            int left = __builtin_popcountll(movers[q] & below & fromMask);
-            for (int j = s[q]; j < i0; ++j) left += (uint32_t(c.binOf[j]) & kMoverBit) ? 1 : 0;
-            rank[q] = (iq - s[q]) - left;
-        } else if (iq >= e[q]) {
-            for (int j = s[q]; j < e[q]; ++j) rank[q] += c.binOf[j] == gb[q] ? 1 : 0;
-        }
-    }
-    // the bins' mover lists, walked side by side (one load per list in flight per round)
-    int jw[kScatterRuns];
-#pragma unroll
-    for (int q = 0; q < kScatterRuns; ++q) jw[q] = active[q] ? head[q] : kNone;
-    for (;;) {
-        bool more = false;
-#pragma unroll
-        for (int q = 0; q < kScatterRuns; ++q)
-            if (jw[q] != kNone) {
-                rank[q] += jw[q] < i[q] ? 1 : 0;
-                more = true;
-            }
-        if (!more) break;
-#pragma unroll
-        for (int q = 0; q < kScatterRuns; ++q) jw[q] = jw[q] != kNone ? c.moverNext[jw[q]] : kNone;
-    }
-#pragma unroll
-    for (int q = 0; q < kScatterRuns; ++q) {
-        if (!active[q]) continue;
-        const int iq = i[q];
-        const int dest = dest0[q] + rank[q];
-        c.sorted[dest] = iq;
-        // the row-staged collision pass reads a copy of the state in map order; the fluid pass
-        // reads the state through `sorted` (a copy for it costs the scatter more than it saves)
-        if (c.params[wi[q]].motion != 0) {
-            c.mpos[dest] = c.A.pos[iq];
-            c.mvel[dest] = c.A.vel[iq];
-            c.mflags[dest] = c.A.flags[iq];
-        }
-        if (c.partStage > 0) part_scatter_staged(c, c.worlds[wi[q]], iq);
-    }
-}
-
-// One launch scatters the cells and, on workgroups of their own (first, so that they start with the
-// cells), the live particles; a cell's thread also takes the particle it emitted this step.  Both need
-// only the scan.  (As launches of their own on a second stream the two particle scatters cost 20 us of
-// the particle chain of a radiating world of 1M cells, which is longer than its fluid pass.)
-__global__ void k_scatter(Ctx c, int partBlocks, int tableBlocks) {
-    const int b = int(blockIdx.x);
-    if (b < partBlocks)
-        part_scatter(c, {b, partBlocks});
-    else
-        cell_scatter(c, b - partBlocks, tableBlocks);
-}
-
 // ---------------------------------------------------------------------------------------------
+// The cells' map.  One wave per group puts every cell of its bins at its rank by A index, i.e. by its place
+// in the last map (R1).  It goes over the bins' reach in that order, 64 cells at a time, with the first
+// rounds' loads of all three stretches in flight together: the wave is a chain of latencies (table,
+// offsets, cells, stores; 9 us at 1024 waves, 33 us at 16384, where the VALU's share is 15).  Each XCD
+// takes one run of groups (the rows that neighbouring waves share: 7 of 40 us).
+//  - The bins' own cells that left are counted per bin; the near movers into the bins are counted and, met
+//    in order, listed in LDS.  That gives the bins' sizes, and with the groups before it their offsets.
+//  - The bins' own cells that stayed hold their old order: a stayer's rank is its place in the bin's
+//    old stretch, minus the cells that left the bin before it, plus the movers into it from lower places.
+//  - A listed mover from a lower place comes behind the listed ones of its bin before it, one from a
+//    higher place behind the stayers as well.  If there are more than the list holds, another run over
+//    the reach places them.
+// Far cells (few, but all of them after seeding) are placed by waves of their own: the cells of the
+// target's group before it are counted over the group's reach, the far ones of its bin along the list;
+// near cells of a bin with a far list add the list's smaller indices.
+// ---------------------------------------------------------------------------------------------
+constexpr int kMapWaves = kMapThreads / 64;
+constexpr int kScatterList = 192;  // movers into a group's bins listed (typically 5 to 25)
+constexpr int kScatterRounds = 5;  // rounds of a stretch loaded at once (258 bins at up to 1.24 cells per bin)
+constexpr int kFarBlocks = 1024;   // workgroups for the far cells, at most
+static_assert(kGroupBins == 4 * 64, "four bins per lane");
+
+struct ScatterShared {
+    int prev[kGroupBins + 4];  // places in the last map, counted from the world's first cell
+    union {
+        int start[kGroupBins + 4];  // the same in the new map
+        uint32_t out[kGroupBins];   // before it is known: cells that left the bin
+    };
+    uint32_t before[kGroupBins], after[kGroupBins];  // near movers into the bin from lower and higher places
+    union {
+        int2 list[kScatterList];   // (A index in the world, bin)
+        uint32_t met[kGroupBins];  // movers placed so far (the other run)
+    };
+};
+
+// cells that the world's groups before global group g gained since the last map
+__device__ __forceinline__ int gained_before(const Ctx& c, const DevWorld& w, int g, int lane) {
+    const int first = w.binOff / kGroupBins;
+    const int s0 = (first + kSuperGroups - 1) / kSuperGroups, s1 = g / kSuperGroups;
+    int n = 0;
+    if (s0 < s1) {
+        for (int k = first + lane; k < s0 * kSuperGroups; k += 64) n += c.groupSum[k];
+        for (int k = s0 + lane; k < s1; k += 64) n += c.superSum[k];
+        for (int k = s1 * kSuperGroups + lane; k < g; k += 64) n += c.groupSum[k];
+    } else {
+        for (int k = first + lane; k < g; k += 64) n += c.groupSum[k];
+    }
+    return wave_last(int(wave_inclusive_scan(uint32_t(n))));
+}
+
+// the next step's sums, and the far lists of the group's bins where there are any, start empty (their last
+// readers ran a step ago)
+__device__ __forceinline__ void clear_next(const Ctx& c, int g, int lane) {
+    if (lane == 0) {
+        c.groupSumNext[g] = 0;
+        if (g % kSuperGroups == 0) c.superSumNext[g / kSuperGroups] = 0;
+    }
+    if (c.farNext.group[g] == 0) return;
+    reinterpret_cast<int4*>(c.farNext.count + g * kGroupBins)[lane] = make_int4(0, 0, 0, 0);
+    reinterpret_cast<int4*>(c.farNext.head + g * kGroupBins)[lane] = make_int4(kNone, kNone, kNone, kNone);
+    if (lane == 0) c.farNext.group[g] = 0;
+}
+
+// far cells of global bin gb with A index below i
+__device__ __forceinline__ int rank_far(const Ctx& c, int gb, int i) {
+    int n = 0;
+    for (int j = c.far.head[gb]; j != kNone; j = c.moverNext[j]) n += j < i ? 1 : 0;
+    return n;
+}
+
+__device__ __forceinline__ void place_cell(const Ctx& c, const DevWorld& w, bool copies, int i, int dest) {
+    const int a = w.cellOff + i, d = w.cellOff + dest;
+    st32(c.sorted, uint32_t(d), a);
+    // the row-staged collision pass reads a copy of the state in map order; the fluid pass
+    // reads the state through `sorted` (a copy for it costs the scatter more than it saves)
+    if (copies) {
+        st32(c.mpos, uint32_t(d), ld32(c.A.pos, uint32_t(a)));
+        st32(c.mvel, uint32_t(d), ld32(c.A.vel, uint32_t(a)));
+        st32(c.mflags, uint32_t(d), ld32(c.A.flags, uint32_t(a)));
+    }
+}
+
+__device__ __forceinline__ void far_scatter(const Ctx& c, int wave, int waves, int lane) {
+    const int total = *c.far.total;
+    for (int q = wave; q < total; q += waves) {
+        const int2 f = c.far.list[q];
+        if (f.y < 0) continue;  // (seeded while its world was left out)
+        const int wi = world_of(c, f.y);
+        const DevWorld& w = c.worlds[wi];
+        if (!w.active) continue;
+        const int g = f.y / kGroupBins, b0 = g * kGroupBins - w.binOff;
+        const uint32_t t = uint32_t(f.y - w.binOff - b0);
+        const int i = f.x - w.cellOff;
+        const uint32_t* prev = c.startPrev + w.binOff;
+        const Places p = places_of(reach_of(w, b0, min(kGroupBins, w.nbx * w.nby - b0)), prev);
+        const int* binOf = c.binOf + w.cellOff;
+        const int4 fc = reinterpret_cast<const int4*>(c.far.count + g * kGroupBins)[lane];
+        const int base = int(prev[b0] - prev[0]) + gained_before(c, w, g, lane);
+        const uint32_t b = uint32_t(4 * lane);
+        uint32_t n = (b < t ? uint32_t(fc.x) : 0u) + (b + 1u < t ? uint32_t(fc.y) : 0u) + (b + 2u < t ? uint32_t(fc.z) : 0u) +
+                     (b + 3u < t ? uint32_t(fc.w) : 0u);
+        for (int k = 0; k < 3; ++k)
+            for (int j0 = p.s[k]; j0 < p.e[k]; j0 += 256) {
+                int x[4];
+                load_rounds(binOf, j0, p.e[k], lane, x);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const uint32_t u = move_of(x[r]) == kFarCode ? ~0u : bin_from(x[r], b0);
+                    n += j0 + 64 * r + lane < p.e[k] && (u < t || (u == t && j0 + 64 * r + lane < i)) ? 1u : 0u;
+                }
+            }
+        const int at = base + wave_last(int(wave_inclusive_scan(n))) + rank_far(c, f.y, f.x);
+        if (lane == 0) place_cell(c, w, c.params[wi].motion != 0, i, at);
+    }
+}
+
+__device__ __forceinline__ void cell_scatter(const Ctx& c, ScatterShared& S, int g, int lane) {
+    const int g0 = g * kGroupBins;
+    if (g0 >= c.numCellBins) return;
+    const int wi = world_of(c, g0);
+    const DevWorld& w = c.worlds[wi];
+    const int b0 = g0 - w.binOff, bins = w.nbx * w.nby;
+    const uint32_t* prev = c.startPrev + w.binOff;
+    const int prevBase = int(prev[0]);
+    const uint4 pv = *reinterpret_cast<const uint4*>(prev + b0 + 4 * lane);
+    const uint32_t pvEnd = prev[b0 + kGroupBins];
+    uint4* startOut = reinterpret_cast<uint4*>(c.start + g0) + lane;
+    const bool last = g0 + kGroupBins == c.numCellBins;  // its end is stored too
+    clear_next(c, g, lane);
+    if (!w.active || b0 >= bins) {
+        // a world left out keeps its map; padding ends with the world
+        const uint32_t d = uint32_t(w.cellOff - prevBase), end = uint32_t(w.cellOff + w.numCells);
+        *startOut = w.active ? make_uint4(end, end, end, end) : make_uint4(pv.x + d, pv.y + d, pv.z + d, pv.w + d);
+        if (last && lane == 0) c.start[c.numCellBins] = end;
+        return;
+    }
+    const int nb = min(kGroupBins, bins - b0);
+    const int p0 = int(prev[b0]) - prevBase, p1 = int(prev[b0 + nb]) - prevBase;  // the bins' own cells
+    const Places p = places_of(reach_of(w, b0, nb), prev);
+    const bool copies = c.params[wi].motion != 0;
+    const int farCells = c.far.group[g];
+    const int* binOf = c.binOf + w.cellOff;
+    const int base = p0 + gained_before(c, w, g, lane);
+    int x[3][kScatterRounds];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) load_rounds(binOf, p.s[k], p.e[k], lane, x[k]);
+    reinterpret_cast<int4*>(S.prev)[lane] =
+        make_int4(int(pv.x) - prevBase, int(pv.y) - prevBase, int(pv.z) - prevBase, int(pv.w) - prevBase);
+    if (lane == 0) S.prev[kGroupBins] = int(pvEnd) - prevBase;
+    reinterpret_cast<uint4*>(S.out)[lane] = make_uint4(0u, 0u, 0u, 0u);
+    reinterpret_cast<uint4*>(S.before)[lane] = make_uint4(0u, 0u, 0u, 0u);
+    reinterpret_cast<uint4*>(S.after)[lane] = make_uint4(0u, 0u, 0u, 0u);
+    __syncwarp();
+    int listed = 0;  // movers into the bins so far (listed up to the list's size)
+    // cells i0 + lane of the stretch around the bins (k == 1), above or below: what they recorded
+    auto meet = [&](int k, int y, int i0) {
+        if (i0 >= p.e[k]) return;
+        const int i = i0 + lane;
+        const uint32_t move = move_of(y), t = bin_from(y, b0);
+        const bool into = i < p.e[k] && move != 0u && move != kFarCode && t < uint32_t(nb);
+        if (k == 1 && move != 0u && i >= p0 && i < p1) {
+            int old;
+            if (move != kFarCode) {
+                old = int(t) - move_bins(w, move);
+            } else {  // the last bin that starts at or before the cell
+                old = 0;
+#pragma unroll
+                for (int s = kGroupBins / 2; s > 0; s >>= 1)
+                    if (S.prev[old + s] <= i) old += s;
+            }
+            atomicAdd(&S.out[old], 1u);
+        }
+        const unsigned long long m = __ballot(into);
+        if (m == 0ull) return;
+        if (into) {
+            atomicAdd(k == 0 || (k == 1 && i < S.prev[t]) ? &S.before[t] : &S.after[t], 1u);
+            const int q = int(__builtin_amdgcn_mbcnt_hi(uint32_t(m >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(m), uint32_t(listed))));
+            if (q < kScatterList) S.list[q] = make_int2(i, int(t));
+        }
+        listed += __builtin_popcountll(m);
+    };
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+#pragma unroll
+        for (int q = 0; q < kScatterRounds; ++q) meet(k, x[k][q], p.s[k] + 64 * q);
+        for (int i0 = p.s[k] + 64 * kScatterRounds; i0 < p.e[k]; i0 += 256) {
+            int y[4];
+            load_rounds(binOf, i0, p.e[k], lane, y);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) meet(k, y[q], i0 + 64 * q);
+        }
+    }
+    __syncwarp();
+    // sizes and offsets
+    {
+        const uint4 o = reinterpret_cast<const uint4*>(S.out)[lane];
+        const uint4 f = reinterpret_cast<const uint4*>(S.before)[lane], a = reinterpret_cast<const uint4*>(S.after)[lane];
+        const int next = S.prev[4 * lane + 4];
+        uint32_t v[4] = {pv.y - pv.x - o.x + f.x + a.x, pv.z - pv.y - o.y + f.y + a.y, pv.w - pv.z - o.z + f.z + a.z,
+                         uint32_t(next + prevBase) - pv.w - o.w + f.w + a.w};
+        if (farCells) {
+            const int4 fc = *reinterpret_cast<const int4*>(c.far.count + g0 + 4 * lane);
+            v[0] += uint32_t(fc.x), v[1] += uint32_t(fc.y), v[2] += uint32_t(fc.z), v[3] += uint32_t(fc.w);
+        }
+        const uint32_t sum = v[0] + v[1] + v[2] + v[3];
+        const int s0 = base + int(wave_inclusive_scan(sum) - sum);
+        const int4 s = make_int4(s0, s0 + int(v[0]), s0 + int(v[0] + v[1]), s0 + int(v[0] + v[1] + v[2]));
+        reinterpret_cast<int4*>(S.start)[lane] = s;
+        const uint32_t off = uint32_t(w.cellOff);
+        *startOut = make_uint4(off + uint32_t(s.x), off + uint32_t(s.y), off + uint32_t(s.z), off + uint32_t(s.w));
+        if (lane == 63) {
+            S.start[kGroupBins] = s0 + int(sum);
+            if (last) c.start[c.numCellBins] = off + uint32_t(w.numCells);
+        }
+    }
+    __syncwarp();
+    const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    unsigned long long leftPrev = 0ull;  // the round before: own cells that left their bin
+    int longStart = -1, longGone = 0;    // the bin that reaches into this round: its cells that left before it
+    auto stay = [&](int y, int i0) {
+        const int i = i0 + lane;
+        const bool own = i >= p0 && i < p1;
+        const uint32_t move = move_of(y), t = bin_from(y, b0);
+        const unsigned long long left = __ballot(own && move != 0u);
+        const bool stays = own && move == 0u;
+        const int sb = stays ? S.prev[t] : i0;
+        const unsigned long long old = __ballot(sb < i0);
+        if (old) {  // (all of one bin)
+            const int from = __builtin_amdgcn_readlane(sb, __builtin_ctzll(old));
+            if (from != longStart) {
+                longStart = from;
+                longGone = __builtin_popcountll(from > i0 - 64 ? leftPrev >> (from - (i0 - 64)) : leftPrev);
+                for (int j0 = from; j0 < i0 - 64; j0 += 64) {
+                    const int j = j0 + lane;
+                    longGone += __builtin_popcountll(__ballot(j < i0 - 64 && move_of(binOf[min(j, i0)]) != 0u));
+                }
+            }
+        }
+        if (stays) {
+            const int gone = sb < i0 ? longGone + __builtin_popcountll(left & below)
+                                     : __builtin_popcountll(left & below & ~((1ull << (sb - i0)) - 1ull));
+            int rank = i - sb - gone + int(S.before[t]);
+            if (farCells) rank += rank_far(c, g0 + int(t), w.cellOff + i);
+            place_cell(c, w, copies, i, S.start[t] + rank);
+        }
+        longGone += __builtin_popcountll(left);
+        leftPrev = left;
+    };
+#pragma unroll
+    for (int q = 0; q < kScatterRounds; ++q)
+        if (p.s[1] + 64 * q < p1) stay(x[1][q], p.s[1] + 64 * q);
+    for (int i0 = p.s[1] + 64 * kScatterRounds; i0 < p1; i0 += 256) {
+        int y[4];
+        load_rounds(binOf, i0, p1, lane, y);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (i0 + 64 * q < p1) stay(y[q], i0 + 64 * q);
+    }
+    // a mover's place, n: movers into its bin before it
+    auto place_mover = [&](int i, int t, int n) {
+        int at = S.start[t] + n;
+        if (i >= S.prev[t]) {  // behind the stayers
+            at += S.start[t + 1] - S.start[t] - int(S.before[t] + S.after[t]);
+            if (farCells) at -= c.far.count[g0 + t];
+        }
+        if (farCells) at += rank_far(c, g0 + t, w.cellOff + i);
+        place_cell(c, w, copies, i, at);
+    };
+    if (listed <= kScatterList) {
+        for (int q0 = 0; q0 < listed; q0 += 64) {
+            const int q = q0 + lane;
+            const bool on = q < listed;
+            const int2 m = S.list[on ? q : 0];
+            int n = 0;
+            // (few bins get more than one)
+            if (__ballot(on && S.before[m.y] + S.after[m.y] > 1u)) {
+                const int end = min(listed, q0 + 64);
+                for (int j = 0; j < end; ++j) n += S.list[j].y == m.y && j < q ? 1 : 0;
+            }
+            if (on) place_mover(m.x, m.y, n);
+        }
+        return;
+    }
+    reinterpret_cast<uint4*>(S.met)[lane] = make_uint4(0u, 0u, 0u, 0u);
+    __syncwarp();
+    for (int k = 0; k < 3; ++k)
+        for (int i0 = p.s[k]; i0 < p.e[k]; i0 += 64) {
+            const int i = i0 + lane;
+            const int y = binOf[min(i, p.e[k] - 1)];
+            const uint32_t move = move_of(y), t = bin_from(y, b0);
+            const bool into = i < p.e[k] && move != 0u && move != kFarCode && t < uint32_t(nb);
+            for (unsigned long long m = __ballot(into); m != 0ull;) {
+                const uint32_t tm = uint32_t(__builtin_amdgcn_readlane(int(t), __builtin_ctzll(m)));
+                const unsigned long long same = __ballot(into && t == tm);
+                const uint32_t n = S.met[tm];
+                __syncwarp();
+                if (into && t == tm) {
+                    const int earlier = __builtin_popcountll(same & below);
+                    if (earlier == 0) S.met[tm] = n + uint32_t(__builtin_popcountll(same));
+                    place_mover(i, int(t), int(n) + earlier);
+                }
+                __syncwarp();
+                m &= ~same;
+            }
+        }
+}
+
+__device__ __forceinline__ void particles_to_bins(const Ctx& c, int b, int partBlocks) {
+    if (b < partBlocks) return part_scatter(c, {b, partBlocks});
+    // the particles that cells emitted this step
+    const int2 blk = c.cellBlocks[b - partBlocks];
+    const DevWorld& w = c.worlds[blk.x];
+    const int i = blk.y + int(threadIdx.x);
+    if (i < w.cellOff + w.numCells) part_scatter_staged(c, w, i);
+}
+__global__ void k_part_scatter(Ctx c, int partBlocks) { particles_to_bins(c, int(blockIdx.x), partBlocks); }
+__global__ void __launch_bounds__(kMapThreads) k_part_scan(Ctx c, int tiles) { part_scan(c, tiles); }
+
+// The map of a step, on workgroups of one launch: the cells, the far cells, and of the particles the offsets of
+// their bins (scanTiles) or, where those were found before, their places (partBlocks live ones,
+// stagedBlocks the cells' emitted ones).  It opens the
+// step: clears the per-step list counters and advances the worlds' timesteps if asked (a step without
+// bond work has no later reader of them).
+__global__ void __launch_bounds__(kMapThreads)
+k_map(Ctx c, int scanTiles, int partBlocks, int stagedBlocks, int groupBlocks, int farBlocks, StepCounters* open, int advance) {
+    __shared__ __align__(16) ScatterShared S[kMapWaves];
+    int b = int(blockIdx.x);
+    const int tid = int(threadIdx.x), lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = int(blockDim.x) >> 6;
+    if (b == 0) {
+        if (tid == 0) *c.farNext.total = 0;
+        if (open && tid == 0) {
+            open->candidates = 0;
+            open->liveParticles = 0;
+        }
+        if (advance)
+            for (int wi = tid; wi < c.numWorlds; wi += int(blockDim.x)) c.ctr[wi].timestep += 1ull;
+    }
+    if (b < scanTiles) return part_scan(c, scanTiles);
+    b -= scanTiles;
+    if (b < groupBlocks) return cell_scatter(c, S[wave], xcd_run(b, groupBlocks) * waves + wave, lane);
+    b -= groupBlocks;
+    if (b < partBlocks + stagedBlocks) return particles_to_bins(c, b, partBlocks);
+    b -= partBlocks + stagedBlocks;
+    if (b < farBlocks) far_scatter(c, b * waves + wave, farBlocks * waves, lane);
+}
+
 void launch_fill_u32(uint32_t* p, uint32_t v, size_t n, hipStream_t s) {
     if (n == 0) return;
     size_t g = (n + 255) / 256;
@@ -347,28 +599,44 @@ void launch_fill_u32(uint32_t* p, uint32_t v, size_t n, hipStream_t s) {
 }
 
 void launch_seed_bins(const Ctx& c, const LaunchShape& sh, hipStream_t s) {
-    // no last map (every bin of it empty), every cell a mover of the coming step
+    // no last map (every bin of it empty), every cell a far one of the coming step
     launch_fill_u32(const_cast<uint32_t*>(c.startPrev), 0u, size_t(c.numBins) + 1, s);
-    launch_fill_u32(reinterpret_cast<uint32_t*>(c.moverHead), uint32_t(kNone), size_t(c.numCellBins), s);
-    launch_fill_u32(reinterpret_cast<uint32_t*>(c.delta), 0u, size_t(c.numCellBins), s);
+    launch_fill_u32(reinterpret_cast<uint32_t*>(c.far.head), uint32_t(kNone), size_t(c.numCellBins), s);
+    launch_fill_u32(reinterpret_cast<uint32_t*>(c.far.count), 0u, size_t(c.numCellBins), s);
+    launch_fill_u32(reinterpret_cast<uint32_t*>(c.far.group), 0u, size_t(c.numCellBins / kGroupBins), s);
+    launch_fill_u32(reinterpret_cast<uint32_t*>(c.far.list), 0xffffffffu, 2 * size_t(c.cellCount), s);
+    launch_fill_u32(reinterpret_cast<uint32_t*>(c.far.total), uint32_t(c.cellCount), 1, s);
+    launch_fill_u32(reinterpret_cast<uint32_t*>(c.superSum), 0u, size_t(c.numCellBins / kGroupBins / kSuperGroups + 1), s);
     if (sh.cellBlocks) hipLaunchKernelGGL(k_cell_bin, dim3(sh.cellBlocks), dim3(sh.cellThreads), 0, s, c);
+    if (c.numCellBins) hipLaunchKernelGGL(k_seed_sums, dim3(c.numCellBins / kGroupBins / 256 + 1), dim3(256), 0, s, c);
     if (sh.partBlocks) hipLaunchKernelGGL(k_part_bin, dim3(sh.partGrid), dim3(sh.partThreads), 0, s, c);
 }
 
-// exclusive scan of the bin sizes into start (c.start); with `open` it also opens the step (its
-// list counters cleared) and with `advanceTimestep` advances the worlds' timesteps
-void launch_map_scan(const Ctx& c, hipStream_t s, StepCounters* open, bool advanceTimestep) {
-    const int tiles = map_scan_tiles(c.numBins);
-    if (tiles == 0) return;
-    hipLaunchKernelGGL(k_map_scan, dim3(tiles), dim3(kMapScanThreads), 0, s, c, tiles, open, advanceTimestep ? 1 : 0);
+int map_scan_tiles(int partBins) { return (partBins + kPartScanTile - 1) / kPartScanTile; }
+
+// The maps of a step; with `open` it also opens the step, with `advanceTimestep` the worlds' timesteps.
+// The particles' takes two launches, one for their bins' offsets and one for their places.  `chain`: the
+// offsets come with the cells' map, and launch_part_scatter is to follow at the head of the particles'
+// chain, beside the next cell pass; otherwise the offsets come first and the places with the cells' map.
+void launch_map(const Ctx& c, const LaunchShape& sh, hipStream_t s, bool chain, StepCounters* open, bool advanceTimestep) {
+    const bool particles = sh.hasParticles && sh.partBlocks;
+    const int tiles = particles ? map_scan_tiles(c.numBins - c.numCellBins) : 0;
+    const int threads = sh.cellThreads, waves = threads / 64;
+    const int blocks = c.cellCount > 0 ? (c.numCellBins / kGroupBins + waves - 1) / waves : 0;
+    const int groups = (blocks + kXcdCount - 1) / kXcdCount * kXcdCount;
+    const int far = std::min(64 * sh.cellBlocks, kFarBlocks);
+    const bool with = chain && threads == kMapThreads;  // (the scan's tiles are of kMapThreads)
+    if (!with && tiles) hipLaunchKernelGGL(k_part_scan, dim3(tiles), dim3(kMapThreads), 0, s, c, tiles);
+    const int scan = with ? tiles : 0, parts = particles && !chain ? sh.partGrid : 0;
+    const int staged = particles && !chain && c.partStage > 0 ? sh.cellBlocks : 0;
+    hipLaunchKernelGGL(k_map, dim3(std::max(scan + groups + parts + staged + far, 1)), dim3(threads), 0, s, c, scan, parts, staged,
+                       groups, far, open, advanceTimestep ? 1 : 0);
 }
 
-int map_scan_tiles(int numBins) { return (numBins + kMapScanTile - 1) / kMapScanTile; }
-
-void launch_scatter(const Ctx& c, const LaunchShape& sh, hipStream_t s) {
-    const int parts = sh.hasParticles && sh.partBlocks ? sh.partGrid : 0;
-    const int cells = (sh.cellBlocks + kScatterRuns - 1) / kScatterRuns;
-    if (parts + cells) hipLaunchKernelGGL(k_scatter, dim3(parts + cells), dim3(sh.cellThreads), 0, s, c, parts, sh.cellBlocks);
+void launch_part_scatter(const Ctx& c, const LaunchShape& sh, hipStream_t s) {
+    if (!sh.hasParticles || !sh.partBlocks) return;
+    const int staged = c.partStage > 0 ? sh.cellBlocks : 0;
+    hipLaunchKernelGGL(k_part_scatter, dim3(sh.partGrid + staged), dim3(sh.cellThreads), 0, s, c, sh.partGrid);
 }
 
 }  // namespace alien

@@ -63,14 +63,39 @@ __device__ __forceinline__ int cell_bin_of(const DevWorld& w, f2 p) {
     return w.binOff + by * w.nbx + bx;
 }
 
-// The map of a step orders cells by bin, and inside a bin by their index in the last step's order
-// (R1).  The kernels that produce a cell's end-of-step position record its next bin (binOf).  A
-// cell that stays in its bin keeps its place among the bin's cells of the last map; a cell that
-// changes bins (a "mover"; after seeding every cell) is marked (kMoverBit), counted out of its old
-// bin and into its new one (delta), and entered in the list of its new bin: head[bin] is the last
-// one entered, next[i] the one before (kNone ends a list; ranks count the list's smaller indices,
-// so its order does not matter).
-__device__ __forceinline__ void push_mover(int* head, int* next, int gb, int k) { next[k] = atomicExch(&head[gb], k); }
+// enters cell k in the far list of global bin gb
+__device__ __forceinline__ void list_far(const FarCells& f, int* next, int gb, int k) {
+    next[k] = atomicExch(&f.head[gb], k);
+    atomicAdd(&f.count[gb], 1);
+    atomicAdd(&f.group[gb / kGroupBins], 1);
+}
+
+// moves the active lanes' cells between groups in the sums of groups: one atomic per group that gains or
+// loses any
+__device__ __forceinline__ void add_per_key(int* sums, int key, int unit) {
+    const int lane = int(threadIdx.x) & 63;
+    for (unsigned long long m = __ballot(true); m != 0ull;) {
+        const int lead = __builtin_ctzll(m), k = __builtin_amdgcn_readlane(key, lead);
+        const unsigned long long same = __ballot(key == k);
+        if (lane == lead) atomicAdd(&sums[k], unit * __builtin_popcountll(same));
+        m &= ~same;
+    }
+}
+__device__ __forceinline__ void shift_groups(int* sums, int* supers, int from, int to) {
+    add_per_key(sums, from, -1);
+    add_per_key(sums, to, 1);
+    const int sf = from / kSuperGroups, st = to / kSuperGroups;
+    if (sf != st) {
+        add_per_key(supers, sf, -1);
+        add_per_key(supers, st, 1);
+    }
+}
+
+// flat bins that a cell with near move code `move` crossed
+__device__ __forceinline__ int move_bins(const DevWorld& w, uint32_t move) {
+    const int m = int(move) - 1, y = m >= 6 ? 1 : (m >= 3 ? 0 : -1);
+    return m - 3 * y - 4 + y * w.nbx;
+}
 
 // base[i] through a 32-bit byte offset, which a 64-bit address of a signed index costs four operations
 // more than (a set's cells times 8 bytes, and a world's bins times 4, stay below 2^32)
@@ -82,22 +107,28 @@ template <class T> __device__ __forceinline__ T ld32(const T* base, uint32_t i) 
 template <class T> __device__ __forceinline__ void st32(T* base, uint32_t i, T v) { *at32(base, i) = v; }
 static_assert(uint64_t(kMaxSetCells) * 8 < (uint64_t(1) << 32), "32-bit byte offsets");
 
-// next-step bin of the cell at end-of-step index k: end-of-step position pNew; bOld, its bin in this
-// step's map (the bin of its start-of-step position, counted from the world's first)
+// Next-step bin of the cell at end-of-step index k: end-of-step position pNew; bOld, its bin in this
+// step's map (the bin of its start-of-step position, counted from the world's first).  The next map
+// looks for a bin's cells in the bins one and one row of bins around (counted along the rows, so a step
+// across the end of a row is near, one across the torus' edge is not).
 __device__ __forceinline__ void bin_next(const Ctx& c, const DevWorld& w, int k, f2 pNew, int bOld) {
     int bx, by;
     cell_bin_xy(w, pNew, bx, by);
     const int b = by * w.nbx + bx;
-    const int gb = w.binOff + b;
-    if (b == bOld) {
-        st32(c.binOf, k, gb);
-        return;
+    const int d = b - bOld;
+    uint32_t move = 0u;
+    if (d != 0) {
+        const int y = d > 1 ? 1 : (d < -1 ? -1 : 0), x = d - y * w.nbx;
+        move = uint32_t(3 * (y + 1) + x + 2);
+        if (x < -1 || x > 1) {
+            move = kFarCode;
+            c.farNext.list[atomicAdd(c.farNext.total, 1)] = make_int2(k, w.binOff + b);
+            list_far(c.farNext, c.moverNext, w.binOff + b, k);
+        }
+        const int from = (w.binOff + bOld) / kGroupBins, to = (w.binOff + b) / kGroupBins;
+        if (from != to) shift_groups(c.groupSumNext, c.superSumNext, from, to);
     }
-    st32(c.binOf, k, int(uint32_t(gb) | kMoverBit));
-    st32(c.moverNext, k, atomicExch(at32(c.moverHeadNext + w.binOff, b), k));
-    int* delta = c.deltaNext + w.binOff;
-    atomicAdd(at32(delta, b), 1);
-    atomicSub(at32(delta, bOld), 1);
+    st32(c.binOf, uint32_t(k), int(uint32_t(b) | move << kMoveShift));
 }
 
 __device__ __forceinline__ void pbin_for_next_step(const Ctx& c, const DevWorld& w, int k, f2 p, uint32_t* hist) {

@@ -11,8 +11,8 @@
 
 namespace alien {
 
-void launch_map_scan(const Ctx& c, hipStream_t s, StepCounters* open, bool advanceTimestep);
-void launch_scatter(const Ctx& c, const LaunchShape& sh, hipStream_t s);
+void launch_map(const Ctx& c, const LaunchShape& sh, hipStream_t s, bool chain, StepCounters* open, bool advanceTimestep);
+void launch_part_scatter(const Ctx& c, const LaunchShape& sh, hipStream_t s);
 void launch_neighbor(const Ctx& c, const LaunchShape& sh, hipStream_t s, bool withPartSort);
 void launch_particles(const Ctx& c, const LaunchShape& sh, hipStream_t s, Recorder* rec);
 void launch_bonds(const Ctx& c, const LaunchShape& sh, hipStream_t s, Recorder* rec);
@@ -28,12 +28,9 @@ void launch_radiation(const Ctx& c, const LaunchShape& sh, hipStream_t s, Record
 void launch_step(const Ctx& c, const LaunchShape& sh, hipStream_t s, Recorder* rec, const SideStream* side) {
     // cell radiation comes first: the particles it emits enter this step's particle map
     launch_radiation(c, sh, s, rec);
-    // without bond work the end-of-step kernel would only advance the timesteps: the map scan does
-    // it
-    if (rec) rec->mark("map_scan");
-    launch_map_scan(c, s, c.sc, !sh.hasBondWork);
-    if (rec) rec->mark("cell_scatter");
-    launch_scatter(c, sh, s);
+    // without bond work the end-of-step kernel would only advance the timesteps: the map does it
+    if (rec) rec->mark("map");
+    launch_map(c, sh, s, !sh.hasBondWork, c.sc, !sh.hasBondWork);
     const bool fork = side && !rec && !sh.hasBondWork && sh.hasParticles && sh.partBlocks;
     if (fork) (void)hipEventRecord(side->fork, s);
     if (rec) rec->mark("neighbor");
@@ -42,6 +39,8 @@ void launch_step(const Ctx& c, const LaunchShape& sh, hipStream_t s, Recorder* r
         launch_bonds(c, sh, s, rec);
     } else {
         if (fork) (void)hipStreamWaitEvent(side->stream, side->fork, 0);
+        if (rec) rec->mark("part_scatter");
+        launch_part_scatter(c, sh, fork ? side->stream : s);
         launch_particles(c, sh, fork ? side->stream : s, rec);
         if (fork) {
             (void)hipEventRecord(side->join, side->stream);
@@ -52,11 +51,10 @@ void launch_step(const Ctx& c, const LaunchShape& sh, hipStream_t s, Recorder* r
     if (rec) rec->mark(nullptr);
 }
 
-// The map of the current state: consumes the seeded bins and mover lists, which seeding restores
+// The map of the current state: consumes the seeded bins and far lists, which seeding restores
 // for the next step.
 void launch_debug_map(const Ctx& c, const LaunchShape& sh, hipStream_t s) {
-    launch_map_scan(c, s, nullptr, false);
-    launch_scatter(c, sh, s);
+    launch_map(c, sh, s, false, nullptr, false);
     launch_seed_bins(c, sh, s);
 }
 

@@ -473,8 +473,7 @@ uint64_t WorldSet::estimateBytes(uint64_t cells, uint64_t particles, int W, int 
     const uint64_t perParticle = 2 * (8 + 8 + 4 + 4 + 4 + 1 + 8) + 6 * 4;
     const uint64_t bins = uint64_t(std::max(1, W / binSize)) * uint64_t(std::max(1, H / binSize)) +
                           uint64_t(std::max(1, W / kParticleBin)) * uint64_t(std::max(1, H / kParticleBin));
-    // per bin: two histograms, two offset arrays, two mover-list heads and deltas (cell bins), scan
-    // partials
+    // per bin: two histograms, two offset arrays, two far-list heads and counts (cell bins), sums
     return cells * perCell + particles * perParticle + bins * 36 + (1u << 20);
 }
 
@@ -584,7 +583,7 @@ void WorldSet::build(const std::vector<Source>& sources) {
         stageChoice.push_back(stage);
         cellOff += h.numCells;
         partOff += w.partCap;
-        bins += int64_t(w.nbx) * w.nby;
+        bins += (int64_t(w.nbx) * w.nby + kGroupBins - 1) / kGroupBins * kGroupBins;
         if (bins + int64_t(w.pnbx) * w.pnby >= (int64_t(1) << 31) - 2)
             throw Error(ALIEN_E_CAPACITY, "too many spatial bins in one world set");
         hosts.push_back(std::move(h));
@@ -669,19 +668,36 @@ void WorldSet::build(const std::vector<Source>& sources) {
     activation_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
     creature_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
     stretched_ = static_cast<uint8_t*>(A(NC));
-    binOf_ = static_cast<int*>(A(sizeof(int) * NC));
+    binOf_ = static_cast<int*>(A(sizeof(int) * (size_t(NC) + kBinOfPad)));
     pbinOf_ = static_cast<int*>(A(sizeof(int) * NP));
     count_[0] = static_cast<uint32_t*>(A(sizeof(uint32_t) * NB));
     count_[1] = static_cast<uint32_t*>(A(sizeof(uint32_t) * NB));
     numCellBins_ = cellBins;
     const size_t NCB = size_t(std::max(cellBins, 1));
+    farList_ = static_cast<int2*>(A(sizeof(int2) * NC));
     for (int b = 0; b < 2; ++b) {
         start_[b] = static_cast<uint32_t*>(A(sizeof(uint32_t) * (size_t(NB) + 1)));
-        moverHead_[b] = static_cast<int*>(A(sizeof(int) * NCB));
-        delta_[b] = static_cast<int*>(A(sizeof(int) * NCB));
+        far_[b].head = static_cast<int*>(A(sizeof(int) * NCB));
+        far_[b].count = static_cast<int*>(A(sizeof(int) * NCB));
+        far_[b].group = static_cast<int*>(A(sizeof(int) * (NCB / kGroupBins + 1)));
+        far_[b].total = far_[b].group + NCB / kGroupBins;
+        far_[b].list = farList_;
     }
     moverNext_ = static_cast<int*>(A(sizeof(int) * NC));
-    mapStatus_ = static_cast<unsigned long long*>(A(sizeof(unsigned long long) * size_t(map_scan_tiles(NB))));
+    std::vector<int> groupWorld;
+    for (size_t w = 0; w < worlds.size(); ++w) {
+        const int64_t groups = (int64_t(worlds[w].nbx) * worlds[w].nby + kGroupBins - 1) / kGroupBins;
+        groupWorld.insert(groupWorld.end(), size_t(groups), int(w));
+    }
+    groupWorld_ = static_cast<int*>(A(sizeof(int) * std::max<size_t>(groupWorld.size(), 1)));
+    if (!groupWorld.empty())
+        check_hip(hipMemcpy(groupWorld_, groupWorld.data(), sizeof(int) * groupWorld.size(), hipMemcpyHostToDevice), "H2D");
+    const size_t groups = NCB / kGroupBins + 1, supers = groups / kSuperGroups + 1;
+    for (int b = 0; b < 2; ++b) {
+        groupSum_[b] = static_cast<int*>(A(sizeof(int) * groups));
+        superSum_[b] = static_cast<int*>(A(sizeof(int) * supers));
+    }
+    mapStatus_ = static_cast<unsigned long long*>(A(sizeof(unsigned long long) * size_t(map_scan_tiles(NB - cellBins) + 1)));
     mapEpochTicket_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * 2));
     sorted_ = static_cast<int*>(A(sizeof(int) * NC));
     mpos_ = static_cast<float2*>(A(sizeof(float2) * NC));
@@ -836,12 +852,17 @@ void WorldSet::build(const std::vector<Source>& sources) {
     launch_fill_u32(count_[1], 0u, size_t(NB), stream_);
     for (int b = 0; b < 2; ++b) {
         launch_fill_u32(start_[b], 0u, size_t(NB) + 1, stream_);
-        launch_fill_u32(reinterpret_cast<uint32_t*>(moverHead_[b]), uint32_t(kNone), NCB, stream_);
-        launch_fill_u32(reinterpret_cast<uint32_t*>(delta_[b]), 0u, NCB, stream_);
+        launch_fill_u32(reinterpret_cast<uint32_t*>(far_[b].head), uint32_t(kNone), NCB, stream_);
+        launch_fill_u32(reinterpret_cast<uint32_t*>(far_[b].count), 0u, NCB, stream_);
+        launch_fill_u32(reinterpret_cast<uint32_t*>(far_[b].group), 0u, NCB / kGroupBins + 1, stream_);
     }
     launch_fill_u32(reinterpret_cast<uint32_t*>(fclaim_), uint32_t(kClaimFree), size_t(NP), stream_);
     launch_fill_u32(reinterpret_cast<uint32_t*>(cclaim_), uint32_t(kClaimFree), size_t(NC), stream_);
-    launch_fill_u32(reinterpret_cast<uint32_t*>(mapStatus_), 0u, 2 * size_t(map_scan_tiles(NB)), stream_);
+    launch_fill_u32(reinterpret_cast<uint32_t*>(mapStatus_), 0u, 2 * size_t(map_scan_tiles(NB - cellBins) + 1), stream_);
+    for (int b = 0; b < 2; ++b) {
+        launch_fill_u32(reinterpret_cast<uint32_t*>(groupSum_[b]), 0u, groups, stream_);
+        launch_fill_u32(reinterpret_cast<uint32_t*>(superSum_[b]), 0u, supers, stream_);
+    }
     launch_fill_u32(mapEpochTicket_, 0u, 2, stream_);
     launch_fill_u32(reinterpret_cast<uint32_t*>(claim_), 0xffffffffu, size_t(NC) * 2, stream_);
     launch_fill_u32(reinterpret_cast<uint32_t*>(buf_[1].pflags), 0u, (size_t(NP) + 3) / 4, stream_);
@@ -1162,13 +1183,17 @@ Ctx WorldSet::makeCtx(int parity) const {
     c.partCap = partCap_;
     c.numBins = numBins_;
     c.numCellBins = numCellBins_;
+    c.cellCount = worlds_.empty() ? 0 : worlds_.back().cellOff + worlds_.back().numCells;
     c.start = start_[parity];
     c.startPrev = start_[parity ^ 1];
-    c.moverHead = moverHead_[parity];
-    c.moverHeadNext = moverHead_[parity ^ 1];
+    c.far = far_[parity];
+    c.farNext = far_[parity ^ 1];
     c.moverNext = moverNext_;
-    c.delta = delta_[parity];
-    c.deltaNext = delta_[parity ^ 1];
+    c.groupWorld = groupWorld_;
+    c.groupSum = groupSum_[parity];
+    c.groupSumNext = groupSum_[parity ^ 1];
+    c.superSum = superSum_[parity];
+    c.superSumNext = superSum_[parity ^ 1];
     c.worlds = dWorlds_;
     c.params = dParams_;
     c.ctr = dCtr_;
@@ -1908,7 +1933,7 @@ void WorldSet::cellMap(int wi, std::vector<int>& bins, std::vector<int>& slots) 
     bins.resize(n);
     slots.resize(n);
     for (int k = 0; k < n; ++k) {
-        bins[k] = int(uint32_t(binOfAll[sorted[k]]) & ~kMoverBit) - w.binOff;
+        bins[k] = int(uint32_t(binOfAll[sorted[k]]) & kBinMask);
         slots[k] = slotAll[sorted[k]];
     }
 }

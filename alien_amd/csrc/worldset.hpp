@@ -262,11 +262,14 @@ private:
     std::vector<uint8_t> livingWork_;  // per world
     int *binOf_ = nullptr, *pbinOf_ = nullptr;
     uint32_t* count_[2] = {nullptr, nullptr};  // bin histograms, alternating with the state buffers
-    // map build: offsets of the map of the step of that parity and the mover lists (per cell bin)
+    // map build: offsets of the map of the step of that parity and the far cells
     // read in it, alternating with the state buffers
     uint32_t* start_[2] = {nullptr, nullptr};
-    int* moverHead_[2] = {nullptr, nullptr};
-    int* delta_[2] = {nullptr, nullptr};
+    FarCells far_[2] = {};
+    int2* farList_ = nullptr;
+    int* groupWorld_ = nullptr;
+    int* groupSum_[2] = {nullptr, nullptr};
+    int* superSum_[2] = {nullptr, nullptr};
     int* moverNext_ = nullptr;
     int numCellBins_ = 0;
     unsigned long long* mapStatus_ = nullptr;

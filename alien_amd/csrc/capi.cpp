@@ -309,7 +309,7 @@ int alien_debug_get_map(alien_world* w, int32_t* cellBin, uint64_t* cellId, uint
         if (binsX) *binsX = w->desc.worldSizeX / alien::bin_size_for(w->params);
         if (binsY) *binsY = w->desc.worldSizeY / alien::bin_size_for(w->params);
         if (bins.size() > cap) throw Error(ALIEN_E_CAPACITY, "output buffer too small (count was written)");
-        const auto& ids = w->set->host(0).cellId;
+        const auto& ids = w->set->host(0).cells->cellId;
         for (size_t k = 0; k < bins.size(); ++k) {
             cellBin[k] = bins[k];
             cellId[k] = ids[slots[k]];
@@ -323,7 +323,7 @@ int alien_debug_neighbors(alien_world* w, uint64_t* offsets, uint64_t offsetsCap
         requireHealthy(w);
         std::vector<std::vector<int>> bySlot;
         w->set->neighbors(0, bySlot);
-        const auto& ids = w->set->host(0).cellId;
+        const auto& ids = w->set->host(0).cells->cellId;
         const int n = int(bySlot.size());
         std::vector<int> order(n);
         for (int i = 0; i < n; ++i) order[i] = i;

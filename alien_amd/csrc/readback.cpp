@@ -118,4 +118,34 @@ void read_records(size_t n, size_t size, void* out, hipStream_t s,
     if (error) std::rethrow_exception(error);
 }
 
+// One thread per 8192 entries: starting one costs about 20 us, the work on an entry 10 to 60 ns.
+void for_ranges(size_t n, const std::function<void(size_t, size_t)>& f) {
+    const size_t cores = std::max<size_t>(1, std::thread::hardware_concurrency());
+    const size_t pieces = std::max<size_t>(1, std::min({size_t(8), cores, n / 8192}));
+    if (pieces == 1) return f(0, n);
+    std::vector<std::exception_ptr> errors(pieces);
+    auto work = [&](size_t k) {
+        try {
+            f(n * k / pieces, n * (k + 1) / pieces);
+        } catch (...) {
+            errors[k] = std::current_exception();
+        }
+    };
+    std::vector<std::thread> others;
+    others.reserve(pieces);
+    size_t started = 1;
+    for (; started < pieces; ++started) {
+        try {
+            others.emplace_back(work, started);
+        } catch (const std::system_error&) {
+            break;  // no more threads: the pieces left are done here
+        }
+    }
+    work(0);
+    for (size_t k = started; k < pieces; ++k) work(k);
+    for (auto& t : others) t.join();
+    for (const auto& e : errors)
+        if (e) std::rethrow_exception(e);
+}
+
 }  // namespace alien

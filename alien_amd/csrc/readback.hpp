@@ -99,4 +99,8 @@ private:
 void read_records(size_t n, size_t size, void* out, hipStream_t s,
                   const std::function<void(size_t, size_t, void*)>& pack);
 
+// f(begin, end) over consecutive pieces of [0, n), on up to eight threads; the exception of the first piece
+// that throws one goes on to the caller
+void for_ranges(size_t n, const std::function<void(size_t, size_t)>& f);
+
 }  // namespace alien

@@ -3,6 +3,7 @@
 #include "worldset.hpp"
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <map>
@@ -170,127 +171,163 @@ WorldImage WorldImage::fromTO(const alien_world_desc& desc, const alien_params& 
     h.params = params;
     h.numCells = n;
     h.particleCap = np;
-    h.cellId.resize(n);
-    h.age.resize(n);
-    h.creatureId.resize(n);
-    h.mutationId.resize(n);
-    h.activationTime.resize(n);
-    h.livingState.resize(n);
-    h.cellFunction.resize(n);
-    h.ancestorMutationId.resize(n);
-    h.selected.resize(n);
-    h.genomeComplexity.resize(n);
+    auto host = std::make_shared<HostCells>();
+    HostCells& hc = *host;
+    hc.cellId.resize(n);
+    hc.age.resize(n);
+    hc.creatureId.resize(n);
+    hc.mutationId.resize(n);
+    hc.activationTime.resize(n);
+    hc.livingState.resize(n);
+    hc.cellFunction.resize(n);
+    hc.ancestorMutationId.resize(n);
+    hc.selected.resize(n);
+    hc.genomeComplexity.resize(n);
     img.pos.resize(n);
     img.vel.resize(n);
-    img.dens.assign(n, 1.0f);
+    img.dens.resize(n);
     img.flags.resize(n);
     img.slot.resize(n);
-    img.btgt.assign(size_t(kMaxBonds) * n, 0);
-    img.brest.assign(size_t(kMaxBonds) * n, 0.0f);
-    img.bang.assign(size_t(kMaxBonds) * n, 0.0f);
+    img.btgt.resize(size_t(kMaxBonds) * n);
+    img.brest.resize(size_t(kMaxBonds) * n);
+    img.bang.resize(size_t(kMaxBonds) * n);
     img.energy.resize(n);
     img.stiff.resize(n);
     // Slots (the cells' stable identities, which index their cold state) are given in spatial
     // order, bin by bin of the cell map: the map keeps cells in bin order, so the cold state of
     // neighbouring map entries then lies close in memory.  Only locality depends on it.
+    // (Every thread counts and numbers the cells of a range of bins, which keeps them in index order.)
     {
         const int bs = bin_size_for(params);
         const int nbx = std::max(1, W / bs), nby = std::max(1, H / bs);
-        std::vector<int> key(n), cnt(size_t(nbx) * nby + 1, 0);
-        for (int i = 0; i < n; ++i) {
-            float x = cells[i].pos[0], y = cells[i].pos[1];
-            int k = 0;
-            if (std::isfinite(x) && std::isfinite(y)) {
-                host_wrap(x, y, W, H);
-                const int bx = std::min(int(x) / bs, nbx - 1), by = std::min(int(y) / bs, nby - 1);
-                k = std::max(0, by) * nbx + std::max(0, bx);
+        const size_t bins = size_t(nbx) * nby;
+        HostArray<int> key(n), next(bins);
+        for_ranges(size_t(n), [&](size_t i0, size_t i1) {
+            for (size_t i = i0; i < i1; ++i) {
+                float x = cells[i].pos[0], y = cells[i].pos[1];
+                int k = 0;
+                if (std::isfinite(x) && std::isfinite(y)) {
+                    host_wrap(x, y, W, H);
+                    const int bx = std::min(int(x) / bs, nbx - 1), by = std::min(int(y) / bs, nby - 1);
+                    k = std::max(0, by) * nbx + std::max(0, bx);
+                }
+                key[i] = k;
             }
-            key[i] = k;
-            ++cnt[size_t(k) + 1];
+        });
+        img.binCells.resize(bins);
+        // (by the cells' number: one piece for few cells, whatever the bins)
+        const size_t pieces = std::max<size_t>(1, std::min(size_t(n), bins));
+        auto binsOf = [&](size_t p) { return bins * p / pieces; };
+        for_ranges(pieces, [&](size_t p0, size_t p1) {
+            const size_t b0 = binsOf(p0), span = binsOf(p1) - b0;
+            std::fill_n(img.binCells.begin() + std::ptrdiff_t(b0), span, 0);
+            for (int i = 0; i < n; ++i)
+                if (size_t(key[i]) - b0 < span) ++img.binCells[size_t(key[i])];
+        });
+        int sum = 0;
+        for (size_t b = 0; b < bins; ++b) {
+            next[b] = sum;
+            sum += img.binCells[b];
         }
-        for (size_t b = 1; b < cnt.size(); ++b) cnt[b] += cnt[b - 1];
-        for (int i = 0; i < n; ++i) img.slot[i] = cnt[size_t(key[i])]++;
+        for_ranges(pieces, [&](size_t p0, size_t p1) {
+            const size_t b0 = binsOf(p0), span = binsOf(p1) - b0;
+            for (int i = 0; i < n; ++i)
+                if (size_t(key[i]) - b0 < span) img.slot[i] = next[size_t(key[i])]++;
+        });
     }
-    for (int i = 0; i < n; ++i) {
-        const alien_cell_to& c = cells[i];
-        if (c.numConnections > kMaxBonds) throw Error(ALIEN_E_ARG, "numConnections above 6");
-        if (c.color >= kColors) throw Error(ALIEN_E_ARG, "cell color must be below 7 (MAX_COLORS)");
-        float x = c.pos[0], y = c.pos[1];
-        if (!std::isfinite(x) || !std::isfinite(y)) throw Error(ALIEN_E_ARG, "non-finite cell position");
-        host_wrap(x, y, W, H);
-        img.pos[i] = make_float2(x, y);
-        img.vel[i] = make_float2(c.vel[0], c.vel[1]);
-        uint32_t maxConn = c.maxConnections > 15 ? 15u : c.maxConnections;
-        img.flags[i] = uint32_t(c.numConnections) | (maxConn << kMaxConnShift) | (uint32_t(c.color) << kColorShift) |
-                       (c.barrier ? kBarrierBit : 0u);
-        const int sl = img.slot[i];
-        for (int b = 0; b < c.numConnections; ++b) {
-            int t = c.connections[b].cellIndex;
-            if (t < 0 || t >= n) throw Error(ALIEN_E_ARG, "bond cellIndex out of range");
-            img.btgt[size_t(b) * n + i] = t;
-            img.brest[size_t(b) * n + i] = c.connections[b].distance;
-            img.bang[size_t(b) * n + i] = c.connections[b].angleFromPrevious;
+    std::atomic<bool> hasExtra{false}, hasSelected{false}, livingWork{false};
+    for_ranges(size_t(n), [&](size_t i0, size_t i1) {
+        bool extra = false, living = false;
+        for (size_t i = i0; i < i1; ++i) {
+            const alien_cell_to& c = cells[i];
+            if (c.numConnections > kMaxBonds) throw Error(ALIEN_E_ARG, "numConnections above 6");
+            if (c.color >= kColors) throw Error(ALIEN_E_ARG, "cell color must be below 7 (MAX_COLORS)");
+            float x = c.pos[0], y = c.pos[1];
+            if (!std::isfinite(x) || !std::isfinite(y)) throw Error(ALIEN_E_ARG, "non-finite cell position");
+            host_wrap(x, y, W, H);
+            img.pos[i] = make_float2(x, y);
+            img.vel[i] = make_float2(c.vel[0], c.vel[1]);
+            img.dens[i] = 1.0f;
+            uint32_t maxConn = c.maxConnections > 15 ? 15u : c.maxConnections;
+            img.flags[i] = uint32_t(c.numConnections) | (maxConn << kMaxConnShift) | (uint32_t(c.color) << kColorShift) |
+                           (c.barrier ? kBarrierBit : 0u);
+            const int sl = img.slot[i];
+            for (int b = 0; b < kMaxBonds; ++b) {
+                const bool on = b < c.numConnections;
+                const int t = on ? c.connections[b].cellIndex : 0;
+                if (on && (t < 0 || t >= n)) throw Error(ALIEN_E_ARG, "bond cellIndex out of range");
+                img.btgt[size_t(b) * n + i] = t;
+                img.brest[size_t(b) * n + i] = on ? c.connections[b].distance : 0.0f;
+                img.bang[size_t(b) * n + i] = on ? c.connections[b].angleFromPrevious : 0.0f;
+            }
+            img.energy[sl] = c.energy;
+            img.stiff[sl] = c.stiffness;
+            for (int b = 0; b < c.numConnections; ++b) {  // bonds come in pairs a->b, b->a (TOs.cuh:30-35)
+                const int t = c.connections[b].cellIndex;
+                const alien_cell_to& o = cells[t];
+                int back = 0, same = 0;
+                for (int k = 0; k < o.numConnections && k < kMaxBonds; ++k) back += o.connections[k].cellIndex == int(i);
+                for (int k = 0; k < c.numConnections; ++k) same += c.connections[k].cellIndex == t;
+                if (t == int(i) || back != 1 || same != 1) throw Error(ALIEN_E_ARG, "bonds must be symmetric and unique");
+            }
+            hc.cellId[sl] = c.id;
+            hc.age[sl] = c.age;
+            hc.creatureId[sl] = c.creatureId;
+            hc.mutationId[sl] = c.mutationId;
+            hc.activationTime[sl] = c.activationTime;
+            hc.livingState[sl] = c.livingState;
+            hc.cellFunction[sl] = c.cellFunction;
+            hc.ancestorMutationId[sl] = c.ancestorMutationId;
+            hc.selected[sl] = c.selected;
+            hc.genomeComplexity[sl] = c.genomeComplexity;
+            uint32_t genome = 0;
+            std::memcpy(&genome, &c.genomeComplexity, sizeof(genome));
+            extra = extra || (c.mutationId | genome | c.cellFunction | c.ancestorMutationId | c.selected) != 0u;
+            living = living || c.livingState != 0 || c.activationTime != 0 ||
+                     (!c.barrier && c.energy < params.cellMinEnergy[c.color]);
         }
-        img.energy[sl] = c.energy;
-        img.stiff[sl] = c.stiffness;
-        for (int b = 0; b < c.numConnections; ++b) {  // bonds come in pairs a->b, b->a (TOs.cuh:30-35)
-            const int t = c.connections[b].cellIndex;
-            const alien_cell_to& o = cells[t];
-            int back = 0, same = 0;
-            for (int k = 0; k < o.numConnections && k < kMaxBonds; ++k) back += o.connections[k].cellIndex == i;
-            for (int k = 0; k < c.numConnections; ++k) same += c.connections[k].cellIndex == t;
-            if (t == i || back != 1 || same != 1) throw Error(ALIEN_E_ARG, "bonds must be symmetric and unique");
-        }
-        h.cellId[sl] = c.id;
-        h.age[sl] = c.age;
-        h.creatureId[sl] = c.creatureId;
-        h.mutationId[sl] = c.mutationId;
-        h.activationTime[sl] = c.activationTime;
-        h.livingState[sl] = c.livingState;
-        h.cellFunction[sl] = c.cellFunction;
-        h.ancestorMutationId[sl] = c.ancestorMutationId;
-        h.selected[sl] = c.selected;
-        h.genomeComplexity[sl] = c.genomeComplexity;
-        uint32_t genome = 0;
-        std::memcpy(&genome, &c.genomeComplexity, sizeof(genome));
-        h.hasExtra = h.hasExtra || (c.mutationId | genome | c.cellFunction | c.ancestorMutationId | c.selected) != 0u;
-    }
+        if (extra) hasExtra = true;
+        if (living) livingWork = true;
+    });
     img.ppos.resize(np);
     img.pvel.resize(np);
     img.pen.resize(np);
-    img.plast.assign(np, kNone);
+    img.plast.resize(np);
     img.pslot.resize(np);
     img.pflags.resize(np);
     img.pid.resize(np);
-    h.particleId.resize(np);
-    h.particleSelected.resize(np);
-    for (int i = 0; i < np; ++i) {
-        const alien_particle_to& p = particles[i];
-        if (p.color >= kColors) throw Error(ALIEN_E_ARG, "particle color must be below 7 (MAX_COLORS)");
-        float x = p.pos[0], y = p.pos[1];
-        if (!std::isfinite(x) || !std::isfinite(y)) throw Error(ALIEN_E_ARG, "non-finite particle position");
-        host_wrap(x, y, W, H);
-        img.ppos[i] = make_float2(x, y);
-        img.pvel[i] = make_float2(p.vel[0], p.vel[1]);
-        img.pen[i] = p.energy;
-        img.pslot[i] = i;
-        img.pflags[i] = uint8_t(p.color & kParticleColorMask);
-        img.pid[i] = p.id;
-        h.particleId[i] = p.id;
-        h.particleSelected[i] = p.selected;
-        h.hasSelected = h.hasSelected || p.selected != 0;
-    }
+    hc.particleId.resize(np);
+    hc.particleSelected.resize(np);
+    for_ranges(size_t(np), [&](size_t i0, size_t i1) {
+        bool selected = false;
+        for (size_t i = i0; i < i1; ++i) {
+            const alien_particle_to& p = particles[i];
+            if (p.color >= kColors) throw Error(ALIEN_E_ARG, "particle color must be below 7 (MAX_COLORS)");
+            float x = p.pos[0], y = p.pos[1];
+            if (!std::isfinite(x) || !std::isfinite(y)) throw Error(ALIEN_E_ARG, "non-finite particle position");
+            host_wrap(x, y, W, H);
+            img.ppos[i] = make_float2(x, y);
+            img.pvel[i] = make_float2(p.vel[0], p.vel[1]);
+            img.pen[i] = p.energy;
+            img.plast[i] = kNone;
+            img.pslot[i] = int(i);
+            img.pflags[i] = uint8_t(p.color & kParticleColorMask);
+            img.pid[i] = p.id;
+            hc.particleId[i] = p.id;
+            hc.particleSelected[i] = p.selected;
+            selected = selected || p.selected != 0;
+        }
+        if (selected) hasSelected = true;
+    });
+    h.hasExtra = hasExtra;
+    h.hasSelected = hasSelected;
+    h.cells = std::move(host);
     img.numParticles = np;
     // Living states need tracking on the device only if some cell is not trivially Ready: a state
     // other than Ready, an activation count, (non-barrier) energy below cellMinEnergy, or cell
     // radiation, the one process of this path that takes energy from cells.  A world without any
     // of these keeps every cell Ready with no count for good (its energies only grow).
-    img.livingWork = radiates(params);
-    for (int i = 0; i < n && !img.livingWork; ++i) {
-        const alien_cell_to& c = cells[i];
-        img.livingWork = c.livingState != 0 || c.activationTime != 0 ||
-                         (!c.barrier && c.energy < params.cellMinEnergy[c.color]);
-    }
+    img.livingWork = radiates(params) || livingWork;
     return img;
 }
 
@@ -300,17 +337,18 @@ void WorldImage::updateLivingWork() {
     for (int i = 0; i < h.numCells && !livingWork; ++i) {
         const int sl = slot[size_t(i)];
         const uint32_t f = flags[size_t(i)];
-        livingWork = h.livingState[sl] != 0 || h.activationTime[sl] != 0 ||
+        livingWork = h.cells->livingState[sl] != 0 || h.cells->activationTime[sl] != 0 ||
                      (!flags_barrier(f) && energy[sl] < h.params.cellMinEnergy[flags_color(f)]);
     }
 }
 
 void WorldImage::toTO(std::vector<alien_cell_to>& cells, std::vector<alien_particle_to>& particles) const {
     const HostWorld& h = host;
+    const HostCells& hc = *h.cells;
     const int n = h.numCells;
     // ascending id (ties by index), sorted as compact (id, index) pairs
     std::vector<std::pair<uint64_t, int>> keys(static_cast<size_t>(n));
-    for (int i = 0; i < n; ++i) keys[size_t(i)] = {h.cellId[slot[i]], i};
+    for (int i = 0; i < n; ++i) keys[size_t(i)] = {hc.cellId[slot[i]], i};
     std::sort(keys.begin(), keys.end());
     std::vector<int> order(n);
     for (int k = 0; k < n; ++k) order[k] = keys[size_t(k)].second;
@@ -322,7 +360,7 @@ void WorldImage::toTO(std::vector<alien_cell_to>& cells, std::vector<alien_parti
         const int sl = slot[i];
         alien_cell_to& c = cells[k];
         const uint32_t f = flags[i];
-        c.id = h.cellId[sl];
+        c.id = hc.cellId[sl];
         c.pos[0] = pos[i].x;
         c.pos[1] = pos[i].y;
         c.vel[0] = vel[i].x;
@@ -338,15 +376,15 @@ void WorldImage::toTO(std::vector<alien_cell_to>& cells, std::vector<alien_parti
             c.connections[b].distance = brest[size_t(b) * n + i];
             c.connections[b].angleFromPrevious = bang[size_t(b) * n + i];
         }
-        c.age = h.age[sl];
-        c.livingState = h.livingState[sl];
-        c.activationTime = h.activationTime[sl];
-        c.cellFunction = h.cellFunction[sl];
-        c.ancestorMutationId = h.ancestorMutationId[sl];
-        c.selected = h.selected[sl];
-        c.creatureId = h.creatureId[sl];
-        c.mutationId = h.mutationId[sl];
-        c.genomeComplexity = h.genomeComplexity[sl];
+        c.age = hc.age[sl];
+        c.livingState = hc.livingState[sl];
+        c.activationTime = hc.activationTime[sl];
+        c.cellFunction = hc.cellFunction[sl];
+        c.ancestorMutationId = hc.ancestorMutationId[sl];
+        c.selected = hc.selected[sl];
+        c.creatureId = hc.creatureId[sl];
+        c.mutationId = hc.mutationId[sl];
+        c.genomeComplexity = hc.genomeComplexity[sl];
     }
     const int np = numParticles;
     std::vector<std::pair<uint64_t, int>> pkeys(static_cast<size_t>(np));
@@ -365,7 +403,7 @@ void WorldImage::toTO(std::vector<alien_cell_to>& cells, std::vector<alien_parti
         p.vel[0] = pvel[i].x;
         p.vel[1] = pvel[i].y;
         p.color = uint8_t(pflags[i] & kParticleColorMask);
-        p.selected = pslot[i] >= 0 ? h.particleSelected[pslot[i]] : 0;
+        p.selected = pslot[i] >= 0 ? hc.particleSelected[pslot[i]] : 0;
     }
 }
 
@@ -417,9 +455,11 @@ WorldSet::WorldSet() {
     check_hip(hipEventCreateWithFlags(&side_.fork, hipEventDisableTiming), "hipEventCreate");
     check_hip(hipEventCreateWithFlags(&side_.join, hipEventDisableTiming), "hipEventCreate");
     check_hip(hipEventCreateWithFlags(&liveReady_, hipEventDisableTiming), "hipEventCreate");
-    check_hip(hipHostMalloc(reinterpret_cast<void**>(&liveHost_), 64 + sizeof(DevCounters), hipHostMallocDefault),
+    check_hip(hipHostMalloc(reinterpret_cast<void**>(&liveHost_), 128 + sizeof(StepCounters), hipHostMallocDefault),
               "hipHostMalloc");
+    static_assert(sizeof(DevCounters) <= 64, "room in the pinned words");
     hostWord_ = reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(liveHost_) + 64);
+    hostSc_ = reinterpret_cast<StepCounters*>(reinterpret_cast<char*>(liveHost_) + 128);
 }
 
 WorldSet::~WorldSet() {
@@ -450,6 +490,7 @@ void* WorldSet::alloc(size_t bytes) {
 void WorldSet::freeAll() {
     for (auto& a : allocs_) (void)hipFree(a.p);
     allocs_.clear();
+    partArena_ = nullptr;
     deviceBytes_ = 0;
 }
 
@@ -540,7 +581,9 @@ void WorldSet::build(const std::vector<Source>& sources) {
                     work = true;
             }
             const int bs = bin_size_for(h.params);
-            strip = choose_strip(im.pos, h.desc.worldSizeX, h.desc.worldSizeY, bs,
+            const int W = h.desc.worldSizeX, H = h.desc.worldSizeY;
+            const bool counted = im.binCells.size() == size_t(W / bs) * size_t(H / bs);
+            strip = choose_strip(im.pos.size(), counted ? im.binCells : bin_cells(im.pos, W, H, bs), W / bs, H / bs,
                                  h.params.motionType == ALIEN_MOTION_COLLISION, stage);
         } else {
             h = src.from->hosts_.at(src.fromIndex);
@@ -602,7 +645,6 @@ void WorldSet::build(const std::vector<Source>& sources) {
     }
     if (bins >= (int64_t(1) << 31) - 2) throw Error(ALIEN_E_CAPACITY, "too many spatial bins in one world set");
 
-    WorldSet& me = *this;
     invalidateGraphs();
 
     bool anyRadiates = false, anySplits = false;
@@ -617,108 +659,127 @@ void WorldSet::build(const std::vector<Source>& sources) {
     partCap_ = NP;
     numBins_ = NB;
     candCap_ = std::max(4 * NC, 4096);
-    auto A = [&](size_t bytes) { return me.alloc(bytes); };
-    dWorlds_ = static_cast<DevWorld*>(A(sizeof(DevWorld) * std::max<size_t>(worlds.size(), 1)));
-    dParams_ = static_cast<DevParams*>(A(sizeof(DevParams) * std::max<size_t>(worlds.size(), 1)));
-    dCtr_ = static_cast<DevCounters*>(A(sizeof(DevCounters) * std::max<size_t>(worlds.size(), 1)));
-    dSc_ = static_cast<StepCounters*>(A(sizeof(StepCounters)));
-    for (int b = 0; b < 2; ++b) {
-        HotBuffers& h = buf_[b];
-        h.pos = static_cast<float2*>(A(sizeof(float2) * NC));
-        h.vel = static_cast<float2*>(A(sizeof(float2) * NC));
-        h.dens = static_cast<float*>(A(sizeof(float) * NC));
-        h.flags = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
-        h.slot = static_cast<int*>(A(sizeof(int) * NC));
-        h.btgt = static_cast<int*>(A(sizeof(int) * kMaxBonds * size_t(NC)));
-        h.brest = static_cast<float*>(A(sizeof(float) * kMaxBonds * size_t(NC)));
-        h.bang = static_cast<float*>(A(sizeof(float) * kMaxBonds * size_t(NC)));
-        h.ppos = static_cast<float2*>(A(sizeof(float2) * NP));
-        h.pvel = static_cast<float2*>(A(sizeof(float2) * NP));
-        h.pen = static_cast<float*>(A(sizeof(float) * NP));
-        h.plast = static_cast<int*>(A(sizeof(int) * NP));
-        h.pslot = static_cast<int*>(A(sizeof(int) * NP));
-        h.pflags = static_cast<uint8_t*>(A(NP));
-        h.pid = static_cast<unsigned long long*>(A(sizeof(unsigned long long) * NP));
-    }
-    energy_ = static_cast<float*>(A(sizeof(float) * NC));
-    stiff_ = static_cast<float*>(A(sizeof(float) * NC));
-    cid_ = static_cast<unsigned long long*>(A(sizeof(unsigned long long) * NC));
-    ageBase_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
+    // Everything comes from two allocations, one for the particles' arrays (which growParticles replaces) and
+    // one for the rest: the layout below runs once to add up the sizes and once to hand out the places.
+    struct Places {
+        char* base = nullptr;
+        size_t used = 0;
+        void* operator()(size_t bytes) {
+            char* p = base ? base + used : nullptr;
+            used += (std::max<size_t>(bytes, 64) + 255) & ~size_t(255);
+            return p;
+        }
+    };
+    const size_t NCB = size_t(std::max(cellBins, 1));
+    const size_t groups = NCB / kGroupBins + 1, supers = groups / kSuperGroups + 1;
     bool anyExtra = false;
     for (const auto& h : hosts) anyExtra = anyExtra || h.hasExtra;
-    extra_ = anyExtra ? static_cast<CellExtra*>(A(sizeof(CellExtra) * NC)) : nullptr;
     selected_.assign(hosts.size(), nullptr);
-    for (size_t w = 0; w < hosts.size(); ++w)
-        if (hosts[w].hasSelected) {
-            selected_[w] = static_cast<uint8_t*>(A(hosts[w].particleSelected.size()));
-            check_hip(hipMemcpy(selected_[w], hosts[w].particleSelected.data(), hosts[w].particleSelected.size(),
-                                hipMemcpyHostToDevice),
-                      "H2D");
+    auto layout = [&](Places& A, Places& B) {
+        dWorlds_ = static_cast<DevWorld*>(A(sizeof(DevWorld) * std::max<size_t>(worlds.size(), 1)));
+        dParams_ = static_cast<DevParams*>(A(sizeof(DevParams) * std::max<size_t>(worlds.size(), 1)));
+        dCtr_ = static_cast<DevCounters*>(A(sizeof(DevCounters) * std::max<size_t>(worlds.size(), 1)));
+        dSc_ = static_cast<StepCounters*>(A(sizeof(StepCounters)));
+        for (int b = 0; b < 2; ++b) {
+            HotBuffers& h = buf_[b];
+            h.pos = static_cast<float2*>(A(sizeof(float2) * NC));
+            h.vel = static_cast<float2*>(A(sizeof(float2) * NC));
+            h.dens = static_cast<float*>(A(sizeof(float) * NC));
+            h.flags = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
+            h.slot = static_cast<int*>(A(sizeof(int) * NC));
+            h.btgt = static_cast<int*>(A(sizeof(int) * kMaxBonds * size_t(NC)));
+            h.brest = static_cast<float*>(A(sizeof(float) * kMaxBonds * size_t(NC)));
+            h.bang = static_cast<float*>(A(sizeof(float) * kMaxBonds * size_t(NC)));
+            h.ppos = static_cast<float2*>(B(sizeof(float2) * NP));
+            h.pvel = static_cast<float2*>(B(sizeof(float2) * NP));
+            h.pen = static_cast<float*>(B(sizeof(float) * NP));
+            h.plast = static_cast<int*>(B(sizeof(int) * NP));
+            h.pslot = static_cast<int*>(B(sizeof(int) * NP));
+            h.pflags = static_cast<uint8_t*>(B(NP));
+            h.pid = static_cast<unsigned long long*>(B(sizeof(unsigned long long) * NP));
         }
-    dWords_ = static_cast<unsigned long long*>(A(sizeof(unsigned long long) * 2));
+        energy_ = static_cast<float*>(A(sizeof(float) * NC));
+        stiff_ = static_cast<float*>(A(sizeof(float) * NC));
+        cid_ = static_cast<unsigned long long*>(A(sizeof(unsigned long long) * NC));
+        ageBase_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
+        extra_ = anyExtra ? static_cast<CellExtra*>(A(sizeof(CellExtra) * NC)) : nullptr;
+        for (size_t w = 0; w < hosts.size(); ++w)
+            if (hosts[w].hasSelected) selected_[w] = static_cast<uint8_t*>(A(hosts[w].cells->particleSelected.size()));
+        dWords_ = static_cast<unsigned long long*>(A(sizeof(unsigned long long) * 2));
+        staged_ = partStage_ > 0 ? static_cast<StagedParticle*>(A(sizeof(StagedParticle) * NC)) : nullptr;
+        splitStaged_ = splitStage_ > 0 ? static_cast<StagedParticle*>(B(sizeof(StagedParticle) * size_t(splitStage_))) : nullptr;
+        living_[0] = static_cast<uint8_t*>(A(NC));
+        living_[1] = static_cast<uint8_t*>(A(NC));
+        activation_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
+        creature_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
+        stretched_ = static_cast<uint8_t*>(A(NC));
+        binOf_ = static_cast<int*>(A(sizeof(int) * (size_t(NC) + kBinOfPad)));
+        pbinOf_ = static_cast<int*>(B(sizeof(int) * NP));
+        count_[0] = static_cast<uint32_t*>(A(sizeof(uint32_t) * NB));
+        count_[1] = static_cast<uint32_t*>(A(sizeof(uint32_t) * NB));
+        numCellBins_ = cellBins;
+        farList_ = static_cast<int2*>(A(sizeof(int2) * NC));
+        for (int b = 0; b < 2; ++b) {
+            start_[b] = static_cast<uint32_t*>(A(sizeof(uint32_t) * (size_t(NB) + 1)));
+            far_[b].head = static_cast<int*>(A(sizeof(int) * NCB));
+            far_[b].count = static_cast<int*>(A(sizeof(int) * NCB));
+            far_[b].group = static_cast<int*>(A(sizeof(int) * (NCB / kGroupBins + 1)));
+            far_[b].total = far_[b].group + NCB / kGroupBins;
+            far_[b].list = farList_;
+        }
+        moverNext_ = static_cast<int*>(A(sizeof(int) * NC));
+        groupWorld_ = static_cast<int*>(A(sizeof(int) * NCB / kGroupBins + sizeof(int)));
+        for (int b = 0; b < 2; ++b) {
+            groupSum_[b] = static_cast<int*>(A(sizeof(int) * groups));
+            superSum_[b] = static_cast<int*>(A(sizeof(int) * supers));
+        }
+        mapStatus_ = static_cast<unsigned long long*>(A(sizeof(unsigned long long) * size_t(map_scan_tiles(NB - cellBins) + 1)));
+        mapEpochTicket_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * 2));
+        sorted_ = static_cast<int*>(A(sizeof(int) * NC));
+        mpos_ = static_cast<float2*>(A(sizeof(float2) * NC));
+        mvel_ = static_cast<float2*>(A(sizeof(float2) * NC));
+        mflags_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
+        newidx_ = static_cast<int*>(A(sizeof(int) * NC));
+        psorted_ = static_cast<int*>(B(sizeof(int) * NP));
+        stage_ = static_cast<uint8_t*>(A(NC));
+        own_ = static_cast<float2*>(A(sizeof(float2) * NC));
+        shift_ = static_cast<float2*>(A(sizeof(float2) * NC));
+        bstiff_ = static_cast<float*>(A(sizeof(float) * NC));
+        s2_ = static_cast<float2*>(A(sizeof(float2) * NC));
+        out1_ = static_cast<float2*>(A(sizeof(float2) * kMaxBonds * size_t(NC)));
+        out2_ = static_cast<float2*>(A(sizeof(float2) * kMaxBonds * size_t(NC)));
+        valid_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
+        claim_ = static_cast<unsigned long long*>(A(sizeof(unsigned long long) * NC));
+        cand_ = static_cast<int4*>(A(sizeof(int4) * size_t(candCap_)));
+        want_ = static_cast<int*>(B(sizeof(int) * NP));
+        fclaim_ = static_cast<int*>(B(sizeof(int) * NP));
+        absorbCell_ = static_cast<int*>(B(sizeof(int) * NP));
+        cclaim_ = static_cast<int*>(A(sizeof(int) * NC));
+    };
+    {
+        Places a, b;
+        layout(a, b);
+        Places arena{static_cast<char*>(alloc(a.used))};
+        Places parts{static_cast<char*>(partArena_ = alloc(b.used))};
+        layout(arena, parts);
+    }
     rankOfSlot_ = nullptr;
     rankState_.assign(hosts.size(), 0);
     idBits_.assign(hosts.size(), 0);
     scratch_ = nullptr;
     scratchBytes_ = 0;
-    staged_ = partStage_ > 0 ? static_cast<StagedParticle*>(A(sizeof(StagedParticle) * NC)) : nullptr;
-    splitStaged_ = splitStage_ > 0 ? static_cast<StagedParticle*>(A(sizeof(StagedParticle) * size_t(splitStage_))) : nullptr;
-    living_[0] = static_cast<uint8_t*>(A(NC));
-    living_[1] = static_cast<uint8_t*>(A(NC));
-    activation_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
-    creature_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
-    stretched_ = static_cast<uint8_t*>(A(NC));
-    binOf_ = static_cast<int*>(A(sizeof(int) * (size_t(NC) + kBinOfPad)));
-    pbinOf_ = static_cast<int*>(A(sizeof(int) * NP));
-    count_[0] = static_cast<uint32_t*>(A(sizeof(uint32_t) * NB));
-    count_[1] = static_cast<uint32_t*>(A(sizeof(uint32_t) * NB));
-    numCellBins_ = cellBins;
-    const size_t NCB = size_t(std::max(cellBins, 1));
-    farList_ = static_cast<int2*>(A(sizeof(int2) * NC));
-    for (int b = 0; b < 2; ++b) {
-        start_[b] = static_cast<uint32_t*>(A(sizeof(uint32_t) * (size_t(NB) + 1)));
-        far_[b].head = static_cast<int*>(A(sizeof(int) * NCB));
-        far_[b].count = static_cast<int*>(A(sizeof(int) * NCB));
-        far_[b].group = static_cast<int*>(A(sizeof(int) * (NCB / kGroupBins + 1)));
-        far_[b].total = far_[b].group + NCB / kGroupBins;
-        far_[b].list = farList_;
-    }
-    moverNext_ = static_cast<int*>(A(sizeof(int) * NC));
+    for (size_t w = 0; w < hosts.size(); ++w)
+        if (selected_[w])
+            check_hip(hipMemcpy(selected_[w], hosts[w].cells->particleSelected.data(), hosts[w].cells->particleSelected.size(),
+                                hipMemcpyHostToDevice),
+                      "H2D");
     std::vector<int> groupWorld;
     for (size_t w = 0; w < worlds.size(); ++w) {
         const int64_t groups = (int64_t(worlds[w].nbx) * worlds[w].nby + kGroupBins - 1) / kGroupBins;
         groupWorld.insert(groupWorld.end(), size_t(groups), int(w));
     }
-    groupWorld_ = static_cast<int*>(A(sizeof(int) * std::max<size_t>(groupWorld.size(), 1)));
     if (!groupWorld.empty())
         check_hip(hipMemcpy(groupWorld_, groupWorld.data(), sizeof(int) * groupWorld.size(), hipMemcpyHostToDevice), "H2D");
-    const size_t groups = NCB / kGroupBins + 1, supers = groups / kSuperGroups + 1;
-    for (int b = 0; b < 2; ++b) {
-        groupSum_[b] = static_cast<int*>(A(sizeof(int) * groups));
-        superSum_[b] = static_cast<int*>(A(sizeof(int) * supers));
-    }
-    mapStatus_ = static_cast<unsigned long long*>(A(sizeof(unsigned long long) * size_t(map_scan_tiles(NB - cellBins) + 1)));
-    mapEpochTicket_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * 2));
-    sorted_ = static_cast<int*>(A(sizeof(int) * NC));
-    mpos_ = static_cast<float2*>(A(sizeof(float2) * NC));
-    mvel_ = static_cast<float2*>(A(sizeof(float2) * NC));
-    mflags_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
-    newidx_ = static_cast<int*>(A(sizeof(int) * NC));
-    psorted_ = static_cast<int*>(A(sizeof(int) * NP));
-    stage_ = static_cast<uint8_t*>(A(NC));
-    own_ = static_cast<float2*>(A(sizeof(float2) * NC));
-    shift_ = static_cast<float2*>(A(sizeof(float2) * NC));
-    bstiff_ = static_cast<float*>(A(sizeof(float) * NC));
-    s2_ = static_cast<float2*>(A(sizeof(float2) * NC));
-    out1_ = static_cast<float2*>(A(sizeof(float2) * kMaxBonds * size_t(NC)));
-    out2_ = static_cast<float2*>(A(sizeof(float2) * kMaxBonds * size_t(NC)));
-    valid_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
-    claim_ = static_cast<unsigned long long*>(A(sizeof(unsigned long long) * NC));
-    cand_ = static_cast<int4*>(A(sizeof(int4) * size_t(candCap_)));
-    want_ = static_cast<int*>(A(sizeof(int) * NP));
-    fclaim_ = static_cast<int*>(A(sizeof(int) * NP));
-    absorbCell_ = static_cast<int*>(A(sizeof(int) * NP));
-    cclaim_ = static_cast<int*>(A(sizeof(int) * NC));
 
     // copy world states into buffer 0 (and, from other sets, the split halves still waiting)
     struct PendingCopy {
@@ -754,11 +815,11 @@ void WorldSet::build(const std::vector<Source>& sources) {
             h2d(energy_ + w.cellOff, im.energy.data(), sizeof(float) * n);
             h2d(stiff_ + w.cellOff, im.stiff.data(), sizeof(float) * n);
             static_assert(sizeof(unsigned long long) == sizeof(uint64_t), "cell ids");
-            h2d(cid_ + w.cellOff, im.host.cellId.data(), sizeof(uint64_t) * n);
-            h2d(ageBase_ + w.cellOff, im.host.age.data(), sizeof(uint32_t) * n);
-            h2d(living_[0] + w.cellOff, im.host.livingState.data(), n);
-            h2d(activation_ + w.cellOff, im.host.activationTime.data(), sizeof(uint32_t) * n);
-            h2d(creature_ + w.cellOff, im.host.creatureId.data(), sizeof(uint32_t) * n);
+            h2d(cid_ + w.cellOff, im.host.cells->cellId.data(), sizeof(uint64_t) * n);
+            h2d(ageBase_ + w.cellOff, im.host.cells->age.data(), sizeof(uint32_t) * n);
+            h2d(living_[0] + w.cellOff, im.host.cells->livingState.data(), n);
+            h2d(activation_ + w.cellOff, im.host.cells->activationTime.data(), sizeof(uint32_t) * n);
+            h2d(creature_ + w.cellOff, im.host.cells->creatureId.data(), sizeof(uint32_t) * n);
             h2d(D.ppos + w.partOff, im.ppos.data(), sizeof(float2) * np);
             h2d(D.pvel + w.partOff, im.pvel.data(), sizeof(float2) * np);
             h2d(D.pen + w.partOff, im.pen.data(), sizeof(float) * np);
@@ -807,11 +868,11 @@ void WorldSet::build(const std::vector<Source>& sources) {
             const HostWorld& h = hosts[wi];
             std::vector<CellExtra> x(static_cast<size_t>(h.numCells));
             for (size_t k = 0; k < x.size(); ++k) {
-                std::memcpy(&x[k].genomeComplexity, &h.genomeComplexity[k], sizeof(uint32_t));
-                x[k].mutationId = h.mutationId[k];
-                x[k].cellFunction = h.cellFunction[k];
-                x[k].ancestorMutationId = h.ancestorMutationId[k];
-                x[k].selected = h.selected[k];
+                std::memcpy(&x[k].genomeComplexity, &h.cells->genomeComplexity[k], sizeof(uint32_t));
+                x[k].mutationId = h.cells->mutationId[k];
+                x[k].cellFunction = h.cells->cellFunction[k];
+                x[k].ancestorMutationId = h.cells->ancestorMutationId[k];
+                x[k].selected = h.cells->selected[k];
             }
             if (!x.empty())
                 check_hip(hipMemcpy(extra_ + worlds[wi].cellOff, x.data(), sizeof(CellExtra) * x.size(), hipMemcpyHostToDevice),
@@ -887,9 +948,9 @@ void WorldSet::build(const std::vector<Source>& sources) {
 
 // Strip shape of the neighbour pass for one world, measured on the given positions.  Only
 // performance depends on it.
-int choose_strip(const std::vector<float2>& pos, int W, int H, int binSize, bool twoRowStages, int& rowsPerStage) {
+HostArray<int> bin_cells(const HostArray<float2>& pos, int W, int H, int binSize) {
     const int nbx = W / binSize, nby = H / binSize;
-    std::vector<int> cnt(size_t(nbx) * nby, 0);
+    HostArray<int> cnt(size_t(nbx) * nby, 0);
     for (const float2& p : pos) {
         int sx = host_floor_int(p.x), sy = host_floor_int(p.y);
         sx = ((sx % W) + W) % W;
@@ -897,10 +958,14 @@ int choose_strip(const std::vector<float2>& pos, int W, int H, int binSize, bool
         const int bx = std::min(sx / binSize, nbx - 1), by = std::min(sy / binSize, nby - 1);
         ++cnt[size_t(by) * nbx + bx];
     }
+    return cnt;
+}
+
+int choose_strip(size_t cells, const HostArray<int>& cnt, int nbx, int nby, bool twoRowStages, int& rowsPerStage) {
     // sparse rows (fewer than half a wave of cells per bin row of a strip on average) are staged
     // two at a time; a chunk where that overflows runs single rows
     auto stages = [&](int sw) {
-        const double perRow = double(pos.size()) / (double(nby) * double((nbx + sw - 1) / sw));
+        const double perRow = double(cells) / (double(nby) * double((nbx + sw - 1) / sw));
         return twoRowStages && perRow < 32.0 && nby % 2 == 0 && nby >= 6 ? 2 : 1;
     };
     // entries of every staged row as the neighbour pass stages it (interior plus the two halo
@@ -911,11 +976,10 @@ int choose_strip(const std::vector<float2>& pos, int W, int H, int binSize, bool
         bool fits = true;
         std::vector<int> rows(static_cast<size_t>(nby));
         for (int x0 = 0; x0 < nbx && fits; x0 += sw) {
-            const int HX = std::min(sw, nbx - x0) + 2;
+            const int x1 = std::min(x0 + sw, nbx);
             for (int y = 0; y < nby; ++y) {
-                int n = 0;
-                for (int hx = 0; hx < HX; ++hx) n += cnt[size_t(y) * nbx + (x0 - 1 + hx + nbx) % nbx];
-                rows[size_t(y)] = n;
+                const int* row = cnt.data() + size_t(y) * nbx;
+                rows[size_t(y)] = std::accumulate(row + x0, row + x1, row[(x0 - 1 + nbx) % nbx] + row[x1 % nbx]);
             }
             for (int y = 0; y < nby && fits; ++y) {
                 const int three = rows[size_t(y)] + rows[size_t((y + 1) % nby)] + rows[size_t((y + 2) % nby)];
@@ -1003,13 +1067,15 @@ void WorldSet::buildTables() {
         }
         for (int s = 0; s < w.pnbx * w.pnby; s += bt) pbins.push_back(make_int2(wi, w.pbinOff + s));
     }
-    auto up = [&](const std::vector<int2>& v) -> int2* {
-        if (v.empty()) return nullptr;
-        void* p = nullptr;
-        check_hip(hipMalloc(&p, sizeof(int2) * v.size()), "hipMalloc");
-        tableAllocs_.push_back({p, sizeof(int2) * v.size()});
-        check_hip(hipMemcpy(p, v.data(), sizeof(int2) * v.size(), hipMemcpyHostToDevice), "H2D");
-        return static_cast<int2*>(p);
+    // (one allocation and one copy for all tables)
+    std::vector<int2> all;
+    std::vector<std::pair<int2**, size_t>> places;
+    auto up = [&](int2*& table, const std::vector<int2>& v) {
+        table = nullptr;
+        if (v.empty()) return;
+        places.push_back({&table, all.size()});
+        all.insert(all.end(), v.begin(), v.end());
+        all.resize((all.size() + 31) / 32 * 32);
     };
     // neighbour-pass tiles, row-major per world; workgroup b runs on XCD b % 8, so each XCD gets
     // one contiguous run of tiles and the halo rows its tiles share stay in that XCD's L2
@@ -1048,20 +1114,26 @@ void WorldSet::buildTables() {
     {
         std::vector<int2> table(std::max<size_t>(partCapBlocks, 1), make_int2(0, 0));
         std::copy(parts.begin(), parts.end(), table.begin());
-        partBlocks_ = up(table);
-        const std::vector<int2> count(1, make_int2(int(parts.size()), 0));
-        numPartBlocks_ = reinterpret_cast<int*>(up(count));
+        up(partBlocks_, table);
     }
+    int2* count = nullptr;
+    up(count, {make_int2(int(parts.size()), 0)});
     shape_.partGrid = int(std::max<int64_t>(64, std::min<int64_t>(65536, (live + pt - 1) / pt + (radCells / 8 + pt - 1) / pt)));
-    cellBlocks_ = up(cells);
-    bondBlocks_ = up(bonds);
-    pbinBlocks_ = up(pbins);
-    tileBlocks_ = up(tileTable);
-    livingBlocks_ = up(living);
-    edgeBlocks_ = up(edges);
+    up(cellBlocks_, cells);
+    up(bondBlocks_, bonds);
+    up(pbinBlocks_, pbins);
+    up(tileBlocks_, tileTable);
+    up(livingBlocks_, living);
+    up(edgeBlocks_, edges);
     shape_.edgeBlocks = int(edges.size());
-    fluidBlocks_ = up(fluids);
+    up(fluidBlocks_, fluids);
     shape_.fluidBlocks = int(fluids.size());
+    void* p = nullptr;
+    check_hip(hipMalloc(&p, sizeof(int2) * all.size()), "hipMalloc");
+    tableAllocs_.push_back({p, sizeof(int2) * all.size()});
+    check_hip(hipMemcpy(p, all.data(), sizeof(int2) * all.size(), hipMemcpyHostToDevice), "H2D");
+    for (const auto& at : places) *at.first = static_cast<int2*>(p) + at.second;
+    numPartBlocks_ = reinterpret_cast<int*>(count);
     shape_.livingBlocks = int(living.size());
     shape_.cellBlocks = int(cells.size());
     shape_.bondBlocks = int(bonds.size());
@@ -1490,9 +1562,8 @@ bool radiates(const alien_params& p) {
 
 // Reads the last step's candidate-list size: reports overflow and grows the grid of the fusion
 // kernels when the list outgrew it (the graphs are captured again on the next step).
-void WorldSet::checkErrors() {
-    StepCounters sc{};
-    check_hip(hipMemcpy(&sc, dSc_, sizeof(sc), hipMemcpyDeviceToHost), "D2H");
+// (what the last step left in the counters)
+void WorldSet::checkErrors(StepCounters sc) {
     if (sc.errors & 1) {
         sc.errors = 0;
         check_hip(hipMemcpy(dSc_, &sc, sizeof(sc), hipMemcpyHostToDevice), "H2D");
@@ -1574,10 +1645,15 @@ void WorldSet::step(uint64_t n) {
     }
     for (size_t i = 0; i < hosts_.size(); ++i)
         if (active_[i]) hosts_[i].stepsSinceSet += n;  // (an inactive world is frozen)
+    check_hip(hipMemcpyAsync(hostSc_, dSc_, sizeof(*hostSc_), hipMemcpyDeviceToHost, stream_), "D2H");
     synchronize();
     if (timing_) recorder_->collect(kernelTimes_);
-    checkErrors();
-    if (shape_.hasParticles) dropParticlesIfNone();
+    checkErrors(*hostSc_);
+    livePending_ = false;  // (a read in flight has landed; the count of the last step is newer)
+    if (shape_.hasParticles && hostSc_->liveParticles == 0 && !shape_.hasRadiation) {
+        shape_.hasParticles = false;
+        invalidateGraphs();
+    }
 }
 
 void WorldSet::checkParticlesAsync() {
@@ -1601,17 +1677,6 @@ void WorldSet::checkParticlesAsync() {
                   "hipMemcpyAsync");
         check_hip(hipEventRecord(liveReady_, stream_), "hipEventRecord");
         livePending_ = true;
-    }
-}
-
-void WorldSet::dropParticlesIfNone() {
-    synchronize();
-    livePending_ = false;  // (a read in flight has landed; the count below is newer)
-    StepCounters sc{};
-    check_hip(hipMemcpy(&sc, dSc_, sizeof(sc), hipMemcpyDeviceToHost), "D2H");
-    if (sc.liveParticles == 0 && !shape_.hasRadiation) {
-        shape_.hasParticles = false;
-        invalidateGraphs();
     }
 }
 
@@ -1721,6 +1786,8 @@ void WorldSet::growParticles(const std::vector<int64_t>& caps) {
     for (void* p : {static_cast<void*>(pbinOf_), static_cast<void*>(psorted_), static_cast<void*>(want_),
                     static_cast<void*>(fclaim_), static_cast<void*>(absorbCell_), static_cast<void*>(splitStaged_)})
         if (p) release(p);
+    if (partArena_) release(partArena_);  // (the arrays the set was built with)
+    partArena_ = nullptr;
     splitStaged_ = splitStaged;
     pbinOf_ = pbinOf;
     psorted_ = static_cast<int*>(alloc(sizeof(int) * NP));
@@ -1779,21 +1846,24 @@ void WorldSet::extract(int wi, WorldImage& img) {
     // one per step to every non-barrier cell; a world with livingWork has its states and counts on
     // the device, any other world is Ready without counts throughout (its barrier cells too)
     HostWorld& h = img.host;
+    auto own = std::make_shared<HostCells>(*h.cells);
     img.livingWork = livingWork_.at(wi) != 0;
     if (img.livingWork) {
-        d2h(h.livingState.data(), living_[parity_] + w.cellOff, size_t(n));
-        d2h(h.activationTime.data(), activation_ + w.cellOff, sizeof(uint32_t) * n);
+        d2h(own->livingState.data(), living_[parity_] + w.cellOff, size_t(n));
+        d2h(own->activationTime.data(), activation_ + w.cellOff, sizeof(uint32_t) * n);
     }
     if (h.stepsSinceSet > 0)
         for (int i = 0; i < n; ++i) {
             const int sl = img.slot[i];
             if (flags_barrier(img.flags[i])) {
-                h.livingState[sl] = 0;
+                own->livingState[sl] = 0;
                 continue;
             }
-            h.age[sl] = uint32_t(uint64_t(h.age[sl]) + h.stepsSinceSet);
+            own->age[sl] = uint32_t(uint64_t(own->age[sl]) + h.stepsSinceSet);
         }
     h.stepsSinceSet = 0;
+    h.cells = std::move(own);
+    img.binCells.clear();
     img.ppos.resize(np);
     img.pvel.resize(np);
     img.pen.resize(np);

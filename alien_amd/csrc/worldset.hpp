@@ -47,10 +47,28 @@ bool splits(const alien_params& p);
 // (one particle per cell and step at most), doubled when its particles can split
 int64_t particle_room(int64_t cells, int64_t particles, const alien_params& p);
 DevParams to_dev_params(const alien_params& p);
-int choose_strip(const std::vector<float2>& pos, int W, int H, int binSize, bool twoRowStages, int& rowsPerStage);
 void strip_shape(DevWorld& w, int strip, int rowsPerStage);
 void chunk_shape(std::vector<DevWorld>& worlds, const std::vector<DevParams>& params, int forcedRows = 0);
 constexpr int kXcds = kXcdCount;  // accelerator complex dies of an MI355X
+
+// A vector whose resize leaves new elements of plain types unset: what is filled right after is written once,
+// by the threads that fill it.
+template <class T> struct UnsetAllocator : std::allocator<T> {
+    template <class U> struct rebind { using other = UnsetAllocator<U>; };
+    template <class U> void construct(U* p) { ::new (static_cast<void*>(p)) U; }
+    template <class U, class... A> void construct(U* p, A&&... a) { ::new (static_cast<void*>(p)) U(std::forward<A>(a)...); }
+};
+template <class T> using HostArray = std::vector<T, UnsetAllocator<T>>;
+
+// the cells' and particles' part of HostWorld (cells by slot)
+struct HostCells {
+    HostArray<uint64_t> cellId;
+    HostArray<uint32_t> age, creatureId, mutationId, activationTime;
+    HostArray<uint8_t> livingState, cellFunction, ancestorMutationId, selected;
+    HostArray<float> genomeComplexity;
+    HostArray<uint64_t> particleId;
+    HostArray<uint8_t> particleSelected;
+};
 
 // host-side identity and pass-through data of one world (fields the physics path never touches).
 // age, activationTime and livingState hold the values at the last set (stepsSinceSet steps ago):
@@ -62,12 +80,7 @@ struct HostWorld {
     int numCells = 0;
     int particleCap = 0;
     uint64_t stepsSinceSet = 0;
-    std::vector<uint64_t> cellId;
-    std::vector<uint32_t> age, creatureId, mutationId, activationTime;
-    std::vector<uint8_t> livingState, cellFunction, ancestorMutationId, selected;
-    std::vector<float> genomeComplexity;
-    std::vector<uint64_t> particleId;
-    std::vector<uint8_t> particleSelected;
+    std::shared_ptr<const HostCells> cells;  // shared by the images and sets it went through
     bool hasExtra = false;     // some cell has a non-zero CellExtra field
     bool hasSelected = false;  // some particle is selected
 };
@@ -78,19 +91,20 @@ struct WorldImage {
     uint64_t timestep = 0;
     int numParticles = 0;
     bool densityResetPending = false;
-    std::vector<float2> pos, vel;
-    std::vector<float> dens;
-    std::vector<uint32_t> flags;
-    std::vector<int> slot;
-    std::vector<int> btgt;  // [kMaxBonds][numCells]
-    std::vector<float> brest, bang;
-    std::vector<float> energy, stiff;  // by slot
-    bool livingWork = false;           // living states tracked on the device (see WorldSet::build)
-    std::vector<float2> ppos, pvel;
-    std::vector<float> pen;
-    std::vector<int> plast, pslot;
-    std::vector<uint8_t> pflags;
-    std::vector<uint64_t> pid;  // particle ids
+    HostArray<float2> pos, vel;
+    HostArray<float> dens;
+    HostArray<uint32_t> flags;
+    HostArray<int> slot;
+    HostArray<int> btgt;  // [kMaxBonds][numCells]
+    HostArray<float> brest, bang;
+    HostArray<float> energy, stiff;  // by slot
+    HostArray<int> binCells;         // cells per bin of the cell map; may be left empty
+    bool livingWork = false;         // living states tracked on the device (see WorldSet::build)
+    HostArray<float2> ppos, pvel;
+    HostArray<float> pen;
+    HostArray<int> plast, pslot;
+    HostArray<uint8_t> pflags;
+    HostArray<uint64_t> pid;  // particle ids
 
     // from transfer objects (ObjectFactory.cuh:46-86: positions wrapped, density 1)
     static WorldImage fromTO(const alien_world_desc& desc, const alien_params& params, const alien_cell_to* cells,
@@ -100,6 +114,11 @@ struct WorldImage {
     // livingWork for the image's current states, energies and parameters (once set, it stays set)
     void updateLivingWork();
 };
+
+// cells per bin of positions on the torus
+HostArray<int> bin_cells(const HostArray<float2>& pos, int W, int H, int binSize);
+// neighbour-pass strip width for these cells per bin (`cells` in all)
+int choose_strip(size_t cells, const HostArray<int>& binCells, int nbx, int nby, bool twoRowStages, int& rowsPerStage);
 
 class WorldSet {
 public:
@@ -193,8 +212,7 @@ private:
     void invalidateGraphs();
     Ctx makeCtx(int parity) const;
     void ensureSorted();
-    void checkErrors();
-    void dropParticlesIfNone();  // stops launching the particle kernels once no particle is left
+    void checkErrors(StepCounters sc);
     // the same without a host synchronisation: acts on the count read at the previous call (if it
     // has arrived) and starts reading the current one
     void checkParticlesAsync();
@@ -219,6 +237,7 @@ private:
     SideStream side_;  // particle kernels beside the neighbour pass
     int* liveHost_ = nullptr;        // pinned: live particles as read by checkParticlesAsync
     unsigned long long* hostWord_ = nullptr;  // pinned, behind it: words and counters read back
+    StepCounters* hostSc_ = nullptr;          // pinned, behind that: the step counters
     hipEvent_t liveReady_ = nullptr;  // recorded after that read
     bool livePending_ = false;
     std::vector<HostWorld> hosts_;
@@ -267,6 +286,7 @@ private:
     uint32_t* start_[2] = {nullptr, nullptr};
     FarCells far_[2] = {};
     int2* farList_ = nullptr;
+    void* partArena_ = nullptr;  // the particles' arrays as built, null once they have grown
     int* groupWorld_ = nullptr;
     int* groupSum_[2] = {nullptr, nullptr};
     int* superSum_[2] = {nullptr, nullptr};

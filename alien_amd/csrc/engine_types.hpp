@@ -33,6 +33,13 @@ constexpr uint32_t kBinMask = (1u << kMoveShift) - 1u, kFarCode = 15u, kFarMove 
 constexpr int kGroupBins = 256;    // bins per wave of the cells' map; a world's bins are padded to a multiple
 constexpr int kBinOfPad = 576;     // entries of binOf that may be read (and not used) past the last cell
 constexpr int kSuperGroups = 256;  // groups per sum of groups
+// Cells per wave of the fluid pass, as a power of two: 64, and in sets with fewer than a wave per SIMD (1024)
+// half as many, down to 16, as long as they give a SIMD one wave at most.  The pass is one wave's latency
+// there (10751 cells in bodies: a step of 106 us with 64, 97 with 32, 92 with 16); with more cells the
+// wave's fixed work counts (134k cells in bodies: 159, 157 and 162 us; 256k free ones: 22, 26 and 32 us).
+constexpr int kFluidShiftMin = 4;
+// waves of the fluid pass for a row's two edge bins (k_fluid.hip), without and with bond work
+constexpr int kEdgeWaves = 2, kEdgeWavesBonds = 8;
 constexpr int kXcdCount = 8;  // XCDs of an MI355X: workgroup b of a launch runs on XCD b % 8
 // Size limits of one world set.  Cell indices, bin offsets and the bond planes ([kMaxBonds][cap],
 // addressed as b * cap + x) are 32-bit ints in the kernels, so a set holds at most
@@ -286,7 +293,8 @@ struct Ctx {
     int* numPartBlocks;
     int partBlockParticles;
     const int2* fluidBlocks;  // per workgroup of the fluid pass: (world, its first wave)
-    const int2* edgeBlocks;  // per workgroup: (world, its first wave's edge unit and half), see k_fluid.hip
+    int fluidShift;           // its waves take 1 << fluidShift cells
+    const int2* edgeBlocks;  // per workgroup: (world, its first wave's edge unit and part), see k_fluid.hip
     const int2* tileBlocks;  // per block: (world, tile index), -1 for padding blocks
     const int2* livingBlocks;  // per block: (world, first global cell index) over livingWork worlds
     int blockThreads;  // cells, bins or living cells per entry of the block tables above

@@ -20,10 +20,13 @@
 // address costs four operations), 1 / density is stored instead of the density, and sets without bond
 // work run a variant without flags, bonds, barriers and fusion.
 // Steps of a fluid world before (lists cut and pairs compacted per 64-candidate round, edge cells alone
-// in their lanes) and now: 1M cells 35 -> 26.5 us, 4M 172 -> 168 us, 4M in bodies with bonds 331 -> 314 us.
+// in their lanes) and now, with the map as it was: 256k cells 35 -> 26.5 us, 4M 172 -> 168 us.
+// Records for all pairs of a wave in bodies (the tests ran up to five times before): 134k cells 158 -> 152
+// us, with the edge waves and fewer cells per wave (kFluidShiftMin) 10751 cells 108 -> 91.5 us.
 //
 // Cells of the first and last bin column have a stencil that wraps around the torus: their ranges
-// come in two pieces.  They are left to waves of their own, two for each row's pair of edge bins, that
+// come in two pieces.  They are left to waves of their own, two for each row's pair of edge bins (eight with
+// bond work: the cells of a body there, one after the other, took 16 of 32 us of a small world), that
 // take a cell at a time with its candidates side by side; walked alone by a lane of the pass, they
 // were its last waves to end.  Cells with more than 64 candidates walk their stencil alone.
 #include "kernels.hpp"
@@ -36,12 +39,14 @@ constexpr int kFluidWaves = 4;   // waves per workgroup at most
 // staged candidates of the three stencil rows: three rows of 66 bins at one cell per bin; with bonds,
 // bodies of four cells a bin next to empty space
 constexpr int kFreeStage = 288, kBondStage = 448;
-constexpr int kFluidPairs = 128;  // pair records at a time
+// pair records at a time: a fluid's cells have about one each at one cell per bin; with bonds, bodies with
+// ten neighbours a cell (the tests run again for what does not fit)
+constexpr int kFreePairs = 128, kBondPairs = 896;
 constexpr int kEdgeAlone = 16;    // more edge cells than this in a unit walk alone, one per lane
 
 // LDS of one wave: 6 KB (9.9 KB with bonds), six (four) waves per SIMD (the owners' velocities,
 // densities and flags come from their registers, by cross-lane permutes)
-template <int kStage> struct FluidShared {
+template <int kStage, int kPairs> struct FluidShared {
     // staged candidates: their positions, and behind them their A indices (the last round of tests reads
     // up to 63 positions past the last list, and counts nothing there)
     float2 cpos[kStage + kStage / 2];
@@ -49,7 +54,7 @@ template <int kStage> struct FluidShared {
     float2 pos[64];  // the wave's own cells; no position for a lane that does not test
     uint16_t first[65];  // each owner's first pair
     uint16_t own[64];    // pairs up to the owner's own place in its list
-    uint16_t pair[kFluidPairs];  // pair records: staged neighbour, owner << 9
+    uint16_t pair[kPairs];  // pair records: staged neighbour, owner << 9
     union {
         struct {
             // per list: its row boundaries (flat, two 16-bit halves) and what to add to a flat index
@@ -63,6 +68,9 @@ template <int kStage> struct FluidShared {
         } r;
     } u;
 };
+template <bool kBonds>
+using FluidWave = FluidShared<kBonds ? kBondStage : kFreeStage, kBonds ? kBondPairs : kFreePairs>;
+static_assert(sizeof(FluidWave<true>) <= 10240 && sizeof(FluidWave<false>) <= 6826, "16 and 24 waves per CU");
 static_assert(kBondStage <= 512 && kFreeStage >= 126, "9-bit staged entries; room to read past the last list");
 
 __device__ __forceinline__ int lanes_below(unsigned long long mask, int add) {
@@ -166,18 +174,19 @@ __device__ __forceinline__ void walk_alone(const Ctx& c, int wi, int m) {
 // The cells of the edge unit u: the last bin of row u - 1 and the first bin of row u, one after the
 // other in the map; the unit's two waves take every other cell.  Returns the cells left to walk alone:
 // this lane's first one, and the end.
-template <bool kBonds> __device__ __forceinline__ int2 edge_unit(const Ctx& c, int wi, int u, int half) {
+template <bool kBonds> __device__ __forceinline__ int2 edge_unit(const Ctx& c, int wi, int u, int part) {
+    constexpr int kWaves = kBonds ? kEdgeWavesBonds : kEdgeWaves;
     const DevWorld& w = c.worlds[wi];
     const DevParams& P = c.params[wi];
     const int lane = int(threadIdx.x) & 63;
     const uint32_t* start = c.start + w.binOff;
     const int off = w.cellOff - int(start[0]);
     const int m0 = off + int(start[max(u * w.nbx - 1, 0)]), m1 = off + int(start[u < w.nby ? u * w.nbx + 1 : u * w.nbx]);
-    if (m1 - m0 > kEdgeAlone) return make_int2(half == 0 ? m0 + lane : m1, m1);
+    if (m1 - m0 > kEdgeAlone) return make_int2(part == 0 ? m0 + lane : m1, m1);
     const float Wf = float(w.W), Hf = float(w.H), reachSq = P.reachSq;
     const float w0 = sph_w(0.0f) * P.invH2;
     uint32_t crowded = 0u;  // cells with more than 64 candidates
-    for (int m = m0 + half; m < m1; m += 2) {
+    for (int m = m0 + part; m < m1; m += kWaves) {
         const Nb s = map_nb(c, m);  // (the same on every lane)
         int bx, by;
         cell_bin_xy(w, s.pos, bx, by);
@@ -257,12 +266,12 @@ template <bool kBonds> __device__ __forceinline__ int2 edge_unit(const Ctx& c, i
     return make_int2((crowded >> lane) & 1u && lane < kEdgeAlone ? m0 + lane : m1, m1);
 }
 
-// Wave v of the world: 64 consecutive map positions of the first bin row, of the last one, or of those
+// Wave v of the world: 64 (fewer in small sets, fluidShift) consecutive map positions of the first bin row, of the last one, or of those
 // between (each of the three parts has its own last wave, so that no wave has lanes whose stencil rows
 // are at different ends of the map).  Returns the map position that this lane is left to walk alone, or -1.
 template <bool kBonds>
-__device__ __forceinline__ int fluid_wave(const Ctx& c, FluidShared<kBonds ? kBondStage : kFreeStage>& S, int wi, int v) {
-    constexpr int kStage = kBonds ? kBondStage : kFreeStage;
+__device__ __forceinline__ int fluid_wave(const Ctx& c, FluidWave<kBonds>& S, int wi, int v) {
+    constexpr int kStage = kBonds ? kBondStage : kFreeStage, kPairs = kBonds ? kBondPairs : kFreePairs;
     const int lane = int(threadIdx.x) & 63;
     // the world and its parameters are read once, before any store: read through references,
     // every use after a global store would load them again
@@ -273,9 +282,11 @@ __device__ __forceinline__ int fluid_wave(const Ctx& c, FluidShared<kBonds ? kBo
     int m0, mEnd;
     {
         const int r1 = int(start[w.nbx] - start[0]), r2 = int(start[(w.nby - 1) * w.nbx] - start[0]);
-        const int v1 = (r1 + 63) / 64, v2 = v1 + (r2 - r1 + 63) / 64;
-        m0 = w.cellOff + (v < v1 ? 64 * v : (v < v2 ? r1 + 64 * (v - v1) : r2 + 64 * (v - v2)));
-        mEnd = w.cellOff + (v < v1 ? r1 : (v < v2 ? r2 : w.numCells));
+        const int sh = c.fluidShift, more = (1 << sh) - 1;
+        const int v1 = (r1 + more) >> sh, v2 = v1 + ((r2 - r1 + more) >> sh);
+        const int at = v < v1 ? v << sh : (v < v2 ? r1 + ((v - v1) << sh) : r2 + ((v - v2) << sh));
+        m0 = w.cellOff + at;
+        mEnd = w.cellOff + min(at + more + 1, v < v1 ? r1 : (v < v2 ? r2 : w.numCells));
     }
     if (P.motion != 0 || m0 >= mEnd) return -1;  // (a wave past its world)
     const int m = m0 + lane;
@@ -393,7 +404,7 @@ __device__ __forceinline__ int fluid_wave(const Ctx& c, FluidShared<kBonds ? kBo
         const int flat = inc - nt, flatAll = wave_last(inc);
         const int selfBase = m0 - u0[1] + un[0];  // the own entry of lane 0
         int numPairs = 0;
-        for (int R0 = 0;; R0 += kFluidPairs) {
+        for (int R0 = 0;; R0 += kPairs) {
             {
                 int4 rec = make_int4(flat | flat << 16, -flat, -flat, -flat);
                 if (tests) {
@@ -437,9 +448,9 @@ __device__ __forceinline__ int fluid_wave(const Ctx& c, FluidShared<kBonds ? kBo
                     if (__builtin_amdgcn_inverse_ballot_w64(starts)) S.first[owner] = uint16_t(rank);
                     if (self) S.own[owner] = uint16_t(rank);
                     // (a wave's pairs nearly always fit one window: then no lane asks)
-                    if (R0 == 0 && numPairs + __builtin_popcountll(hits) <= kFluidPairs) {
+                    if (R0 == 0 && numPairs + __builtin_popcountll(hits) <= kPairs) {
                         if (hit) S.pair[rank] = uint16_t(x | owner << 9);
-                    } else if (hit && uint32_t(rank - R0) < uint32_t(kFluidPairs)) {
+                    } else if (hit && uint32_t(rank - R0) < uint32_t(kPairs)) {
                         S.pair[rank - R0] = uint16_t(x | owner << 9);
                     }
                     numPairs += __builtin_popcountll(hits);
@@ -453,7 +464,7 @@ __device__ __forceinline__ int fluid_wave(const Ctx& c, FluidShared<kBonds ? kBo
             __syncwarp();
             const int pairs0 = S.first[lane], pairs1 = S.first[lane + 1];
             const int ownAt = kBonds && flags_barrier(flags) ? -1 : S.own[lane];
-            const int rend = min(numPairs, R0 + kFluidPairs);
+            const int rend = min(numPairs, R0 + kPairs);
             for (int p0 = R0; p0 < rend; p0 += 64) {
                 // pair terms, one pair per lane
                 float4 ra = make_float4(0.0f, 0.0f, 0.0f, 0.0f), rb = ra;
@@ -543,7 +554,7 @@ __device__ __forceinline__ int fluid_wave(const Ctx& c, FluidShared<kBonds ? kBo
                     acc.Fv = add(acc.Fv, f2{tb.z, tb.w});
                 }
             }
-            if (R0 + kFluidPairs >= numPairs) {
+            if (R0 + kPairs >= numPairs) {
                 if (tests && ownAt == pairs1) acc.rho = acc.rho + w0;  // the own term after all pairs
                 break;
             }
@@ -572,7 +583,7 @@ __device__ __forceinline__ int fluid_wave(const Ctx& c, FluidShared<kBonds ? kBo
 template <bool kBonds>
 __global__ void __launch_bounds__(64 * kFluidWaves) __attribute__((amdgpu_waves_per_eu(kBonds ? 4 : 6)))
 k_fluid(Ctx c, int sortBlocks, int edgeBlocks, int tableBlocks) {
-    __shared__ FluidShared<kBonds ? kBondStage : kFreeStage> SS[kFluidWaves];
+    __shared__ FluidWave<kBonds> SS[kFluidWaves];
     const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
     int block = int(blockIdx.x);
     if constexpr (kBonds) {
@@ -584,8 +595,9 @@ k_fluid(Ctx c, int sortBlocks, int edgeBlocks, int tableBlocks) {
     if (block < edgeBlocks) {
         const int2 blk = c.edgeBlocks[block];
         wi = blk.x;
+        constexpr int kWaves = kBonds ? kEdgeWavesBonds : kEdgeWaves;
         const int u = blk.y + wave;
-        if (u / 2 <= c.worlds[wi].nby) walk = edge_unit<kBonds>(c, wi, u / 2, u % 2);
+        if (u / kWaves <= c.worlds[wi].nby) walk = edge_unit<kBonds>(c, wi, u / kWaves, u % kWaves);
     } else {
         block -= edgeBlocks;
         // XCD-aware: workgroup b runs on XCD b % 8, which sweeps one contiguous band of the map, so the

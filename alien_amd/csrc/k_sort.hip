@@ -14,8 +14,8 @@
 // (Recording every mover in a list of its new bin and counting it out of the old one cost three
 // device-scope atomics each, which the memory side executes: 40 of 143 us of the fluid pass with 4M
 // cells; clearing those lists and a scan over all bins with tiles that wait for the tiles before them,
-// 34 us more.  Steps then and now: 256k cells 26.5 and 22.1 us, 4M 168 and 139 us, 4M in bodies with
-// bonds 314 and 300 us.  A launch of its own that counts the groups took 18 us at 4M.)
+// 34 us more.  Steps then and now: 256k cells 26.5 and 22.1 us, 4M 168 and 139 us, 0.84M in bodies
+// with bonds 314 and 300 us.  A launch of its own that counts the groups took 18 us at 4M.)
 // Only cells that moved further, or across the torus' edge, or that are in no map yet are entered in a
 // list per bin ("far").  Particles: counted with atomics, scattered, then sorted inside their bins.
 #include "kernels.hpp"

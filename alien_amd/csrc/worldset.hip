@@ -1053,6 +1053,14 @@ void WorldSet::buildTables() {
     tableAllocs_.clear();
     std::vector<int2> cells, bonds, pbins, parts, living, edges, fluids;
     const int ct = shape_.cellThreads, pt = shape_.partThreads, bt = shape_.binThreads;
+    int64_t fluidCells = 0;
+    for (int wi = 0; wi < int(worlds_.size()); ++wi)
+        if (active_[wi] && params_[wi].motion == 0) fluidCells += worlds_[wi].numCells;
+    fluidShift_ = 6;
+    while (fluidShift_ > kFluidShiftMin && fluidCells >> (fluidShift_ - 1) <= 1024) --fluidShift_;
+    bool bondWork = false;
+    for (int wi = 0; wi < int(worlds_.size()); ++wi) bondWork = bondWork || (active_[wi] && bondWork_[wi] && worlds_[wi].numCells > 0);
+    const int edgeWaves = bondWork ? kEdgeWavesBonds : kEdgeWaves;
     for (int wi = 0; wi < int(worlds_.size()); ++wi) {
         if (!active_[wi]) continue;
         const DevWorld& w = worlds_[wi];
@@ -1062,8 +1070,8 @@ void WorldSet::buildTables() {
         if (livingWork_[wi])
             for (int s = 0; s < w.numCells; s += ct) living.push_back(make_int2(wi, w.cellOff + s));
         if (params_[wi].motion == 0 && w.numCells > 0) {  // waves of the fluid pass, see k_fluid.hip
-            for (int s = 0; s < 2 * (w.nby + 1); s += ct / 64) edges.push_back(make_int2(wi, s));
-            for (int s = 0; s < (w.numCells + 63) / 64 + 2; s += ct / 64) fluids.push_back(make_int2(wi, s));
+            for (int s = 0; s < edgeWaves * (w.nby + 1); s += ct / 64) edges.push_back(make_int2(wi, s));
+            for (int s = 0; s < (w.numCells >> fluidShift_) + 3; s += ct / 64) fluids.push_back(make_int2(wi, s));
         }
         for (int s = 0; s < w.pnbx * w.pnby; s += bt) pbins.push_back(make_int2(wi, w.pbinOff + s));
     }
@@ -1138,7 +1146,7 @@ void WorldSet::buildTables() {
     shape_.cellBlocks = int(cells.size());
     shape_.bondBlocks = int(bonds.size());
     // the bond kernels run when an active world can have a bonded or barrier cell
-    shape_.hasBondWork = !bonds.empty();
+    shape_.hasBondWork = bondWork;
     shape_.partBlocks = int(partCapBlocks);
     shape_.pbinBlocks = int(pbins.size());
     shape_.tileBlocks = int(tileTable.size());
@@ -1322,6 +1330,7 @@ Ctx WorldSet::makeCtx(int parity) const {
     c.tileBlocks = tileBlocks_;
     c.edgeBlocks = edgeBlocks_;
     c.fluidBlocks = fluidBlocks_;
+    c.fluidShift = fluidShift_;
     c.numPartBlocks = numPartBlocks_;
     c.partBlockParticles = shape_.partThreads;
     c.blockThreads = shape_.cellThreads;

@@ -308,6 +308,7 @@ private:
     int2* partBlocks_ = nullptr;
     int2* tileBlocks_ = nullptr;
     int2 *edgeBlocks_ = nullptr, *fluidBlocks_ = nullptr;
+    int fluidShift_ = 6;
     int* numPartBlocks_ = nullptr;  // (device) entries of partBlocks_
     std::vector<uint8_t> bondWork_;  // per world: a bonded or barrier cell exists or can appear by fusion
     std::vector<uint8_t> active_;    // per world: included in the launch tables

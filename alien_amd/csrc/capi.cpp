@@ -62,7 +62,6 @@ void readWorld(WorldSet& set, int w, alien_cell_to* cells, uint64_t cellCap, uin
     set.readCells(w, cells);
 }
 
-constexpr int kStripCapMax = alien::kStripMax;
 
 double nowSeconds() {
     using namespace std::chrono;
@@ -389,16 +388,12 @@ struct alien_batch {
     int resident = 0;
     uint64_t cells = 0, particles = 0;  // totals of the resident and pending worlds
     int blockSize = 256;
-    int stripCap = kStripCapMax;  // launch shape chosen by the autotuner, kept when worlds are added
-    int chunkRows = 0;
     bool useGraph = true;
     bool timing = false;
     void flush() {
         if (pending.empty()) return;
         auto fresh = std::make_unique<WorldSet>();
         fresh->setBlockSize(blockSize);
-        fresh->setStripCap(stripCap);
-        fresh->setChunkRows(chunkRows);
         fresh->setUseGraph(useGraph);
         fresh->setKernelTiming(timing);
         std::vector<WorldSet::Source> src;
@@ -541,45 +536,27 @@ int alien_batch_autotune(alien_batch* b, uint32_t trialSteps, int32_t* blockSize
         trial.setUseGraph(b->useGraph);
         trial.build(src);
         double best = 1e300;
-        int bestBlock = b->blockSize, bestStrip = b->set->stripCap(), bestRows = 0;
+        int bestBlock = b->blockSize;
         auto time = [&]() {
             trial.step(1);  // captures the graphs of this shape
             const double t0 = nowSeconds();
             trial.step(trialSteps);
             return (nowSeconds() - t0) / double(trialSteps);
         };
-        // block size x strip cap with the default chunk rows, then the chunk rows for the best
-        trial.setChunkRows(0);
-        for (int blk : {64, 128, 256})
-            for (int sc : {kStripCapMax, 32, 16}) {
-                trial.setBlockSize(blk);
-                trial.setStripCap(sc);
-                const double dt = time();
-                if (dt < best) {
-                    best = dt;
-                    bestBlock = blk;
-                    bestStrip = sc;
-                }
-            }
-        trial.setBlockSize(bestBlock);
-        trial.setStripCap(bestStrip);
-        for (int rows : {2, 4, alien::kChunkMax}) {
-            trial.setChunkRows(rows);
+        for (int blk : {64, 128, 256}) {
+            trial.setBlockSize(blk);
             const double dt = time();
             if (dt < best) {
                 best = dt;
-                bestRows = rows;
+                bestBlock = blk;
             }
         }
         b->blockSize = bestBlock;
-        b->stripCap = bestStrip;
-        b->chunkRows = bestRows;
         b->set->setBlockSize(bestBlock);
-        b->set->setStripCap(bestStrip);
-        b->set->setChunkRows(bestRows);
         if (blockSize) *blockSize = bestBlock;
-        if (stripCap) *stripCap = bestStrip;
-        if (chunkRows) *chunkRows = bestRows;
+        // (the neighbour pass has no strips and chunks to choose from any more)
+        if (stripCap) *stripCap = 64;
+        if (chunkRows) *chunkRows = 0;
         if (msPerStep) *msPerStep = best * 1000.0;
     });
 }

@@ -16,14 +16,6 @@ constexpr int kMaxBonds = 6;
 constexpr int kColors = 7;
 constexpr int kParticleBin = 8;  // edge of the energy-particle bins, in world units
 constexpr int kNone = -1;
-// neighbour pass: one wave per strip of bin columns, three staged bin rows (strip plus two halo
-// columns each) in LDS; at most kRowCap entries per staged row (two per lane while in flight);
-// widest strip
-constexpr int kRowThreads = 64;
-constexpr int kRowCap = 128;
-constexpr int kRowPool = 256;  // entries of three consecutive staged rows
-constexpr int kStripMax = 64;
-constexpr int kChunkMax = 8;  // bin rows per neighbour-pass chunk
 constexpr int kClaimFree = 0x7fffffff;
 // binOf: the cell's next bin, counted from its world's first (below 2^28: bins are at least two units wide
 // and worlds span at most 2^30 square units), and in the bits above it how the cell came there: 0 it stayed,
@@ -38,7 +30,7 @@ constexpr int kSuperGroups = 256;  // groups per sum of groups
 // there (10751 cells in bodies: a step of 106 us with 64, 97 with 32, 92 with 16); with more cells the
 // wave's fixed work counts (134k cells in bodies: 159, 157 and 162 us; 256k free ones: 22, 26 and 32 us).
 constexpr int kFluidShiftMin = 4;
-// waves of the fluid pass for a row's two edge bins (k_fluid.hip), without and with bond work
+// waves of the fluid pass for a row's two edge bins (k_neighbor.hip), without and with bond work
 constexpr int kEdgeWaves = 2, kEdgeWavesBonds = 8;
 constexpr int kXcdCount = 8;  // XCDs of an MI355X: workgroup b of a launch runs on XCD b % 8
 // Size limits of one world set.  Cell indices, bin offsets and the bond planes ([kMaxBonds][cap],
@@ -118,9 +110,6 @@ struct DevWorld {
     int binOff;             // first cell bin in the combined bin arrays
     int pbinOff;            // first particle bin in the combined bin arrays
     int partOff, partCap;   // particle arrays
-    int tileX, tileY;       // neighbour pass: bins per strip, staged rows per chunk (launch shape only)
-    int ntx, nty;           // strips, chunks
-    int rowsPerStage;       // bin rows per staged row of the neighbour pass (1, or 2 for sparse rows)
     int bondWork;           // 1 if a bonded or barrier cell exists or can appear by fusion
     int livingWork;         // 1 if living states are tracked on the device (see WorldSet::build)
     unsigned long long seed;  // key of the world's random draws
@@ -257,12 +246,6 @@ struct Ctx {
     uint32_t* mapEpoch;
     uint32_t* mapTicket;
     int* sorted;   // [cellCap] map order (bin, then previous index) -> A index
-    // [cellCap] the start-of-step state of the cells of collision worlds in map order, written next
-    // to `sorted`, so that the row-staged neighbour pass reads each row of bins as one contiguous
-    // range (the fluid pass reads the state through `sorted`)
-    float2* mpos;
-    float2* mvel;
-    uint32_t* mflags;
     int* newidx;   // [cellCap] A index -> new index
     int* psorted;  // [partCap]
     // [cellCap] kStagedCell: the end-of-step cell is staged (bonded or barrier at the neighbour pass);
@@ -294,8 +277,9 @@ struct Ctx {
     int partBlockParticles;
     const int2* fluidBlocks;  // per workgroup of the fluid pass: (world, its first wave)
     int fluidShift;           // its waves take 1 << fluidShift cells
-    const int2* edgeBlocks;  // per workgroup: (world, its first wave's edge unit and part), see k_fluid.hip
-    const int2* tileBlocks;  // per block: (world, tile index), -1 for padding blocks
+    const int2 *collideBlocks, *collideEdgeBlocks;  // the same of the collision pass
+    int collideShift;
+    const int2* edgeBlocks;  // per workgroup: (world, its first wave's edge unit and part), see k_neighbor.hip
     const int2* livingBlocks;  // per block: (world, first global cell index) over livingWork worlds
     int blockThreads;  // cells, bins or living cells per entry of the block tables above
 };

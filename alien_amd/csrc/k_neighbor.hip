@@ -1,615 +1,715 @@
-// k_neighbor.hip — the collision neighbour pass, and the launch of both passes.
+// k_neighbor.hip — the neighbour passes: fluid (SPH pressure and viscosity, overlap push, barriers, fusion
+// candidates) and collision (repulsion, momentum exchange, overlap push, fusion candidates), with the
+// end-of-step state of the cells that have no bonds (CellProcessor::calcFluidForces_reconnectCells_
+// correctOverlap and calcCollisions_reconnectCells_correctOverlap, source/EngineGpuKernels/
+// CellProcessor.cuh:122-365).
 //
-// One wave owns a strip of bin columns and walks it row by row (see "Row streaming" below).  Per
-// row it (1) tests the 3x3 bin stencil of every cell with the neighbour predicate on squared
-// lengths and records the neighbours as a bit mask in visiting order, (2) evaluates all neighbour
-// pairs of the row one pair per lane, and (3) lets every cell add its pairs' terms in visiting
-// order, which gives the float sums of a sequential stencil walk bit for bit.  A cell with more
-// than 64 stencil candidates, or a strip whose rows do not fit LDS, walks its stencil
-// sequentially instead (same order, same results).  A workgroup of a fluid world exits at once.
-#include <type_traits>
-
+// The map is in logical order (cells by bin, inside a bin by previous index), so the three stencil
+// bins of a cell in one bin row are one contiguous range of the map, and one wave takes 64
+// consecutive map positions:
+//  1. Every lane finds its three ranges, without the bins and bin rows that lie beyond its reach (the
+//     squared distance to the bin's edge, in the same rounded operations as the test itself, so no
+//     neighbour is lost): 5 candidates a cell instead of 9.6 at one cell per bin.
+//  2. The union of the lanes' ranges, one stretch of the map per stencil row, is staged in LDS.
+//  3. The lanes' lists are laid end to end and tested 64 candidates at a time, whoever they belong
+//     to: a wave spends its total over 64, not its longest list.  A bit per list start tells a lane
+//     its list's owner; the hits of a round, in lane order, go straight to the wave's list of pairs,
+//     which is thereby ordered by owner and inside by visiting order.
+//  4. The pairs are evaluated one per lane, and every owner adds its pairs' terms in visiting order
+//     (the float sums of a sequential stencil walk, bit for bit).
+// The pass is bound by VALU issue, so the pair terms use the short exact reciprocals and roots
+// (mid_rcp, mid_sqrt; one range check per pair), indices become 32-bit byte offsets (a 64-bit
+// address costs four operations), 1 / density is stored instead of the density, and sets without bond
+// work run a variant without flags, bonds, barriers and fusion.
+// Steps of a fluid world before (lists cut and pairs compacted per 64-candidate round, edge cells alone
+// in their lanes) and now, with the map as it was: 256k cells 35 -> 26.5 us, 4M 172 -> 168 us.
+// Records for all pairs of a wave in bodies (the tests ran up to five times before): 134k cells 158 -> 152
+// us, with the edge waves and fewer cells per wave (kFluidShiftMin) 10751 cells 108 -> 91.5 us.
+//
+// Cells of the first and last bin column have a stencil that wraps around the torus: their ranges
+// come in two pieces.  They are left to waves of their own, two for each row's pair of edge bins (eight with
+// bond work: the cells of a body there, one after the other, took 16 of 32 us of a small world), that
+// take a cell at a time with its candidates side by side; walked alone by a lane of the pass, they
+// were its last waves to end.  Cells with more than 64 candidates walk their stencil alone.
+// Collision worlds run the same pass.  In a body most neighbours are bonded, and a bonded pair adds nothing
+// but a rare push, so the pairs found are first sifted (8 to 2 a cell).  The pass before walked strips of
+// bin columns row by row, with the rows' halo staged again by every chunk, all nine bins tested and a list
+// as long as the longest lane's: 3300 VALU operations for 64 cells of a body; now 0.84M cells in bodies 110
+// -> 84 us (a step, with no copy of the cells' state in the map any more, 300 -> 260), 18k cells 25 -> 12.5
+// us (85 -> 68), eight worlds of 1024^2 in one set: a step 210 -> 175 us.
 #include "kernels.hpp"
 #include "neighbor_device.hpp"
 #include "particle_steps.hpp"
 
 namespace alien {
 
-// ---------------------------------------------------------------------------------------------
-// Row streaming.  A workgroup (one wave) owns a strip of up to kStripMax bin columns and a chunk of
-// staged rows, and walks them top to bottom with staged rows Y-1, Y, Y+1 in LDS.  A staged row is
-// kSub consecutive bin rows (1, or 2 for sparse worlds, so that one pass has enough cells for the
-// 64 lanes); each bin row covers the strip plus one halo column on each side, its entries stored
-// bin by bin in rank order (R1), so the three stencil bins of a cell in one bin row are one
-// contiguous range.  While row Y is computed, the entries of row Y+2 and the bin counters of row
-// Y+3 are on their way into registers; row Y+2 is committed once row Y-1 is no longer needed.  The
-// three staged rows share one ring pool of entries (positions counted up without wrapping, stored
-// modulo kPool): a row takes the pool space right after the previous one, so any three
-// consecutive rows of up to kPool entries together fit, however they are distributed.
-// ---------------------------------------------------------------------------------------------
-constexpr int kRowBins = kStripMax + 2;            // halo columns of one bin row
-constexpr int kSubMax = 2;                         // bin rows per staged row, at most
-constexpr int kPool = kRowPool;
-constexpr int kPoolMask = kPool - 1;
-constexpr int kPairCap = 128;  // pair records per evaluation window
-constexpr int kPosMirror = 64;
-static_assert((kPool & kPoolMask) == 0 && kPool <= 256, "pair records keep an 8-bit pool position");
-static_assert(kRowCap <= 2 * kRowThreads, "a row in flight holds at most two entries per lane");
-static_assert(kSubMax * kRowBins <= 3 * kRowThreads && kSubMax * kRowBins < 256,
-              "bin slots: three per lane, 8-bit ids");
+// The pass's variants: fluid worlds of sets without bond work, and with; collision worlds.
+enum class Pass { kFree, kBonds, kCollide };
+template <Pass kPass> constexpr bool kBonded = kPass != Pass::kFree;  // (collision worlds have bonds in general)
+constexpr int kFluidWaves = 4;   // waves per workgroup at most
+// staged candidates of the three stencil rows: three rows of 66 bins at one cell per bin; with bonds,
+// bodies of four cells a bin next to empty space
+constexpr int kFreeStage = 288, kBondStage = 448;
+// pair records at a time: a fluid's cells have about one each at one cell per bin; with bonds, bodies with
+// ten neighbours a cell (the tests run again for what does not fit)
+constexpr int kFreePairs = 128, kBondPairs = 896;
+constexpr int kEdgeAlone = 16;    // more edge cells than this in a unit walk alone, one per lane
 
-// LDS of one wave, for staged rows of up to kMaxSub bin rows
-template <int kMaxSub>
-struct RowShared {
-    static constexpr int kStageBins = kMaxSub * kRowBins;  // bin slots of one staged row (row major)
-    // per ring row: pool position of the first entry of every bin slot, then the end; per ring
-    // row and bin row, map positions of the first entries of the left halo bin, the first interior
-    // bin and the right halo bin (the interior bins of a bin row are contiguous in the map)
-    int rs[3][kStageBins + 1];
-    int rm[3][kMaxSub][3];
-    // entries of the staged rows, by pool position modulo kPool; positions 0..kPosMirror-1 are
-    // repeated after the end so that a stencil range of up to 64 entries reads without wrapping
-    float2 pos[kPool + kPosMirror];
-    float2 vel[kPool];
-    uint16_t flags[kPool];  // the bits the pass reads of an entry's flags (flags16)
-    int aidx[kPool];
-    uint8_t sbin[kPool];  // bin slot: bin row * HX + halo column
-    // the row in flight
-    int nrs[kStageBins + 1];
-    int nrm[kMaxSub][3];
-    uint8_t nebin[kRowCap];  // entry of the row -> bin slot
+// LDS of one wave: 6 KB (9.9 KB with bonds), six (four) waves per SIMD (the owners' velocities,
+// densities and flags come from their registers, by cross-lane permutes)
+template <int kStage, int kPairs> struct FluidShared {
+    // staged candidates: their positions, and behind them their A indices (the last round of tests reads
+    // up to 63 positions past the last list, and counts nothing there)
+    float2 cpos[kStage + kStage / 2];
+    __device__ int& caidx(int x) { return reinterpret_cast<int*>(cpos + kStage)[x]; }
+    float2 pos[64];  // the wave's own cells; no position for a lane that does not test
+    uint16_t first[65];  // each owner's first pair
+    uint16_t own[64];    // pairs up to the owner's own place in its list
+    uint16_t pair[kPairs];  // pair records: staged neighbour, owner << 9
     union {
         struct {
-            // while a row is computed, the pair records of the current window: the cell's pool
-            // position, and the neighbour as bonded << 15 | ring row << 8 | pool position
-            uint8_t pself[kPairCap];
-            uint16_t pnb[kPairCap];
-        } pr;
+            // per list: its row boundaries (flat, two 16-bit halves) and what to add to a flat index
+            // for the candidate's place, row by row
+            int4 rec[64];
+            uint32_t start[128];  // bit f: a list starts at flat index f (64 lists of at most 64)
+        } t;
+        struct {
+            float4 a[64];  // density term, overlap push, barrier (A index + 1)
+            float4 b[64];  // pressure and viscosity terms
+        } r;
     } u;
 };
+template <bool kBonds>
+using FluidWave = FluidShared<kBonds ? kBondStage : kFreeStage, kBonds ? kBondPairs : kFreePairs>;
+static_assert(sizeof(FluidWave<true>) <= 10240 && sizeof(FluidWave<false>) <= 6826, "16 and 24 waves per CU");
+static_assert(kBondStage <= 512 && kFreeStage >= 126, "9-bit staged entries; room to read past the last list");
 
-// registers of a row in flight: bin counters of the bin slots lane, lane + 64, lane + 128, then
-// the entries lane and lane + 64 in map order
-template <int kSub>
-struct RowFlight {
-    static constexpr int kSlots = kSub == 2 ? 3 : 2;  // bin slots per lane
-    uint32_t s0[kSlots], s1[kSlots];
-    int aidx[2];
-    float2 pos[2], vel[2];
-    uint32_t flags[2];
-    int total;
-};
-
-struct StripGeom {
-    int x0, IX, HX;  // first interior bin column, interior columns, halo columns (IX + 2)
-    int nbx, nby, binOff, cellOff;
-    uint32_t base;   // start[] value of the world's first bin
-    bool seam;       // the staged rows or columns wrap around the torus
-};
-
-// map segment of halo column hx: 0 the left halo bin, 1 the interior, 2 the right halo bin; and
-// the segment's first halo column
-__device__ __forceinline__ int seg_of(int hx, int HX) { return hx == 0 ? 0 : (hx == HX - 1 ? 2 : 1); }
-__device__ __forceinline__ int seg_first(int seg, int HX) { return seg == 0 ? 0 : (seg == 2 ? HX - 1 : 1); }
-
-// bin row (0 or 1) of bin slot j
-template <int kSub>
-__device__ __forceinline__ int slot_row(int j, int HX) { return kSub == 2 && j >= HX ? 1 : 0; }
-
-// An entry's flags in LDS: bond counts (bits 0..7) and the barrier bit (moved to bit 8), the only
-// bits the pass reads of a neighbour; a cell's own full flags are read again before its writes.
-__device__ __forceinline__ uint16_t flags16(uint32_t f) { return uint16_t((f & 0xFFu) | ((f & kBarrierBit) >> 8)); }
-__device__ __forceinline__ uint32_t flags32(uint16_t p) { return (uint32_t(p) & 0xFFu) | ((uint32_t(p) & 0x100u) << 8); }
-
-// logical index of the staged entry at pool position pp (already reduced modulo kPool) of ring row r
-template <int kSub, class RS>
-__device__ __forceinline__ int row_lidx(const RS& S, const StripGeom& g, int r, int pp) {
-    const int j = S.sbin[pp];
-    const int t = slot_row<kSub>(j, g.HX);
-    const int seg = seg_of(j - t * g.HX, g.HX);
-    return S.rm[r][t][seg] + ((pp - S.rs[r][t * g.HX + seg_first(seg, g.HX)]) & kPoolMask);
+__device__ __forceinline__ int lanes_below(unsigned long long mask, int add) {
+    return int(__builtin_amdgcn_mbcnt_hi(uint32_t(mask >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(mask), uint32_t(add))));
 }
 
-// the staged entry at pool position pp of ring row r; without its logical index if !kLidx
-template <int kSub, class RS, bool kLidx = true>
-__device__ __forceinline__ Nb row_nb(const RS& S, const StripGeom& g, int r, int pp) {
+// the cell at map position m
+__device__ __forceinline__ Nb map_nb(const Ctx& c, int m) {
     Nb o;
-    o.pos = to_f2(S.pos[pp]);
-    o.vel = to_f2(S.vel[pp]);
-    o.dens = 0.0f;
-    o.flags = flags32(S.flags[pp]);
-    o.aidx = S.aidx[pp];
-    o.lidx = kLidx ? row_lidx<kSub>(S, g, r, pp) : -1;
+    o.aidx = c.sorted[m];
+    o.pos = to_f2(ld32(c.A.pos, o.aidx));
+    o.vel = to_f2(ld32(c.A.vel, o.aidx));
+    o.dens = ld32(c.A.dens, o.aidx);
+    o.flags = ld32(c.A.flags, o.aidx);
+    o.lidx = m;
     return o;
 }
 
-template <bool kFluid>
-__device__ __forceinline__ Nb global_nb(const Ctx& c, int a, int l) {
-    Nb o;
-    o.pos = to_f2(c.A.pos[a]);
-    o.vel = to_f2(c.A.vel[a]);
-    o.dens = kFluid ? c.A.dens[a] : 0.0f;
-    o.flags = c.A.flags[a];
-    o.aidx = a;
-    o.lidx = l;
-    return o;
+// the terms of a pair of fluid cells (pair_term<true>, CellProcessor.cuh:144-231): a = density term,
+// overlap push; b = pressure, viscosity
+struct FluidTerms {
+    float rho;
+    f2 D, Fp, Fv;
+};
+template <bool kForce>
+__device__ __forceinline__ FluidTerms fluid_terms(const DevParams& P, f2 pd, f2 vd, float si, float oi, bool force) {
+    const float d2 = lensq(pd);
+    float d = mid_sqrt(d2);
+    float invD = mid_rcp(d);
+    if (!mid_range(d2)) {
+        d = __builtin_sqrtf(d2);
+        invD = 1.0f / d;
+    }
+    const float q = d * P.invH;
+    const float r = 2.0f - q;
+    const float wNear = kTwoThirds - q * q + 0.5f * q * q * q, wFar = mid_div<6>(r * r * r);
+    const float gNear = -2.0f * q + 1.5f * q * q, gFar = -0.5f * r * r;
+    const bool near = q < 1.0f, far = q < 2.0f;
+    FluidTerms t;
+    t.rho = (near ? wNear : (far ? wFar : 0.0f)) * kKernelNorm * P.invH2;
+    const float kd = (near ? gNear : (far ? gFar : 0.0f)) * kKernelNorm * P.invH3;
+    t.D = {0.0f, 0.0f};
+    if (d < P.minDistance) {
+        const f2 p = mul(pd, P.minDistance);
+        t.D = f2{mid_div<5>(p.x), mid_div<5>(p.y)};
+        if (!mid_range(p.x) || !mid_range(p.y)) t.D = dvd(p, 5.0f);
+    }
+    t.Fp = t.Fv = f2{0.0f, 0.0f};
+    const bool on = d > kNearZero && (!kForce || force);
+    const f2 fp = mul(mul(mul(pd, -invD), si + oi), kd);
+    // (d * d + 0.25 lies in the middle range: d is a neighbour's distance, at most 64)
+    const f2 fv = mul(mul(mul(mul(vd, oi), d), kd), mid_rcp(d * d + 0.25f));
+    if (on) {
+        t.Fp = fp;
+        t.Fv = fv;
+    }
+    return t;
 }
 
-// bin of halo column hx in bin row yy (both wrapped around the torus)
-__device__ __forceinline__ int strip_bin(const StripGeom& g, int yy, int hx) {
-    return g.binOff + wrap_small(yy, g.nby) * g.nbx + wrap_small(g.x0 - 1 + hx, g.nbx);
+// end of the pass for a cell of a set without bond work (cell_finish without bonds and barriers)
+__device__ __forceinline__ void finish_free(const Ctx& c, const DevWorld& w, const DevParams& P, int k, f2 pos, f2 vel,
+                                            uint32_t flags, int slot, float rho, f2 D, f2 Fp, f2 Fv, int bOld) {
+    const f2 F = add(f2{0.0f, 0.0f}, add(mul(Fp, P.pressure), mul(Fv, P.viscosity)));
+    const f2 pc = add(pos, D);
+    f2 v = add(vel, F);
+    if (lensq(v) > P.maxVelSq) v = mul(unit(v), P.maxVelocity);
+    const f2 zero = {0.0f, 0.0f};
+    const float dt = P.dt;
+    const f2 p2 = torus_pos(add(pc, add(mul(v, dt), mul(mul(mul(zero, dt), dt), 0.5f))), w.W, w.H);
+    v = add(v, mul(mul(add(zero, zero), 0.5f), dt));
+    v = mul(v, 1.0f - P.friction);
+    float inv = mid_rcp(rho);
+    if (!mid_range(rho)) inv = 1.0f / rho;
+    st32(c.B.flags, k, flags);
+    st32(c.B.slot, k, slot);
+    st32(c.B.dens, k, inv);
+    st32(c.B.pos, k, to_float2(p2));
+    st32(c.B.vel, k, to_float2(v));
+    bin_next(c, w, k, p2, bOld);
 }
 
-// A: bin counters of staged row Y
-template <int kSub>
-__device__ __forceinline__ void row_issue_counts(const Ctx& c, const StripGeom& g, int Y, RowFlight<kSub>& F) {
-    const int lane = threadIdx.x;
-#pragma unroll
-    for (int q = 0; q < RowFlight<kSub>::kSlots; ++q) {
-        const int j = lane + q * kRowThreads;
-        F.s0[q] = F.s1[q] = 0u;
-        if (j < kSub * g.HX) {
-            const int t = slot_row<kSub>(j, g.HX);
-            const int gb = strip_bin(g, kSub * Y + t, j - t * g.HX);
-            F.s0[q] = c.start[gb];
-            F.s1[q] = c.start[gb + 1];
+// a cell whose stencil is walked by one lane, entry by entry
+template <bool kFluid> __device__ __forceinline__ void walk_alone(const Ctx& c, int wi, int m) {
+    const DevWorld& w = c.worlds[wi];
+    const DevParams& P = c.params[wi];
+    const uint32_t* start = c.start + w.binOff;
+    const int off = w.cellOff - int(start[0]);
+    const Nb s = map_nb(c, m);
+    int bx, by;
+    cell_bin_xy(w, s.pos, bx, by);
+    atomicAdd(&c.sc->directCells, 1ull);
+    cell_direct<kFluid>(c, w, P, wi, s, [&](auto&& visit) {
+        for (int k = 0; k < 9; ++k) {
+            const int b = wrap_small(by + k / 3 - 1, w.nby) * w.nbx + wrap_small(bx + k % 3 - 1, w.nbx);
+            const int e = off + int(start[b + 1]);
+            for (int j = off + int(start[b]); j < e; ++j) visit(map_nb(c, j));
         }
-    }
+    });
 }
 
-// B: slots of the row's bins, then the entry loads (map-order copy, contiguous per bin)
-template <int kSub, class RS>
-__device__ __forceinline__ void row_issue_entries(const Ctx& c, const StripGeom& g, RS& S, RowFlight<kSub>& F) {
-    constexpr int kSlots = RowFlight<kSub>::kSlots;
-    const int lane = threadIdx.x;
-    const int SB = kSub * g.HX;
-    int n[kSlots], inc[kSlots];
-#pragma unroll
-    for (int q = 0; q < kSlots; ++q) {
-        n[q] = lane + q * kRowThreads < SB ? int(F.s1[q] - F.s0[q]) : 0;
-        inc[q] = int(wave_inclusive_scan(uint32_t(n[q])));
-    }
-    const int tot0 = wave_last(inc[0]), tot1 = wave_last(inc[1]);
-    F.total = tot0 + tot1 + (kSlots > 2 ? wave_last(inc[kSlots - 1]) : 0);
-#pragma unroll
-    for (int q = 0; q < kSlots; ++q) {
-        const int j = lane + q * kRowThreads;
-        if (j >= SB) continue;
-        const int off = inc[q] - n[q] + (q >= 1 ? tot0 : 0) + (q >= 2 ? tot1 : 0);
-        const int t = slot_row<kSub>(j, g.HX);
-        const int hx = j - t * g.HX;
-        S.nrs[j] = off;
-        if (hx <= 1 || hx == g.HX - 1) S.nrm[t][seg_of(hx, g.HX)] = g.cellOff + int(F.s0[q] - g.base);
-        for (int e = 0; e < n[q]; ++e) S.nebin[off + e] = uint8_t(j);
-    }
-    if (lane == 0) S.nrs[SB] = F.total;
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-        const int e = lane + q * kRowThreads;
-        if (e < F.total) {
-            const int j = S.nebin[e];
-            const int t = slot_row<kSub>(j, g.HX);
-            const int seg = seg_of(j - t * g.HX, g.HX);
-            const int m = S.nrm[t][seg] + (e - S.nrs[t * g.HX + seg_first(seg, g.HX)]);
-            F.aidx[q] = c.sorted[m];
-            F.pos[q] = c.mpos[m];
-            F.vel[q] = c.mvel[m];
-            F.flags[q] = c.mflags[m];
+// The cells of the edge unit u: the last bin of row u - 1 and the first bin of row u, one after the
+// other in the map; the unit's two waves take every other cell.  Returns the cells left to walk alone:
+// this lane's first one, and the end.
+template <Pass kPass> __device__ __forceinline__ int2 edge_unit(const Ctx& c, int wi, int u, int part) {
+    constexpr bool kFluid = kPass != Pass::kCollide;
+    constexpr int kWaves = kBonded<kPass> ? kEdgeWavesBonds : kEdgeWaves;
+    const DevWorld& w = c.worlds[wi];
+    const DevParams& P = c.params[wi];
+    const int lane = int(threadIdx.x) & 63;
+    const uint32_t* start = c.start + w.binOff;
+    const int off = w.cellOff - int(start[0]);
+    const int m0 = off + int(start[max(u * w.nbx - 1, 0)]), m1 = off + int(start[u < w.nby ? u * w.nbx + 1 : u * w.nbx]);
+    if (m1 - m0 > kEdgeAlone) return make_int2(part == 0 ? m0 + lane : m1, m1);
+    const float Wf = float(w.W), Hf = float(w.H), reachSq = P.reachSq;
+    const float w0 = sph_w(0.0f) * P.invH2;
+    uint32_t crowded = 0u;  // cells with more than 64 candidates
+    for (int m = m0 + part; m < m1; m += kWaves) {
+        const Nb s = map_nb(c, m);  // (the same on every lane)
+        int bx, by;
+        cell_bin_xy(w, s.pos, bx, by);
+        // lane k < 9: the stencil bin k in visiting order
+        int lo = 0, n = 0;
+        if (lane < 9) {
+            const int b = wrap_small(by + lane / 3 - 1, w.nby) * w.nbx + wrap_small(bx + lane % 3 - 1, w.nbx);
+            lo = off + int(start[b]);
+            n = off + int(start[b + 1]) - lo;
         }
-    }
-}
-
-// C: the row into ring row r at pool position head.  The row was read from the map copy bin by
-// bin, and the map holds every bin's cells by previous index (R1): an entry's place in the row is
-// its rank in its bin.
-template <int kSub, class RS>
-__device__ __forceinline__ void row_commit(const StripGeom& g, RS& S, const RowFlight<kSub>& F, int r, int head) {
-    const int lane = threadIdx.x;
-    const int SB = kSub * g.HX;
-    for (int i = lane; i <= SB; i += kRowThreads) S.rs[r][i] = head + S.nrs[i];
-    if (lane < 3 * kSub) S.rm[r][lane / 3][lane % 3] = S.nrm[lane / 3][lane % 3];
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-        const int e = lane + q * kRowThreads;
-        if (e < F.total) {
-            const int j = S.nebin[e];
-            const int a = F.aidx[q];
-            const int pp = (head + e) & kPoolMask;
-            S.pos[pp] = F.pos[q];
-            if (pp < kPosMirror) S.pos[kPool + pp] = F.pos[q];
-            S.vel[pp] = F.vel[q];
-            S.flags[pp] = flags16(F.flags[q]);
-            S.aidx[pp] = a;
-            S.sbin[pp] = uint8_t(j);
+        const int inc = int(wave_inclusive_scan(uint32_t(n)));
+        const int total = wave_last(inc);
+        if (total > 64) {
+            crowded |= 1u << (m - m0);
+            continue;
         }
-    }
-    __syncthreads();
-}
-
-// element r (0..2) of a three-element register array, without indexing it at run time (which
-// would place the array in scratch memory)
-__device__ __forceinline__ int pick3(const int (&a)[3], int r) { return r == 0 ? a[0] : (r == 1 ? a[1] : a[2]); }
-
-// The cells of staged row Y (ring row rc; rows Y-1 and Y+1 in rm_ and rp).
-template <bool kFluid, int kSub, class RS>
-__device__ __forceinline__ void row_compute(const Ctx& c, const DevWorld& w, const DevParams& P, int wi,
-                                            const StripGeom& g, RS& S, int rm_, int rc, int rp) {
-    const int lane = threadIdx.x;
-    const float Wf = float(w.W), Hf = float(w.H);
-    // the cells: the interior bins of each bin row of the staged row
-    const int cs0 = S.rs[rc][1];
-    const int n0 = S.rs[rc][g.IX + 1] - cs0;
-    const int cs1 = kSub == 2 ? S.rs[rc][g.HX + 1] : 0;
-    const int ncell = n0 + (kSub == 2 ? S.rs[rc][g.HX + g.IX + 1] - cs1 : 0);
-    const float w0 = kFluid ? sph_w(0.0f) * P.invH2 : 0.0f;  // a fluid cell's own density term
-    for (int q0 = 0; q0 < ncell; q0 += kRowThreads) {
-        // candidates of this lane's cell: three contiguous pool ranges, one per stencil bin row
-        const int q = q0 + lane;
-        const bool active = q < ncell;
-        Nb self;
-        int bt[kMaxBonds];
-        int a0s[3] = {0, 0, 0}, ns[3] = {0, 0, 0}, ringOf[3] = {rm_, rc, rp};
-        unsigned long long mask = 0ull, bmask = 0ull;
-        bool direct = false;
-        int selfIdx = -1;  // fluid: number of the cell's pairs that come before its own density term
-        const int t = kSub == 2 && q >= n0 ? 1 : 0;    // the cell's bin row in the staged row
-        const int su = t == 0 ? cs0 + q : cs1 + (q - n0);  // pool position, not wrapped
-        const int sp = su & kPoolMask;
-        int slot = 0;
-        if (active) {
-            self = row_nb<kSub>(S, g, rc, sp);
-            slot = c.A.slot[self.aidx];  // needed only at the end: loaded early
-            load_bonds(c, self, bt);
-            const int hx = S.sbin[sp] - t * g.HX;
-            // stencil bin rows (ring row, bin row): above, own, below
-            int subOf[3] = {0, 0, 0};
-            if (kSub == 2) {
-                ringOf[0] = t == 0 ? rm_ : rc;
-                subOf[0] = t == 0 ? 1 : 0;
-                ringOf[1] = rc;
-                subOf[1] = t;
-                ringOf[2] = t == 0 ? rc : rp;
-                subOf[2] = t == 0 ? 1 : 0;
-            }
+        // candidate `lane` of the list
+        int at = 0;
 #pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                const int b0 = subOf[k] * g.HX + hx;
-                a0s[k] = S.rs[ringOf[k]][b0 - 1];
-                ns[k] = S.rs[ringOf[k]][b0 + 2] - a0s[k];
-            }
-            if (ns[0] + ns[1] + ns[2] > 64) {
-                direct = true;
-            } else {
-                const bool hasBonds = flags_num_conn(self.flags) > 0;
-                // fluid: the cell's own density term needs no pair evaluation; only its place in
-                // the visiting order is kept (a barrier cell meets itself as a barrier instead);
-                // collision: the cell is not its own neighbour
-                const bool keepSelf = kFluid && flags_barrier(self.flags);
-                const int selfFlat = ns[0] + (su - a0s[1]);  // the cell's own visiting index
-                // predicated tests, one mask bit per candidate in visiting order (one copy of the
-                // loop for chunks on the torus seam, one for the rest)
-                auto test = [&](auto seamTag) {
-                    constexpr bool kSeam = decltype(seamTag)::value;
-                    auto dsq = [&](f2 o) {
-                        return kFluid ? lensq(kSeam ? torus_delta(self.pos, o, Wf, Hf) : sub(self.pos, o))
-                                      : lensq(sub(o, self.pos));  // R13
-                    };
-                    int cidx = 0;
-#pragma unroll
-                    for (int r = 0; r < 3; ++r) {
-                        const int pb = a0s[r] & kPoolMask, n = ns[r];
-                        unsigned long long rowMask = 0ull;
-                        for (int u = 0; u < n; u += 2) {
-                            // two candidates per iteration; the second is read even past the
-                            // range end (within the mirrored pool) and trimmed below
-                            const f2 p0 = to_f2(S.pos[pb + u]);
-                            const f2 p1 = to_f2(S.pos[pb + u + 1]);
-                            rowMask |= dsq(p0) <= P.reachSq ? (1ull << u) : 0ull;
-                            rowMask |= dsq(p1) <= P.reachSq ? (2ull << u) : 0ull;
-                        }
-                        rowMask &= n >= 64 ? ~0ull : (1ull << n) - 1ull;
-                        mask |= rowMask << cidx;
-                        cidx += n;
-                    }
-                };
-                if (g.seam)
-                    test(std::true_type{});
-                else
-                    test(std::false_type{});
-                if (!keepSelf) mask &= ~(1ull << selfFlat);
-                if (kFluid && !keepSelf) selfIdx = __builtin_popcountll(mask & ((1ull << selfFlat) - 1ull));
-                if (hasBonds) {
-                    // which of the neighbours are bonded
-                    const bool bari = flags_barrier(self.flags);
-                    unsigned long long m = mask;
-                    while (m) {
-                        const int ci = __builtin_ctzll(m);
-                        m &= m - 1ull;
-                        const int r = ci < ns[0] ? 0 : (ci < ns[0] + ns[1] ? 1 : 2);
-                        const int rest = ci - (r == 0 ? 0 : (r == 1 ? ns[0] : ns[0] + ns[1]));
-                        const int np = (pick3(a0s, r) + rest) & kPoolMask;
-                        if (!is_bonded(bt, S.aidx[np] - w.cellOff)) continue;
-                        if constexpr (!kFluid) {
-                            // a bonded collision pair adds only its overlap push (closer than
-                            // minDistance, not for a barrier cell): otherwise it adds nothing and
-                            // leaves the list (the distance as the pair term takes it)
-                            const f2 o = to_f2(S.pos[np]);
-                            const float d2 = lensq(g.seam ? torus_delta(self.pos, o, Wf, Hf) : sub(self.pos, o));
-                            if (bari || d2 > P.overlapBelowSq) {
-                                mask &= ~(1ull << ci);
-                                continue;
-                            }
-                        }
-                        bmask |= 1ull << ci;
-                    }
-                }
-            }
+        for (int k = 0; k < 9; ++k) {
+            const int begin = __builtin_amdgcn_readlane(inc - n, k);
+            at = lane >= begin ? __builtin_amdgcn_readlane(lo, k) + lane - begin : at;
         }
-        const int count = __builtin_popcountll(mask);
-        const int inc = int(wave_inclusive_scan(uint32_t(count)));
-        const int numPairs = wave_last(inc);
-        const int pbase = inc - count;
-
+        const bool in = lane < total;
+        const bool keepSelf = kFluid && flags_barrier(s.flags);
+        Nb o = s;
+        if (in) o = map_nb(c, at);
+        const float d2 = lensq(kFluid ? torus_delta(s.pos, o.pos, Wf, Hf) : sub(o.pos, s.pos));
+        const bool hit = in && d2 <= reachSq && (o.aidx != s.aidx || keepSelf);
+        const unsigned long long self = __ballot(in && o.aidx == s.aidx);
+        unsigned long long hits = __ballot(hit);
+        const int selfAt = keepSelf || self == 0ull ? 64 : __builtin_ctzll(self);
+        bool pending = kFluid && !keepSelf;  // the own density term, at its place in the order
         Acc a;
-        if (active) acc_init(a, self);
-        for (int W0 = 0; W0 < numPairs; W0 += kPairCap) {
-            const int wend = min(numPairs, W0 + kPairCap);
-            // owners write the records of their pairs inside this window
-            if (count > 0 && pbase < wend && pbase + count > W0) {
-                unsigned long long m = mask;
-                for (int p = pbase; m; ++p) {
-                    const int ci = __builtin_ctzll(m);
-                    m &= m - 1ull;
-                    if (p < W0 || p >= wend) continue;
-                    int r = 0, rest = ci;
-                    if (rest >= ns[0]) {
-                        rest -= ns[0];
-                        r = 1;
-                        if (rest >= ns[1]) {
-                            rest -= ns[1];
-                            r = 2;
-                        }
-                    }
-                    const int np = (pick3(a0s, r) + rest) & kPoolMask;
-                    const uint32_t bonded = uint32_t((bmask >> ci) & 1ull);
-                    S.u.pr.pself[p - W0] = uint8_t(sp);
-                    S.u.pr.pnb[p - W0] = uint16_t((bonded << 15) | (uint32_t(pick3(ringOf, r)) << 8) | uint32_t(np));
-                }
+        acc_init(a, s);
+        auto add_own = [&](int l) {
+            if (pending && l > selfAt) {
+                a.rho = a.rho + w0;
+                pending = false;
             }
-            __syncthreads();
-            for (int off = W0; off < wend; off += kRowThreads) {
-                // pair terms, one pair per lane
-                const int p = off + lane;
-                float tm[kPairTerms];
-#pragma unroll
-                for (int v = 0; v < kPairTerms; ++v) tm[v] = 0.0f;
-                uint32_t f = 0u;
-                if (p < wend) {
-                    const uint32_t rec = S.u.pr.pnb[p - W0];
-                    const int ps = S.u.pr.pself[p - W0], ro = int((rec >> 8) & 3u), po = int(rec & 0xFFu);
-                    const Nb s = row_nb<kSub, RS, false>(S, g, rc, ps);
-                    const Nb o = row_nb<kSub, RS, false>(S, g, ro, po);
-                    f = pair_term<kFluid>(c, w, P, wi, s, o, (rec >> 15) != 0u, tm, g.seam, [&] {
-                        return make_int2(row_lidx<kSub>(S, g, rc, ps), row_lidx<kSub>(S, g, ro, po));
-                    });
-                }
-                // the owner adds its pairs of this round in visiting order, reading each from the
-                // lane that evaluated it (every lane takes part in every exchange)
-                const int lo = max(pbase, off), hi = min(pbase + count, min(off + kRowThreads, wend));
-                const int n = count > 0 ? max(0, hi - lo) : 0;
-                for (int j = 0; __any(j < n); ++j) {
-                    const int src = (lo + j - off) & (kRowThreads - 1);
-                    float tt[kPairTerms];
-#pragma unroll
-                    for (int v = 0; v < kPairTerms; ++v) tt[v] = __shfl(tm[v], src, kRowThreads);
-                    const uint32_t ff = uint32_t(__shfl(int(f), src, kRowThreads));
-                    const bool on = j < n;
-                    if constexpr (kFluid) a.rho = on && lo + j - pbase == selfIdx ? a.rho + w0 : a.rho;
-                    acc_add_sel<kFluid>(a, on, ff, tt);
-                }
+        };
+        auto from = [](float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
+        const int slot = c.A.slot[s.aidx];
+        if constexpr (kPass == Pass::kFree) {
+            const FluidTerms t = fluid_terms<false>(P, torus_delta(s.pos, o.pos, Wf, Hf), sub(s.vel, o.vel), s.dens, o.dens, true);
+            for (; hits; hits &= hits - 1ull) {
+                const int l = __builtin_ctzll(hits);
+                add_own(l);
+                a.rho = a.rho + from(t.rho, l);
+                a.D = add(a.D, f2{from(t.D.x, l), from(t.D.y, l)});
+                a.Fp = add(a.Fp, f2{from(t.Fp.x, l), from(t.Fp.y, l)});
+                a.Fv = add(a.Fv, f2{from(t.Fv.x, l), from(t.Fv.y, l)});
             }
-            __syncthreads();
-        }
-        if (active && selfIdx == count) a.rho = a.rho + w0;  // the own term after all pairs
-        if (active) {
-            // the cell's full flags, from the start-of-step arrays (the map copy holds a bin's
-            // entries in arrival order, not at their logical indices)
-            self.flags = c.A.flags[self.aidx];
-            if (direct) {
-                atomicAdd(&c.sc->directCells, 1ull);
-                cell_direct<kFluid>(c, w, P, wi, self, [&](auto&& visit) {
+            add_own(65);
+            if (lane == 0) finish_free(c, w, P, m, s.pos, s.vel, s.flags, slot, a.rho, a.D, a.Fp, a.Fv, by * w.nbx + bx);
+        } else {
+            int bt[kMaxBonds];
+            load_bonds(c, s, bt);
+            float t[kPairTerms];
 #pragma unroll
-                    for (int r = 0; r < 3; ++r)
-                        for (int u = a0s[r]; u < a0s[r] + ns[r]; ++u)
-                            visit(row_nb<kSub>(S, g, ringOf[r], u & kPoolMask));
-                });
-            } else {
-                // the bond targets are loaded again rather than kept in registers through the pair
-                // work (few cells have bonds in a fluid world; the loads hit the cache)
-                int bt2[kMaxBonds];
-                load_bonds(c, self, bt2);
-                cell_finish<kFluid>(c, w, P, wi, self, slot, bt2, a);
+            for (int v = 0; v < kPairTerms; ++v) t[v] = 0.0f;
+            uint32_t f = 0u;
+            if (hit)
+                f = pair_term<kFluid>(c, w, P, wi, s, o, is_bonded(bt, o.aidx - w.cellOff), t, true,
+                                    [&] { return make_int2(s.lidx, o.lidx); });
+            for (; hits; hits &= hits - 1ull) {
+                const int l = __builtin_ctzll(hits);
+                add_own(l);
+                float tt[kPairTerms];
+#pragma unroll
+                for (int v = 0; v < kPairTerms; ++v) tt[v] = from(t[v], l);
+                acc_add<kFluid>(a, uint32_t(__builtin_amdgcn_readlane(int(f), l)), tt);
             }
+            add_own(65);
+            if (lane == 0) cell_finish<kFluid>(c, w, P, wi, s, slot, bt, a, by * w.nbx + bx);
         }
     }
+    return make_int2((crowded >> lane) & 1u && lane < kEdgeAlone ? m0 + lane : m1, m1);
 }
 
-// A chunk with a row too dense for LDS: every cell walks its stencil in global memory, entries of
-// a bin by increasing previous index (selection over the bin), same order and results.
-template <bool kFluid>
-__device__ __forceinline__ void rows_direct(const Ctx& c, const DevWorld& w, const DevParams& P, int wi, const StripGeom& g, int y0,
-                            int IY) {
-    const uint32_t base = g.base;
-    auto binRange = [&](int gb, int& s0, int& n) {
-        s0 = g.cellOff + int(c.start[gb] - base);
-        n = int(c.start[gb + 1] - c.start[gb]);
-    };
-    for (int y = y0; y < y0 + IY; ++y) {
-        const int rowFirst = g.binOff + y * g.nbx + g.x0;
-        const int m0 = g.cellOff + int(c.start[rowFirst] - base);
-        const int m1 = g.cellOff + int(c.start[rowFirst + g.IX] - base);
-        for (int m = m0 + int(threadIdx.x); m < m1; m += kRowThreads) {
-            // the bin of map position m: the last bin of the row segment starting at or before m
-            int lo = 0, hi = g.IX;
-            while (hi - lo > 1) {
-                const int mid = (lo + hi) >> 1;
-                if (g.cellOff + int(c.start[rowFirst + mid] - base) <= m)
-                    lo = mid;
-                else
-                    hi = mid;
-            }
-            const int hx = lo + 1;
-            // (the map holds every bin's cells by previous index: a cell's logical index is its map
-            // position)
-            const int i = c.sorted[m];
-            const Nb self = global_nb<kFluid>(c, i, m);
-            cell_direct<kFluid>(c, w, P, wi, self, [&](auto&& visit) {
-                for (int dy = -1; dy <= 1; ++dy)
-                    for (int dx = -1; dx <= 1; ++dx) {
-                        int s0, n;
-                        binRange(strip_bin(g, y + dy, hx + dx), s0, n);
-                        for (int t = 0; t < n; ++t) visit(global_nb<kFluid>(c, c.sorted[s0 + t], s0 + t));
-                    }
-            });
-        }
-    }
-}
-
-// Whether staged rows y0-1 .. y0+IY (kSub bin rows each) each fit a row in flight and every three
-// consecutive ones the pool (the same answer on every lane).
-template <int kSub>
-__device__ __forceinline__ bool stage_fits(const Ctx& c, const StripGeom& g, int y0, int IY) {
-    const int lane = threadIdx.x;
-    int total = 0;
-    if (lane < IY + 2) {
-        const int Y = y0 - 1 + lane;
-#pragma unroll
-        for (int t = 0; t < kSub; ++t) {
-            const int yy = kSub * Y + t;
-            const int rowFirst = g.binOff + wrap_small(yy, g.nby) * g.nbx + g.x0;
-            total += int(c.start[rowFirst + g.IX] - c.start[rowFirst]);
-            const int gl = strip_bin(g, yy, 0), gr = strip_bin(g, yy, g.IX + 1);
-            total += int(c.start[gl + 1] - c.start[gl]) + int(c.start[gr + 1] - c.start[gr]);
-        }
-    }
-    const int three = total + __shfl_down(total, 1, kRowThreads) + __shfl_down(total, 2, kRowThreads);
-    return !__any(total > kRowCap || (lane < IY && three > kPool));
-}
-
-// One chunk of IY staged rows from staged row y0 (kSub bin rows each); false (and nothing done)
-// when its staged rows do not fit the LDS.
-template <bool kFluid, int kSub, class RS>
-__device__ __forceinline__ bool chunk_rows(const Ctx& c, const DevWorld& w, const DevParams& P, int wi,
-                                           StripGeom& g, RS& S, int y0, int IY) {
-    const int nbyS = g.nby / kSub;
-    // Away from the seam no staged bin wraps, and two stencil neighbours lie less than three bin
-    // edges apart (the last column and row absorb less than one edge of remainder) while half the
-    // world is at least four: the torus difference is the plain difference there, bit for bit.
-    g.seam = g.x0 == 0 || g.x0 + g.IX >= g.nbx || y0 == 0 || y0 + IY >= nbyS || g.nbx < 8 || g.nby < 8;
-    if (!stage_fits<kSub>(c, g, y0, IY)) return false;
-
-    RowFlight<kSub> F, G;
-    int head = 0;  // pool position of the next committed row
-    // rows y0-1, y0, y0+1 into ring rows 0, 1, 2
-    for (int r = 0; r < 3; ++r) {
-        row_issue_counts<kSub>(c, g, y0 - 1 + r, F);
-        row_issue_entries<kSub>(c, g, S, F);
-        row_commit<kSub>(g, S, F, r, head);
-        head += F.total;
-    }
-    if (IY >= 2) row_issue_counts<kSub>(c, g, y0 + 2, F);
-    for (int y = y0; y < y0 + IY; ++y) {
-        const int rc = (y - y0 + 1) % 3;
-        const int rm_ = (rc + 2) % 3, rp = (rc + 1) % 3;
-        const bool next = y + 2 <= y0 + IY;  // row y+2 is the lower halo of row y+1
-        if (next) {
-            row_issue_entries<kSub>(c, g, S, F);
-            if (y + 3 <= y0 + IY) row_issue_counts<kSub>(c, g, y + 3, G);
-        }
-        row_compute<kFluid, kSub>(c, w, P, wi, g, S, rm_, rc, rp);
-        if (next) {
-            row_commit<kSub>(g, S, F, rm_, head);  // row y+2 replaces row y-1
-            head += F.total;
-#pragma unroll
-            for (int q = 0; q < RowFlight<kSub>::kSlots; ++q) {
-                F.s0[q] = G.s0[q];
-                F.s1[q] = G.s1[q];
-            }
-        }
-    }
-    return true;
-}
-
-// A collision world staged two bin rows at a time (sparse rows) runs a chunk whose two-row stages
-// do not fit as single bin rows over the same bins.
-// (four waves per SIMD, 128 VGPRs without scratch: at 133 VGPRs and three waves the eight-world batch ran
-// 13 % slower)
-template <bool kFluid>
-__global__ void __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
-k_neighbor_rows(Ctx c, int sortBlocks) {
-    __shared__ RowShared<kFluid ? 1 : kSubMax> S;
-    // (the particles' bin sort, on workgroups of its own, in sets with bond work)
-    if (int(blockIdx.x) < sortBlocks) {
-        part_binsort(c, {int(blockIdx.x), sortBlocks});
-        return;
-    }
-    const int2 tb = c.tileBlocks[int(blockIdx.x) - sortBlocks];
-    if (tb.x < 0) return;
-    const int wi = tb.x;
+// Wave v of the world: 64 (fewer in small sets, fluidShift) consecutive map positions of the first bin row, of the last one, or of those
+// between (each of the three parts has its own last wave, so that no wave has lanes whose stencil rows
+// are at different ends of the map).  Returns the map position that this lane is left to walk alone, or -1.
+template <Pass kPass>
+__device__ __forceinline__ int fluid_wave(const Ctx& c, FluidWave<kBonded<kPass>>& S, int wi, int v) {
+    constexpr bool kBonds = kBonded<kPass>, kCollide = kPass == Pass::kCollide;
+    constexpr int kStage = kBonds ? kBondStage : kFreeStage, kPairs = kBonds ? kBondPairs : kFreePairs;
+    const int lane = int(threadIdx.x) & 63;
     // the world and its parameters are read once, before any store: read through references,
     // every use after a global store would load them again
     const DevWorld w = c.worlds[wi];
     const DevParams P = c.params[wi];
-    if ((P.motion == 0) != kFluid) return;
-    const int strip = tb.y % w.ntx, chunk = tb.y / w.ntx;
-    StripGeom g;
-    g.x0 = strip * w.tileX;
-    g.IX = min(w.tileX, w.nbx - g.x0);
-    g.HX = g.IX + 2;
-    g.nbx = w.nbx;
-    g.nby = w.nby;
-    g.binOff = w.binOff;
-    g.cellOff = w.cellOff;
-    g.base = c.start[w.binOff];
-    g.seam = true;
-    const int y0 = chunk * w.tileY;  // in staged rows of w.rowsPerStage bin rows
-    const int IY = min(w.tileY, w.nby / w.rowsPerStage - y0);
-    const int by0 = w.rowsPerStage * y0, bIY = w.rowsPerStage * IY;  // the chunk in bin rows
-    bool done = false;
-    // (fluid worlds are always staged one bin row at a time: the two-row variant would cost the
-    // fluid kernel a third of its resident waves in registers)
-    if constexpr (!kFluid)
-        if (w.rowsPerStage == 2) done = chunk_rows<kFluid, 2>(c, w, P, wi, g, S, y0, IY);
-    if (!done) done = chunk_rows<kFluid, 1>(c, w, P, wi, g, S, by0, bIY);
-    if (!done) {
-        // too crowded for the LDS staging: every cell walks its stencil in global memory, and the
-        // owner-counted part of the region's bins is empty
-        if (threadIdx.x == 0) atomicAdd(&c.sc->fallbackChunks, 1ull);
-        rows_direct<kFluid>(c, w, P, wi, g, by0, bIY);
+    const uint32_t* start = c.start + w.binOff;
+    const int off = w.cellOff - int(start[0]);
+    int m0, mEnd;
+    {
+        const int r1 = int(start[w.nbx] - start[0]), r2 = int(start[(w.nby - 1) * w.nbx] - start[0]);
+        const int sh = kCollide ? c.collideShift : c.fluidShift, more = (1 << sh) - 1;
+        const int v1 = (r1 + more) >> sh, v2 = v1 + ((r2 - r1 + more) >> sh);
+        const int at = v < v1 ? v << sh : (v < v2 ? r1 + ((v - v1) << sh) : r2 + ((v - v2) << sh));
+        m0 = w.cellOff + at;
+        mEnd = w.cellOff + min(at + more + 1, v < v1 ? r1 : (v < v2 ? r2 : w.numCells));
     }
+    if ((P.motion == 0) == kCollide || m0 >= mEnd) return -1;  // (a wave past its world)
+    const int m = m0 + lane;
+    const bool active = m < mEnd;
+    const float Wf = float(w.W), Hf = float(w.H);
+    const float w0 = kCollide ? 0.0f : sph_w(0.0f) * P.invH2;  // a cell's own density term
+
+    int aidx = 0, slot = 0;
+    f2 pos = {0.0f, 0.0f}, vel = {0.0f, 0.0f};
+    float inv = 0.0f;
+    uint32_t flags = 0u;
+    if (active) {
+        aidx = ld32(c.sorted, m);
+        pos = to_f2(ld32(c.A.pos, aidx));
+        vel = to_f2(ld32(c.A.vel, aidx));
+        if (!kCollide) inv = ld32(c.A.dens, aidx);
+        flags = ld32(c.A.flags, aidx);
+        slot = ld32(c.A.slot, aidx);
+    }
+    // the own bonds, early: the pairs ask the owners for them
+    int bt[kMaxBonds];
+#pragma unroll
+    for (int b = 0; b < kMaxBonds; ++b)
+        bt[b] = kBonds && active && b < flags_num_conn(flags) ? c.A.btgt[b * c.cellCap + aidx] : -1;
+    int bx, by;
+    cell_bin_xy(w, pos, bx, by);
+    // (rounding may put a position on the far edge itself, which is bin 0, or it may be no number)
+    const bool plain = pos.x < Wf && pos.y < Hf;
+    const bool edge = bx == 0 || bx == w.nbx - 1;
+    const bool mine = active && !edge;  // (edge cells belong to the edge waves)
+    bool alone = mine && !plain;
+    // the ranges; a bin (or bin row) next to the cell's is left out when its near edge is out of reach
+    int lo[3] = {0, 0, 0}, ns[3] = {0, 0, 0};
+    if (mine && !alone) {
+        const float X0 = float(bx * w.binSize);
+        const float l = pos.x - X0, r = pos.x - (X0 + float(w.binSize));
+        const int b0 = l * l <= P.reachSq ? bx - 1 : bx, b1 = r * r <= P.reachSq ? bx + 2 : bx + 1;
+        const int rows[3] = {by == 0 ? w.nby - 1 : by - 1, by, by == w.nby - 1 ? 0 : by + 1};
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const uint32_t rb = uint32_t(rows[k] * w.nbx);
+            lo[k] = off + int(ld32(start, rb + uint32_t(b0)));
+            ns[k] = off + int(ld32(start, rb + uint32_t(b1))) - lo[k];
+        }
+    }
+    // up and down rows out of reach
+    if (mine && !alone) {
+        const float Y0 = float(by * w.binSize);
+        const float up = pos.y - Y0, down = pos.y - (by == w.nby - 1 ? Hf : Y0 + float(w.binSize));
+        if (up * up > P.reachSq) ns[0] = 0;
+        if (down * down > P.reachSq) ns[2] = 0;
+        alone = ns[0] + ns[1] + ns[2] > 64;
+    }
+    Acc acc;
+    {
+        Nb self;
+        self.pos = pos;
+        acc_init(acc, self);
+    }
+    if constexpr (kCollide) {
+        // (counted: waves too crowded for the stage)
+        const unsigned long long all = __ballot(mine);
+        if (__ballot(alone) & all) {
+            const int first = __builtin_ctzll(all), last = 63 - __builtin_clzll(all);
+            const int bF = __builtin_amdgcn_readlane(by, first) * w.nbx + __builtin_amdgcn_readlane(bx, first);
+            const int bL = __builtin_amdgcn_readlane(by, last) * w.nbx + __builtin_amdgcn_readlane(bx, last);
+            if (int(start[bL + 1]) - int(start[bF]) > kStage / 3 && lane == 0) atomicAdd(&c.sc->fallbackChunks, 1ull);
+        }
+    }
+    // The staged stretch of each stencil row, [u0, u0 + un): from the left bin of the first testing lane to
+    // the right bin of the last one (both grow with the lane: a wave is in the torus' first bin row, in its
+    // last one, or in neither).  Lanes whose rows do not fit the stage walk alone.
+    unsigned long long group = __ballot(mine && !alone);
+    {
+        const int first = group ? __builtin_ctzll(group) : 0;
+        const int bxF = __builtin_amdgcn_readlane(bx, first), byF = __builtin_amdgcn_readlane(by, first);
+        int u0[3], un[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            u0[k] = group ? off + int(start[wrap_small(byF + k - 1, w.nby) * w.nbx + bxF - 1]) : 0;
+            un[k] = 0;
+        }
+        for (int keep = 32; group;) {
+            const int last = 63 - __builtin_clzll(group);
+            const int bxL = __builtin_amdgcn_readlane(bx, last), byL = __builtin_amdgcn_readlane(by, last);
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+                un[k] = off + int(start[wrap_small(byL + k - 1, w.nby) * w.nbx + bxL + 2]) - u0[k];
+            if (__builtin_expect(un[0] + un[1] + un[2] <= kStage, 1)) break;
+            group &= keep ? ((1ull << keep) - 1ull) << first : 0ull;
+            keep >>= 1;
+            if (!group) un[0] = un[1] = un[2] = 0;
+        }
+        const int un01 = un[0] + un[1], unAll = un01 + un[2];
+        const bool tests = __builtin_amdgcn_inverse_ballot_w64(group);
+        alone = mine && !tests;
+        {
+            const int g0 = u0[0], g1 = u0[1] - un[0], g2 = u0[2] - un01;
+            constexpr int kLoads = (kStage + 63) / 64;
+            int a[kLoads];
+            float2 v[kLoads];
+#pragma unroll
+            for (int q = 0; q < kLoads; ++q) {
+                const int x = lane + 64 * q;
+                a[q] = x < unAll ? ld32(c.sorted, uint32_t(x + (x < un[0] ? g0 : (x < un01 ? g1 : g2)))) : 0;
+            }
+#pragma unroll
+            for (int q = 0; q < kLoads; ++q)
+                if (64 * q < unAll) v[q] = ld32(c.A.pos, uint32_t(a[q]));
+#pragma unroll
+            for (int q = 0; q < kLoads; ++q)
+                if (lane + 64 * q < unAll) {
+                    S.cpos[lane + 64 * q] = v[q];
+                    S.caidx(lane + 64 * q) = a[q];
+                }
+        }
+        // (in grids of at least eight bins each way, two stencil neighbours lie less than three bin edges
+        // apart, less than half the world: away from the seam rows the plain difference equals the torus
+        // difference bit for bit)
+        // (collision pairs are tested by their plain difference, R13: no neighbours across the seam)
+        const bool seam = !kCollide && (byF == 0 || byF == w.nby - 1 || w.nbx < 8 || w.nby < 8);
+        S.pos[lane] = tests ? to_float2(pos) : make_float2(__builtin_nanf(""), 0.0f);
+        // A lane without a list gets one entry that no test accepts, so that list k belongs to lane k.
+        const int nt = tests ? ns[0] + ns[1] + ns[2] : 1;
+        const int inc = int(wave_inclusive_scan(uint32_t(nt)));
+        const int flat = inc - nt, flatAll = wave_last(inc);
+        const int selfBase = m0 - u0[1] + un[0];  // the own entry of lane 0
+        int numPairs = 0;
+        for (int R0 = 0;; R0 += kPairs) {
+            {
+                int4 rec = make_int4(flat | flat << 16, -flat, -flat, -flat);
+                if (tests) {
+                    const int b1 = flat + ns[0], b2 = b1 + ns[1];
+                    rec.x = b1 | b2 << 16 | (kPass == Pass::kBonds && flags_barrier(flags) ? int(0x80000000u) : 0);
+                    rec.y = lo[0] - u0[0] - flat;
+                    rec.z = lo[1] - u0[1] + un[0] - b1;
+                    rec.w = lo[2] - u0[2] + un01 - b2;
+                }
+                S.u.t.start[lane] = 0u;
+                S.u.t.start[lane + 64] = 0u;
+                S.u.t.rec[lane] = rec;
+                __syncwarp();
+                atomicOr(&S.u.t.start[flat >> 5], 1u << (flat & 31));
+                __syncwarp();
+            }
+            numPairs = 0;
+            auto test = [&](auto seamTag) {
+                constexpr bool kSeam = decltype(seamTag)::value;
+                int owners = -1;  // lists that started before this round, minus one
+                for (int f0 = 0; f0 < flatAll; f0 += 64) {
+                    const uint32_t s0 = __builtin_amdgcn_readfirstlane(S.u.t.start[f0 >> 5]);
+                    const uint32_t s1 = __builtin_amdgcn_readfirstlane(S.u.t.start[(f0 >> 5) + 1]);
+                    const unsigned long long starts = (static_cast<unsigned long long>(s1) << 32) | s0;
+                    const int owner = lanes_below(starts >> 1, owners + int(s0 & 1u));
+                    owners += __builtin_popcountll(starts);
+                    const int f = f0 + lane;
+                    const bool in = f < flatAll;
+                    const int4 rec = S.u.t.rec[owner];
+                    const f2 ps = to_f2(S.pos[owner]);
+                    const int b1 = rec.x & 0xffff, b2 = kBonds ? (rec.x >> 16) & 0x7fff : rec.x >> 16;
+                    const int x = f + (f < b1 ? rec.y : (f < b2 ? rec.z : rec.w));
+                    const f2 pn = to_f2(S.cpos[x]);
+                    const float d2 = lensq(kSeam ? torus_delta(ps, pn, Wf, Hf) : sub(ps, pn));
+                    // a barrier cell meets itself as a barrier neighbour; any other cell adds its own
+                    // density term at its place in the visiting order, without a pair
+                    const bool self = in && x == owner + selfBase;
+                    const bool hit = in && d2 <= P.reachSq && (!self || (kPass == Pass::kBonds && rec.x < 0));
+                    const unsigned long long hits = __ballot(hit);
+                    const int rank = lanes_below(hits, numPairs);
+                    if (__builtin_amdgcn_inverse_ballot_w64(starts)) S.first[owner] = uint16_t(rank);
+                    if (!kCollide && self) S.own[owner] = uint16_t(rank);
+                    // (a wave's pairs nearly always fit one window: then no lane asks)
+                    if (R0 == 0 && numPairs + __builtin_popcountll(hits) <= kPairs) {
+                        if (hit) S.pair[rank] = uint16_t(x | owner << 9);
+                    } else if (hit && uint32_t(rank - R0) < uint32_t(kPairs)) {
+                        S.pair[rank - R0] = uint16_t(x | owner << 9);
+                    }
+                    numPairs += __builtin_popcountll(hits);
+                }
+            };
+            if (seam)
+                test(std::true_type{});
+            else
+                test(std::false_type{});
+            if (lane == 0) S.first[64] = uint16_t(numPairs);
+            __syncwarp();
+            int pairs0 = S.first[lane], pairs1 = S.first[lane + 1];
+            const int ownAt = kCollide || (kBonds && flags_barrier(flags)) ? -1 : S.own[lane];
+            int rend = min(numPairs, R0 + kPairs);
+            if constexpr (kCollide) {
+                // Most neighbours in a body are bonded, and a bonded pair adds only its overlap push (closer
+                // than minDistance, not for a barrier cell): the other records go, bit 15 marks what stays of
+                // the bonded ones.  (In place: a round's records land at or before their own places.)
+                int to = R0;
+                const int from0 = pairs0, from1 = pairs1;
+                pairs0 = from0 <= R0 ? R0 : rend;
+                pairs1 = from1 <= R0 ? R0 : rend;
+                for (int p0 = R0; p0 < rend; p0 += 64) {
+                    const int p = p0 + lane;
+                    const int r = p < rend ? S.pair[p - R0] : 0;
+                    const int x = r & 0x1ff, ol = r >> 9;
+                    const uint32_t sf = uint32_t(__shfl(int(flags), ol, 64));
+                    bool bonded = false;
+                    if (__any(p < rend && flags_num_conn(sf) > 0)) {
+                        const int oa = S.caidx(x) - w.cellOff;
+#pragma unroll
+                        for (int b = 0; b < kMaxBonds; ++b) {
+                            const int partner = __shfl(bt[b], ol, 64);  // (every lane takes part)
+                            bonded = bonded || partner == oa;
+                        }
+                    }
+                    const bool push = !flags_barrier(sf) && lensq(sub(to_f2(S.pos[ol]), to_f2(S.cpos[x]))) <= P.overlapBelowSq;
+                    const bool stays = p < rend && (!bonded || push);
+                    const unsigned long long m = __ballot(stays);
+                    if (stays) S.pair[lanes_below(m, to) - R0] = uint16_t(r | (bonded ? 0x8000 : 0));
+                    // the owners' first and last records move along
+                    if (from0 > p0 && from0 <= p0 + 64) pairs0 = to + __builtin_popcountll(m & (~0ull >> (p0 + 64 - from0)));
+                    if (from1 > p0 && from1 <= p0 + 64) pairs1 = to + __builtin_popcountll(m & (~0ull >> (p0 + 64 - from1)));
+                    to += __builtin_popcountll(m);
+                }
+                if (from0 > rend) pairs0 = to;
+                if (from1 > rend) pairs1 = to;
+                rend = to;
+                __syncwarp();
+            }
+            for (int p0 = R0; p0 < rend; p0 += 64) {
+                // pair terms, one pair per lane
+                float4 ra = make_float4(0.0f, 0.0f, 0.0f, 0.0f), rb = ra;
+                const int p = p0 + lane;
+                int x = 0, ol = 0, bonded = 0;  // (bonded: of a collision pair)
+                if (p < rend) {
+                    const int r = S.pair[p - R0];
+                    x = r & 0x1ff;
+                    ol = (r >> 9) & 63;
+                    bonded = r >> 15;
+                }
+                // the owner's state, from its registers
+                const f2 sv = {__shfl(vel.x, ol, 64), __shfl(vel.y, ol, 64)};
+                const float si = kCollide ? 0.0f : __shfl(inv, ol, 64);
+                const f2 sp = to_f2(S.pos[ol]);
+                const uint32_t sf = kBonds ? uint32_t(__shfl(int(flags), ol, 64)) : 0u;
+                const int sa = kBonds ? __shfl(aidx, ol, 64) : 0;
+                int sb[kMaxBonds];
+                if constexpr (kPass == Pass::kBonds) {
+                    // (no permutes for a round without a bonded owner)
+                    if (__any(flags_num_conn(sf) > 0)) {
+    #pragma unroll
+                        for (int b = 0; b < kMaxBonds; ++b) sb[b] = __shfl(bt[b], ol, 64);
+                    } else {
+    #pragma unroll
+                        for (int b = 0; b < kMaxBonds; ++b) sb[b] = -1;
+                    }
+                }
+                if (p < rend) {
+                    const int oa = S.caidx(x);
+                    const f2 op = to_f2(S.cpos[x]);
+                    const f2 ov = to_f2(ld32(c.A.vel, uint32_t(oa)));
+                    const float oi = kCollide ? 0.0f : ld32(c.A.dens, uint32_t(oa));
+                    const f2 pd = stencil_delta(sp, op, Wf, Hf, seam);
+                    const f2 vd = sub(sv, ov);
+                    if constexpr (kCollide) {
+                        Nb s, o;
+                        s.pos = sp, s.vel = sv, s.flags = sf, s.aidx = sa;
+                        o.pos = op, o.vel = ov, o.flags = ld32(c.A.flags, uint32_t(oa)), o.aidx = oa;
+                        float t[kPairTerms] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+                        const uint32_t f = pair_term<false>(c, w, P, wi, s, o, bonded != 0, t, false, [&] {
+                            return make_int2(m0 + ol, x + (x < un[0] ? u0[0] : (x < un01 ? u0[1] - un[0] : u0[2] - un01)));
+                        });
+                        ra = make_float4(t[0], t[1], t[2], t[3]);
+                        rb = make_float4(t[4], t[5], __int_as_float(int(f)), 0.0f);
+                    } else if constexpr (!kBonds) {
+                        const FluidTerms t = fluid_terms<false>(P, pd, vd, si, oi, true);
+                        ra = make_float4(t.rho, t.D.x, t.D.y, 0.0f);
+                        rb = make_float4(t.Fp.x, t.Fp.y, t.Fv.x, t.Fv.y);
+                    } else {
+                        const uint32_t of = ld32(c.A.flags, uint32_t(oa));
+                        if (flags_barrier(of)) {
+                            ra.x = len2(pd);
+                            ra.w = __int_as_float(oa + 1);
+                        } else {
+                            const bool bonded = is_bonded(sb, oa - w.cellOff);
+                            const int nc = flags_num_conn(sf);
+                            const bool bari = flags_barrier(sf);
+                            const FluidTerms t = fluid_terms<true>(P, pd, vd, si, oi, !bonded);
+                            ra = make_float4(t.rho, bari ? 0.0f : t.D.x, bari ? 0.0f : t.D.y, 0.0f);
+                            rb = make_float4(t.Fp.x, t.Fp.y, t.Fv.x, t.Fv.y);
+                            if (!bonded && !bari && nc < flags_max_conn(sf) && flags_num_conn(of) < flags_max_conn(of) &&
+                                lensq(vd) > P.fusionBelowSq) {
+                                const int sl = m0 + ol, olx = x + (x < un[0] ? u0[0] : (x < un01 ? u0[1] - un[0] : u0[2] - un01));
+                                if (sl < olx) {
+                                    const float ei = c.energy[w.cellOff + c.A.slot[sa]];
+                                    const float ej = c.energy[w.cellOff + c.A.slot[oa]];
+                                    if (ei <= P.maxBindingEnergy && ej <= P.maxBindingEnergy) push_candidate(c, sl, olx, wi);
+                                }
+                            }
+                        }
+                    }
+                }
+                __syncwarp();  // (the test's records, and the round before, are done with)
+                S.u.r.a[lane] = ra;
+                S.u.r.b[lane] = rb;
+                __syncwarp();
+                // every owner adds its pairs of this round in visiting order; terms a pair does not have
+                // are zero, which leaves a sum that started at +0 unchanged bit for bit
+                const int j1 = min(pairs1, min(p0 + 64, rend));
+                for (int j = max(pairs0, p0); j < j1; ++j) {
+                    const float4 ta = S.u.r.a[j - p0], tb = S.u.r.b[j - p0];
+                    if constexpr (kCollide) {
+                        acc_add_collision(acc, uint32_t(__float_as_int(tb.z)), f2{ta.x, ta.y}, f2{ta.z, ta.w}, f2{tb.x, tb.y});
+                        continue;
+                    }
+                    acc.rho = j == ownAt ? acc.rho + w0 : acc.rho;
+                    if constexpr (kBonds) {
+                        // of the barrier neighbours only the first ten count, and of those the first
+                        // nearest one (CellProcessor.cuh:234-246)
+                        const bool bar = __float_as_int(ta.w) != 0;
+                        const bool nearest = bar && acc.numBarrier < 10 && (acc.cb < 0 || ta.x < acc.cbDist);
+                        acc.cb = nearest ? __float_as_int(ta.w) - 1 : acc.cb;
+                        acc.cbDist = nearest ? ta.x : acc.cbDist;
+                        acc.numBarrier += bar ? 1 : 0;
+                        acc.rho = bar ? acc.rho : acc.rho + ta.x;
+                    } else {
+                        acc.rho = acc.rho + ta.x;
+                    }
+                    acc.D = add(acc.D, f2{ta.y, ta.z});
+                    acc.Fp = add(acc.Fp, f2{tb.x, tb.y});
+                    acc.Fv = add(acc.Fv, f2{tb.z, tb.w});
+                }
+            }
+            if (R0 + kPairs >= numPairs) {
+                if (!kCollide && tests && ownAt == pairs1) acc.rho = acc.rho + w0;  // the own term after all pairs
+                break;
+            }
+            __syncwarp();
+        }
+    }
+    if (!mine) return -1;
+    if (alone) return m;
+    const int bOld = by * w.nbx + bx;
+    if constexpr (kBonds) {
+        Nb self;
+        self.pos = pos;
+        self.vel = vel;
+        self.dens = inv;
+        self.flags = flags;
+        self.aidx = aidx;
+        self.lidx = m;
+        cell_finish<!kCollide>(c, w, P, wi, self, slot, bt, acc, bOld);
+    } else {
+        finish_free(c, w, P, m, pos, vel, flags, slot, acc.rho, acc.D, acc.Fp, acc.Fv, bOld);
+    }
+    return -1;
 }
 
-int neighbor_blocks_per_cu() {
-    int n = 0;
-    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_neighbor_rows<false>, kRowThreads, 0);
-    return e == hipSuccess ? std::max(1, n) : 1;
+// With bonds also the particles' bin sort, on the launch's first workgroups (sets with bond work)
+template <Pass kPass>
+__global__ void __launch_bounds__(64 * kFluidWaves) __attribute__((amdgpu_waves_per_eu(kBonded<kPass> ? 4 : 6)))
+k_neighbor(Ctx c, int sortBlocks, int edgeBlocks, int tableBlocks) {
+    constexpr bool kBonds = kBonded<kPass>, kFluid = kPass != Pass::kCollide;
+    __shared__ FluidWave<kBonds> SS[kFluidWaves];
+    const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+    int block = int(blockIdx.x);
+    if constexpr (kBonds) {
+        if (block < sortBlocks) return part_binsort(c, {block, sortBlocks});
+        block -= sortBlocks;
+    }
+    int wi;
+    int2 walk = make_int2(0, 0);  // cells this lane walks alone: walk.x, walk.x + 64, ... below walk.y
+    if (block < edgeBlocks) {
+        const int2 blk = (kFluid ? c.edgeBlocks : c.collideEdgeBlocks)[block];
+        wi = blk.x;
+        constexpr int kWaves = kBonds ? kEdgeWavesBonds : kEdgeWaves;
+        const int u = blk.y + wave;
+        if (u / kWaves <= c.worlds[wi].nby) walk = edge_unit<kPass>(c, wi, u / kWaves, u % kWaves);
+    } else {
+        block -= edgeBlocks;
+        // XCD-aware: workgroup b runs on XCD b % 8, which sweeps one contiguous band of the map, so the
+        // stencil rows its waves share stay in its L2
+        const int per = (tableBlocks + kXcdCount - 1) / kXcdCount;
+        const int e = (block % kXcdCount) * per + block / kXcdCount;
+        if (e >= tableBlocks) return;
+        const int2 blk = (kFluid ? c.fluidBlocks : c.collideBlocks)[e];
+        wi = blk.x;
+        const int m = fluid_wave<kPass>(c, SS[wave], wi, blk.y + wave);
+        if (m >= 0) walk = make_int2(m, m + 1);
+    }
+    // (rare: its parameters are read again, so that the waves above do not carry them)
+    for (int m = walk.x; m < walk.y; m += 64) walk_alone<kFluid>(c, wi, m);
 }
 
-void launch_fluid(const Ctx& c, const LaunchShape& sh, hipStream_t s, int sortBlocks);
-
+// The bin sort goes with the first launch.  A set with collision worlds but no bond work at all still runs
+// the one collision variant.
 void launch_neighbor(const Ctx& c, const LaunchShape& sh, hipStream_t s, bool withPartSort) {
-    // (the bin sort goes with the first launch)
     int sort = withPartSort && sh.hasParticles && sh.partBlocks ? sh.pbinBlocks : 0;
-    const bool collision = sh.hasCollision && sh.tileBlocks;
-    if (sh.fluidBlocks || (sort && !collision)) {
-        launch_fluid(c, sh, s, sort);
+    const auto grid = [&](int edges, int table) {
+        return dim3(sort + edges + (table + kXcdCount - 1) / kXcdCount * kXcdCount);
+    };
+    const dim3 threads(sh.cellThreads);
+    if (sh.collideBlocks) {
+        hipLaunchKernelGGL(k_neighbor<Pass::kCollide>, grid(sh.collideEdgeBlocks, sh.collideBlocks), threads, 0, s, c, sort,
+                           sh.collideEdgeBlocks, sh.collideBlocks);
         sort = 0;
     }
-    if (collision) {
-        sort *= sh.binThreads / kRowThreads;
-        hipLaunchKernelGGL(k_neighbor_rows<false>, dim3(sort + sh.tileBlocks), dim3(kRowThreads), 0, s, c, sort);
-    }
+    if (sh.hasBondWork && (sh.fluidBlocks || sort))
+        hipLaunchKernelGGL(k_neighbor<Pass::kBonds>, grid(sh.edgeBlocks, sh.fluidBlocks), threads, 0, s, c, sort, sh.edgeBlocks,
+                           sh.fluidBlocks);
+    else if (sh.fluidBlocks)
+        hipLaunchKernelGGL(k_neighbor<Pass::kFree>, grid(sh.edgeBlocks, sh.fluidBlocks), threads, 0, s, c, 0, sh.edgeBlocks,
+                           sh.fluidBlocks);
 }
 
 }  // namespace alien

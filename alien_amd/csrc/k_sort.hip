@@ -314,16 +314,9 @@ __device__ __forceinline__ int rank_far(const Ctx& c, int gb, int i) {
     return n;
 }
 
-__device__ __forceinline__ void place_cell(const Ctx& c, const DevWorld& w, bool copies, int i, int dest) {
-    const int a = w.cellOff + i, d = w.cellOff + dest;
-    st32(c.sorted, uint32_t(d), a);
-    // the row-staged collision pass reads a copy of the state in map order; the fluid pass
-    // reads the state through `sorted` (a copy for it costs the scatter more than it saves)
-    if (copies) {
-        st32(c.mpos, uint32_t(d), ld32(c.A.pos, uint32_t(a)));
-        st32(c.mvel, uint32_t(d), ld32(c.A.vel, uint32_t(a)));
-        st32(c.mflags, uint32_t(d), ld32(c.A.flags, uint32_t(a)));
-    }
+// (the passes read the cells' state through `sorted`: a copy of it in map order costs more than it saves)
+__device__ __forceinline__ void place_cell(const Ctx& c, const DevWorld& w, int i, int dest) {
+    st32(c.sorted, uint32_t(w.cellOff + dest), w.cellOff + i);
 }
 
 __device__ __forceinline__ void far_scatter(const Ctx& c, int wave, int waves, int lane) {
@@ -331,8 +324,7 @@ __device__ __forceinline__ void far_scatter(const Ctx& c, int wave, int waves, i
     for (int q = wave; q < total; q += waves) {
         const int2 f = c.far.list[q];
         if (f.y < 0) continue;  // (seeded while its world was left out)
-        const int wi = world_of(c, f.y);
-        const DevWorld& w = c.worlds[wi];
+        const DevWorld& w = c.worlds[world_of(c, f.y)];
         if (!w.active) continue;
         const int g = f.y / kGroupBins, b0 = g * kGroupBins - w.binOff;
         const uint32_t t = uint32_t(f.y - w.binOff - b0);
@@ -356,15 +348,14 @@ __device__ __forceinline__ void far_scatter(const Ctx& c, int wave, int waves, i
                 }
             }
         const int at = base + wave_last(int(wave_inclusive_scan(n))) + rank_far(c, f.y, f.x);
-        if (lane == 0) place_cell(c, w, c.params[wi].motion != 0, i, at);
+        if (lane == 0) place_cell(c, w, i, at);
     }
 }
 
 __device__ __forceinline__ void cell_scatter(const Ctx& c, ScatterShared& S, int g, int lane) {
     const int g0 = g * kGroupBins;
     if (g0 >= c.numCellBins) return;
-    const int wi = world_of(c, g0);
-    const DevWorld& w = c.worlds[wi];
+    const DevWorld& w = c.worlds[world_of(c, g0)];
     const int b0 = g0 - w.binOff, bins = w.nbx * w.nby;
     const uint32_t* prev = c.startPrev + w.binOff;
     const int prevBase = int(prev[0]);
@@ -383,7 +374,6 @@ __device__ __forceinline__ void cell_scatter(const Ctx& c, ScatterShared& S, int
     const int nb = min(kGroupBins, bins - b0);
     const int p0 = int(prev[b0]) - prevBase, p1 = int(prev[b0 + nb]) - prevBase;  // the bins' own cells
     const Places p = places_of(reach_of(w, b0, nb), prev);
-    const bool copies = c.params[wi].motion != 0;
     const int farCells = c.far.group[g];
     const int* binOf = c.binOf + w.cellOff;
     const int base = p0 + gained_before(c, w, g, lane);
@@ -487,7 +477,7 @@ __device__ __forceinline__ void cell_scatter(const Ctx& c, ScatterShared& S, int
                                      : __builtin_popcountll(left & below & ~((1ull << (sb - i0)) - 1ull));
             int rank = i - sb - gone + int(S.before[t]);
             if (farCells) rank += rank_far(c, g0 + int(t), w.cellOff + i);
-            place_cell(c, w, copies, i, S.start[t] + rank);
+            place_cell(c, w, i, S.start[t] + rank);
         }
         longGone += __builtin_popcountll(left);
         leftPrev = left;
@@ -510,7 +500,7 @@ __device__ __forceinline__ void cell_scatter(const Ctx& c, ScatterShared& S, int
             if (farCells) at -= c.far.count[g0 + t];
         }
         if (farCells) at += rank_far(c, g0 + t, w.cellOff + i);
-        place_cell(c, w, copies, i, at);
+        place_cell(c, w, i, at);
     };
     if (listed <= kScatterList) {
         for (int q0 = 0; q0 < listed; q0 += 64) {

@@ -15,11 +15,10 @@ struct LaunchShape {
     int partBlocks = 0, partThreads = 256;
     int pbinBlocks = 0, binThreads = 256;
     int fluidBlocks = 0, edgeBlocks = 0;  // workgroups of the fluid pass: inner cells, edge columns
-    int tileBlocks = 0;    // neighbour-pass workgroups (including XCD padding)
+    int collideBlocks = 0, collideEdgeBlocks = 0;  // of the collision pass
     int partGrid = 64;     // grid-stride particle kernels
     int bondBlocks = 0;    // bond kernels: cell blocks of the worlds that can have bonded cells
     int candGrid = 16;     // grid-stride kernels over fusion candidates
-    bool hasFluid = false, hasCollision = false;  // motion modes present in the set
     bool hasBondWork = true;  // some active world has (or can get by fusion) a bonded or barrier cell
     // some world has live energy particles or radiates (only cell radiation creates particles, so
     // once all are absorbed or merged in a set without it the particle kernels, which would find
@@ -42,14 +41,12 @@ void launch_fill_u32(uint32_t* p, uint32_t v, size_t n, hipStream_t s);
 int map_scan_tiles(int partBins);
 // bins of the current state (A) for the next sort; the step keeps them up to date itself
 void launch_seed_bins(const Ctx& c, const LaunchShape& sh, hipStream_t s);
-// workgroups of the row-streaming (collision) neighbour pass one CU keeps resident
-int neighbor_blocks_per_cu();
 // A second stream of the same priority and two events: in sets without bond work the particles' chain
 // runs on it beside the neighbour pass (which then reads none of the energies it changes), joined
 // before the kernels after the pass.
 struct SideStream {
     hipStream_t stream = nullptr;
-    hipEvent_t fork = nullptr, join = nullptr;  // after the scatter, after the particles
+    hipEvent_t fork = nullptr, join = nullptr;  // after the map, after the particles
 };
 // rec != nullptr (per-kernel timing) launches everything on s, one kernel after another
 void launch_step(const Ctx& c, const LaunchShape& sh, hipStream_t s, Recorder* rec = nullptr,

@@ -192,35 +192,13 @@ __device__ __forceinline__ void acc_add(Acc& a, uint32_t f, const float* t) {
     }
 }
 
-// acc_add without branches, for terms zeroed before pair_term wrote them (lanes with !on add
-// nothing).  Adding a zero term leaves a sum that started at +0 unchanged bit for bit (such a sum
-// is never -0), so the flags select only what is not a plain zero: a barrier neighbour's data, and
-// the collision position sum, which starts at the cell's position.
-template <bool kFluid>
-__device__ __forceinline__ void acc_add_sel(Acc& a, bool on, uint32_t f, const float* t) {
-    if constexpr (kFluid) {
-        const bool bar = on && (f & kPairBarrier) != 0u;
-        const bool sum = on && !bar;
-        const bool near = bar && a.numBarrier < 10 && (a.cb < 0 || t[1] < a.cbDist);
-        a.cb = near ? __float_as_int(t[0]) : a.cb;
-        a.cbDist = near ? t[1] : a.cbDist;
-        a.numBarrier += bar ? 1 : 0;
-        a.rho = sum ? a.rho + t[0] : a.rho;
-        a.D.x = sum ? a.D.x + t[1] : a.D.x;
-        a.D.y = sum ? a.D.y + t[2] : a.D.y;
-        a.Fp.x = on ? a.Fp.x + t[3] : a.Fp.x;
-        a.Fp.y = on ? a.Fp.y + t[4] : a.Fp.y;
-        a.Fv.x = on ? a.Fv.x + t[5] : a.Fv.x;
-        a.Fv.y = on ? a.Fv.y + t[6] : a.Fv.y;
-    } else {
-        const bool ov = on && (f & kPairOverlap) != 0u;
-        a.pc.x = ov ? a.pc.x + t[0] : a.pc.x;
-        a.pc.y = ov ? a.pc.y + t[1] : a.pc.y;
-        f2 F = add(a.F, f2{t[2], t[3]});
-        F = add(F, f2{t[4], t[5]});
-        a.F.x = on ? F.x : a.F.x;
-        a.F.y = on ? F.y : a.F.y;
-    }
+// acc_add of a collision pair without branches, for terms zeroed before pair_term wrote them.  Adding a
+// zero term leaves a sum that started at +0 unchanged bit for bit (such a sum is never -0), so the flags
+// select only for the position sum, which starts at the cell's position.
+__device__ __forceinline__ void acc_add_collision(Acc& a, uint32_t f, f2 push, f2 f1, f2 f2nd) {
+    const f2 pc = add(a.pc, push);
+    if (f & kPairOverlap) a.pc = pc;
+    a.F = add(add(a.F, f1), f2nd);
 }
 
 __device__ __forceinline__ void load_bonds(const Ctx& c, const Nb& s, int bt[kMaxBonds]) {

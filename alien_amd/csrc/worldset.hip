@@ -201,7 +201,7 @@ WorldImage WorldImage::fromTO(const alien_world_desc& desc, const alien_params& 
         const int bs = bin_size_for(params);
         const int nbx = std::max(1, W / bs), nby = std::max(1, H / bs);
         const size_t bins = size_t(nbx) * nby;
-        HostArray<int> key(n), next(bins);
+        HostArray<int> key(n), count(bins);
         for_ranges(size_t(n), [&](size_t i0, size_t i1) {
             for (size_t i = i0; i < i1; ++i) {
                 float x = cells[i].pos[0], y = cells[i].pos[1];
@@ -214,25 +214,25 @@ WorldImage WorldImage::fromTO(const alien_world_desc& desc, const alien_params& 
                 key[i] = k;
             }
         });
-        img.binCells.resize(bins);
         // (by the cells' number: one piece for few cells, whatever the bins)
         const size_t pieces = std::max<size_t>(1, std::min(size_t(n), bins));
         auto binsOf = [&](size_t p) { return bins * p / pieces; };
         for_ranges(pieces, [&](size_t p0, size_t p1) {
             const size_t b0 = binsOf(p0), span = binsOf(p1) - b0;
-            std::fill_n(img.binCells.begin() + std::ptrdiff_t(b0), span, 0);
+            std::fill_n(count.begin() + std::ptrdiff_t(b0), span, 0);
             for (int i = 0; i < n; ++i)
-                if (size_t(key[i]) - b0 < span) ++img.binCells[size_t(key[i])];
+                if (size_t(key[i]) - b0 < span) ++count[size_t(key[i])];
         });
         int sum = 0;
         for (size_t b = 0; b < bins; ++b) {
-            next[b] = sum;
-            sum += img.binCells[b];
+            const int cells = count[b];
+            count[b] = sum;  // (the bin's next slot)
+            sum += cells;
         }
         for_ranges(pieces, [&](size_t p0, size_t p1) {
             const size_t b0 = binsOf(p0), span = binsOf(p1) - b0;
             for (int i = 0; i < n; ++i)
-                if (size_t(key[i]) - b0 < span) img.slot[i] = next[size_t(key[i])]++;
+                if (size_t(key[i]) - b0 < span) img.slot[i] = count[size_t(key[i])]++;
         });
     }
     std::atomic<bool> hasExtra{false}, hasSelected{false}, livingWork{false};
@@ -541,7 +541,6 @@ void WorldSet::build(const std::vector<Source>& sources) {
     std::vector<int> liveParticles;
     std::vector<uint8_t> pending;
     std::vector<uint8_t> bondWork, livingWork;
-    std::vector<int> stripChoice, stageChoice;
     // A set is built once, into fresh allocations; a failed build then leaves nothing behind (the
     // destructor frees what was allocated).  Sizes are checked before anything is read or allocated.
     if (!allocs_.empty() || !worlds_.empty())
@@ -566,7 +565,6 @@ void WorldSet::build(const std::vector<Source>& sources) {
         int live = 0;
         uint64_t ts = 0;
         bool pend = false;
-        int strip = kStripMax, stage = 1;
         bool work = false, living = false;
         if (src.image) {
             h = src.image->host;
@@ -580,18 +578,11 @@ void WorldSet::build(const std::vector<Source>& sources) {
                 if (flags_num_conn(im.flags[i]) > 0 || flags_barrier(im.flags[i]) || flags_max_conn(im.flags[i]) > 0)
                     work = true;
             }
-            const int bs = bin_size_for(h.params);
-            const int W = h.desc.worldSizeX, H = h.desc.worldSizeY;
-            const bool counted = im.binCells.size() == size_t(W / bs) * size_t(H / bs);
-            strip = choose_strip(im.pos.size(), counted ? im.binCells : bin_cells(im.pos, W, H, bs), W / bs, H / bs,
-                                 h.params.motionType == ALIEN_MOTION_COLLISION, stage);
         } else {
             h = src.from->hosts_.at(src.fromIndex);
             live = src.from->numParticles(src.fromIndex);
             ts = src.from->timestep(src.fromIndex);
             pend = src.from->densityPending_.at(src.fromIndex) != 0;
-            strip = src.from->stripChoice_.at(src.fromIndex);
-            stage = src.from->stageChoice_.at(src.fromIndex);
             work = src.from->bondWork_.at(src.fromIndex) != 0;
             living = src.from->livingWork_.at(src.fromIndex) != 0;
         }
@@ -621,9 +612,6 @@ void WorldSet::build(const std::vector<Source>& sources) {
         w.bondWork = work ? 1 : 0;
         w.livingWork = living ? 1 : 0;
         w.seed = h.desc.randomSeed;
-        strip_shape(w, std::min(strip, stripCap_), stage);
-        stripChoice.push_back(strip);
-        stageChoice.push_back(stage);
         cellOff += h.numCells;
         partOff += w.partCap;
         bins += (int64_t(w.nbx) * w.nby + kGroupBins - 1) / kGroupBins * kGroupBins;
@@ -736,9 +724,6 @@ void WorldSet::build(const std::vector<Source>& sources) {
         mapStatus_ = static_cast<unsigned long long*>(A(sizeof(unsigned long long) * size_t(map_scan_tiles(NB - cellBins) + 1)));
         mapEpochTicket_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * 2));
         sorted_ = static_cast<int*>(A(sizeof(int) * NC));
-        mpos_ = static_cast<float2*>(A(sizeof(float2) * NC));
-        mvel_ = static_cast<float2*>(A(sizeof(float2) * NC));
-        mflags_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
         newidx_ = static_cast<int*>(A(sizeof(int) * NC));
         psorted_ = static_cast<int*>(B(sizeof(int) * NP));
         stage_ = static_cast<uint8_t*>(A(NC));
@@ -887,9 +872,6 @@ void WorldSet::build(const std::vector<Source>& sources) {
     bondWork_ = std::move(bondWork);
     livingWork_ = std::move(livingWork);
     active_.assign(worlds_.size(), 1);
-    stripChoice_ = std::move(stripChoice);
-    stageChoice_ = std::move(stageChoice);
-    chunk_shape(worlds_, params_, chunkRows_);
     shape_.hasParticles = anyRadiates;
     for (int lp : liveParticles) shape_.hasParticles = shape_.hasParticles || lp > 0;
     parity_ = 0;
@@ -946,121 +928,24 @@ void WorldSet::build(const std::vector<Source>& sources) {
     synchronize();
 }
 
-// Strip shape of the neighbour pass for one world, measured on the given positions.  Only
-// performance depends on it.
-HostArray<int> bin_cells(const HostArray<float2>& pos, int W, int H, int binSize) {
-    const int nbx = W / binSize, nby = H / binSize;
-    HostArray<int> cnt(size_t(nbx) * nby, 0);
-    for (const float2& p : pos) {
-        int sx = host_floor_int(p.x), sy = host_floor_int(p.y);
-        sx = ((sx % W) + W) % W;
-        sy = ((sy % H) + H) % H;
-        const int bx = std::min(sx / binSize, nbx - 1), by = std::min(sy / binSize, nby - 1);
-        ++cnt[size_t(by) * nbx + bx];
-    }
-    return cnt;
-}
-
-int choose_strip(size_t cells, const HostArray<int>& cnt, int nbx, int nby, bool twoRowStages, int& rowsPerStage) {
-    // sparse rows (fewer than half a wave of cells per bin row of a strip on average) are staged
-    // two at a time; a chunk where that overflows runs single rows
-    auto stages = [&](int sw) {
-        const double perRow = double(cells) / (double(nby) * double((nbx + sw - 1) / sw));
-        return twoRowStages && perRow < 32.0 && nby % 2 == 0 && nby >= 6 ? 2 : 1;
-    };
-    // entries of every staged row as the neighbour pass stages it (interior plus the two halo
-    // columns, both wrapped around the torus), for each candidate width; a chunk whose rows exceed
-    // the row capacity, or whose three consecutive rows exceed the LDS pool, takes the slower
-    // global path, so the widest strip where no row does that at the start is taken
-    for (int sw : {kStripMax, 32, 16, 8}) {
-        bool fits = true;
-        std::vector<int> rows(static_cast<size_t>(nby));
-        for (int x0 = 0; x0 < nbx && fits; x0 += sw) {
-            const int x1 = std::min(x0 + sw, nbx);
-            for (int y = 0; y < nby; ++y) {
-                const int* row = cnt.data() + size_t(y) * nbx;
-                rows[size_t(y)] = std::accumulate(row + x0, row + x1, row[(x0 - 1 + nbx) % nbx] + row[x1 % nbx]);
-            }
-            for (int y = 0; y < nby && fits; ++y) {
-                const int three = rows[size_t(y)] + rows[size_t((y + 1) % nby)] + rows[size_t((y + 2) % nby)];
-                fits = rows[size_t(y)] <= kRowCap && three <= kRowPool;
-            }
-        }
-        if (fits) {
-            rowsPerStage = stages(sw);
-            return sw;
-        }
-    }
-    rowsPerStage = stages(4);
-    return 4;
-}
-
-// Strip width (capped by the world's columns), strip count and staging; chunk_shape sets the rows.
-void strip_shape(DevWorld& w, int strip, int rowsPerStage) {
-    w.tileX = std::max(1, std::min(strip, w.nbx));
-    w.ntx = (w.nbx + w.tileX - 1) / w.tileX;
-    w.rowsPerStage = rowsPerStage;
-    w.tileY = 1;
-    w.nty = w.nby / rowsPerStage;
-}
-
-// Rows per chunk of the row-streaming (collision) pass, one value for all worlds of a set
-// (forcedRows if nonzero).  Tall chunks stage fewer halo rows per computed row; short ones even
-// out the work of the workgroups, whose cell counts vary.  Measured on MI355X, the pass ran fastest
-// with the tallest chunks that still give at least 5 workgroups per resident slot on the
-// 3.4M-cell soft-body world, whose bodies make the workgroups' loads unequal (2 % faster than at
-// 3.5); sets too small for that take the shortest chunks.
-void chunk_shape(std::vector<DevWorld>& worlds, const std::vector<DevParams>& params, int forcedRows) {
-    static const int numCUs = [] {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-            return 256;
-        return std::max(1, n);
-    }();
-    // (only collision worlds run the row-streaming pass; the fluid pass is cell-parallel)
-    bool collision = false;
-    for (size_t i = 0; i < worlds.size(); ++i) collision = collision || params[i].motion != 0;
-    const int perCU = collision ? neighbor_blocks_per_cu() : 1;
-    const int64_t slots = int64_t(perCU) * numCUs;
-    const double minRounds = 5.0;
-    int best = 2;
-    // staged rows per chunk of a world for `rows` bin rows (a chunk covers at most kChunkMax bin
-    // rows: the LDS histogram of its region)
-    auto stagedRows = [](const DevWorld& w, int rows) {
-        return std::max(1, std::min(rows, w.nby) / w.rowsPerStage);
-    };
-    for (int rows = 2; rows <= kChunkMax; ++rows) {
-        int64_t tiles = 0;
-        for (size_t i = 0; i < worlds.size(); ++i) {
-            const DevWorld& w = worlds[i];
-            if (w.numCells == 0 || params[i].motion == 0) continue;
-            const int ty = stagedRows(w, rows), nyS = w.nby / w.rowsPerStage;
-            tiles += int64_t(w.ntx) * ((nyS + ty - 1) / ty);
-        }
-        if (double(tiles) >= minRounds * double(slots)) best = rows;
-    }
-    if (forcedRows > 0) best = forcedRows;
-    for (DevWorld& w : worlds) {
-        const int nyS = w.nby / w.rowsPerStage;
-        w.tileY = stagedRows(w, best);
-        w.nty = (nyS + w.tileY - 1) / w.tileY;
-    }
-}
-
 void WorldSet::buildTables() {
     if (stream_) synchronize();  // (the tables and the live counts read below are in use until then)
     for (auto& a : tableAllocs_) (void)hipFree(a.p);
     tableAllocs_.clear();
-    std::vector<int2> cells, bonds, pbins, parts, living, edges, fluids;
+    std::vector<int2> cells, bonds, pbins, parts, living, edges, fluids, collides, collideEdges;
     const int ct = shape_.cellThreads, pt = shape_.partThreads, bt = shape_.binThreads;
-    int64_t fluidCells = 0;
+    int64_t fluidCells = 0, collideCells = 0;
     for (int wi = 0; wi < int(worlds_.size()); ++wi)
-        if (active_[wi] && params_[wi].motion == 0) fluidCells += worlds_[wi].numCells;
-    fluidShift_ = 6;
-    while (fluidShift_ > kFluidShiftMin && fluidCells >> (fluidShift_ - 1) <= 1024) --fluidShift_;
+        if (active_[wi]) (params_[wi].motion == 0 ? fluidCells : collideCells) += worlds_[wi].numCells;
+    auto shift = [](int64_t n) {
+        int s = 6;
+        while (s > kFluidShiftMin && n >> (s - 1) <= 1024) --s;
+        return s;
+    };
+    fluidShift_ = shift(fluidCells);
+    collideShift_ = shift(collideCells);
     bool bondWork = false;
     for (int wi = 0; wi < int(worlds_.size()); ++wi) bondWork = bondWork || (active_[wi] && bondWork_[wi] && worlds_[wi].numCells > 0);
-    const int edgeWaves = bondWork ? kEdgeWavesBonds : kEdgeWaves;
     for (int wi = 0; wi < int(worlds_.size()); ++wi) {
         if (!active_[wi]) continue;
         const DevWorld& w = worlds_[wi];
@@ -1069,9 +954,12 @@ void WorldSet::buildTables() {
             for (int s = 0; s < w.numCells; s += ct) bonds.push_back(make_int2(wi, w.cellOff + s));
         if (livingWork_[wi])
             for (int s = 0; s < w.numCells; s += ct) living.push_back(make_int2(wi, w.cellOff + s));
-        if (params_[wi].motion == 0 && w.numCells > 0) {  // waves of the fluid pass, see k_fluid.hip
-            for (int s = 0; s < edgeWaves * (w.nby + 1); s += ct / 64) edges.push_back(make_int2(wi, s));
-            for (int s = 0; s < (w.numCells >> fluidShift_) + 3; s += ct / 64) fluids.push_back(make_int2(wi, s));
+        if (w.numCells > 0) {  // waves of the neighbour passes, see k_neighbor.hip
+            const bool fluid = params_[wi].motion == 0;
+            const int waves = (w.numCells >> (fluid ? fluidShift_ : collideShift_)) + 3;
+            const int edgeWaves = (fluid && !bondWork ? kEdgeWaves : kEdgeWavesBonds) * (w.nby + 1);
+            for (int s = 0; s < edgeWaves; s += ct / 64) (fluid ? edges : collideEdges).push_back(make_int2(wi, s));
+            for (int s = 0; s < waves; s += ct / 64) (fluid ? fluids : collides).push_back(make_int2(wi, s));
         }
         for (int s = 0; s < w.pnbx * w.pnby; s += bt) pbins.push_back(make_int2(wi, w.pbinOff + s));
     }
@@ -1085,24 +973,6 @@ void WorldSet::buildTables() {
         all.insert(all.end(), v.begin(), v.end());
         all.resize((all.size() + 31) / 32 * 32);
     };
-    // neighbour-pass tiles, row-major per world; workgroup b runs on XCD b % 8, so each XCD gets
-    // one contiguous run of tiles and the halo rows its tiles share stay in that XCD's L2
-    std::vector<int2> tiles;
-    for (int wi = 0; wi < int(worlds_.size()); ++wi) {
-        const DevWorld& w = worlds_[wi];
-        if (w.numCells == 0 || !active_[wi] || params_[wi].motion == 0) continue;
-        for (int t = 0; t < w.ntx * w.nty; ++t) tiles.push_back(make_int2(wi, t));
-    }
-    std::vector<int2> tileTable;
-    if (!tiles.empty()) {
-        const int T = int(tiles.size());
-        const int chunk = (T + kXcds - 1) / kXcds;
-        tileTable.assign(size_t(chunk) * kXcds, make_int2(-1, -1));
-        for (int b = 0; b < int(tileTable.size()); ++b) {
-            const int t = (b % kXcds) * chunk + b / kXcds;
-            if (t < T) tileTable[b] = tiles[t];
-        }
-    }
     // particle blocks: a table sized for every active world's particle capacity, holding the
     // blocks of the live particles (the particle bin sort rewrites it every step); the grid of the
     // particle kernels follows the live particles (and the cells that can radiate)
@@ -1130,11 +1000,14 @@ void WorldSet::buildTables() {
     up(cellBlocks_, cells);
     up(bondBlocks_, bonds);
     up(pbinBlocks_, pbins);
-    up(tileBlocks_, tileTable);
     up(livingBlocks_, living);
     up(edgeBlocks_, edges);
     shape_.edgeBlocks = int(edges.size());
     up(fluidBlocks_, fluids);
+    up(collideBlocks_, collides);
+    up(collideEdgeBlocks_, collideEdges);
+    shape_.collideBlocks = int(collides.size());
+    shape_.collideEdgeBlocks = int(collideEdges.size());
     shape_.fluidBlocks = int(fluids.size());
     void* p = nullptr;
     check_hip(hipMalloc(&p, sizeof(int2) * all.size()), "hipMalloc");
@@ -1149,9 +1022,6 @@ void WorldSet::buildTables() {
     shape_.hasBondWork = bondWork;
     shape_.partBlocks = int(partCapBlocks);
     shape_.pbinBlocks = int(pbins.size());
-    shape_.tileBlocks = int(tileTable.size());
-    shape_.hasFluid = shape_.hasCollision = false;
-    for (const DevParams& p : params_) (p.motion == 0 ? shape_.hasFluid : shape_.hasCollision) = true;
     updateRadiation();
     invalidateGraphs();
 }
@@ -1207,27 +1077,6 @@ void WorldSet::setActive(int w, bool on) {
     }
     buildTables();
     invalidateGraphs();
-}
-
-void WorldSet::setStripCap(int cap) {
-    if (cap != 8 && cap != 16 && cap != 32 && cap != kStripMax)
-        throw Error(ALIEN_E_ARG, "strip cap must be 8, 16, 32 or 64");
-    stripCap_ = cap;
-    if (worlds_.empty()) return;
-    for (size_t i = 0; i < worlds_.size(); ++i)
-        strip_shape(worlds_[i], std::min(stripChoice_[i], cap), stageChoice_[i]);
-    chunk_shape(worlds_, params_, chunkRows_);
-    check_hip(hipMemcpy(dWorlds_, worlds_.data(), sizeof(DevWorld) * worlds_.size(), hipMemcpyHostToDevice), "H2D");
-    buildTables();
-}
-
-void WorldSet::setChunkRows(int rows) {
-    if (rows != 0 && (rows < 2 || rows > kChunkMax)) throw Error(ALIEN_E_ARG, "chunk rows must be 0 or 2..8");
-    chunkRows_ = rows;
-    if (worlds_.empty()) return;
-    chunk_shape(worlds_, params_, chunkRows_);
-    check_hip(hipMemcpy(dWorlds_, worlds_.data(), sizeof(DevWorld) * worlds_.size(), hipMemcpyHostToDevice), "H2D");
-    buildTables();
 }
 
 void WorldSet::setUseGraph(bool on) {
@@ -1303,9 +1152,6 @@ Ctx WorldSet::makeCtx(int parity) const {
     c.mapEpoch = mapEpochTicket_;
     c.mapTicket = mapEpochTicket_ + 1;
     c.sorted = sorted_;
-    c.mpos = mpos_;
-    c.mvel = mvel_;
-    c.mflags = mflags_;
     c.newidx = newidx_;
     c.psorted = psorted_;
     c.stage = stage_;
@@ -1327,10 +1173,12 @@ Ctx WorldSet::makeCtx(int parity) const {
     c.bondBlocks = bondBlocks_;
     c.pbinBlocks = pbinBlocks_;
     c.partBlocks = partBlocks_;
-    c.tileBlocks = tileBlocks_;
     c.edgeBlocks = edgeBlocks_;
     c.fluidBlocks = fluidBlocks_;
     c.fluidShift = fluidShift_;
+    c.collideBlocks = collideBlocks_;
+    c.collideEdgeBlocks = collideEdgeBlocks_;
+    c.collideShift = collideShift_;
     c.numPartBlocks = numPartBlocks_;
     c.partBlockParticles = shape_.partThreads;
     c.blockThreads = shape_.cellThreads;
@@ -1523,17 +1371,8 @@ void WorldSet::setParams(int w, const alien_params& p) {
     params_.at(w) = to_dev_params(p);
     check_hip(hipMemcpy(dParams_ + w, &params_[w], sizeof(DevParams), hipMemcpyHostToDevice), "H2D");
     densityPending_.at(w) = 1;  // prepareForSimulationParametersChanges, SimulationCudaFacade.cu:667-669
-    // the set of motion modes selects which neighbour-pass variants the step launches
-    const bool fluid = shape_.hasFluid, collision = shape_.hasCollision;
-    shape_.hasFluid = shape_.hasCollision = false;
-    for (const DevParams& q : params_) (q.motion == 0 ? shape_.hasFluid : shape_.hasCollision) = true;
-    if (wasFluid != (params_[w].motion == 0)) {
-        // only collision worlds run the row-streaming pass: its chunks and tiles follow the switch
-        chunk_shape(worlds_, params_, chunkRows_);
-        check_hip(hipMemcpy(dWorlds_, worlds_.data(), sizeof(DevWorld) * worlds_.size(), hipMemcpyHostToDevice), "H2D");
+    if (wasFluid != (params_[w].motion == 0)) {  // the neighbour passes' tables follow the switch
         buildTables();
-        invalidateGraphs();
-    } else if (fluid != shape_.hasFluid || collision != shape_.hasCollision) {
         invalidateGraphs();
     }
     updateRadiation();  // (the room for emitted particles is made before the next step)
@@ -1872,7 +1711,6 @@ void WorldSet::extract(int wi, WorldImage& img) {
         }
     h.stepsSinceSet = 0;
     h.cells = std::move(own);
-    img.binCells.clear();
     img.ppos.resize(np);
     img.pvel.resize(np);
     img.pen.resize(np);

@@ -47,9 +47,6 @@ bool splits(const alien_params& p);
 // (one particle per cell and step at most), doubled when its particles can split
 int64_t particle_room(int64_t cells, int64_t particles, const alien_params& p);
 DevParams to_dev_params(const alien_params& p);
-void strip_shape(DevWorld& w, int strip, int rowsPerStage);
-void chunk_shape(std::vector<DevWorld>& worlds, const std::vector<DevParams>& params, int forcedRows = 0);
-constexpr int kXcds = kXcdCount;  // accelerator complex dies of an MI355X
 
 // A vector whose resize leaves new elements of plain types unset: what is filled right after is written once,
 // by the threads that fill it.
@@ -98,7 +95,6 @@ struct WorldImage {
     HostArray<int> btgt;  // [kMaxBonds][numCells]
     HostArray<float> brest, bang;
     HostArray<float> energy, stiff;  // by slot
-    HostArray<int> binCells;         // cells per bin of the cell map; may be left empty
     bool livingWork = false;         // living states tracked on the device (see WorldSet::build)
     HostArray<float2> ppos, pvel;
     HostArray<float> pen;
@@ -114,11 +110,6 @@ struct WorldImage {
     // livingWork for the image's current states, energies and parameters (once set, it stays set)
     void updateLivingWork();
 };
-
-// cells per bin of positions on the torus
-HostArray<int> bin_cells(const HostArray<float2>& pos, int W, int H, int binSize);
-// neighbour-pass strip width for these cells per bin (`cells` in all)
-int choose_strip(size_t cells, const HostArray<int>& binCells, int nbx, int nby, bool twoRowStages, int& rowsPerStage);
 
 class WorldSet {
 public:
@@ -176,15 +167,9 @@ public:
 
     void setBlockSize(int threads);
     int blockSize() const { return shape_.cellThreads; }
-    // neighbour-pass strips no wider than cap bins (8, 16, 32 or 64); launch shape only
-    void setStripCap(int cap);
     // An inactive world stays in place but is left out of every launch (its state is frozen);
     // all worlds are active after build.
     void setActive(int w, bool on);
-    int stripCap() const { return stripCap_; }
-    // bin rows per neighbour-pass chunk (2..kChunkMax), or 0 for the occupancy rule; launch shape only
-    void setChunkRows(int rows);
-    int chunkRows() const { return chunkRows_; }
     void setUseGraph(bool on);
     // kernel timing mode: no graphs, every launch bracketed by events (see alien_set_kernel_timing)
     void setKernelTiming(bool on);
@@ -295,8 +280,6 @@ private:
     unsigned long long* mapStatus_ = nullptr;
     uint32_t* mapEpochTicket_ = nullptr;  // [2]: epoch, ticket
     int *sorted_ = nullptr, *newidx_ = nullptr, *psorted_ = nullptr;
-    float2 *mpos_ = nullptr, *mvel_ = nullptr;
-    uint32_t* mflags_ = nullptr;
     uint8_t* stage_ = nullptr;
     float2 *own_ = nullptr, *shift_ = nullptr, *s2_ = nullptr, *out1_ = nullptr, *out2_ = nullptr;
     float* bstiff_ = nullptr;
@@ -306,16 +289,13 @@ private:
     int *want_ = nullptr, *fclaim_ = nullptr, *absorbCell_ = nullptr, *cclaim_ = nullptr;
     int2 *cellBlocks_ = nullptr, *bondBlocks_ = nullptr, *pbinBlocks_ = nullptr;
     int2* partBlocks_ = nullptr;
-    int2* tileBlocks_ = nullptr;
     int2 *edgeBlocks_ = nullptr, *fluidBlocks_ = nullptr;
     int fluidShift_ = 6;
+    int2 *collideEdgeBlocks_ = nullptr, *collideBlocks_ = nullptr;
+    int collideShift_ = 6;
     int* numPartBlocks_ = nullptr;  // (device) entries of partBlocks_
     std::vector<uint8_t> bondWork_;  // per world: a bonded or barrier cell exists or can appear by fusion
     std::vector<uint8_t> active_;    // per world: included in the launch tables
-    std::vector<int> stripChoice_;   // per world: strip width chosen from its cell density
-    std::vector<int> stageChoice_;   // per world: bin rows per staged row (1 or 2)
-    int stripCap_ = kStripMax;
-    int chunkRows_ = 0;
     void adaptGrids();
     std::vector<Arr> tableAllocs_;
 

@@ -228,9 +228,9 @@ int alien_set_kernel_timing(alien_world* w, int32_t enable);
 int alien_get_kernel_timing(alien_world* w, alien_kernel_time* out, int32_t cap, int32_t* count);
 
 /* Neighbour-pass path counts since the world's data was last set (no counterpart in ALIEN; a
- * performance diagnostic, results never depend on the path): chunks of bin rows too crowded for
- * the LDS staging (a row above 128 entries or three consecutive rows above 256), which walk their
- * stencils in global memory, and cells with more than 64 candidates, which walk theirs alone. */
+ * performance diagnostic, results never depend on the path): waves of the collision pass with cells
+ * that have more than 64 candidates among too many for their staged rows, and cells with more than 64
+ * candidates, which walk their stencils alone. */
 int alien_get_path_counts(alien_world* w, uint64_t* fallbackChunks, uint64_t* directCells);
 
 /* ---- batched worlds ------------------------------------------------------------------------ */
@@ -259,10 +259,9 @@ uint64_t alien_batch_get_timestep(const alien_batch* b, int32_t world);
 int alien_batch_set_block_size(alien_batch* b, int32_t threads);
 int alien_batch_set_use_graph(alien_batch* b, int32_t enable);
 /* Autotuner (no counterpart in ALIEN): times trialSteps steps of a device copy of the batch for
- * candidate launch shapes (cell-kernel block size 64/128/256 x neighbour-pass strip cap 64/32/16
- * bins, then bin rows per neighbour-pass chunk 2/4/8 against the default rule, reported as 0)
- * and keeps the fastest, also for worlds added later.  The batch's own worlds do not advance and
- * no result depends on the choice.  Outputs may be NULL. */
+ * candidate launch shapes (cell-kernel block size 64/128/256) and keeps the fastest, also for worlds
+ * added later.  The batch's own worlds do not advance and no result depends on the choice.  Outputs may
+ * be NULL; stripCap and chunkRows are 64 and 0 (shapes of an earlier neighbour pass). */
 int alien_batch_autotune(alien_batch* b, uint32_t trialSteps, int32_t* blockSize, int32_t* stripCap,
                          int32_t* chunkRows, double* msPerStep);
 int alien_batch_set_kernel_timing(alien_batch* b, int32_t enable);

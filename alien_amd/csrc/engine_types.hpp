@@ -246,14 +246,14 @@ struct Ctx {
     uint32_t* mapEpoch;
     uint32_t* mapTicket;
     int* sorted;   // [cellCap] map order (bin, then previous index) -> A index
-    int* newidx;   // [cellCap] A index -> new index
+    float4* bonded;  // [cellCap] by A index, of bonded cells: position after the neighbour pass, stiffness, new index
     int* psorted;  // [partCap]
     // [cellCap] kStagedCell: the end-of-step cell is staged (bonded or barrier at the neighbour pass);
     // kDropBonds: it loses all its bonds at the end of the step; kMarkedCell: it or a bond partner
     // does.  The neighbour pass writes the byte of every cell of the bond-work worlds.
     uint8_t* stage;
     float2* own;    // [cellCap]
-    float2* shift;  // [cellCap] Verlet displacement of a staged cell, applied after the second force pass
+    float4* moved;  // [cellCap] position after the neighbour pass, and displacement of the first Verlet step
     float* bstiff;  // [cellCap] stiffness of a bonded cell in end-of-step order (written by the neighbour pass)
     float2* s2;     // [cellCap] connection force of the first pass
     float2* out1;  // [kMaxBonds][cellCap]

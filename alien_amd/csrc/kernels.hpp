@@ -51,7 +51,7 @@ struct SideStream {
 // rec != nullptr (per-kernel timing) launches everything on s, one kernel after another
 void launch_step(const Ctx& c, const LaunchShape& sh, hipStream_t s, Recorder* rec = nullptr,
                  const SideStream* side = nullptr);
-// cell map of the current state in logical order (sorted/newidx), for introspection; consumes
+// cell map of the current state in logical order (sorted), for introspection; consumes
 // the seeded bins and seeds them again afterwards
 void launch_debug_map(const Ctx& c, const LaunchShape& sh, hipStream_t s);
 // per-colour statistics of one world: block count for its cells and particle slots, and the

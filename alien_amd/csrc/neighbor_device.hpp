@@ -268,6 +268,7 @@ __device__ __forceinline__ void cell_finish(const Ctx& c, const DevWorld& w, con
     c.B.flags[k] = fi;
     c.B.slot[k] = slot;
     if constexpr (kFluid) c.B.dens[k] = 1.0f / a.rho;
+    float stiff = 0.0f;
     if constexpr (kFluid) {
         // (unrolled: a loop to nci would index bt at run time and place it in scratch memory)
 #pragma unroll
@@ -277,7 +278,7 @@ __device__ __forceinline__ void cell_finish(const Ctx& c, const DevWorld& w, con
                 c.B.brest[b * cap + k] = c.A.brest[b * cap + i];
                 c.B.bang[b * cap + k] = c.A.bang[b * cap + i];
             }
-        if (nci > 0) c.bstiff[k] = c.stiff[w.cellOff + slot];
+        if (nci > 0) stiff = c.stiff[w.cellOff + slot];
     } else {
         // (collision worlds are mostly bonded cells: their bond data is loaded before any of it
         // is stored, so that the loads are in flight together)
@@ -287,7 +288,7 @@ __device__ __forceinline__ void cell_finish(const Ctx& c, const DevWorld& w, con
             brest[b] = b < nci ? c.A.brest[b * cap + i] : 0.0f;
             bang[b] = b < nci ? c.A.bang[b * cap + i] : 0.0f;
         }
-        const float stiff = nci > 0 ? c.stiff[w.cellOff + slot] : 0.0f;
+        stiff = nci > 0 ? c.stiff[w.cellOff + slot] : 0.0f;
 #pragma unroll
         for (int b = 0; b < kMaxBonds; ++b)
             if (b < nci) {
@@ -295,9 +296,11 @@ __device__ __forceinline__ void cell_finish(const Ctx& c, const DevWorld& w, con
                 c.B.brest[b * cap + k] = brest[b];
                 c.B.bang[b * cap + k] = bang[b];
             }
-        if (nci > 0) c.bstiff[k] = stiff;
     }
-    if (nci > 0) c.newidx[i] = k;
+    if (nci > 0) {
+        c.bstiff[k] = stiff;
+        c.bonded[i] = make_float4(pc.x, pc.y, stiff, __int_as_float(k));
+    }
     // checkForces (CellProcessor.cuh:367-386): a bonded cell whose force is above cellMaxForce loses
     // all its bonds with probability cellMaxForceDecayProb (deleting the bonds of an unbonded cell
     // would change nothing)

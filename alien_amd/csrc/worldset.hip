@@ -724,11 +724,11 @@ void WorldSet::build(const std::vector<Source>& sources) {
         mapStatus_ = static_cast<unsigned long long*>(A(sizeof(unsigned long long) * size_t(map_scan_tiles(NB - cellBins) + 1)));
         mapEpochTicket_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * 2));
         sorted_ = static_cast<int*>(A(sizeof(int) * NC));
-        newidx_ = static_cast<int*>(A(sizeof(int) * NC));
+        bonded_ = static_cast<float4*>(A(sizeof(float4) * NC));
         psorted_ = static_cast<int*>(B(sizeof(int) * NP));
         stage_ = static_cast<uint8_t*>(A(NC));
         own_ = static_cast<float2*>(A(sizeof(float2) * NC));
-        shift_ = static_cast<float2*>(A(sizeof(float2) * NC));
+        moved_ = static_cast<float4*>(A(sizeof(float4) * NC));
         bstiff_ = static_cast<float*>(A(sizeof(float) * NC));
         s2_ = static_cast<float2*>(A(sizeof(float2) * NC));
         out1_ = static_cast<float2*>(A(sizeof(float2) * kMaxBonds * size_t(NC)));
@@ -1152,11 +1152,11 @@ Ctx WorldSet::makeCtx(int parity) const {
     c.mapEpoch = mapEpochTicket_;
     c.mapTicket = mapEpochTicket_ + 1;
     c.sorted = sorted_;
-    c.newidx = newidx_;
+    c.bonded = bonded_;
     c.psorted = psorted_;
     c.stage = stage_;
     c.own = own_;
-    c.shift = shift_;
+    c.moved = moved_;
     c.bstiff = bstiff_;
     c.s2 = s2_;
     c.out1 = out1_;

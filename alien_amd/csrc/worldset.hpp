@@ -279,9 +279,10 @@ private:
     int numCellBins_ = 0;
     unsigned long long* mapStatus_ = nullptr;
     uint32_t* mapEpochTicket_ = nullptr;  // [2]: epoch, ticket
-    int *sorted_ = nullptr, *newidx_ = nullptr, *psorted_ = nullptr;
+    int *sorted_ = nullptr, *psorted_ = nullptr;
+    float4 *bonded_ = nullptr, *moved_ = nullptr;
     uint8_t* stage_ = nullptr;
-    float2 *own_ = nullptr, *shift_ = nullptr, *s2_ = nullptr, *out1_ = nullptr, *out2_ = nullptr;
+    float2 *own_ = nullptr, *s2_ = nullptr, *out1_ = nullptr, *out2_ = nullptr;
     float* bstiff_ = nullptr;
     uint32_t* valid_ = nullptr;
     unsigned long long* claim_ = nullptr;

@@ -253,6 +253,7 @@ struct Ctx {
     // does.  The neighbour pass writes the byte of every cell of the bond-work worlds.
     uint8_t* stage;
     float2* own;    // [cellCap]
+    int4* lists;    // [2 * cellCap] on angle steps, of bonded cells: their bond targets (-1: none), flags, unused
     float4* moved;  // [cellCap] position after the neighbour pass, and displacement of the first Verlet step
     float* bstiff;  // [cellCap] stiffness of a bonded cell in end-of-step order (written by the neighbour pass)
     float2* s2;     // [cellCap] connection force of the first pass

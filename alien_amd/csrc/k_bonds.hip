@@ -38,6 +38,13 @@ __device__ __forceinline__ bool staged_cell(const Ctx& c, int block, int& x, int
 // Angle forces act every third step; on the others no partner has written any.
 __device__ __forceinline__ bool angle_step(const Ctx& c, int wi) { return (c.ctr[wi].timestep % 3ull) == 0ull; }
 
+// a partner's bond targets (-1: none) and flags, from the record the first pass leaves on an angle step
+__device__ __forceinline__ uint32_t partner_list(const Ctx& c, int o, int (&t)[kMaxBonds]) {
+    const int4 a = c.lists[2 * o], b = c.lists[2 * o + 1];
+    t[0] = a.x, t[1] = a.y, t[2] = a.z, t[3] = a.w, t[4] = b.x, t[5] = b.y;
+    return uint32_t(b.z);
+}
+
 // Connection forces of a staged cell: own force plus per-bond angle forces for the partners; pass 1
 // also runs checkConnections (CellProcessor.cuh:493-523) on the moved positions.  The partners' data of
 // all the cell's bonds is loaded up front, so the loads are in flight together (lanes skip the slots
@@ -47,7 +54,8 @@ __device__ __forceinline__ bool angle_step(const Ctx& c, int wi) { return (c.ctr
 // partners' lists from A, so that no thread reads a list another rewrites.
 // What a pass needs of a partner lies in one 16-byte record (bonded, moved): a gather costs the L1 a line
 // per lane whatever its width.  Records, and no markers read or written on the steps without angle forces:
-// 0.84M cells in bodies, a step 260 -> 248 us.
+// 0.84M cells in bodies, a step 260 -> 248 us; with the bond lists of an angle step in records too (its
+// partners' planes: seven gathers for each bond and pass), 242 us, eight worlds 172 -> 162 us.
 // In the second pass the cells stand at pos + shift; the bond vector is taken as the start-of-pass
 // difference plus the difference of the shifts, which keeps the FP32 result close to the exact one
 // (rounding pos + shift first would cost up to ulp(world size)).
@@ -60,9 +68,7 @@ template <int kPass> __device__ __forceinline__ void conn_own(const Ctx& c, int 
     const DevParams& P = c.params[wi];
     const uint32_t fx = c.B.flags[x];
     const int nc = flags_num_conn(fx);
-    // the partners' indices in the arrays their bond lists are read from (pass 0: A, pass 1: B), and
-    // in B
-    const HotBuffers& L = kPass == 0 ? c.A : c.B;
+    // the partners' indices, in A (pass 0) or B (pass 1)
     int tl[kMaxBonds];
     float4 part[kMaxBonds];  // (what the bonds' partners have in the pass's record)
 #pragma unroll
@@ -78,6 +84,13 @@ template <int kPass> __device__ __forceinline__ void conn_own(const Ctx& c, int 
             if (b < nc) c.B.btgt[b * cap + x] = __float_as_int(part[b].w) - w.cellOff;
     }
     const bool considerAngles = angle_step(c, wi);
+    if (kPass == 0 && considerAngles && nc > 0) {
+        int own[kMaxBonds];
+#pragma unroll
+        for (int b = 0; b < kMaxBonds; ++b) own[b] = b < nc ? __float_as_int(part[b].w) - w.cellOff : -1;
+        c.lists[2 * x] = make_int4(own[0], own[1], own[2], own[3]);
+        c.lists[2 * x + 1] = make_int4(own[4], own[5], int(fx), 0);
+    }
     if (nc == 0 || flags_barrier(fx)) {
         if (considerAngles) c.valid[x] = 0u;
         if (kPass == 1) c.stretched[x] = 0;  // checkConnections skips barrier cells
@@ -134,12 +147,17 @@ template <int kPass> __device__ __forceinline__ void conn_own(const Ctx& c, int 
         bool skipped = false;  // a bond whose actual angle is negative keeps the previous vector
         if (considerAngles && (nc > 2 || (nc == 2 && b == 0))) {
             const int lc = b == 0 ? lastTarget : tl[b > 0 ? b - 1 : 0];
-            const uint32_t fo = L.flags[o];
-            const int no = flags_num_conn(fo);
-            // (the partner's list: its loads in flight together)
+            uint32_t fo;
             int lt[kMaxBonds];
+            if constexpr (kPass == 0) {
+                fo = c.A.flags[o];
+                const int no = flags_num_conn(fo);
+                // (the partner's list: its loads in flight together)
 #pragma unroll
-            for (int j = 0; j < kMaxBonds; ++j) lt[j] = j < no ? L.btgt[j * cap + o] : -1;
+                for (int j = 0; j < kMaxBonds; ++j) lt[j] = j < no ? c.A.btgt[j * cap + o] : -1;
+            } else {
+                fo = partner_list(c, o, lt);
+            }
             bool tri = false;
 #pragma unroll
             for (int j = 0; j < kMaxBonds; ++j) tri = tri || lt[j] == lc - w.cellOff;
@@ -164,7 +182,7 @@ template <int kPass> __device__ __forceinline__ void conn_own(const Ctx& c, int 
                         c.out1[b * cap + x] = to_float2(f1);
                         v |= 1u << b;
                     }
-                    if (!flags_barrier(L.flags[lc])) {
+                    if (!flags_barrier((kPass == 0 ? c.A : c.B).flags[lc])) {
                         c.out2[b * cap + x] = to_float2(fb);
                         v |= 1u << (6 + b);
                     }
@@ -216,10 +234,8 @@ __device__ __forceinline__ f2 gather_conn(const Ctx& c, const DevWorld& w, int w
         const uint32_t vp = vps[q];
         if (vp == 0u) continue;  // the partner wrote no angle force this pass
         const int p = pt[q];
-        const int np = flags_num_conn(c.B.flags[p]);
         int lt[kMaxBonds];
-#pragma unroll
-        for (int kk = 0; kk < kMaxBonds; ++kk) lt[kk] = kk < np ? c.B.btgt[kk * cap + p] : -1;
+        const int np = flags_num_conn(partner_list(c, p, lt));
         int b = -1;
 #pragma unroll
         for (int kk = kMaxBonds - 1; kk >= 0; --kk) b = lt[kk] == xl ? kk : b;

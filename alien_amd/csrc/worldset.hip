@@ -729,6 +729,7 @@ void WorldSet::build(const std::vector<Source>& sources) {
         stage_ = static_cast<uint8_t*>(A(NC));
         own_ = static_cast<float2*>(A(sizeof(float2) * NC));
         moved_ = static_cast<float4*>(A(sizeof(float4) * NC));
+        lists_ = static_cast<int4*>(A(2 * sizeof(int4) * NC));
         bstiff_ = static_cast<float*>(A(sizeof(float) * NC));
         s2_ = static_cast<float2*>(A(sizeof(float2) * NC));
         out1_ = static_cast<float2*>(A(sizeof(float2) * kMaxBonds * size_t(NC)));
@@ -1157,6 +1158,7 @@ Ctx WorldSet::makeCtx(int parity) const {
     c.stage = stage_;
     c.own = own_;
     c.moved = moved_;
+    c.lists = lists_;
     c.bstiff = bstiff_;
     c.s2 = s2_;
     c.out1 = out1_;

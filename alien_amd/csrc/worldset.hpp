@@ -281,6 +281,7 @@ private:
     uint32_t* mapEpochTicket_ = nullptr;  // [2]: epoch, ticket
     int *sorted_ = nullptr, *psorted_ = nullptr;
     float4 *bonded_ = nullptr, *moved_ = nullptr;
+    int4* lists_ = nullptr;
     uint8_t* stage_ = nullptr;
     float2 *own_ = nullptr, *s2_ = nullptr, *out1_ = nullptr, *out2_ = nullptr;
     float* bstiff_ = nullptr;

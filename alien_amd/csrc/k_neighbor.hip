@@ -49,14 +49,15 @@ template <Pass kPass> constexpr bool kBonded = kPass != Pass::kFree;  // (collis
 constexpr int kFluidWaves = 4;   // waves per workgroup at most
 // staged candidates of the three stencil rows: three rows of 66 bins at one cell per bin; with bonds,
 // bodies of four cells a bin next to empty space
-constexpr int kFreeStage = 288, kBondStage = 448;
+constexpr int kFreeStage = 288, kBondStage = 344;
 // pair records at a time: a fluid's cells have about one each at one cell per bin; with bonds, bodies with
 // ten neighbours a cell (the tests run again for what does not fit)
-constexpr int kFreePairs = 128, kBondPairs = 896;
+constexpr int kFreePairs = 128, kBondPairs = 512;
 constexpr int kEdgeAlone = 16;    // more edge cells than this in a unit walk alone, one per lane
 
-// LDS of one wave: 6 KB (9.9 KB with bonds), six (four) waves per SIMD (the owners' velocities,
-// densities and flags come from their registers, by cross-lane permutes)
+// LDS of one wave: 6 KB (8 KB with bonds), six (five) waves per SIMD (the owners' velocities, densities
+// and flags come from their registers, by cross-lane permutes).  With bonds: room for 448 staged cells and
+// 896 pairs at four waves ran 1 % slower in bodies, for 288 and 384 5 to 10 % (the tests run again).
 template <int kStage, int kPairs> struct FluidShared {
     // staged candidates: their positions, and behind them their A indices (the last round of tests reads
     // up to 63 positions past the last list, and counts nothing there)
@@ -81,7 +82,7 @@ template <int kStage, int kPairs> struct FluidShared {
 };
 template <bool kBonds>
 using FluidWave = FluidShared<kBonds ? kBondStage : kFreeStage, kBonds ? kBondPairs : kFreePairs>;
-static_assert(sizeof(FluidWave<true>) <= 10240 && sizeof(FluidWave<false>) <= 6826, "16 and 24 waves per CU");
+static_assert(sizeof(FluidWave<true>) <= 8000 && sizeof(FluidWave<false>) <= 6826, "20 and 24 waves per CU");
 static_assert(kBondStage <= 512 && kFreeStage >= 126, "9-bit staged entries; room to read past the last list");
 
 __device__ __forceinline__ int lanes_below(unsigned long long mask, int add) {
@@ -657,7 +658,7 @@ __device__ __forceinline__ int fluid_wave(const Ctx& c, FluidWave<kBonded<kPass>
 
 // With bonds also the particles' bin sort, on the launch's first workgroups (sets with bond work)
 template <Pass kPass>
-__global__ void __launch_bounds__(64 * kFluidWaves) __attribute__((amdgpu_waves_per_eu(kBonded<kPass> ? 4 : 6)))
+__global__ void __launch_bounds__(64 * kFluidWaves) __attribute__((amdgpu_waves_per_eu(kBonded<kPass> ? 5 : 6)))
 k_neighbor(Ctx c, int sortBlocks, int edgeBlocks, int tableBlocks) {
     constexpr bool kBonds = kBonded<kPass>, kFluid = kPass != Pass::kCollide;
     __shared__ FluidWave<kBonds> SS[kFluidWaves];

@@ -199,18 +199,18 @@ template <int kPass> __device__ __forceinline__ void conn_own(const Ctx& c, int 
 }
 
 // (at most 80 VGPRs, six waves per SIMD: the partner loads are latency-bound)
-__global__ void __attribute__((amdgpu_waves_per_eu(6))) k_conn_first(Ctx c, int partBlocks) {
+template <bool kLate> __global__ void __attribute__((amdgpu_waves_per_eu(6))) k_conn_first(Ctx c, int partBlocks) {
     const int b = int(blockIdx.x);
     if (b < partBlocks)
-        part_move(c, {b, partBlocks});
+        kLate ? part_binsort(c, {b, partBlocks}) : part_move(c, {b, partBlocks});
     else
         conn_own<0>(c, b - partBlocks);
 }
 
-__global__ void __attribute__((amdgpu_waves_per_eu(6))) k_conn_second(Ctx c, int partBlocks) {
+template <bool kLate> __global__ void __attribute__((amdgpu_waves_per_eu(6))) k_conn_second(Ctx c, int partBlocks) {
     const int b = int(blockIdx.x);
     if (b < partBlocks)
-        part_apply(c, {b, partBlocks});
+        kLate ? part_target(c, {b, partBlocks}) : part_apply(c, {b, partBlocks});
     else
         conn_own<1>(c, b - partBlocks);
 }
@@ -269,10 +269,10 @@ __device__ __forceinline__ void conn_pos(const Ctx& c, int block) {
     c.s2[x] = to_float2(s1);
 }
 
-__global__ void k_conn_pos(Ctx c, int partBlocks) {
+template <bool kLate> __global__ void k_conn_pos(Ctx c, int partBlocks) {
     const int b = int(blockIdx.x);
     if (b < partBlocks)
-        part_target(c, {b, partBlocks});
+        kLate ? part_move(c, {b, partBlocks}) : part_target(c, {b, partBlocks});
     else
         conn_pos(c, b - partBlocks);
 }
@@ -492,16 +492,18 @@ __global__ void k_living_unbonded(Ctx c) {
 
 // the velocity step, the marks and ages of the living states (from this step's overstretched bonds),
 // and the absorptions
-__global__ void k_conn_vel(Ctx c, int partBlocks, int bondBlocks) {
+template <bool kLate> __global__ void k_conn_vel(Ctx c, int partBlocks, int bondBlocks) {
     int b = int(blockIdx.x);
-    if (b < partBlocks) return part_absorb(c, {b, partBlocks});
+    if (b < partBlocks) return kLate ? part_apply(c, {b, partBlocks}) : part_absorb(c, {b, partBlocks});
     b -= partBlocks;
     if (b < bondBlocks) return conn_vel(c, b);
     living_mark_age(c, b - bondBlocks);
 }
 
-__global__ void k_marks(Ctx c, int bondBlocks) {
-    const int b = int(blockIdx.x);
+__global__ void k_marks(Ctx c, int absorbBlocks, int bondBlocks) {
+    int b = int(blockIdx.x);
+    if (b < absorbBlocks) return part_absorb(c, {b, absorbBlocks});
+    b -= absorbBlocks;
     if (b < bondBlocks)
         friction_and_marks(c, b);
     else
@@ -749,8 +751,12 @@ __global__ void k_fuse_end(Ctx c, int candBlocks) {
 // the particles' chain from the movement on: their bin sort ran with the neighbour pass.  Energies
 // change in the absorptions only; before them the neighbour pass read them for fusion candidates, after
 // them the marks and the decay do.
+// The particles' chain goes along: movement in the first launch to absorption in the fourth, or all of it a
+// launch later (lateParticles), which lets the scan of their bins share the launch of the cells' map (a
+// launch of its own was 4.5 us of a step's 64.5 with 18k cells in bodies; now 59.4).
 void launch_bonds(const Ctx& c, const LaunchShape& sh, hipStream_t s, Recorder* rec) {
     const int parts = sh.hasParticles && sh.partBlocks ? sh.partGrid : 0;
+    const int sort = parts ? sh.pbinBlocks : 0;
     const int bonds = sh.bondBlocks, living = sh.livingBlocks, cand = sh.candGrid;
     const dim3 t(sh.cellThreads);
 #define L(name, kernel, grid, ...)                                         \
@@ -758,11 +764,19 @@ void launch_bonds(const Ctx& c, const LaunchShape& sh, hipStream_t s, Recorder* 
         if (rec) rec->mark(name);                                          \
         hipLaunchKernelGGL(kernel, dim3(grid), t, 0, s, __VA_ARGS__);      \
     } while (0)
-    L("conn_first", k_conn_first, parts + bonds, c, parts);
-    L("conn_pos", k_conn_pos, parts + bonds, c, parts);
-    L("conn_second", k_conn_second, parts + bonds, c, parts);
-    L("conn_vel", k_conn_vel, parts + bonds + living, c, parts, bonds);
-    L("marks", k_marks, bonds + living, c, bonds);
+    if (sh.lateParticles) {
+        L("conn_first", k_conn_first<true>, sort + bonds, c, sort);
+        L("conn_pos", k_conn_pos<true>, parts + bonds, c, parts);
+        L("conn_second", k_conn_second<true>, parts + bonds, c, parts);
+        L("conn_vel", k_conn_vel<true>, parts + bonds + living, c, parts, bonds);
+    } else {
+        L("conn_first", k_conn_first<false>, parts + bonds, c, parts);
+        L("conn_pos", k_conn_pos<false>, parts + bonds, c, parts);
+        L("conn_second", k_conn_second<false>, parts + bonds, c, parts);
+        L("conn_vel", k_conn_vel<false>, parts + bonds + living, c, parts, bonds);
+    }
+    const int absorb = sh.lateParticles ? parts : 0;
+    L("marks", k_marks, absorb + bonds + living, c, absorb, bonds);
     L("fuse_claim", k_fuse_claim, cand + living, c, cand);
     L("fuse_apply", k_fuse_apply, cand, c);
     L("fuse_end", k_fuse_end, cand + bonds, c, cand);

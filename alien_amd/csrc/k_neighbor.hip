@@ -656,17 +656,19 @@ __device__ __forceinline__ int fluid_wave(const Ctx& c, FluidWave<kBonded<kPass>
     return -1;
 }
 
-// With bonds also the particles' bin sort, on the launch's first workgroups (sets with bond work)
+// With bonds also a stage of the particles' chain, on the launch's first workgroups (sets with bond work):
+// their bin sort, or with the late chain their scatter
 template <Pass kPass>
 __global__ void __launch_bounds__(64 * kFluidWaves) __attribute__((amdgpu_waves_per_eu(kBonded<kPass> ? 5 : 6)))
-k_neighbor(Ctx c, int sortBlocks, int edgeBlocks, int tableBlocks) {
+k_neighbor(Ctx c, int partBlocks, int late, int edgeBlocks, int tableBlocks) {
     constexpr bool kBonds = kBonded<kPass>, kFluid = kPass != Pass::kCollide;
     __shared__ FluidWave<kBonds> SS[kFluidWaves];
     const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
     int block = int(blockIdx.x);
     if constexpr (kBonds) {
-        if (block < sortBlocks) return part_binsort(c, {block, sortBlocks});
-        block -= sortBlocks;
+        if (block < partBlocks)
+            return late ? part_scatter(c, {block, partBlocks}) : part_binsort(c, {block, partBlocks});
+        block -= partBlocks;
     }
     int wi;
     int2 walk = make_int2(0, 0);  // cells this lane walks alone: walk.x, walk.x + 64, ... below walk.y
@@ -692,24 +694,25 @@ k_neighbor(Ctx c, int sortBlocks, int edgeBlocks, int tableBlocks) {
     for (int m = walk.x; m < walk.y; m += 64) walk_alone<kFluid>(c, wi, m);
 }
 
-// The bin sort goes with the first launch.  A set with collision worlds but no bond work at all still runs
-// the one collision variant.
-void launch_neighbor(const Ctx& c, const LaunchShape& sh, hipStream_t s, bool withPartSort) {
-    int sort = withPartSort && sh.hasParticles && sh.partBlocks ? sh.pbinBlocks : 0;
+// The particles' stage goes with the first launch.  A set with collision worlds but no bond work at all still
+// runs the one collision variant.
+void launch_neighbor(const Ctx& c, const LaunchShape& sh, hipStream_t s, bool withParticles) {
+    int parts = withParticles && sh.hasParticles && sh.partBlocks ? (sh.lateParticles ? sh.partGrid : sh.pbinBlocks) : 0;
+    const int late = sh.lateParticles ? 1 : 0;
     const auto grid = [&](int edges, int table) {
-        return dim3(sort + edges + (table + kXcdCount - 1) / kXcdCount * kXcdCount);
+        return dim3(parts + edges + (table + kXcdCount - 1) / kXcdCount * kXcdCount);
     };
     const dim3 threads(sh.cellThreads);
     if (sh.collideBlocks) {
-        hipLaunchKernelGGL(k_neighbor<Pass::kCollide>, grid(sh.collideEdgeBlocks, sh.collideBlocks), threads, 0, s, c, sort,
+        hipLaunchKernelGGL(k_neighbor<Pass::kCollide>, grid(sh.collideEdgeBlocks, sh.collideBlocks), threads, 0, s, c, parts, late,
                            sh.collideEdgeBlocks, sh.collideBlocks);
-        sort = 0;
+        parts = 0;
     }
-    if (sh.hasBondWork && (sh.fluidBlocks || sort))
-        hipLaunchKernelGGL(k_neighbor<Pass::kBonds>, grid(sh.edgeBlocks, sh.fluidBlocks), threads, 0, s, c, sort, sh.edgeBlocks,
-                           sh.fluidBlocks);
+    if (sh.hasBondWork && (sh.fluidBlocks || parts))
+        hipLaunchKernelGGL(k_neighbor<Pass::kBonds>, grid(sh.edgeBlocks, sh.fluidBlocks), threads, 0, s, c, parts, late,
+                           sh.edgeBlocks, sh.fluidBlocks);
     else if (sh.fluidBlocks)
-        hipLaunchKernelGGL(k_neighbor<Pass::kFree>, grid(sh.edgeBlocks, sh.fluidBlocks), threads, 0, s, c, 0, sh.edgeBlocks,
+        hipLaunchKernelGGL(k_neighbor<Pass::kFree>, grid(sh.edgeBlocks, sh.fluidBlocks), threads, 0, s, c, 0, 0, sh.edgeBlocks,
                            sh.fluidBlocks);
 }
 

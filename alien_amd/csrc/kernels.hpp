@@ -19,6 +19,10 @@ struct LaunchShape {
     int partGrid = 64;     // grid-stride particle kernels
     int bondBlocks = 0;    // bond kernels: cell blocks of the worlds that can have bonded cells
     int candGrid = 16;     // grid-stride kernels over fusion candidates
+    // With bond work: the particles' chain starts a launch later, with their scatter beside the neighbour pass and
+    // the scan of their bins beside the cells' map, and absorbs beside the marks.  Not where the marks or
+    // living states read energies (a finite cellMaxBindingEnergy, living states), nor with emissions.
+    bool lateParticles = false;
     bool hasBondWork = true;  // some active world has (or can get by fusion) a bonded or barrier cell
     // some world has live energy particles or radiates (only cell radiation creates particles, so
     // once all are absorbed or merged in a set without it the particle kernels, which would find

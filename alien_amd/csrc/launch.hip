@@ -30,7 +30,7 @@ void launch_step(const Ctx& c, const LaunchShape& sh, hipStream_t s, Recorder* r
     launch_radiation(c, sh, s, rec);
     // without bond work the end-of-step kernel would only advance the timesteps: the map does it
     if (rec) rec->mark("map");
-    launch_map(c, sh, s, !sh.hasBondWork, c.sc, !sh.hasBondWork);
+    launch_map(c, sh, s, !sh.hasBondWork || sh.lateParticles, c.sc, !sh.hasBondWork);
     const bool fork = side && !rec && !sh.hasBondWork && sh.hasParticles && sh.partBlocks;
     if (fork) (void)hipEventRecord(side->fork, s);
     if (rec) rec->mark("neighbor");

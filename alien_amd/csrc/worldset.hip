@@ -1033,7 +1033,11 @@ void WorldSet::updateRadiation() {
         on = on || (active_[w] && params_[w].radiates);
         split = split || (active_[w] && params_[w].splits);
     }
-    if (on != shape_.hasRadiation || split != shape_.hasSplitting) invalidateGraphs();
+    bool late = shape_.hasBondWork && shape_.livingBlocks == 0;
+    for (size_t w = 0; w < params_.size(); ++w)
+        late = late && !(active_[w] && (params_[w].radiates || params_[w].splits || std::isfinite(params_[w].maxBindingEnergy)));
+    if (on != shape_.hasRadiation || split != shape_.hasSplitting || late != shape_.lateParticles) invalidateGraphs();
+    shape_.lateParticles = late;
     shape_.hasRadiation = on;
     shape_.hasSplitting = split;
     if (on) shape_.hasParticles = true;  // (particles can appear)

@@ -725,7 +725,7 @@ struct alien_server {
                     if (id && !jobs.count(id)) id = 0;  // cancelled and erased: inactive in place
                 running = oldRunning;
                 for (size_t i = 0; i < running.size(); ++i)
-                    if (!running[i] && set && i < size_t(set->numWorlds())) set->setActive(int(i), false);
+                    if (!running[i] && set && i < size_t(set->numWorlds())) set->setInactive(int(i));
                 bool anyLive = false;
                 for (auto id : running) anyLive = anyLive || id != 0;
                 if (!anyLive) {
@@ -776,7 +776,7 @@ struct alien_server {
                     std::vector<alien_cell_to> c(size_t(set->numCells(f.second)));
                     set->readCells(f.second, c.data());
                     snaps.push_back({f.first, {std::move(c), std::move(p)}});
-                    set->setActive(f.second, false);
+                    set->setInactive(f.second);
                 }
             } catch (const std::exception& e) {
                 snapErr = e.what();

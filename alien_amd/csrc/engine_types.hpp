@@ -179,7 +179,7 @@ struct CellExtra {
 // Cells that the map cannot find near their new bin (k_sort.hip): all of them in one list, and a
 // list per bin.
 struct FarCells {
-    int* head;   // [numCellBins] one of the bin's, kNone without any; Ctx::moverNext goes on
+    int* head;   // [numCellBins] one of the bin's, kNone without any; Ctx::farLink goes on
     int* count;  // [numCellBins]
     int* group;  // [numCellBins / kGroupBins] number in the group's bins
     int* total;  // entries in the list
@@ -239,7 +239,7 @@ struct Ctx {
     const uint32_t* startPrev;  // [numBins + 1] the last step's map
     // far cells of this step's map, and of the next (entered during this step)
     FarCells far, farNext;
-    int* moverNext;  // [cellCap] the bin's next far cell (kNone ends a list)
+    int* farLink;  // [cellCap] the bin's next far cell (kNone ends a list)
     // one-pass scan of the particle bins: per tile of bins a status word (flag, launch epoch, sum), the launch epoch
     // and the tile ticket
     unsigned long long* mapStatus;

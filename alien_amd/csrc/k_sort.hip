@@ -42,7 +42,7 @@ __global__ void k_cell_bin(Ctx c) {
     const int gb = w.binOff + by * w.nbx + bx;
     c.binOf[i] = int(uint32_t(gb - w.binOff) | kFarMove);
     c.far.list[i] = make_int2(i, gb);
-    list_far(c.far, c.moverNext, gb, i);
+    list_far(c.far, c.farLink, gb, i);
 }
 
 // (the groups gain their far cells)
@@ -310,7 +310,7 @@ __device__ __forceinline__ void clear_next(const Ctx& c, int g, int lane) {
 // far cells of global bin gb with A index below i
 __device__ __forceinline__ int rank_far(const Ctx& c, int gb, int i) {
     int n = 0;
-    for (int j = c.far.head[gb]; j != kNone; j = c.moverNext[j]) n += j < i ? 1 : 0;
+    for (int j = c.far.head[gb]; j != kNone; j = c.farLink[j]) n += j < i ? 1 : 0;
     return n;
 }
 

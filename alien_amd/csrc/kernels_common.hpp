@@ -123,7 +123,7 @@ __device__ __forceinline__ void bin_next(const Ctx& c, const DevWorld& w, int k,
         if (x < -1 || x > 1) {
             move = kFarCode;
             c.farNext.list[atomicAdd(c.farNext.total, 1)] = make_int2(k, w.binOff + b);
-            list_far(c.farNext, c.moverNext, w.binOff + b, k);
+            list_far(c.farNext, c.farLink, w.binOff + b, k);
         }
         const int from = (w.binOff + bOld) / kGroupBins, to = (w.binOff + b) / kGroupBins;
         if (from != to) shift_groups(c.groupSumNext, c.superSumNext, from, to);

@@ -264,7 +264,7 @@ __device__ __forceinline__ void cell_finish(const Ctx& c, const DevWorld& w, con
     }
 
     // the cell in the end-of-step order; bond targets stay in start-of-step indices until the
-    // staged cells are renumbered (k_remap)
+    // first connection pass renumbers them
     c.B.flags[k] = fi;
     c.B.slot[k] = slot;
     if constexpr (kFluid) c.B.dens[k] = 1.0f / a.rho;

@@ -715,7 +715,7 @@ void WorldSet::build(const std::vector<Source>& sources) {
             far_[b].total = far_[b].group + NCB / kGroupBins;
             far_[b].list = farList_;
         }
-        moverNext_ = static_cast<int*>(A(sizeof(int) * NC));
+        farLink_ = static_cast<int*>(A(sizeof(int) * NC));
         groupWorld_ = static_cast<int*>(A(sizeof(int) * NCB / kGroupBins + sizeof(int)));
         for (int b = 0; b < 2; ++b) {
             groupSum_[b] = static_cast<int*>(A(sizeof(int) * groups));
@@ -1068,18 +1068,14 @@ void WorldSet::setBlockSize(int threads) {
     if (!worlds_.empty()) buildTables();
 }
 
-// The kernels reach a world only through the launch tables, and every offset they derive from the
-// shared scan is relative to the world's own first bin, so the frozen counters of an inactive
-// world change nothing for the others.
-void WorldSet::setActive(int w, bool on) {
-    if (active_.at(w) == uint8_t(on)) return;
-    active_[w] = on;
-    worlds_[w].active = on ? 1 : 0;
+// The kernels reach a world only through the launch tables, and a world's offsets in the map start at its
+// first cell, so a world left out changes nothing for the others.  It does not come back: the records its
+// next map would be built from are gone.
+void WorldSet::setInactive(int w) {
+    if (!active_.at(w)) return;
+    active_[w] = 0;
+    worlds_[w].active = 0;
     check_hip(hipMemcpy(dWorlds_ + w, &worlds_[w], sizeof(DevWorld), hipMemcpyHostToDevice), "H2D");
-    if (on) {
-        synchronize();
-        anchorAges(w);
-    }
     buildTables();
     invalidateGraphs();
 }
@@ -1122,7 +1118,7 @@ Ctx WorldSet::makeCtx(int parity) const {
     c.startPrev = start_[parity ^ 1];
     c.far = far_[parity];
     c.farNext = far_[parity ^ 1];
-    c.moverNext = moverNext_;
+    c.farLink = farLink_;
     c.groupWorld = groupWorld_;
     c.groupSum = groupSum_[parity];
     c.groupSumNext = groupSum_[parity ^ 1];
@@ -1356,8 +1352,7 @@ void WorldSet::setTimestep(int w, uint64_t t) {
 }
 
 // The device derives a cell's age from the world's timestep (ageBase + timestep - ageTs); after
-// the timestep is set, or while the world was inactive (frozen, its ages too, though the step
-// advances every world's timestep), the anchor moves so that the ages stay base + steps simulated.
+// the timestep is set, the anchor moves so that the ages stay base + steps simulated.
 void WorldSet::anchorAges(int w) {
     DevCounters c{};
     check_hip(hipMemcpy(&c, dCtr_ + w, sizeof(c), hipMemcpyDeviceToHost), "D2H");

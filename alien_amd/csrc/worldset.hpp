@@ -167,9 +167,9 @@ public:
 
     void setBlockSize(int threads);
     int blockSize() const { return shape_.cellThreads; }
-    // An inactive world stays in place but is left out of every launch (its state is frozen);
-    // all worlds are active after build.
-    void setActive(int w, bool on);
+    // An inactive world stays in place but is left out of every launch from then on (its state is
+    // frozen); all worlds are active after build.
+    void setInactive(int w);
     void setUseGraph(bool on);
     // kernel timing mode: no graphs, every launch bracketed by events (see alien_set_kernel_timing)
     void setKernelTiming(bool on);
@@ -275,7 +275,7 @@ private:
     int* groupWorld_ = nullptr;
     int* groupSum_[2] = {nullptr, nullptr};
     int* superSum_[2] = {nullptr, nullptr};
-    int* moverNext_ = nullptr;
+    int* farLink_ = nullptr;
     int numCellBins_ = 0;
     unsigned long long* mapStatus_ = nullptr;
     uint32_t* mapEpochTicket_ = nullptr;  // [2]: epoch, ticket

@@ -357,8 +357,8 @@ class Batch:
         check(lib().alien_batch_set_kernel_timing(self._h, 1 if on else 0))
 
     def autotune(self, trial_steps=20):
-        """Picks the fastest launch shape on a device copy; returns (block, strip cap, chunk rows
-        (0: the default rule), ms/step)."""
+        """Picks the fastest launch shape on a device copy; returns (block, 64, 0, ms/step):
+        the neighbour pass has no strips and chunks to choose from any more."""
         blk, strip, rows, ms = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int32(), ctypes.c_double()
         check(lib().alien_batch_autotune(self._h, int(trial_steps), ctypes.byref(blk), ctypes.byref(strip),
                                          ctypes.byref(rows), ctypes.byref(ms)))

@@ -27,7 +27,7 @@ HBM_PEAK_GBS = 8000.0  # MI355X HBM3E peak
 # algorithmic (compulsory) bytes per unit and step: fluid cell 56 B, energy particle 52 B
 BYTES_PER_FLUID_CELL = 56
 BYTES_PER_PARTICLE = 52
-NEIGHBOR_KERNEL = "k_neighbor_cells"  # the neighbour pass of fluid worlds (the dominant kernel)
+NEIGHBOR_KERNEL = "k_neighbor<kFree>"  # the neighbour pass of fluid worlds (the dominant kernel)
 
 
 def parse():

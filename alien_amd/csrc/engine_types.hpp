@@ -248,6 +248,7 @@ struct Ctx {
     int* sorted;   // [cellCap] map order (bin, then previous index) -> A index
     float4* bonded;  // [cellCap] by A index, of bonded cells: position after the neighbour pass, stiffness, new index
     int* psorted;  // [partCap]
+    uint8_t* pcode;  // [partCap] by map position: the particle's slot inside its bin before the movement
     // [cellCap] kStagedCell: the end-of-step cell is staged (bonded or barrier at the neighbour pass);
     // kDropBonds: it loses all its bonds at the end of the step; kMarkedCell: it or a bond partner
     // does.  The neighbour pass writes the byte of every cell of the bond-work worlds.

@@ -726,6 +726,7 @@ void WorldSet::build(const std::vector<Source>& sources) {
         sorted_ = static_cast<int*>(A(sizeof(int) * NC));
         bonded_ = static_cast<float4*>(A(sizeof(float4) * NC));
         psorted_ = static_cast<int*>(B(sizeof(int) * NP));
+        pcode_ = static_cast<uint8_t*>(B(NP));
         stage_ = static_cast<uint8_t*>(A(NC));
         own_ = static_cast<float2*>(A(sizeof(float2) * NC));
         moved_ = static_cast<float4*>(A(sizeof(float4) * NC));
@@ -1155,6 +1156,7 @@ Ctx WorldSet::makeCtx(int parity) const {
     c.sorted = sorted_;
     c.bonded = bonded_;
     c.psorted = psorted_;
+    c.pcode = pcode_;
     c.stage = stage_;
     c.own = own_;
     c.moved = moved_;
@@ -1632,7 +1634,7 @@ void WorldSet::growParticles(const std::vector<int64_t>& caps) {
             release(p);
         buf_[b] = nb[b];
     }
-    for (void* p : {static_cast<void*>(pbinOf_), static_cast<void*>(psorted_), static_cast<void*>(want_),
+    for (void* p : {static_cast<void*>(pbinOf_), static_cast<void*>(psorted_), static_cast<void*>(pcode_), static_cast<void*>(want_),
                     static_cast<void*>(fclaim_), static_cast<void*>(absorbCell_), static_cast<void*>(splitStaged_)})
         if (p) release(p);
     if (partArena_) release(partArena_);  // (the arrays the set was built with)
@@ -1640,6 +1642,7 @@ void WorldSet::growParticles(const std::vector<int64_t>& caps) {
     splitStaged_ = splitStaged;
     pbinOf_ = pbinOf;
     psorted_ = static_cast<int*>(alloc(sizeof(int) * NP));
+    pcode_ = static_cast<uint8_t*>(alloc(NP));
     want_ = static_cast<int*>(alloc(sizeof(int) * NP));
     fclaim_ = static_cast<int*>(alloc(sizeof(int) * NP));
     absorbCell_ = static_cast<int*>(alloc(sizeof(int) * NP));

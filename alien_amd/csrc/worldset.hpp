@@ -280,6 +280,7 @@ private:
     unsigned long long* mapStatus_ = nullptr;
     uint32_t* mapEpochTicket_ = nullptr;  // [2]: epoch, ticket
     int *sorted_ = nullptr, *psorted_ = nullptr;
+    uint8_t* pcode_ = nullptr;
     float4 *bonded_ = nullptr, *moved_ = nullptr;
     int4* lists_ = nullptr;
     uint8_t* stage_ = nullptr;

@@ -256,13 +256,14 @@ __device__ __forceinline__ void part_scan(const Ctx& c, int tiles) {
 //  - A listed mover from a lower place comes behind the listed ones of its bin before it, one from a
 //    higher place behind the stayers as well.  If there are more than the list holds, another run over
 //    the reach places them.
-// Far cells (few, but all of them after seeding) are placed by waves of their own: the cells of the
+// Far cells are placed by waves of their own (after seeding, when all are far, by their bins' lanes): the cells of the
 // target's group before it are counted over the group's reach, the far ones of its bin along the list;
 // near cells of a bin with a far list add the list's smaller indices.
 // ---------------------------------------------------------------------------------------------
 constexpr int kMapWaves = kMapThreads / 64;
 constexpr int kScatterList = 192;  // movers into a group's bins listed (typically 5 to 25)
 constexpr int kScatterRounds = 5;  // rounds of a stretch loaded at once (258 bins at up to 1.24 cells per bin)
+constexpr int kFarWalk = 16;       // far cells of a seeded bin that one lane places
 constexpr int kFarBlocks = 1024;   // workgroups for the far cells, at most
 static_assert(kGroupBins == 4 * 64, "four bins per lane");
 
@@ -319,36 +320,52 @@ __device__ __forceinline__ void place_cell(const Ctx& c, const DevWorld& w, int 
     st32(c.sorted, uint32_t(w.cellOff + dest), w.cellOff + i);
 }
 
+// Whether the world's last map is empty: it was seeded, and every cell is a far one.  Its groups' waves then
+// place the cells of bins with few of them themselves, the whole list of a bin in one lane (a first step of
+// 4M cells 4.9 -> 1.5 ms).
+__device__ __forceinline__ bool seeded(const Ctx& c, const DevWorld& w) {
+    return c.startPrev[w.binOff + w.nbx * w.nby] == c.startPrev[w.binOff];
+}
+
 __device__ __forceinline__ void far_scatter(const Ctx& c, int wave, int waves, int lane) {
     const int total = *c.far.total;
-    for (int q = wave; q < total; q += waves) {
-        const int2 f = c.far.list[q];
-        if (f.y < 0) continue;  // (seeded while its world was left out)
-        const DevWorld& w = c.worlds[world_of(c, f.y)];
-        if (!w.active) continue;
-        const int g = f.y / kGroupBins, b0 = g * kGroupBins - w.binOff;
-        const uint32_t t = uint32_t(f.y - w.binOff - b0);
-        const int i = f.x - w.cellOff;
-        const uint32_t* prev = c.startPrev + w.binOff;
-        const Places p = places_of(reach_of(w, b0, min(kGroupBins, w.nbx * w.nby - b0)), prev);
-        const int* binOf = c.binOf + w.cellOff;
-        const int4 fc = reinterpret_cast<const int4*>(c.far.count + g * kGroupBins)[lane];
-        const int base = int(prev[b0] - prev[0]) + gained_before(c, w, g, lane);
-        const uint32_t b = uint32_t(4 * lane);
-        uint32_t n = (b < t ? uint32_t(fc.x) : 0u) + (b + 1u < t ? uint32_t(fc.y) : 0u) + (b + 2u < t ? uint32_t(fc.z) : 0u) +
-                     (b + 3u < t ? uint32_t(fc.w) : 0u);
-        for (int k = 0; k < 3; ++k)
-            for (int j0 = p.s[k]; j0 < p.e[k]; j0 += 256) {
-                int x[4];
-                load_rounds(binOf, j0, p.e[k], lane, x);
+    // (a lane looks at one entry of 64 rounds: few entries go to a wave each)
+    for (int q0 = wave; q0 < total; q0 += 64 * waves) {
+        const long long q = q0 + (long long)(lane) * waves;
+        const int2 own = q < total ? c.far.list[q] : make_int2(-1, -1);
+        bool mine = own.y >= 0;  // (not while seeded with its world left out)
+        if (mine) {
+            const DevWorld& w = c.worlds[world_of(c, own.y)];
+            mine = w.active && !(c.far.count[own.y] <= kFarWalk && seeded(c, w));
+        }
+        for (unsigned long long todo = __ballot(mine); todo != 0ull; todo &= todo - 1ull) {
+            const int at0 = __builtin_ctzll(todo);
+            const int2 f = make_int2(__builtin_amdgcn_readlane(own.x, at0), __builtin_amdgcn_readlane(own.y, at0));
+            const DevWorld& w = c.worlds[world_of(c, f.y)];
+            const int g = f.y / kGroupBins, b0 = g * kGroupBins - w.binOff;
+            const uint32_t t = uint32_t(f.y - w.binOff - b0);
+            const int i = f.x - w.cellOff;
+            const uint32_t* prev = c.startPrev + w.binOff;
+            const Places p = places_of(reach_of(w, b0, min(kGroupBins, w.nbx * w.nby - b0)), prev);
+            const int* binOf = c.binOf + w.cellOff;
+            const int4 fc = reinterpret_cast<const int4*>(c.far.count + g * kGroupBins)[lane];
+            const int base = int(prev[b0] - prev[0]) + gained_before(c, w, g, lane);
+            const uint32_t b = uint32_t(4 * lane);
+            uint32_t n = (b < t ? uint32_t(fc.x) : 0u) + (b + 1u < t ? uint32_t(fc.y) : 0u) + (b + 2u < t ? uint32_t(fc.z) : 0u) +
+                         (b + 3u < t ? uint32_t(fc.w) : 0u);
+            for (int k = 0; k < 3; ++k)
+                for (int j0 = p.s[k]; j0 < p.e[k]; j0 += 256) {
+                    int x[4];
+                    load_rounds(binOf, j0, p.e[k], lane, x);
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const uint32_t u = move_of(x[r]) == kFarCode ? ~0u : bin_from(x[r], b0);
-                    n += j0 + 64 * r + lane < p.e[k] && (u < t || (u == t && j0 + 64 * r + lane < i)) ? 1u : 0u;
+                    for (int r = 0; r < 4; ++r) {
+                        const uint32_t u = move_of(x[r]) == kFarCode ? ~0u : bin_from(x[r], b0);
+                        n += j0 + 64 * r + lane < p.e[k] && (u < t || (u == t && j0 + 64 * r + lane < i)) ? 1u : 0u;
+                    }
                 }
-            }
-        const int at = base + wave_last(int(wave_inclusive_scan(n))) + rank_far(c, f.y, f.x);
-        if (lane == 0) place_cell(c, w, i, at);
+            const int at = base + wave_last(int(wave_inclusive_scan(n))) + rank_far(c, f.y, f.x);
+            if (lane == 0) place_cell(c, w, i, at);
+        }
     }
 }
 
@@ -450,6 +467,15 @@ __device__ __forceinline__ void cell_scatter(const Ctx& c, ScatterShared& S, int
         }
     }
     __syncwarp();
+    if (farCells && seeded(c, w)) {
+        for (int k = 0; k < 4; ++k) {
+            const int t = 4 * lane + k;
+            if (c.far.count[g0 + t] > kFarWalk) continue;
+            for (int j = c.far.head[g0 + t]; j != kNone; j = c.farLink[j])
+                place_cell(c, w, j - w.cellOff, S.start[t] + rank_far(c, g0 + t, j));
+        }
+        return;
+    }
     const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
     unsigned long long leftPrev = 0ull;  // the round before: own cells that left their bin
     int longStart = -1, longGone = 0;    // the bin that reaches into this round: its cells that left before it

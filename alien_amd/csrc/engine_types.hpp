@@ -176,14 +176,15 @@ struct CellExtra {
     uint8_t cellFunction, ancestorMutationId, selected, pad;
 };
 
-// Cells that the map cannot find near their new bin (k_sort.hip): all of them in one list, and a
-// list per bin.
+// Cells that the map cannot find near their new bin (k_sort.hip): a list per bin, and of the bins with
+// more than kFarWalk of them a list of their parts of 64.
+constexpr int kFarWalk = 16;
 struct FarCells {
     int* head;   // [numCellBins] one of the bin's, kNone without any; Ctx::farLink goes on
     int* count;  // [numCellBins]
-    int* group;  // [numCellBins / kGroupBins] number in the group's bins
+    int* group;  // [numCellBins / kGroupBins] whether the group's bins have any
     int* total;  // entries in the list
-    int2* list;  // [cellCap] (A index, global bin); one array for both steps: read before it is written
+    int2* list;  // (global bin, part); one array for both steps: read before it is written
 };
 
 struct Ctx {

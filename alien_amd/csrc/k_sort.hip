@@ -41,18 +41,18 @@ __global__ void k_cell_bin(Ctx c) {
     cell_bin_xy(w, to_f2(c.A.pos[i]), bx, by);
     const int gb = w.binOff + by * w.nbx + bx;
     c.binOf[i] = int(uint32_t(gb - w.binOff) | kFarMove);
-    c.far.list[i] = make_int2(i, gb);
     list_far(c.far, c.farLink, gb, i);
 }
 
-// (the groups gain their far cells)
+// (the groups gain their far cells; a wave each)
 __global__ void k_seed_sums(Ctx c) {
-    const int g = int(blockIdx.x) * int(blockDim.x) + int(threadIdx.x);
-    const bool in = g < c.numCellBins / kGroupBins;
-    const int n = in ? c.far.group[g] : 0;
-    if (in) c.groupSum[g] = n;
-    const int sum = wave_last(int(wave_inclusive_scan(uint32_t(n))));  // (of one sum of groups)
-    if (in && g % 64 == 0) atomicAdd(&c.superSum[g / kSuperGroups], sum);
+    const int g = (int(blockIdx.x) * int(blockDim.x) + int(threadIdx.x)) / 64, lane = int(threadIdx.x) & 63;
+    if (g >= c.numCellBins / kGroupBins) return;
+    const int4 n = reinterpret_cast<const int4*>(c.far.count + g * kGroupBins)[lane];
+    const int sum = wave_last(int(wave_inclusive_scan(uint32_t(n.x + n.y + n.z + n.w))));
+    if (lane != 0) return;
+    c.groupSum[g] = sum;
+    if (sum) atomicAdd(&c.superSum[g / kSuperGroups], sum);
 }
 
 __global__ void k_part_bin(Ctx c) {
@@ -255,16 +255,18 @@ __device__ __forceinline__ void part_scan(const Ctx& c, int tiles) {
 //    old stretch, minus the cells that left the bin before it, plus the movers into it from lower places.
 //  - A listed mover from a lower place comes behind the listed ones of its bin before it, one from a
 //    higher place behind the stayers as well.  If there are more than the list holds, another run over
-//    the reach places them.
-// Far cells are placed by waves of their own (after seeding, when all are far, by their bins' lanes): the cells of the
-// target's group before it are counted over the group's reach, the far ones of its bin along the list;
-// near cells of a bin with a far list add the list's smaller indices.
+//    the reach places them, the lanes of one bin in turns (256k cells of 1 to 2 units a step: the map 61 us
+//    with one bin of a round after the other, 26 with turns).
+//  - Far cells: the near cells of a bin with few of them take its first places, and at the end the bin's lane
+//    merges its far cells in (256k cells that move 5 units a step: a step of 158 us with a wave for each far
+//    cell, 62 so; 1M of them 500 and 117).  Bins with more far cells than a lane takes (kFarWalk) get a wave
+//    per 64 of them: it counts the cells of the group before them over the group's reach, and their ranks
+//    along the list; the near cells of such a bin add the list's smaller indices.
 // ---------------------------------------------------------------------------------------------
 constexpr int kMapWaves = kMapThreads / 64;
-constexpr int kScatterList = 192;  // movers into a group's bins listed (typically 5 to 25)
+constexpr int kScatterList = 192;  // movers into a group's bins listed (typically 5 to 25), a multiple of 8
 constexpr int kScatterRounds = 5;  // rounds of a stretch loaded at once (258 bins at up to 1.24 cells per bin)
-constexpr int kFarWalk = 16;       // far cells of a seeded bin that one lane places
-constexpr int kFarBlocks = 1024;   // workgroups for the far cells, at most
+constexpr int kFarBlocks = 256;    // workgroups for the bins with many far cells, at most
 static_assert(kGroupBins == 4 * 64, "four bins per lane");
 
 struct ScatterShared {
@@ -276,7 +278,10 @@ struct ScatterShared {
     uint32_t before[kGroupBins], after[kGroupBins];  // near movers into the bin from lower and higher places
     union {
         int2 list[kScatterList];   // (A index in the world, bin)
-        uint32_t met[kGroupBins];  // movers placed so far (the other run)
+        struct {                   // the other run
+            uint32_t met[kGroupBins];   // movers placed so far
+            uint16_t turn[kGroupBins];  // lane whose turn it is
+        } run;
     };
 };
 
@@ -320,53 +325,77 @@ __device__ __forceinline__ void place_cell(const Ctx& c, const DevWorld& w, int 
     st32(c.sorted, uint32_t(w.cellOff + dest), w.cellOff + i);
 }
 
-// Whether the world's last map is empty: it was seeded, and every cell is a far one.  Its groups' waves then
-// place the cells of bins with few of them themselves, the whole list of a bin in one lane (a first step of
-// 4M cells 4.9 -> 1.5 ms).
-__device__ __forceinline__ bool seeded(const Ctx& c, const DevWorld& w) {
-    return c.startPrev[w.binOff + w.nbx * w.nby] == c.startPrev[w.binOff];
-}
-
+// The far cells of bins with more than kFarWalk: one wave per entry, 64 of a bin's list
 __device__ __forceinline__ void far_scatter(const Ctx& c, int wave, int waves, int lane) {
     const int total = *c.far.total;
-    // (a lane looks at one entry of 64 rounds: few entries go to a wave each)
-    for (int q0 = wave; q0 < total; q0 += 64 * waves) {
-        const long long q = q0 + (long long)(lane) * waves;
-        const int2 own = q < total ? c.far.list[q] : make_int2(-1, -1);
-        bool mine = own.y >= 0;  // (not while seeded with its world left out)
-        if (mine) {
-            const DevWorld& w = c.worlds[world_of(c, own.y)];
-            mine = w.active && !(c.far.count[own.y] <= kFarWalk && seeded(c, w));
-        }
-        for (unsigned long long todo = __ballot(mine); todo != 0ull; todo &= todo - 1ull) {
-            const int at0 = __builtin_ctzll(todo);
-            const int2 f = make_int2(__builtin_amdgcn_readlane(own.x, at0), __builtin_amdgcn_readlane(own.y, at0));
-            const DevWorld& w = c.worlds[world_of(c, f.y)];
-            const int g = f.y / kGroupBins, b0 = g * kGroupBins - w.binOff;
-            const uint32_t t = uint32_t(f.y - w.binOff - b0);
-            const int i = f.x - w.cellOff;
-            const uint32_t* prev = c.startPrev + w.binOff;
-            const Places p = places_of(reach_of(w, b0, min(kGroupBins, w.nbx * w.nby - b0)), prev);
-            const int* binOf = c.binOf + w.cellOff;
-            const int4 fc = reinterpret_cast<const int4*>(c.far.count + g * kGroupBins)[lane];
-            const int base = int(prev[b0] - prev[0]) + gained_before(c, w, g, lane);
-            const uint32_t b = uint32_t(4 * lane);
-            uint32_t n = (b < t ? uint32_t(fc.x) : 0u) + (b + 1u < t ? uint32_t(fc.y) : 0u) + (b + 2u < t ? uint32_t(fc.z) : 0u) +
-                         (b + 3u < t ? uint32_t(fc.w) : 0u);
-            for (int k = 0; k < 3; ++k)
-                for (int j0 = p.s[k]; j0 < p.e[k]; j0 += 256) {
-                    int x[4];
-                    load_rounds(binOf, j0, p.e[k], lane, x);
+    for (int q = wave; q < total; q += waves) {
+        const int2 entry = c.far.list[q];
+        const int gb = entry.x, first = 64 * entry.y;
+        const DevWorld& w = c.worlds[world_of(c, gb)];
+        if (!w.active) continue;
+        // this lane's cell, and its rank among the list's
+        int own = kNone, rank = 0;
+        for (int j = c.far.head[gb], n = 0; j != kNone && n < first + 64; j = c.farLink[j], ++n) own = n - first == lane ? j : own;
+        for (int j = c.far.head[gb]; j != kNone; j = c.farLink[j]) rank += j < own ? 1 : 0;
+        const int g = gb / kGroupBins, b0 = g * kGroupBins - w.binOff;
+        const uint32_t t = uint32_t(gb - w.binOff - b0);
+        const int i = own - w.cellOff;
+        const uint32_t* prev = c.startPrev + w.binOff;
+        const Places p = places_of(reach_of(w, b0, min(kGroupBins, w.nbx * w.nby - b0)), prev);
+        const int* binOf = c.binOf + w.cellOff;
+        const int4 fc = reinterpret_cast<const int4*>(c.far.count + g * kGroupBins)[lane];
+        const int base = int(prev[b0] - prev[0]) + gained_before(c, w, g, lane);
+        const uint32_t b = uint32_t(4 * lane);
+        // cells of the group's bins before this one, and the bin's near cells before the lane's
+        uint32_t n = (b < t ? uint32_t(fc.x) : 0u) + (b + 1u < t ? uint32_t(fc.y) : 0u) + (b + 2u < t ? uint32_t(fc.z) : 0u) +
+                     (b + 3u < t ? uint32_t(fc.w) : 0u);
+        for (int k = 0; k < 3; ++k)
+            for (int j0 = p.s[k]; j0 < p.e[k]; j0 += 256) {
+                int x[4];
+                load_rounds(binOf, j0, p.e[k], lane, x);
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const uint32_t u = move_of(x[r]) == kFarCode ? ~0u : bin_from(x[r], b0);
-                        n += j0 + 64 * r + lane < p.e[k] && (u < t || (u == t && j0 + 64 * r + lane < i)) ? 1u : 0u;
-                    }
+                for (int r = 0; r < 4; ++r) {
+                    const bool in = j0 + 64 * r + lane < p.e[k] && move_of(x[r]) != kFarCode;
+                    const uint32_t u = in ? bin_from(x[r], b0) : ~0u;
+                    n += u < t ? 1u : 0u;
+                    for (unsigned long long m = __ballot(u == t); m != 0ull; m &= m - 1ull)
+                        rank += j0 + 64 * r + __builtin_ctzll(m) < i ? 1 : 0;
                 }
-            const int at = base + wave_last(int(wave_inclusive_scan(n))) + rank_far(c, f.y, f.x);
-            if (lane == 0) place_cell(c, w, i, at);
-        }
+            }
+        const int at = base + wave_last(int(wave_inclusive_scan(n))) + rank;
+        if (own != kNone) place_cell(c, w, i, at);
     }
+}
+
+// Merges the k far cells of a bin (at most kMax) into its places `seg`, whose first m hold its other cells in
+// order
+template <int kMax> __device__ __forceinline__ void merge_far(int* seg, const int* link, int head, int k, int m) {
+    int f[kMax], to[kMax];
+#pragma unroll
+    for (int s = 0; s < kMax; ++s) {
+        f[s] = s < k ? head : 0x7fffffff;
+        if (s + 1 < k) head = link[head];
+    }
+#pragma unroll
+    for (int s = 0; s < kMax; ++s) {
+        to[s] = 0;
+#pragma unroll
+        for (int j = 0; j < kMax; ++j) to[s] += f[j] < f[s] ? 1 : 0;
+    }
+    // the others from the last one on, up behind the far cells before them; those before all stay
+    for (; m > 0; --m) {
+        const int e = seg[m - 1];
+        int n = 0;
+#pragma unroll
+        for (int s = 0; s < kMax; ++s) n += f[s] < e ? 1 : 0;
+        if (n == 0) break;
+#pragma unroll
+        for (int s = 0; s < kMax; ++s) to[s] += f[s] > e ? 1 : 0;
+        seg[m - 1 + n] = e;
+    }
+#pragma unroll
+    for (int s = 0; s < kMax; ++s)
+        if (s < k) seg[m + to[s]] = f[s];
 }
 
 __device__ __forceinline__ void cell_scatter(const Ctx& c, ScatterShared& S, int g, int lane) {
@@ -391,7 +420,8 @@ __device__ __forceinline__ void cell_scatter(const Ctx& c, ScatterShared& S, int
     const int nb = min(kGroupBins, bins - b0);
     const int p0 = int(prev[b0]) - prevBase, p1 = int(prev[b0 + nb]) - prevBase;  // the bins' own cells
     const Places p = places_of(reach_of(w, b0, nb), prev);
-    const int farCells = c.far.group[g];
+    const bool farCells = c.far.group[g] != 0;
+    bool manyFar = false;  // some bin has more than its lane merges in
     const int* binOf = c.binOf + w.cellOff;
     const int base = p0 + gained_before(c, w, g, lane);
     int x[3][kScatterRounds];
@@ -453,6 +483,7 @@ __device__ __forceinline__ void cell_scatter(const Ctx& c, ScatterShared& S, int
                          uint32_t(next + prevBase) - pv.w - o.w + f.w + a.w};
         if (farCells) {
             const int4 fc = *reinterpret_cast<const int4*>(c.far.count + g0 + 4 * lane);
+            manyFar = __any(max(max(fc.x, fc.y), max(fc.z, fc.w)) > kFarWalk);
             v[0] += uint32_t(fc.x), v[1] += uint32_t(fc.y), v[2] += uint32_t(fc.z), v[3] += uint32_t(fc.w);
         }
         const uint32_t sum = v[0] + v[1] + v[2] + v[3];
@@ -467,15 +498,10 @@ __device__ __forceinline__ void cell_scatter(const Ctx& c, ScatterShared& S, int
         }
     }
     __syncwarp();
-    if (farCells && seeded(c, w)) {
-        for (int k = 0; k < 4; ++k) {
-            const int t = 4 * lane + k;
-            if (c.far.count[g0 + t] > kFarWalk) continue;
-            for (int j = c.far.head[g0 + t]; j != kNone; j = c.farLink[j])
-                place_cell(c, w, j - w.cellOff, S.start[t] + rank_far(c, g0 + t, j));
-        }
-        return;
-    }
+    // far cells before cell i in bin t, where they are not merged in at the end
+    auto far_before = [&](int t, int i) {
+        return manyFar && c.far.count[g0 + t] > kFarWalk ? rank_far(c, g0 + t, w.cellOff + i) : 0;
+    };
     const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
     unsigned long long leftPrev = 0ull;  // the round before: own cells that left their bin
     int longStart = -1, longGone = 0;    // the bin that reaches into this round: its cells that left before it
@@ -501,9 +527,7 @@ __device__ __forceinline__ void cell_scatter(const Ctx& c, ScatterShared& S, int
         if (stays) {
             const int gone = sb < i0 ? longGone + __builtin_popcountll(left & below)
                                      : __builtin_popcountll(left & below & ~((1ull << (sb - i0)) - 1ull));
-            int rank = i - sb - gone + int(S.before[t]);
-            if (farCells) rank += rank_far(c, g0 + int(t), w.cellOff + i);
-            place_cell(c, w, i, S.start[t] + rank);
+            place_cell(c, w, i, S.start[t] + i - sb - gone + int(S.before[t]) + far_before(int(t), i));
         }
         longGone += __builtin_popcountll(left);
         leftPrev = left;
@@ -525,8 +549,7 @@ __device__ __forceinline__ void cell_scatter(const Ctx& c, ScatterShared& S, int
             at += S.start[t + 1] - S.start[t] - int(S.before[t] + S.after[t]);
             if (farCells) at -= c.far.count[g0 + t];
         }
-        if (farCells) at += rank_far(c, g0 + t, w.cellOff + i);
-        place_cell(c, w, i, at);
+        place_cell(c, w, i, at + far_before(t, i));
     };
     if (listed <= kScatterList) {
         for (int q0 = 0; q0 < listed; q0 += 64) {
@@ -537,34 +560,62 @@ __device__ __forceinline__ void cell_scatter(const Ctx& c, ScatterShared& S, int
             // (few bins get more than one)
             if (__ballot(on && S.before[m.y] + S.after[m.y] > 1u)) {
                 const int end = min(listed, q0 + 64);
-                for (int j = 0; j < end; ++j) n += S.list[j].y == m.y && j < q ? 1 : 0;
+                for (int j = 0; j < end; j += 8) {
+                    int4 v[4];  // (two of the list each; the reads in flight together)
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) v[u] = reinterpret_cast<const int4*>(S.list)[j / 2 + u];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                        n += (v[u].y == m.y && j + 2 * u < q ? 1 : 0) + (v[u].w == m.y && j + 2 * u + 1 < q ? 1 : 0);
+                }
             }
             if (on) place_mover(m.x, m.y, n);
         }
-        return;
-    }
-    reinterpret_cast<uint4*>(S.met)[lane] = make_uint4(0u, 0u, 0u, 0u);
-    __syncwarp();
-    for (int k = 0; k < 3; ++k)
-        for (int i0 = p.s[k]; i0 < p.e[k]; i0 += 64) {
-            const int i = i0 + lane;
-            const int y = binOf[min(i, p.e[k] - 1)];
-            const uint32_t move = move_of(y), t = bin_from(y, b0);
-            const bool into = i < p.e[k] && move != 0u && move != kFarCode && t < uint32_t(nb);
-            for (unsigned long long m = __ballot(into); m != 0ull;) {
-                const uint32_t tm = uint32_t(__builtin_amdgcn_readlane(int(t), __builtin_ctzll(m)));
-                const unsigned long long same = __ballot(into && t == tm);
-                const uint32_t n = S.met[tm];
-                __syncwarp();
-                if (into && t == tm) {
-                    const int earlier = __builtin_popcountll(same & below);
-                    if (earlier == 0) S.met[tm] = n + uint32_t(__builtin_popcountll(same));
-                    place_mover(i, int(t), int(n) + earlier);
+    } else {
+        reinterpret_cast<uint4*>(S.run.met)[lane] = make_uint4(0u, 0u, 0u, 0u);
+        reinterpret_cast<uint2*>(S.run.turn)[lane] = make_uint2(~0u, ~0u);
+        __syncwarp();
+        for (int k = 0; k < 3; ++k)
+            for (int i0 = p.s[k]; i0 < p.e[k]; i0 += 64) {
+                const int i = i0 + lane;
+                const int y = binOf[min(i, p.e[k] - 1)];
+                const uint32_t move = move_of(y), t = bin_from(y, b0);
+                const bool into = i < p.e[k] && move != 0u && move != kFarCode && t < uint32_t(nb);
+                // Lanes of one bin take turns, whoever comes first: a lane's movers before it are those met in
+                // the rounds before, and the turns of lower lanes
+                bool waits = into;
+                int n = into ? int(S.run.met[t]) : 0;
+                for (uint32_t turn = 0; __any(waits); turn += 64u) {
+                    if (waits) S.run.turn[t] = uint16_t(turn + uint32_t(lane));
+                    __syncwarp();
+                    const uint32_t who = into ? S.run.turn[t] : ~0u;
+                    if ((who ^ turn) < uint32_t(lane)) ++n;
+                    waits = waits && who != turn + uint32_t(lane);
+                    __syncwarp();
+                }
+                if (into) {
+                    atomicAdd(&S.run.met[t], 1u);
+                    place_mover(i, int(t), n);
                 }
                 __syncwarp();
-                m &= ~same;
             }
+    }
+    if (farCells) {
+        __threadfence_block();  // (the near cells' places)
+        const int4 fc = *reinterpret_cast<const int4*>(c.far.count + g0 + 4 * lane);
+        const int4 head = *reinterpret_cast<const int4*>(c.far.head + g0 + 4 * lane);
+        for (int k = 0; k < 4; ++k) {
+            const int t = 4 * lane + k, n = k < 2 ? (k == 0 ? fc.x : fc.y) : (k == 2 ? fc.z : fc.w);
+            const int h = k < 2 ? (k == 0 ? head.x : head.y) : (k == 2 ? head.z : head.w);
+            if (n == 0 || n > kFarWalk) continue;
+            int* seg = c.sorted + w.cellOff + S.start[t];
+            const int m = S.start[t + 1] - S.start[t] - n;
+            if (__any(n > 4))
+                merge_far<kFarWalk>(seg, c.farLink, h, n, m);
+            else
+                merge_far<4>(seg, c.farLink, h, n, m);
         }
+    }
 }
 
 __device__ __forceinline__ void particles_to_bins(const Ctx& c, int b, int partBlocks) {
@@ -620,11 +671,10 @@ void launch_seed_bins(const Ctx& c, const LaunchShape& sh, hipStream_t s) {
     launch_fill_u32(reinterpret_cast<uint32_t*>(c.far.head), uint32_t(kNone), size_t(c.numCellBins), s);
     launch_fill_u32(reinterpret_cast<uint32_t*>(c.far.count), 0u, size_t(c.numCellBins), s);
     launch_fill_u32(reinterpret_cast<uint32_t*>(c.far.group), 0u, size_t(c.numCellBins / kGroupBins), s);
-    launch_fill_u32(reinterpret_cast<uint32_t*>(c.far.list), 0xffffffffu, 2 * size_t(c.cellCount), s);
-    launch_fill_u32(reinterpret_cast<uint32_t*>(c.far.total), uint32_t(c.cellCount), 1, s);
+    launch_fill_u32(reinterpret_cast<uint32_t*>(c.far.total), 0u, 1, s);
     launch_fill_u32(reinterpret_cast<uint32_t*>(c.superSum), 0u, size_t(c.numCellBins / kGroupBins / kSuperGroups + 1), s);
     if (sh.cellBlocks) hipLaunchKernelGGL(k_cell_bin, dim3(sh.cellBlocks), dim3(sh.cellThreads), 0, s, c);
-    if (c.numCellBins) hipLaunchKernelGGL(k_seed_sums, dim3(c.numCellBins / kGroupBins / 256 + 1), dim3(256), 0, s, c);
+    if (c.numCellBins) hipLaunchKernelGGL(k_seed_sums, dim3(c.numCellBins / kGroupBins / 4 + 1), dim3(256), 0, s, c);
     if (sh.partBlocks) hipLaunchKernelGGL(k_part_bin, dim3(sh.partGrid), dim3(sh.partThreads), 0, s, c);
 }
 

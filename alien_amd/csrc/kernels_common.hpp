@@ -63,11 +63,13 @@ __device__ __forceinline__ int cell_bin_of(const DevWorld& w, f2 p) {
     return w.binOff + by * w.nbx + bx;
 }
 
-// enters cell k in the far list of global bin gb
+// enters cell k in the far list of global bin gb; the bin's parts are listed once it has more than a lane merges
+// in (k_sort.hip)
 __device__ __forceinline__ void list_far(const FarCells& f, int* next, int gb, int k) {
     next[k] = atomicExch(&f.head[gb], k);
-    atomicAdd(&f.count[gb], 1);
-    atomicAdd(&f.group[gb / kGroupBins], 1);
+    const int n = atomicAdd(&f.count[gb], 1);
+    f.group[gb / kGroupBins] = 1;
+    if (n == kFarWalk || (n > kFarWalk && n % 64 == 0)) f.list[atomicAdd(f.total, 1)] = make_int2(gb, n / 64);
 }
 
 // moves the active lanes' cells between groups in the sums of groups: one atomic per group that gains or
@@ -122,7 +124,6 @@ __device__ __forceinline__ void bin_next(const Ctx& c, const DevWorld& w, int k,
         move = uint32_t(3 * (y + 1) + x + 2);
         if (x < -1 || x > 1) {
             move = kFarCode;
-            c.farNext.list[atomicAdd(c.farNext.total, 1)] = make_int2(k, w.binOff + b);
             list_far(c.farNext, c.farLink, w.binOff + b, k);
         }
         const int from = (w.binOff + bOld) / kGroupBins, to = (w.binOff + b) / kGroupBins;

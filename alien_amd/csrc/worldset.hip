@@ -706,7 +706,7 @@ void WorldSet::build(const std::vector<Source>& sources) {
         count_[0] = static_cast<uint32_t*>(A(sizeof(uint32_t) * NB));
         count_[1] = static_cast<uint32_t*>(A(sizeof(uint32_t) * NB));
         numCellBins_ = cellBins;
-        farList_ = static_cast<int2*>(A(sizeof(int2) * NC));
+        farList_ = static_cast<int2*>(A(sizeof(int2) * (size_t(NC) / 8 + 1)));  // (17 or 64 cells for an entry)
         for (int b = 0; b < 2; ++b) {
             start_[b] = static_cast<uint32_t*>(A(sizeof(uint32_t) * (size_t(NB) + 1)));
             far_[b].head = static_cast<int*>(A(sizeof(int) * NCB));

@@ -132,8 +132,8 @@ struct StepCounters {
     int errors;      // bit 0: candidate list overflow; bit 1: map-build look-back gave up;
                      // bit 2: a world's particles exceeded its particle capacity
     int liveParticles;  // energy particles alive after this step's particle sort, all worlds
-    // neighbour-pass paths since the data was set (not reset per step): chunks that walked their
-    // stencils in global memory, and cells of staged rows that walked theirs alone
+    // neighbour-pass paths since the data was set (not reset per step): waves with too many candidates to
+    // stage or to list at once, and the cells that went over their candidates alone
     unsigned long long fallbackChunks;
     unsigned long long directCells;
 };

@@ -30,7 +30,14 @@
 // come in two pieces.  They are left to waves of their own, two for each row's pair of edge bins (eight with
 // bond work: the cells of a body there, one after the other, took 16 of 32 us of a small world), that
 // take a cell at a time with its candidates side by side; walked alone by a lane of the pass, they
-// were its last waves to end.  Cells with more than 64 candidates walk their stencil alone.
+// were its last waves to end.
+// A wave whose stretches do not fit the stage (uneven density: bodies next to empty space, drops) tests the lists of
+// its first lanes; the other lanes go over their ranges by themselves, and so do all of a wave with long lists
+// (dense worlds, wide reach: above 72 candidates a cell).  A list of any length fits otherwise: the tests go on
+// until the pair records are full, and again after their pairs.  (When cells with more than 64 candidates and the
+// lanes beyond the stage walked all nine bins, a candidate at a time: bodies 210k cells in fluid 146 -> 117 us a
+// step, in collision 147 -> 124, drops of 2.7 cells a unit square 115 -> 54, a million cells at 2 a unit square, reach
+// 1.3, 376 -> 147, at 1 and reach 4, 375 -> 286.)
 // Collision worlds run the same pass.  In a body most neighbours are bonded, and a bonded pair adds nothing
 // but a rare push, so the pairs found are first sifted (8 to 2 a cell).  The pass before walked strips of
 // bin columns row by row, with the rows' halo staged again by every chunk, all nine bins tested and a list
@@ -43,6 +50,7 @@
 
 namespace alien {
 
+constexpr int kEdgeAlone = 16;    // more edge cells than this in a unit walk alone, one per lane
 // The pass's variants: fluid worlds of sets without bond work, and with; collision worlds.
 enum class Pass { kFree, kBonds, kCollide };
 template <Pass kPass> constexpr bool kBonded = kPass != Pass::kFree;  // (collision worlds have bonds in general)
@@ -51,20 +59,26 @@ constexpr int kFluidWaves = 4;   // waves per workgroup at most
 // bodies of four cells a bin next to empty space
 constexpr int kFreeStage = 288, kBondStage = 344;
 // pair records at a time: a fluid's cells have about one each at one cell per bin; with bonds, bodies with
-// ten neighbours a cell (the tests run again for what does not fit)
+// ten neighbours a cell
 constexpr int kFreePairs = 128, kBondPairs = 512;
-constexpr int kEdgeAlone = 16;    // more edge cells than this in a unit walk alone, one per lane
+// Lists longer than this in the mean are not laid out: their pairs come to one owner after the other, whose sums are
+// a serial chain, and the lanes go over their ranges by themselves (walk_ranges).  Steps of fluid cells with 48 | 64 |
+// 80 as the limit: 1 a unit square and reach 2.4, 223, 160 and 153 us; 0.25 and 8, 152, 152 and 153 (280 with lists);
+// drops of 2.7 in sparse surroundings and reach 4, 186, 184 and 197.
+constexpr int kLongLists = 72;
+static_assert(64 * kLongLists + 64 <= 8192, "a bit for each candidate of a wave's lists, and of a lane without one");
 
 // LDS of one wave: 6 KB (8 KB with bonds), six (five) waves per SIMD (the owners' velocities, densities
-// and flags come from their registers, by cross-lane permutes).  With bonds: room for 448 staged cells and
-// 896 pairs at four waves ran 1 % slower in bodies, for 288 and 384 5 to 10 % (the tests run again).
+// and flags come from their registers, by cross-lane permutes).  With bonds, while the tests ran again for pairs
+// without a record: room for 448 staged cells and 896 pairs at four waves was 1 % slower in bodies, for 288
+// and 384 5 to 10 %.
 template <int kStage, int kPairs> struct FluidShared {
     // staged candidates: their positions, and behind them their A indices (the last round of tests reads
     // up to 63 positions past the last list, and counts nothing there)
     float2 cpos[kStage + kStage / 2];
     __device__ int& caidx(int x) { return reinterpret_cast<int*>(cpos + kStage)[x]; }
     float2 pos[64];  // the wave's own cells; no position for a lane that does not test
-    uint16_t first[65];  // each owner's first pair
+    uint16_t first[64];  // each owner's first pair
     uint16_t own[64];    // pairs up to the owner's own place in its list
     uint16_t pair[kPairs];  // pair records: staged neighbour, owner << 9
     union {
@@ -72,7 +86,7 @@ template <int kStage, int kPairs> struct FluidShared {
             // per list: its row boundaries (flat, two 16-bit halves) and what to add to a flat index
             // for the candidate's place, row by row
             int4 rec[64];
-            uint32_t start[128];  // bit f: a list starts at flat index f (64 lists of at most 64)
+            uint32_t start[256];  // bit f: a list starts at flat index f
         } t;
         struct {
             float4 a[64];  // density term, overlap push, barrier (A index + 1)
@@ -181,6 +195,59 @@ template <bool kFluid> __device__ __forceinline__ void walk_alone(const Ctx& c, 
             for (int j = off + int(start[b]); j < e; ++j) visit(map_nb(c, j));
         }
     });
+}
+
+// A cell of the pass whose lane goes over its ranges by itself: the map positions lo[k] on, ns[k] of each stencil
+// row, with the loads of four candidates in flight.  Adds up in visiting order, as the pairs of a wave's lists do.
+template <Pass kPass>
+__device__ __forceinline__ void walk_ranges(const Ctx& c, const DevWorld& w, const DevParams& P, int wi, int m, int aidx, f2 pos,
+                                            f2 vel, float inv, uint32_t flags, const int bt[kMaxBonds], const int lo[3],
+                                            const int ns[3], bool seam, Acc& acc) {
+    constexpr bool kFluid = kPass != Pass::kCollide, kBonds = kBonded<kPass>;
+    constexpr int kAhead = 4;
+    const float Wf = float(w.W), Hf = float(w.H);
+    Nb s;
+    s.pos = pos, s.vel = vel, s.dens = inv, s.flags = flags, s.aidx = aidx, s.lidx = m;
+    int3 at = make_int3(lo[0], lo[1], lo[2]), n = make_int3(ns[0], ns[1], ns[2]);
+#pragma unroll 1
+    for (int k = 0; k < 3; ++k) {
+        int x = at.x;
+        const int end = x + n.x;
+        at.x = at.y, at.y = at.z, n.x = n.y, n.y = n.z;
+        for (; x < end; x += kAhead) {
+            Nb o[kAhead];
+#pragma unroll
+            for (int q = 0; q < kAhead; ++q) o[q].aidx = ld32(c.sorted, uint32_t(min(x + q, end - 1)));
+#pragma unroll
+            for (int q = 0; q < kAhead; ++q) {
+                const uint32_t a = uint32_t(o[q].aidx);
+                o[q].pos = to_f2(ld32(c.A.pos, a));
+                o[q].vel = to_f2(ld32(c.A.vel, a));
+                if (kFluid) o[q].dens = ld32(c.A.dens, a);
+                if (kBonds) o[q].flags = ld32(c.A.flags, a);
+            }
+#pragma unroll
+            for (int q = 0; q < kAhead; ++q) {
+                o[q].lidx = x + q;
+                const f2 pd = stencil_delta(pos, o[q].pos, Wf, Hf, kFluid && seam);
+                if (!(lensq(pd) <= P.reachSq) || x + q >= end) continue;
+                if constexpr (kPass == Pass::kFree) {
+                    // (the cell itself, at distance 0, adds its own density term and zeros)
+                    const FluidTerms t = fluid_terms<false>(P, pd, sub(vel, o[q].vel), inv, o[q].dens, true);
+                    acc.rho = acc.rho + t.rho;
+                    acc.D = add(acc.D, t.D);
+                    acc.Fp = add(acc.Fp, t.Fp);
+                    acc.Fv = add(acc.Fv, t.Fv);
+                } else {
+                    if (!kFluid && x + q == m) continue;
+                    float t[kPairTerms];
+                    const uint32_t f = pair_term<kFluid>(c, w, P, wi, s, o[q], is_bonded(bt, o[q].aidx - w.cellOff), t, kFluid && seam,
+                                                         [&] { return make_int2(m, o[q].lidx); });
+                    acc_add<kFluid>(acc, f, t);
+                }
+            }
+        }
+    }
 }
 
 // The cells of the edge unit u: the last bin of row u - 1 and the first bin of row u, one after the
@@ -295,6 +362,7 @@ __device__ __forceinline__ int fluid_wave(const Ctx& c, FluidWave<kBonded<kPass>
     const uint32_t* start = c.start + w.binOff;
     const int off = w.cellOff - int(start[0]);
     int m0, mEnd;
+    bool seam = false;
     {
         const int r1 = int(start[w.nbx] - start[0]), r2 = int(start[(w.nby - 1) * w.nbx] - start[0]);
         const int sh = kCollide ? c.collideShift : c.fluidShift, more = (1 << sh) - 1;
@@ -302,6 +370,11 @@ __device__ __forceinline__ int fluid_wave(const Ctx& c, FluidWave<kBonded<kPass>
         const int at = v < v1 ? v << sh : (v < v2 ? r1 + ((v - v1) << sh) : r2 + ((v - v2) << sh));
         m0 = w.cellOff + at;
         mEnd = w.cellOff + min(at + more + 1, v < v1 ? r1 : (v < v2 ? r2 : w.numCells));
+        // (in grids of at least eight bins each way, two stencil neighbours lie less than three bin edges
+        // apart, less than half the world: away from the seam rows the plain difference equals the torus
+        // difference bit for bit)
+        // (collision pairs are tested by their plain difference, R13: no neighbours across the seam)
+        if (!kCollide) seam = v < v1 || v >= v2 || w.nbx < 8 || w.nby < 8;
     }
     if ((P.motion == 0) == kCollide || m0 >= mEnd) return -1;  // (a wave past its world)
     const int m = m0 + lane;
@@ -353,7 +426,6 @@ __device__ __forceinline__ int fluid_wave(const Ctx& c, FluidWave<kBonded<kPass>
         const float up = pos.y - Y0, down = pos.y - (by == w.nby - 1 ? Hf : Y0 + float(w.binSize));
         if (up * up > P.reachSq) ns[0] = 0;
         if (down * down > P.reachSq) ns[2] = 0;
-        alone = ns[0] + ns[1] + ns[2] > 64;
     }
     Acc acc;
     {
@@ -361,20 +433,13 @@ __device__ __forceinline__ int fluid_wave(const Ctx& c, FluidWave<kBonded<kPass>
         self.pos = pos;
         acc_init(acc, self);
     }
-    if constexpr (kCollide) {
-        // (counted: waves too crowded for the stage)
-        const unsigned long long all = __ballot(mine);
-        if (__ballot(alone) & all) {
-            const int first = __builtin_ctzll(all), last = 63 - __builtin_clzll(all);
-            const int bF = __builtin_amdgcn_readlane(by, first) * w.nbx + __builtin_amdgcn_readlane(bx, first);
-            const int bL = __builtin_amdgcn_readlane(by, last) * w.nbx + __builtin_amdgcn_readlane(bx, last);
-            if (int(start[bL + 1]) - int(start[bF]) > kStage / 3 && lane == 0) atomicAdd(&c.sc->fallbackChunks, 1ull);
-        }
-    }
     // The staged stretch of each stencil row, [u0, u0 + un): from the left bin of the first testing lane to
     // the right bin of the last one (both grow with the lane: a wave is in the torus' first bin row, in its
-    // last one, or in neither).  Lanes whose rows do not fit the stage walk alone.
+    // last one, or in neither).  Lists that are long in the mean are not laid out.  If the rows do not fit the
+    // stage, the first lanes take what fits.  The other lanes go over their ranges each for itself, as all do
+    // where fewer than 16 would fit.
     unsigned long long group = __ballot(mine && !alone);
+    if (wave_last(int(wave_inclusive_scan(uint32_t(ns[0] + ns[1] + ns[2])))) > kLongLists * __builtin_popcountll(group)) group = 0ull;
     {
         const int first = group ? __builtin_ctzll(group) : 0;
         const int bxF = __builtin_amdgcn_readlane(bx, first), byF = __builtin_amdgcn_readlane(by, first);
@@ -384,20 +449,19 @@ __device__ __forceinline__ int fluid_wave(const Ctx& c, FluidWave<kBonded<kPass>
             u0[k] = group ? off + int(start[wrap_small(byF + k - 1, w.nby) * w.nbx + bxF - 1]) : 0;
             un[k] = 0;
         }
-        for (int keep = 32; group;) {
+        for (int keep = 64; group;) {
             const int last = 63 - __builtin_clzll(group);
             const int bxL = __builtin_amdgcn_readlane(bx, last), byL = __builtin_amdgcn_readlane(by, last);
 #pragma unroll
             for (int k = 0; k < 3; ++k)
                 un[k] = off + int(start[wrap_small(byL + k - 1, w.nby) * w.nbx + bxL + 2]) - u0[k];
             if (__builtin_expect(un[0] + un[1] + un[2] <= kStage, 1)) break;
-            group &= keep ? ((1ull << keep) - 1ull) << first : 0ull;
             keep >>= 1;
+            group &= keep >= 16 ? ((1ull << keep) - 1ull) << first : 0ull;
             if (!group) un[0] = un[1] = un[2] = 0;
         }
         const int un01 = un[0] + un[1], unAll = un01 + un[2];
         const bool tests = __builtin_amdgcn_inverse_ballot_w64(group);
-        alone = mine && !tests;
         {
             const int g0 = u0[0], g1 = u0[1] - un[0], g2 = u0[2] - un01;
             constexpr int kLoads = (kStage + 63) / 64;
@@ -418,19 +482,14 @@ __device__ __forceinline__ int fluid_wave(const Ctx& c, FluidWave<kBonded<kPass>
                     S.caidx(lane + 64 * q) = a[q];
                 }
         }
-        // (in grids of at least eight bins each way, two stencil neighbours lie less than three bin edges
-        // apart, less than half the world: away from the seam rows the plain difference equals the torus
-        // difference bit for bit)
-        // (collision pairs are tested by their plain difference, R13: no neighbours across the seam)
-        const bool seam = !kCollide && (byF == 0 || byF == w.nby - 1 || w.nbx < 8 || w.nby < 8);
         S.pos[lane] = tests ? to_float2(pos) : make_float2(__builtin_nanf(""), 0.0f);
         // A lane without a list gets one entry that no test accepts, so that list k belongs to lane k.
         const int nt = tests ? ns[0] + ns[1] + ns[2] : 1;
         const int inc = int(wave_inclusive_scan(uint32_t(nt)));
-        const int flat = inc - nt, flatAll = wave_last(inc);
+        const int flat = inc - nt, flatAll = group ? wave_last(inc) : 0;
         const int selfBase = m0 - u0[1] + un[0];  // the own entry of lane 0
-        int numPairs = 0;
-        for (int R0 = 0;; R0 += kPairs) {
+        // the lists' tests and pairs, as many rounds of tests at a time as there is room for their pairs
+        for (int from = 0, to = 0; from < flatAll; from = to) {
             {
                 int4 rec = make_int4(flat | flat << 16, -flat, -flat, -flat);
                 if (tests) {
@@ -442,16 +501,22 @@ __device__ __forceinline__ int fluid_wave(const Ctx& c, FluidWave<kBonded<kPass>
                 }
                 S.u.t.start[lane] = 0u;
                 S.u.t.start[lane + 64] = 0u;
+                if (flatAll > 4096 - 64) {
+                    S.u.t.start[lane + 128] = 0u;
+                    S.u.t.start[lane + 192] = 0u;
+                }
                 S.u.t.rec[lane] = rec;
+                if (!kCollide) S.own[lane] = 0xffff;
                 __syncwarp();
                 atomicOr(&S.u.t.start[flat >> 5], 1u << (flat & 31));
                 __syncwarp();
             }
-            numPairs = 0;
+            int numPairs = 0;
             auto test = [&](auto seamTag) {
                 constexpr bool kSeam = decltype(seamTag)::value;
-                int owners = -1;  // lists that started before this round, minus one
-                for (int f0 = 0; f0 < flatAll; f0 += 64) {
+                int owners = __builtin_popcountll(__ballot(flat < from)) - 1;  // lists that started before this round, minus one
+                int f0 = from;
+                for (; f0 < flatAll; f0 += 64) {
                     const uint32_t s0 = __builtin_amdgcn_readfirstlane(S.u.t.start[f0 >> 5]);
                     const uint32_t s1 = __builtin_amdgcn_readfirstlane(S.u.t.start[(f0 >> 5) + 1]);
                     const unsigned long long starts = (static_cast<unsigned long long>(s1) << 32) | s0;
@@ -471,37 +536,34 @@ __device__ __forceinline__ int fluid_wave(const Ctx& c, FluidWave<kBonded<kPass>
                     const bool hit = in && d2 <= P.reachSq && (!self || (kPass == Pass::kBonds && rec.x < 0));
                     const unsigned long long hits = __ballot(hit);
                     const int rank = lanes_below(hits, numPairs);
+                    if (numPairs + __builtin_popcountll(hits) > kPairs) break;
                     if (__builtin_amdgcn_inverse_ballot_w64(starts)) S.first[owner] = uint16_t(rank);
                     if (!kCollide && self) S.own[owner] = uint16_t(rank);
-                    // (a wave's pairs nearly always fit one window: then no lane asks)
-                    if (R0 == 0 && numPairs + __builtin_popcountll(hits) <= kPairs) {
-                        if (hit) S.pair[rank] = uint16_t(x | owner << 9);
-                    } else if (hit && uint32_t(rank - R0) < uint32_t(kPairs)) {
-                        S.pair[rank - R0] = uint16_t(x | owner << 9);
-                    }
+                    if (hit) S.pair[rank] = uint16_t(x | owner << 9);
                     numPairs += __builtin_popcountll(hits);
                 }
+                to = min(f0, flatAll);
             };
             if (seam)
                 test(std::true_type{});
             else
                 test(std::false_type{});
-            if (lane == 0) S.first[64] = uint16_t(numPairs);
             __syncwarp();
-            int pairs0 = S.first[lane], pairs1 = S.first[lane + 1];
+            // (a list may have started before these tests, or start after them)
+            int pairs0 = flat < from ? 0 : (flat < to ? S.first[lane] : numPairs);
+            int pairs1 = inc < from ? 0 : (inc < to ? S.first[lane + 1] : numPairs);
             const int ownAt = kCollide || (kBonds && flags_barrier(flags)) ? -1 : S.own[lane];
-            int rend = min(numPairs, R0 + kPairs);
+            int rend = numPairs;
             if constexpr (kCollide) {
                 // Most neighbours in a body are bonded, and a bonded pair adds only its overlap push (closer
                 // than minDistance, not for a barrier cell): the other records go, bit 15 marks what stays of
                 // the bonded ones.  (In place: a round's records land at or before their own places.)
-                int to = R0;
+                int kept = 0;
                 const int from0 = pairs0, from1 = pairs1;
-                pairs0 = from0 <= R0 ? R0 : rend;
-                pairs1 = from1 <= R0 ? R0 : rend;
-                for (int p0 = R0; p0 < rend; p0 += 64) {
+                pairs0 = pairs1 = 0;
+                for (int p0 = 0; p0 < rend; p0 += 64) {
                     const int p = p0 + lane;
-                    const int r = p < rend ? S.pair[p - R0] : 0;
+                    const int r = p < rend ? S.pair[p] : 0;
                     const int x = r & 0x1ff, ol = r >> 9;
                     const uint32_t sf = uint32_t(__shfl(int(flags), ol, 64));
                     bool bonded = false;
@@ -516,24 +578,22 @@ __device__ __forceinline__ int fluid_wave(const Ctx& c, FluidWave<kBonded<kPass>
                     const bool push = !flags_barrier(sf) && lensq(sub(to_f2(S.pos[ol]), to_f2(S.cpos[x]))) <= P.overlapBelowSq;
                     const bool stays = p < rend && (!bonded || push);
                     const unsigned long long m = __ballot(stays);
-                    if (stays) S.pair[lanes_below(m, to) - R0] = uint16_t(r | (bonded ? 0x8000 : 0));
+                    if (stays) S.pair[lanes_below(m, kept)] = uint16_t(r | (bonded ? 0x8000 : 0));
                     // the owners' first and last records move along
-                    if (from0 > p0 && from0 <= p0 + 64) pairs0 = to + __builtin_popcountll(m & (~0ull >> (p0 + 64 - from0)));
-                    if (from1 > p0 && from1 <= p0 + 64) pairs1 = to + __builtin_popcountll(m & (~0ull >> (p0 + 64 - from1)));
-                    to += __builtin_popcountll(m);
+                    if (from0 > p0 && from0 <= p0 + 64) pairs0 = kept + __builtin_popcountll(m & (~0ull >> (p0 + 64 - from0)));
+                    if (from1 > p0 && from1 <= p0 + 64) pairs1 = kept + __builtin_popcountll(m & (~0ull >> (p0 + 64 - from1)));
+                    kept += __builtin_popcountll(m);
                 }
-                if (from0 > rend) pairs0 = to;
-                if (from1 > rend) pairs1 = to;
-                rend = to;
+                rend = kept;
                 __syncwarp();
             }
-            for (int p0 = R0; p0 < rend; p0 += 64) {
+            for (int p0 = 0; p0 < rend; p0 += 64) {
                 // pair terms, one pair per lane
                 float4 ra = make_float4(0.0f, 0.0f, 0.0f, 0.0f), rb = ra;
                 const int p = p0 + lane;
                 int x = 0, ol = 0, bonded = 0;  // (bonded: of a collision pair)
                 if (p < rend) {
-                    const int r = S.pair[p - R0];
+                    const int r = S.pair[p];
                     x = r & 0x1ff;
                     ol = (r >> 9) & 63;
                     bonded = r >> 15;
@@ -631,12 +691,19 @@ __device__ __forceinline__ int fluid_wave(const Ctx& c, FluidWave<kBonded<kPass>
                     acc.Fv = add(acc.Fv, f2{tb.z, tb.w});
                 }
             }
-            if (R0 + kPairs >= numPairs) {
-                if (!kCollide && tests && ownAt == pairs1) acc.rho = acc.rho + w0;  // the own term after all pairs
-                break;
-            }
+            if (!kCollide && tests && ownAt == pairs1) acc.rho = acc.rho + w0;  // the own term after all pairs
             __syncwarp();
         }
+    }
+    const bool walks = mine && !alone && !__builtin_amdgcn_inverse_ballot_w64(group);
+    if (__builtin_expect(__any(walks), 0)) {
+        const unsigned long long all = __ballot(walks);
+        // (counted here: after a store the compiler would read the map's offsets through the vector path)
+        if (lane == 0) {
+            atomicAdd(&c.sc->fallbackChunks, 1ull);
+            atomicAdd(&c.sc->directCells, (unsigned long long)(__builtin_popcountll(all)));
+        }
+        if (walks) walk_ranges<kPass>(c, w, P, wi, m, aidx, pos, vel, inv, flags, bt, lo, ns, seam, acc);
     }
     if (!mine) return -1;
     if (alone) return m;

@@ -174,7 +174,7 @@ public:
     // kernel timing mode: no graphs, every launch bracketed by events (see alien_set_kernel_timing)
     void setKernelTiming(bool on);
     bool kernelTiming() const { return timing_; }
-    // neighbour-pass fallback counts since the data was set: chunks, cells
+    // neighbour-pass fallback counts since the data was set: waves, cells
     void pathCounts(uint64_t& fallbackChunks, uint64_t& directCells);
     struct KernelTime {
         uint64_t launches = 0;

@@ -228,9 +228,8 @@ int alien_set_kernel_timing(alien_world* w, int32_t enable);
 int alien_get_kernel_timing(alien_world* w, alien_kernel_time* out, int32_t cap, int32_t* count);
 
 /* Neighbour-pass path counts since the world's data was last set (no counterpart in ALIEN; a
- * performance diagnostic, results never depend on the path): waves of the collision pass with cells
- * that have more than 64 candidates among too many for their staged rows, and cells with more than 64
- * candidates, which walk their stencils alone. */
+ * performance diagnostic, results never depend on the path): waves with too many candidates to stage or
+ * to list at once, and the cells that go over their candidates alone (some or all of such a wave's). */
 int alien_get_path_counts(alien_world* w, uint64_t* fallbackChunks, uint64_t* directCells);
 
 /* ---- batched worlds ------------------------------------------------------------------------ */

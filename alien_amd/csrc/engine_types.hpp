@@ -30,8 +30,9 @@ constexpr int kSuperGroups = 256;  // groups per sum of groups
 // there (10751 cells in bodies: a step of 106 us with 64, 97 with 32, 92 with 16); with more cells the
 // wave's fixed work counts (134k cells in bodies: 159, 157 and 162 us; 256k free ones: 22, 26 and 32 us).
 constexpr int kFluidShiftMin = 4;
-// waves of the fluid pass for a row's two edge bins (k_neighbor.hip), without and with bond work
-constexpr int kEdgeWaves = 2, kEdgeWavesBonds = 8;
+// waves of the neighbour passes for a group of units of two edge bins (k_neighbor.hip); units per group: as few as
+// keep a set's edge waves below kEdgeWavesMost
+constexpr int kEdgeWaves = 8, kEdgeUnitsMost = 8, kEdgeWavesMost = 4096;
 constexpr int kXcdCount = 8;  // XCDs of an MI355X: workgroup b of a launch runs on XCD b % 8
 // Size limits of one world set.  Cell indices, bin offsets and the bond planes ([kMaxBonds][cap],
 // addressed as b * cap + x) are 32-bit ints in the kernels, so a set holds at most
@@ -282,7 +283,8 @@ struct Ctx {
     int fluidShift;           // its waves take 1 << fluidShift cells
     const int2 *collideBlocks, *collideEdgeBlocks;  // the same of the collision pass
     int collideShift;
-    const int2* edgeBlocks;  // per workgroup: (world, its first wave's edge unit and part), see k_neighbor.hip
+    const int2* edgeBlocks;  // per workgroup: (world, its first edge wave), see k_neighbor.hip
+    int edgeUnits, collideEdgeUnits;  // edge units that kEdgeWaves waves share
     const int2* livingBlocks;  // per block: (world, first global cell index) over livingWork worlds
     int blockThreads;  // cells, bins or living cells per entry of the block tables above
 };

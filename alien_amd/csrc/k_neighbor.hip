@@ -27,10 +27,12 @@
 // us, with the edge waves and fewer cells per wave (kFluidShiftMin) 10751 cells 108 -> 91.5 us.
 //
 // Cells of the first and last bin column have a stencil that wraps around the torus: their ranges
-// come in two pieces.  They are left to waves of their own, two for each row's pair of edge bins (eight with
-// bond work: the cells of a body there, one after the other, took 16 of 32 us of a small world), that
-// take a cell at a time with its candidates side by side; walked alone by a lane of the pass, they
-// were its last waves to end.
+// come in two pieces.  They are left to waves of their own, eight for a group of rows' pairs of edge bins (one row
+// in small sets; the cells of a body there, one after the other, took 16 of 32 us of a small world), that take a
+// cell at a time with 64 of its candidates side by side; walked alone by a lane of the pass, they were its last
+// waves to end.  (With eight waves for every row, a tall world spent its time on empty ones, and more than 16 cells
+// or 64 candidates were walked by a lane each: 256k cells of 64 x 8192 units, reach 2.5, a step of 340 us, 151 so;
+// bodies there 117 and 96; 64k fluid cells with reach 8, 281 and 152.)
 // A wave whose stretches do not fit the stage (uneven density: bodies next to empty space, drops) tests the lists of
 // its first lanes; the other lanes go over their ranges by themselves, and so do all of a wave with long lists
 // (dense worlds, wide reach: above 72 candidates a cell).  A list of any length fits otherwise: the tests go on
@@ -50,7 +52,6 @@
 
 namespace alien {
 
-constexpr int kEdgeAlone = 16;    // more edge cells than this in a unit walk alone, one per lane
 // The pass's variants: fluid worlds of sets without bond work, and with; collision worlds.
 enum class Pass { kFree, kBonds, kCollide };
 template <Pass kPass> constexpr bool kBonded = kPass != Pass::kFree;  // (collision worlds have bonds in general)
@@ -250,23 +251,28 @@ __device__ __forceinline__ void walk_ranges(const Ctx& c, const DevWorld& w, con
     }
 }
 
-// The cells of the edge unit u: the last bin of row u - 1 and the first bin of row u, one after the
-// other in the map; the unit's two waves take every other cell.  Returns the cells left to walk alone:
-// this lane's first one, and the end.
-template <Pass kPass> __device__ __forceinline__ int2 edge_unit(const Ctx& c, int wi, int u, int part) {
+// The cells of the first and last bin column, in units: the last bin of row u - 1 and the first bin of row u, which
+// follow each other in the map.  A group of units (edgeUnits) is shared by kEdgeWaves waves, this one number `part`, a
+// cell at a time in turn, with 64 of its candidates side by side.
+template <Pass kPass> __device__ __forceinline__ void edge_cells(const Ctx& c, int wi, int group, int part) {
     constexpr bool kFluid = kPass != Pass::kCollide;
-    constexpr int kWaves = kBonded<kPass> ? kEdgeWavesBonds : kEdgeWaves;
     const DevWorld& w = c.worlds[wi];
     const DevParams& P = c.params[wi];
     const int lane = int(threadIdx.x) & 63;
     const uint32_t* start = c.start + w.binOff;
     const int off = w.cellOff - int(start[0]);
-    const int m0 = off + int(start[max(u * w.nbx - 1, 0)]), m1 = off + int(start[u < w.nby ? u * w.nbx + 1 : u * w.nbx]);
-    if (m1 - m0 > kEdgeAlone) return make_int2(part == 0 ? m0 + lane : m1, m1);
+    const int units = kFluid ? c.edgeUnits : c.collideEdgeUnits, u = group * units + lane;
+    int unitAt = 0, unitN = 0;
+    if (lane < units && u <= w.nby) {
+        unitAt = off + int(start[max(u * w.nbx - 1, 0)]);
+        unitN = off + int(start[u < w.nby ? u * w.nbx + 1 : u * w.nbx]) - unitAt;
+    }
+    const int unitEnd = int(wave_inclusive_scan(uint32_t(unitN))), cells = wave_last(unitEnd);
     const float Wf = float(w.W), Hf = float(w.H), reachSq = P.reachSq;
     const float w0 = sph_w(0.0f) * P.invH2;
-    uint32_t crowded = 0u;  // cells with more than 64 candidates
-    for (int m = m0 + part; m < m1; m += kWaves) {
+    for (int t = part; t < cells; t += kEdgeWaves) {
+        const int k = __builtin_popcountll(__ballot(unitEnd <= t));
+        const int m = t + __builtin_amdgcn_readlane(unitAt - (unitEnd - unitN), k);
         const Nb s = map_nb(c, m);  // (the same on every lane)
         int bx, by;
         cell_bin_xy(w, s.pos, bx, by);
@@ -279,72 +285,72 @@ template <Pass kPass> __device__ __forceinline__ int2 edge_unit(const Ctx& c, in
         }
         const int inc = int(wave_inclusive_scan(uint32_t(n)));
         const int total = wave_last(inc);
-        if (total > 64) {
-            crowded |= 1u << (m - m0);
-            continue;
-        }
-        // candidate `lane` of the list
-        int at = 0;
-#pragma unroll
-        for (int k = 0; k < 9; ++k) {
-            const int begin = __builtin_amdgcn_readlane(inc - n, k);
-            at = lane >= begin ? __builtin_amdgcn_readlane(lo, k) + lane - begin : at;
-        }
-        const bool in = lane < total;
         const bool keepSelf = kFluid && flags_barrier(s.flags);
-        Nb o = s;
-        if (in) o = map_nb(c, at);
-        const float d2 = lensq(kFluid ? torus_delta(s.pos, o.pos, Wf, Hf) : sub(o.pos, s.pos));
-        const bool hit = in && d2 <= reachSq && (o.aidx != s.aidx || keepSelf);
-        const unsigned long long self = __ballot(in && o.aidx == s.aidx);
-        unsigned long long hits = __ballot(hit);
-        const int selfAt = keepSelf || self == 0ull ? 64 : __builtin_ctzll(self);
-        bool pending = kFluid && !keepSelf;  // the own density term, at its place in the order
+        const int slot = c.A.slot[s.aidx];
+        int bt[kMaxBonds];
+        if constexpr (kPass != Pass::kFree) load_bonds(c, s, bt);
         Acc a;
         acc_init(a, s);
-        auto add_own = [&](int l) {
-            if (pending && l > selfAt) {
-                a.rho = a.rho + w0;
-                pending = false;
-            }
-        };
         auto from = [](float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
-        const int slot = c.A.slot[s.aidx];
-        if constexpr (kPass == Pass::kFree) {
-            const FluidTerms t = fluid_terms<false>(P, torus_delta(s.pos, o.pos, Wf, Hf), sub(s.vel, o.vel), s.dens, o.dens, true);
-            for (; hits; hits &= hits - 1ull) {
-                const int l = __builtin_ctzll(hits);
-                add_own(l);
-                a.rho = a.rho + from(t.rho, l);
-                a.D = add(a.D, f2{from(t.D.x, l), from(t.D.y, l)});
-                a.Fp = add(a.Fp, f2{from(t.Fp.x, l), from(t.Fp.y, l)});
-                a.Fv = add(a.Fv, f2{from(t.Fv.x, l), from(t.Fv.y, l)});
+        for (int f0 = 0; f0 < total; f0 += 64) {
+            // candidate f0 + lane of the list
+            int at = 0;
+#pragma unroll
+            for (int q = 0; q < 9; ++q) {
+                const int begin = __builtin_amdgcn_readlane(inc - n, q);
+                at = f0 + lane >= begin ? __builtin_amdgcn_readlane(lo, q) + f0 + lane - begin : at;
+            }
+            const bool in = f0 + lane < total;
+            Nb o = s;
+            if (in) o = map_nb(c, at);
+            const float d2 = lensq(kFluid ? torus_delta(s.pos, o.pos, Wf, Hf) : sub(o.pos, s.pos));
+            const bool hit = in && d2 <= reachSq && (o.aidx != s.aidx || keepSelf);
+            unsigned long long hits = __ballot(hit);
+            // the own density term, at its place in the order (after the round's hits before it, or after all)
+            const unsigned long long self = __ballot(in && o.aidx == s.aidx);
+            bool pending = kFluid && !keepSelf && self != 0ull;
+            const int selfAt = pending ? __builtin_ctzll(self) : 64;
+            auto add_own = [&](int l) {
+                if (pending && l > selfAt) {
+                    a.rho = a.rho + w0;
+                    pending = false;
+                }
+            };
+            if constexpr (kPass == Pass::kFree) {
+                const FluidTerms t = fluid_terms<false>(P, torus_delta(s.pos, o.pos, Wf, Hf), sub(s.vel, o.vel), s.dens, o.dens, true);
+                for (; hits; hits &= hits - 1ull) {
+                    const int l = __builtin_ctzll(hits);
+                    add_own(l);
+                    a.rho = a.rho + from(t.rho, l);
+                    a.D = add(a.D, f2{from(t.D.x, l), from(t.D.y, l)});
+                    a.Fp = add(a.Fp, f2{from(t.Fp.x, l), from(t.Fp.y, l)});
+                    a.Fv = add(a.Fv, f2{from(t.Fv.x, l), from(t.Fv.y, l)});
+                }
+            } else {
+                float t[kPairTerms];
+#pragma unroll
+                for (int v = 0; v < kPairTerms; ++v) t[v] = 0.0f;
+                uint32_t f = 0u;
+                if (hit)
+                    f = pair_term<kFluid>(c, w, P, wi, s, o, is_bonded(bt, o.aidx - w.cellOff), t, true,
+                                          [&] { return make_int2(s.lidx, o.lidx); });
+                for (; hits; hits &= hits - 1ull) {
+                    const int l = __builtin_ctzll(hits);
+                    add_own(l);
+                    float tt[kPairTerms];
+#pragma unroll
+                    for (int v = 0; v < kPairTerms; ++v) tt[v] = from(t[v], l);
+                    acc_add<kFluid>(a, uint32_t(__builtin_amdgcn_readlane(int(f), l)), tt);
+                }
             }
             add_own(65);
-            if (lane == 0) finish_free(c, w, P, m, s.pos, s.vel, s.flags, slot, a.rho, a.D, a.Fp, a.Fv, by * w.nbx + bx);
-        } else {
-            int bt[kMaxBonds];
-            load_bonds(c, s, bt);
-            float t[kPairTerms];
-#pragma unroll
-            for (int v = 0; v < kPairTerms; ++v) t[v] = 0.0f;
-            uint32_t f = 0u;
-            if (hit)
-                f = pair_term<kFluid>(c, w, P, wi, s, o, is_bonded(bt, o.aidx - w.cellOff), t, true,
-                                    [&] { return make_int2(s.lidx, o.lidx); });
-            for (; hits; hits &= hits - 1ull) {
-                const int l = __builtin_ctzll(hits);
-                add_own(l);
-                float tt[kPairTerms];
-#pragma unroll
-                for (int v = 0; v < kPairTerms; ++v) tt[v] = from(t[v], l);
-                acc_add<kFluid>(a, uint32_t(__builtin_amdgcn_readlane(int(f), l)), tt);
-            }
-            add_own(65);
-            if (lane == 0) cell_finish<kFluid>(c, w, P, wi, s, slot, bt, a, by * w.nbx + bx);
         }
+        if (lane != 0) continue;
+        if constexpr (kPass == Pass::kFree)
+            finish_free(c, w, P, m, s.pos, s.vel, s.flags, slot, a.rho, a.D, a.Fp, a.Fv, by * w.nbx + bx);
+        else
+            cell_finish<kFluid>(c, w, P, wi, s, slot, bt, a, by * w.nbx + bx);
     }
-    return make_int2((crowded >> lane) & 1u && lane < kEdgeAlone ? m0 + lane : m1, m1);
 }
 
 // Wave v of the world: 64 (fewer in small sets, fluidShift) consecutive map positions of the first bin row, of the last one, or of those
@@ -737,28 +743,22 @@ k_neighbor(Ctx c, int partBlocks, int late, int edgeBlocks, int tableBlocks) {
             return late ? part_scatter(c, {block, partBlocks}) : part_binsort(c, {block, partBlocks});
         block -= partBlocks;
     }
-    int wi;
-    int2 walk = make_int2(0, 0);  // cells this lane walks alone: walk.x, walk.x + 64, ... below walk.y
     if (block < edgeBlocks) {
         const int2 blk = (kFluid ? c.edgeBlocks : c.collideEdgeBlocks)[block];
-        wi = blk.x;
-        constexpr int kWaves = kBonds ? kEdgeWavesBonds : kEdgeWaves;
-        const int u = blk.y + wave;
-        if (u / kWaves <= c.worlds[wi].nby) walk = edge_unit<kPass>(c, wi, u / kWaves, u % kWaves);
-    } else {
-        block -= edgeBlocks;
-        // XCD-aware: workgroup b runs on XCD b % 8, which sweeps one contiguous band of the map, so the
-        // stencil rows its waves share stay in its L2
-        const int per = (tableBlocks + kXcdCount - 1) / kXcdCount;
-        const int e = (block % kXcdCount) * per + block / kXcdCount;
-        if (e >= tableBlocks) return;
-        const int2 blk = (kFluid ? c.fluidBlocks : c.collideBlocks)[e];
-        wi = blk.x;
-        const int m = fluid_wave<kPass>(c, SS[wave], wi, blk.y + wave);
-        if (m >= 0) walk = make_int2(m, m + 1);
+        const int wi = blk.x;
+        edge_cells<kPass>(c, wi, (blk.y + wave) / kEdgeWaves, (blk.y + wave) % kEdgeWaves);
+        return;
     }
+    block -= edgeBlocks;
+    // XCD-aware: workgroup b runs on XCD b % 8, which sweeps one contiguous band of the map, so the
+    // stencil rows its waves share stay in its L2
+    const int per = (tableBlocks + kXcdCount - 1) / kXcdCount;
+    const int e = (block % kXcdCount) * per + block / kXcdCount;
+    if (e >= tableBlocks) return;
+    const int2 blk = (kFluid ? c.fluidBlocks : c.collideBlocks)[e];
+    const int m = fluid_wave<kPass>(c, SS[wave], blk.x, blk.y + wave);
     // (rare: its parameters are read again, so that the waves above do not carry them)
-    for (int m = walk.x; m < walk.y; m += 64) walk_alone<kFluid>(c, wi, m);
+    if (m >= 0) walk_alone<kFluid>(c, blk.x, m);
 }
 
 // The particles' stage goes with the first launch.  A set with collision worlds but no bond work at all still

@@ -946,6 +946,20 @@ void WorldSet::buildTables() {
     };
     fluidShift_ = shift(fluidCells);
     collideShift_ = shift(collideCells);
+    auto units = [&](bool fluid) {
+        int n = 1;
+        auto waves = [&] {
+            int64_t sum = 0;
+            for (size_t wi = 0; wi < worlds_.size(); ++wi)
+                if (active_[wi] && worlds_[wi].numCells > 0 && (params_[wi].motion == 0) == fluid)
+                    sum += int64_t(kEdgeWaves) * (worlds_[wi].nby / n + 1);
+            return sum;
+        };
+        while (n < kEdgeUnitsMost && waves() > kEdgeWavesMost) n *= 2;
+        return n;
+    };
+    edgeUnits_ = units(true);
+    collideEdgeUnits_ = units(false);
     bool bondWork = false;
     for (int wi = 0; wi < int(worlds_.size()); ++wi) bondWork = bondWork || (active_[wi] && bondWork_[wi] && worlds_[wi].numCells > 0);
     for (int wi = 0; wi < int(worlds_.size()); ++wi) {
@@ -959,7 +973,7 @@ void WorldSet::buildTables() {
         if (w.numCells > 0) {  // waves of the neighbour passes, see k_neighbor.hip
             const bool fluid = params_[wi].motion == 0;
             const int waves = (w.numCells >> (fluid ? fluidShift_ : collideShift_)) + 3;
-            const int edgeWaves = (fluid && !bondWork ? kEdgeWaves : kEdgeWavesBonds) * (w.nby + 1);
+            const int edgeWaves = kEdgeWaves * (w.nby / (fluid ? edgeUnits_ : collideEdgeUnits_) + 1);
             for (int s = 0; s < edgeWaves; s += ct / 64) (fluid ? edges : collideEdges).push_back(make_int2(wi, s));
             for (int s = 0; s < waves; s += ct / 64) (fluid ? fluids : collides).push_back(make_int2(wi, s));
         }
@@ -1183,6 +1197,8 @@ Ctx WorldSet::makeCtx(int parity) const {
     c.collideBlocks = collideBlocks_;
     c.collideEdgeBlocks = collideEdgeBlocks_;
     c.collideShift = collideShift_;
+    c.edgeUnits = edgeUnits_;
+    c.collideEdgeUnits = collideEdgeUnits_;
     c.numPartBlocks = numPartBlocks_;
     c.partBlockParticles = shape_.partThreads;
     c.blockThreads = shape_.cellThreads;

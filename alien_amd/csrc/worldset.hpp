@@ -296,6 +296,7 @@ private:
     int fluidShift_ = 6;
     int2 *collideEdgeBlocks_ = nullptr, *collideBlocks_ = nullptr;
     int collideShift_ = 6;
+    int edgeUnits_ = 1, collideEdgeUnits_ = 1;
     int* numPartBlocks_ = nullptr;  // (device) entries of partBlocks_
     std::vector<uint8_t> bondWork_;  // per world: a bonded or barrier cell exists or can appear by fusion
     std::vector<uint8_t> active_;    // per world: included in the launch tables

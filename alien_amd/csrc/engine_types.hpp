@@ -22,7 +22,13 @@ constexpr int kClaimFree = 0x7fffffff;
 // 1 to 9 from the bin around in that direction, kFarCode from further
 constexpr int kMoveShift = 28;
 constexpr uint32_t kBinMask = (1u << kMoveShift) - 1u, kFarCode = 15u, kFarMove = kFarCode << kMoveShift;
-constexpr int kGroupBins = 256;    // bins per wave of the cells' map; a world's bins are padded to a multiple
+// Bins per wave of the cells' map (a group): 256, in sets with more than kDenseBins cells per bin 64, with twice that
+// 16 (Ctx::groupShift).  With many cells to a bin there are few bins, and a wave goes over the cells of its own and
+// of the rows next to them: 262k cells at nine to a bin, 114 waves for the whole map, 173 us of a step of 329 with
+// 256, 251 with 64, 224 with 16; at four to a bin 76, 58 and 55; at 16 to a bin 286, 250 and 236.  At one to a bin
+// the groups' sums cost more: 4M cells 151 us with 256, 190 with 64; 0.84M in bodies 224 and 235.
+// A world's bins are padded to a multiple of kGroupBins.
+constexpr int kGroupBins = 256, kDenseBins = 3;
 constexpr int kBinOfPad = 576;     // entries of binOf that may be read (and not used) past the last cell
 constexpr int kSuperGroups = 256;  // groups per sum of groups
 // Cells per wave of the fluid pass, as a power of two: 64, and in sets with fewer than a wave per SIMD (1024)
@@ -183,7 +189,7 @@ constexpr int kFarWalk = 16;
 struct FarCells {
     int* head;   // [numCellBins] one of the bin's, kNone without any; Ctx::farLink goes on
     int* count;  // [numCellBins]
-    int* group;  // [numCellBins / kGroupBins] whether the group's bins have any
+    int* group;  // [groups] whether the group's bins have any
     int* total;  // entries in the list
     int2* list;  // (global bin, part); one array for both steps: read before it is written
 };
@@ -231,7 +237,8 @@ struct Ctx {
     int numCellBins;      // cell bins of all worlds, each world's padded to a multiple of kGroupBins
     int cellCount;        // cells of all worlds
     const int* groupWorld;  // [numCellBins / kGroupBins] the bins' world
-    // Cells that groups of kGroupBins cell bins, and kSuperGroups of those, gained (or lost) since the
+    int groupShift;         // 1 << groupShift bins per group of the map: 8, 6 or 4
+    // Cells that the groups of cell bins, and kSuperGroups of those, gained (or lost) since the
     // last map; ...Next: for the next step (built during this step)
     int* groupSum;
     int* groupSumNext;

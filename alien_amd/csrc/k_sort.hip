@@ -41,16 +41,19 @@ __global__ void k_cell_bin(Ctx c) {
     cell_bin_xy(w, to_f2(c.A.pos[i]), bx, by);
     const int gb = w.binOff + by * w.nbx + bx;
     c.binOf[i] = int(uint32_t(gb - w.binOff) | kFarMove);
-    list_far(c.far, c.farLink, gb, i);
+    list_far(c.far, c.groupShift, c.farLink, gb, i);
 }
 
-// (the groups gain their far cells; a wave each)
+// (the groups gain their far cells; a wave for 256 bins)
 __global__ void k_seed_sums(Ctx c) {
-    const int g = (int(blockIdx.x) * int(blockDim.x) + int(threadIdx.x)) / 64, lane = int(threadIdx.x) & 63;
-    if (g >= c.numCellBins / kGroupBins) return;
-    const int4 n = reinterpret_cast<const int4*>(c.far.count + g * kGroupBins)[lane];
-    const int sum = wave_last(int(wave_inclusive_scan(uint32_t(n.x + n.y + n.z + n.w))));
-    if (lane != 0) return;
+    const int g0 = (int(blockIdx.x) * int(blockDim.x) + int(threadIdx.x)) / 64 * kGroupBins, lane = int(threadIdx.x) & 63;
+    if (g0 >= c.numCellBins) return;
+    const int4 n = reinterpret_cast<const int4*>(c.far.count + g0)[lane];
+    const int lanes = (1 << c.groupShift) / 4;
+    int sum = n.x + n.y + n.z + n.w;
+    for (int o = 1; o < lanes; o *= 2) sum += __shfl_xor(sum, o, 64);
+    if (lane % lanes != 0) return;
+    const int g = (g0 + 4 * lane) >> c.groupShift;
     c.groupSum[g] = sum;
     if (sum) atomicAdd(&c.superSum[g / kSuperGroups], sum);
 }
@@ -269,25 +272,25 @@ constexpr int kScatterRounds = 5;  // rounds of a stretch loaded at once (258 bi
 constexpr int kFarBlocks = 256;    // workgroups for the bins with many far cells, at most
 static_assert(kGroupBins == 4 * 64, "four bins per lane");
 
-struct ScatterShared {
-    int prev[kGroupBins + 4];  // places in the last map, counted from the world's first cell
+template <int kBins> struct ScatterShared {
+    int prev[kBins + 4];  // places in the last map, counted from the world's first cell
     union {
-        int start[kGroupBins + 4];  // the same in the new map
-        uint32_t out[kGroupBins];   // before it is known: cells that left the bin
+        int start[kBins + 4];  // the same in the new map
+        uint32_t out[kBins];   // before it is known: cells that left the bin
     };
-    uint32_t before[kGroupBins], after[kGroupBins];  // near movers into the bin from lower and higher places
+    uint32_t before[kBins], after[kBins];  // near movers into the bin from lower and higher places
     union {
         int2 list[kScatterList];   // (A index in the world, bin)
         struct {                   // the other run
-            uint32_t met[kGroupBins];   // movers placed so far
-            uint16_t turn[kGroupBins];  // lane whose turn it is
+            uint32_t met[kBins];   // movers placed so far
+            uint16_t turn[kBins];  // lane whose turn it is
         } run;
     };
 };
 
 // cells that the world's groups before global group g gained since the last map
 __device__ __forceinline__ int gained_before(const Ctx& c, const DevWorld& w, int g, int lane) {
-    const int first = w.binOff / kGroupBins;
+    const int first = w.binOff >> c.groupShift;
     const int s0 = (first + kSuperGroups - 1) / kSuperGroups, s1 = g / kSuperGroups;
     int n = 0;
     if (s0 < s1) {
@@ -302,14 +305,16 @@ __device__ __forceinline__ int gained_before(const Ctx& c, const DevWorld& w, in
 
 // the next step's sums, and the far lists of the group's bins where there are any, start empty (their last
 // readers ran a step ago)
-__device__ __forceinline__ void clear_next(const Ctx& c, int g, int lane) {
+template <int kBins> __device__ __forceinline__ void clear_next(const Ctx& c, int g, int lane) {
     if (lane == 0) {
         c.groupSumNext[g] = 0;
         if (g % kSuperGroups == 0) c.superSumNext[g / kSuperGroups] = 0;
     }
     if (c.farNext.group[g] == 0) return;
-    reinterpret_cast<int4*>(c.farNext.count + g * kGroupBins)[lane] = make_int4(0, 0, 0, 0);
-    reinterpret_cast<int4*>(c.farNext.head + g * kGroupBins)[lane] = make_int4(kNone, kNone, kNone, kNone);
+    if (lane < kBins / 4) {
+        reinterpret_cast<int4*>(c.farNext.count + g * kBins)[lane] = make_int4(0, 0, 0, 0);
+        reinterpret_cast<int4*>(c.farNext.head + g * kBins)[lane] = make_int4(kNone, kNone, kNone, kNone);
+    }
     if (lane == 0) c.farNext.group[g] = 0;
 }
 
@@ -326,7 +331,7 @@ __device__ __forceinline__ void place_cell(const Ctx& c, const DevWorld& w, int 
 }
 
 // The far cells of bins with more than kFarWalk: one wave per entry, 64 of a bin's list
-__device__ __forceinline__ void far_scatter(const Ctx& c, int wave, int waves, int lane) {
+template <int kBins> __device__ __forceinline__ void far_scatter(const Ctx& c, int wave, int waves, int lane) {
     const int total = *c.far.total;
     for (int q = wave; q < total; q += waves) {
         const int2 entry = c.far.list[q];
@@ -337,13 +342,13 @@ __device__ __forceinline__ void far_scatter(const Ctx& c, int wave, int waves, i
         int own = kNone, rank = 0;
         for (int j = c.far.head[gb], n = 0; j != kNone && n < first + 64; j = c.farLink[j], ++n) own = n - first == lane ? j : own;
         for (int j = c.far.head[gb]; j != kNone; j = c.farLink[j]) rank += j < own ? 1 : 0;
-        const int g = gb / kGroupBins, b0 = g * kGroupBins - w.binOff;
+        const int g = gb / kBins, b0 = g * kBins - w.binOff;
         const uint32_t t = uint32_t(gb - w.binOff - b0);
         const int i = own - w.cellOff;
         const uint32_t* prev = c.startPrev + w.binOff;
-        const Places p = places_of(reach_of(w, b0, min(kGroupBins, w.nbx * w.nby - b0)), prev);
+        const Places p = places_of(reach_of(w, b0, min(kBins, w.nbx * w.nby - b0)), prev);
         const int* binOf = c.binOf + w.cellOff;
-        const int4 fc = reinterpret_cast<const int4*>(c.far.count + g * kGroupBins)[lane];
+        const int4 fc = lane < kBins / 4 ? reinterpret_cast<const int4*>(c.far.count + g * kBins)[lane] : make_int4(0, 0, 0, 0);
         const int base = int(prev[b0] - prev[0]) + gained_before(c, w, g, lane);
         const uint32_t b = uint32_t(4 * lane);
         // cells of the group's bins before this one, and the bin's near cells before the lane's
@@ -398,26 +403,28 @@ template <int kMax> __device__ __forceinline__ void merge_far(int* seg, const in
         if (s < k) seg[m + to[s]] = f[s];
 }
 
-__device__ __forceinline__ void cell_scatter(const Ctx& c, ScatterShared& S, int g, int lane) {
-    const int g0 = g * kGroupBins;
+template <int kBins>
+__device__ __forceinline__ void cell_scatter(const Ctx& c, ScatterShared<kBins>& S, int g, int lane) {
+    const bool binLane = lane < kBins / 4;  // (four bins each)
+    const int g0 = g * kBins;
     if (g0 >= c.numCellBins) return;
     const DevWorld& w = c.worlds[world_of(c, g0)];
     const int b0 = g0 - w.binOff, bins = w.nbx * w.nby;
     const uint32_t* prev = c.startPrev + w.binOff;
     const int prevBase = int(prev[0]);
-    const uint4 pv = *reinterpret_cast<const uint4*>(prev + b0 + 4 * lane);
-    const uint32_t pvEnd = prev[b0 + kGroupBins];
+    const uint4 pv = binLane ? *reinterpret_cast<const uint4*>(prev + b0 + 4 * lane) : make_uint4(0u, 0u, 0u, 0u);
+    const uint32_t pvEnd = prev[b0 + kBins];
     uint4* startOut = reinterpret_cast<uint4*>(c.start + g0) + lane;
-    const bool last = g0 + kGroupBins == c.numCellBins;  // its end is stored too
-    clear_next(c, g, lane);
+    const bool last = g0 + kBins == c.numCellBins;  // its end is stored too
+    clear_next<kBins>(c, g, lane);
     if (!w.active || b0 >= bins) {
         // a world left out keeps its map; padding ends with the world
         const uint32_t d = uint32_t(w.cellOff - prevBase), end = uint32_t(w.cellOff + w.numCells);
-        *startOut = w.active ? make_uint4(end, end, end, end) : make_uint4(pv.x + d, pv.y + d, pv.z + d, pv.w + d);
+        if (binLane) *startOut = w.active ? make_uint4(end, end, end, end) : make_uint4(pv.x + d, pv.y + d, pv.z + d, pv.w + d);
         if (last && lane == 0) c.start[c.numCellBins] = end;
         return;
     }
-    const int nb = min(kGroupBins, bins - b0);
+    const int nb = min(kBins, bins - b0);
     const int p0 = int(prev[b0]) - prevBase, p1 = int(prev[b0 + nb]) - prevBase;  // the bins' own cells
     const Places p = places_of(reach_of(w, b0, nb), prev);
     const bool farCells = c.far.group[g] != 0;
@@ -427,12 +434,14 @@ __device__ __forceinline__ void cell_scatter(const Ctx& c, ScatterShared& S, int
     int x[3][kScatterRounds];
 #pragma unroll
     for (int k = 0; k < 3; ++k) load_rounds(binOf, p.s[k], p.e[k], lane, x[k]);
-    reinterpret_cast<int4*>(S.prev)[lane] =
-        make_int4(int(pv.x) - prevBase, int(pv.y) - prevBase, int(pv.z) - prevBase, int(pv.w) - prevBase);
-    if (lane == 0) S.prev[kGroupBins] = int(pvEnd) - prevBase;
-    reinterpret_cast<uint4*>(S.out)[lane] = make_uint4(0u, 0u, 0u, 0u);
-    reinterpret_cast<uint4*>(S.before)[lane] = make_uint4(0u, 0u, 0u, 0u);
-    reinterpret_cast<uint4*>(S.after)[lane] = make_uint4(0u, 0u, 0u, 0u);
+    if (binLane) {
+        reinterpret_cast<int4*>(S.prev)[lane] =
+            make_int4(int(pv.x) - prevBase, int(pv.y) - prevBase, int(pv.z) - prevBase, int(pv.w) - prevBase);
+        reinterpret_cast<uint4*>(S.out)[lane] = make_uint4(0u, 0u, 0u, 0u);
+        reinterpret_cast<uint4*>(S.before)[lane] = make_uint4(0u, 0u, 0u, 0u);
+        reinterpret_cast<uint4*>(S.after)[lane] = make_uint4(0u, 0u, 0u, 0u);
+    }
+    if (lane == 0) S.prev[kBins] = int(pvEnd) - prevBase;
     __syncwarp();
     int listed = 0;  // movers into the bins so far (listed up to the list's size)
     // cells i0 + lane of the stretch around the bins (k == 1), above or below: what they recorded
@@ -448,7 +457,7 @@ __device__ __forceinline__ void cell_scatter(const Ctx& c, ScatterShared& S, int
             } else {  // the last bin that starts at or before the cell
                 old = 0;
 #pragma unroll
-                for (int s = kGroupBins / 2; s > 0; s >>= 1)
+                for (int s = kBins / 2; s > 0; s >>= 1)
                     if (S.prev[old + s] <= i) old += s;
             }
             atomicAdd(&S.out[old], 1u);
@@ -476,24 +485,29 @@ __device__ __forceinline__ void cell_scatter(const Ctx& c, ScatterShared& S, int
     __syncwarp();
     // sizes and offsets
     {
-        const uint4 o = reinterpret_cast<const uint4*>(S.out)[lane];
-        const uint4 f = reinterpret_cast<const uint4*>(S.before)[lane], a = reinterpret_cast<const uint4*>(S.after)[lane];
-        const int next = S.prev[4 * lane + 4];
-        uint32_t v[4] = {pv.y - pv.x - o.x + f.x + a.x, pv.z - pv.y - o.y + f.y + a.y, pv.w - pv.z - o.z + f.z + a.z,
-                         uint32_t(next + prevBase) - pv.w - o.w + f.w + a.w};
+        uint32_t v[4] = {0u, 0u, 0u, 0u};
+        if (binLane) {
+            const uint4 o = reinterpret_cast<const uint4*>(S.out)[lane];
+            const uint4 f = reinterpret_cast<const uint4*>(S.before)[lane], a = reinterpret_cast<const uint4*>(S.after)[lane];
+            const int next = S.prev[4 * lane + 4];
+            v[0] = pv.y - pv.x - o.x + f.x + a.x, v[1] = pv.z - pv.y - o.y + f.y + a.y;
+            v[2] = pv.w - pv.z - o.z + f.z + a.z, v[3] = uint32_t(next + prevBase) - pv.w - o.w + f.w + a.w;
+        }
         if (farCells) {
-            const int4 fc = *reinterpret_cast<const int4*>(c.far.count + g0 + 4 * lane);
+            const int4 fc = binLane ? *reinterpret_cast<const int4*>(c.far.count + g0 + 4 * lane) : make_int4(0, 0, 0, 0);
             manyFar = __any(max(max(fc.x, fc.y), max(fc.z, fc.w)) > kFarWalk);
             v[0] += uint32_t(fc.x), v[1] += uint32_t(fc.y), v[2] += uint32_t(fc.z), v[3] += uint32_t(fc.w);
         }
         const uint32_t sum = v[0] + v[1] + v[2] + v[3];
         const int s0 = base + int(wave_inclusive_scan(sum) - sum);
         const int4 s = make_int4(s0, s0 + int(v[0]), s0 + int(v[0] + v[1]), s0 + int(v[0] + v[1] + v[2]));
-        reinterpret_cast<int4*>(S.start)[lane] = s;
         const uint32_t off = uint32_t(w.cellOff);
-        *startOut = make_uint4(off + uint32_t(s.x), off + uint32_t(s.y), off + uint32_t(s.z), off + uint32_t(s.w));
+        if (binLane) {
+            reinterpret_cast<int4*>(S.start)[lane] = s;
+            *startOut = make_uint4(off + uint32_t(s.x), off + uint32_t(s.y), off + uint32_t(s.z), off + uint32_t(s.w));
+        }
         if (lane == 63) {
-            S.start[kGroupBins] = s0 + int(sum);
+            S.start[kBins] = s0 + int(sum);
             if (last) c.start[c.numCellBins] = off + uint32_t(w.numCells);
         }
     }
@@ -572,8 +586,10 @@ __device__ __forceinline__ void cell_scatter(const Ctx& c, ScatterShared& S, int
             if (on) place_mover(m.x, m.y, n);
         }
     } else {
-        reinterpret_cast<uint4*>(S.run.met)[lane] = make_uint4(0u, 0u, 0u, 0u);
-        reinterpret_cast<uint2*>(S.run.turn)[lane] = make_uint2(~0u, ~0u);
+        if (binLane) {
+            reinterpret_cast<uint4*>(S.run.met)[lane] = make_uint4(0u, 0u, 0u, 0u);
+            reinterpret_cast<uint2*>(S.run.turn)[lane] = make_uint2(~0u, ~0u);
+        }
         __syncwarp();
         for (int k = 0; k < 3; ++k)
             for (int i0 = p.s[k]; i0 < p.e[k]; i0 += 64) {
@@ -600,7 +616,7 @@ __device__ __forceinline__ void cell_scatter(const Ctx& c, ScatterShared& S, int
                 __syncwarp();
             }
     }
-    if (farCells) {
+    if (farCells && binLane) {
         __threadfence_block();  // (the near cells' places)
         const int4 fc = *reinterpret_cast<const int4*>(c.far.count + g0 + 4 * lane);
         const int4 head = *reinterpret_cast<const int4*>(c.far.head + g0 + 4 * lane);
@@ -634,9 +650,10 @@ __global__ void __launch_bounds__(kMapThreads) k_part_scan(Ctx c, int tiles) { p
 // stagedBlocks the cells' emitted ones).  It opens the
 // step: clears the per-step list counters and advances the worlds' timesteps if asked (a step without
 // bond work has no later reader of them).
+template <int kBins>
 __global__ void __launch_bounds__(kMapThreads)
 k_map(Ctx c, int scanTiles, int partBlocks, int stagedBlocks, int groupBlocks, int farBlocks, StepCounters* open, int advance) {
-    __shared__ __align__(16) ScatterShared S[kMapWaves];
+    __shared__ __align__(16) ScatterShared<kBins> S[kMapWaves];
     int b = int(blockIdx.x);
     const int tid = int(threadIdx.x), lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = int(blockDim.x) >> 6;
@@ -651,11 +668,11 @@ k_map(Ctx c, int scanTiles, int partBlocks, int stagedBlocks, int groupBlocks, i
     }
     if (b < scanTiles) return part_scan(c, scanTiles);
     b -= scanTiles;
-    if (b < groupBlocks) return cell_scatter(c, S[wave], xcd_run(b, groupBlocks) * waves + wave, lane);
+    if (b < groupBlocks) return cell_scatter<kBins>(c, S[wave], xcd_run(b, groupBlocks) * waves + wave, lane);
     b -= groupBlocks;
     if (b < partBlocks + stagedBlocks) return particles_to_bins(c, b, partBlocks);
     b -= partBlocks + stagedBlocks;
-    if (b < farBlocks) far_scatter(c, b * waves + wave, farBlocks * waves, lane);
+    if (b < farBlocks) far_scatter<kBins>(c, b * waves + wave, farBlocks * waves, lane);
 }
 
 void launch_fill_u32(uint32_t* p, uint32_t v, size_t n, hipStream_t s) {
@@ -670,9 +687,9 @@ void launch_seed_bins(const Ctx& c, const LaunchShape& sh, hipStream_t s) {
     launch_fill_u32(const_cast<uint32_t*>(c.startPrev), 0u, size_t(c.numBins) + 1, s);
     launch_fill_u32(reinterpret_cast<uint32_t*>(c.far.head), uint32_t(kNone), size_t(c.numCellBins), s);
     launch_fill_u32(reinterpret_cast<uint32_t*>(c.far.count), 0u, size_t(c.numCellBins), s);
-    launch_fill_u32(reinterpret_cast<uint32_t*>(c.far.group), 0u, size_t(c.numCellBins / kGroupBins), s);
+    launch_fill_u32(reinterpret_cast<uint32_t*>(c.far.group), 0u, size_t(c.numCellBins >> c.groupShift), s);
     launch_fill_u32(reinterpret_cast<uint32_t*>(c.far.total), 0u, 1, s);
-    launch_fill_u32(reinterpret_cast<uint32_t*>(c.superSum), 0u, size_t(c.numCellBins / kGroupBins / kSuperGroups + 1), s);
+    launch_fill_u32(reinterpret_cast<uint32_t*>(c.superSum), 0u, size_t((c.numCellBins >> c.groupShift) / kSuperGroups + 1), s);
     if (sh.cellBlocks) hipLaunchKernelGGL(k_cell_bin, dim3(sh.cellBlocks), dim3(sh.cellThreads), 0, s, c);
     if (c.numCellBins) hipLaunchKernelGGL(k_seed_sums, dim3(c.numCellBins / kGroupBins / 4 + 1), dim3(256), 0, s, c);
     if (sh.partBlocks) hipLaunchKernelGGL(k_part_bin, dim3(sh.partGrid), dim3(sh.partThreads), 0, s, c);
@@ -688,15 +705,18 @@ void launch_map(const Ctx& c, const LaunchShape& sh, hipStream_t s, bool chain, 
     const bool particles = sh.hasParticles && sh.partBlocks;
     const int tiles = particles ? map_scan_tiles(c.numBins - c.numCellBins) : 0;
     const int threads = sh.cellThreads, waves = threads / 64;
-    const int blocks = c.cellCount > 0 ? (c.numCellBins / kGroupBins + waves - 1) / waves : 0;
+    const int blocks = c.cellCount > 0 ? ((c.numCellBins >> c.groupShift) + waves - 1) / waves : 0;
     const int groups = (blocks + kXcdCount - 1) / kXcdCount * kXcdCount;
     const int far = std::min(64 * sh.cellBlocks, kFarBlocks);
     const bool with = chain && threads == kMapThreads;  // (the scan's tiles are of kMapThreads)
     if (!with && tiles) hipLaunchKernelGGL(k_part_scan, dim3(tiles), dim3(kMapThreads), 0, s, c, tiles);
     const int scan = with ? tiles : 0, parts = particles && !chain ? sh.partGrid : 0;
     const int staged = particles && !chain && c.partStage > 0 ? sh.cellBlocks : 0;
-    hipLaunchKernelGGL(k_map, dim3(std::max(scan + groups + parts + staged + far, 1)), dim3(threads), 0, s, c, scan, parts, staged,
-                       groups, far, open, advanceTimestep ? 1 : 0);
+    const auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(std::max(scan + groups + parts + staged + far, 1)), dim3(threads), 0, s, c, scan, parts,
+                           staged, groups, far, open, advanceTimestep ? 1 : 0);
+    };
+    c.groupShift == 8 ? run(k_map<256>) : (c.groupShift == 6 ? run(k_map<64>) : run(k_map<16>));
 }
 
 void launch_part_scatter(const Ctx& c, const LaunchShape& sh, hipStream_t s) {

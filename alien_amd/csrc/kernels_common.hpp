@@ -65,10 +65,10 @@ __device__ __forceinline__ int cell_bin_of(const DevWorld& w, f2 p) {
 
 // enters cell k in the far list of global bin gb; the bin's parts are listed once it has more than a lane merges
 // in (k_sort.hip)
-__device__ __forceinline__ void list_far(const FarCells& f, int* next, int gb, int k) {
+__device__ __forceinline__ void list_far(const FarCells& f, int groupShift, int* next, int gb, int k) {
     next[k] = atomicExch(&f.head[gb], k);
     const int n = atomicAdd(&f.count[gb], 1);
-    f.group[gb / kGroupBins] = 1;
+    f.group[gb >> groupShift] = 1;
     if (n == kFarWalk || (n > kFarWalk && n % 64 == 0)) f.list[atomicAdd(f.total, 1)] = make_int2(gb, n / 64);
 }
 
@@ -124,9 +124,9 @@ __device__ __forceinline__ void bin_next(const Ctx& c, const DevWorld& w, int k,
         move = uint32_t(3 * (y + 1) + x + 2);
         if (x < -1 || x > 1) {
             move = kFarCode;
-            list_far(c.farNext, c.farLink, w.binOff + b, k);
+            list_far(c.farNext, c.groupShift, c.farLink, w.binOff + b, k);
         }
-        const int from = (w.binOff + bOld) / kGroupBins, to = (w.binOff + b) / kGroupBins;
+        const int from = (w.binOff + bOld) >> c.groupShift, to = (w.binOff + b) >> c.groupShift;
         if (from != to) shift_groups(c.groupSumNext, c.superSumNext, from, to);
     }
     st32(c.binOf, uint32_t(k), int(uint32_t(b) | move << kMoveShift));

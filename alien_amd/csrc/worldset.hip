@@ -659,7 +659,10 @@ void WorldSet::build(const std::vector<Source>& sources) {
         }
     };
     const size_t NCB = size_t(std::max(cellBins, 1));
-    const size_t groups = NCB / kGroupBins + 1, supers = groups / kSuperGroups + 1;
+    int64_t usedBins = 1;
+    for (const DevWorld& w : worlds) usedBins += int64_t(w.nbx) * w.nby;
+    groupShift_ = cellOff <= kDenseBins * usedBins ? 8 : (cellOff <= 2 * kDenseBins * usedBins ? 6 : 4);
+    const size_t groups = (NCB >> groupShift_) + 1, supers = groups / kSuperGroups + 1;
     bool anyExtra = false;
     for (const auto& h : hosts) anyExtra = anyExtra || h.hasExtra;
     selected_.assign(hosts.size(), nullptr);
@@ -711,8 +714,8 @@ void WorldSet::build(const std::vector<Source>& sources) {
             start_[b] = static_cast<uint32_t*>(A(sizeof(uint32_t) * (size_t(NB) + 1)));
             far_[b].head = static_cast<int*>(A(sizeof(int) * NCB));
             far_[b].count = static_cast<int*>(A(sizeof(int) * NCB));
-            far_[b].group = static_cast<int*>(A(sizeof(int) * (NCB / kGroupBins + 1)));
-            far_[b].total = far_[b].group + NCB / kGroupBins;
+            far_[b].group = static_cast<int*>(A(sizeof(int) * groups));
+            far_[b].total = far_[b].group + groups - 1;
             far_[b].list = farList_;
         }
         farLink_ = static_cast<int*>(A(sizeof(int) * NC));
@@ -899,7 +902,7 @@ void WorldSet::build(const std::vector<Source>& sources) {
         launch_fill_u32(start_[b], 0u, size_t(NB) + 1, stream_);
         launch_fill_u32(reinterpret_cast<uint32_t*>(far_[b].head), uint32_t(kNone), NCB, stream_);
         launch_fill_u32(reinterpret_cast<uint32_t*>(far_[b].count), 0u, NCB, stream_);
-        launch_fill_u32(reinterpret_cast<uint32_t*>(far_[b].group), 0u, NCB / kGroupBins + 1, stream_);
+        launch_fill_u32(reinterpret_cast<uint32_t*>(far_[b].group), 0u, groups, stream_);
     }
     launch_fill_u32(reinterpret_cast<uint32_t*>(fclaim_), uint32_t(kClaimFree), size_t(NP), stream_);
     launch_fill_u32(reinterpret_cast<uint32_t*>(cclaim_), uint32_t(kClaimFree), size_t(NC), stream_);
@@ -1135,6 +1138,7 @@ Ctx WorldSet::makeCtx(int parity) const {
     c.farNext = far_[parity ^ 1];
     c.farLink = farLink_;
     c.groupWorld = groupWorld_;
+    c.groupShift = groupShift_;
     c.groupSum = groupSum_[parity];
     c.groupSumNext = groupSum_[parity ^ 1];
     c.superSum = superSum_[parity];

@@ -273,6 +273,7 @@ private:
     int2* farList_ = nullptr;
     void* partArena_ = nullptr;  // the particles' arrays as built, null once they have grown
     int* groupWorld_ = nullptr;
+    int groupShift_ = 8;
     int* groupSum_[2] = {nullptr, nullptr};
     int* superSum_[2] = {nullptr, nullptr};
     int* farLink_ = nullptr;

@@ -50,3 +50,34 @@ def test_far_movers(name, motion):
         ref.step(steps)
         assert_identical(sim.get_data(), ref.get_data(), f"{name} after {steps} more steps")
     sim.close()
+
+
+# worlds of many cells to a bin, whose map's waves take 64 and 16 bins: cells per bin, bin edge, speed
+@pytest.mark.parametrize("motion", [MOTION_FLUID, MOTION_COLLISION])
+@pytest.mark.parametrize("size,per_bin,edge,speed", [((70, 66), 4, 2, 0.5), ((70, 66), 4, 2, 6.0), ((64, 512), 5, 2, 1.0),
+                                                     ((40, 42), 12, 2, 0.5), ((40, 42), 12, 2, 5.0), ((61, 57), 25, 3, 2.0),
+                                                     ((9, 300), 9, 3, 3.0), ((300, 9), 9, 3, 3.0), ((33, 35), 70, 3, 4.0)])
+def test_dense_maps(size, per_bin, edge, speed, motion):
+    print("dense map", size, per_bin, edge, speed, motion, flush=True)
+    n = per_bin * (size[0] // edge) * (size[1] // edge)
+    rng = np.random.default_rng(n + motion)
+    cells = H.cells(n)
+    cells["connections"]["cellIndex"] = 0
+    cells["pos"] = np.minimum((rng.uniform(0, 1, (n, 2)) * np.array(size)).astype(np.float32),
+                              np.nextafter(np.float32(size), np.float32(0)))
+    cells["vel"] = rng.normal(0, speed, (n, 2))
+    cells["maxConnections"] = 0
+    parts = H.particles(0)
+    worlds.assign_ids(cells, parts)
+    w = worlds.World("dense", size, H.params(motion, cellMaxVelocity=15.0, smoothingLength=edge / 2 - 0.1,
+                                             cellMaxCollisionDistance=edge - 0.2), cells, parts, 5, 3)
+    sim, ref = engine.Simulation.from_world(w), from_world(w, precision=32, threads=8)
+    for steps in (1, 1, 2):
+        sim.step(steps)
+        ref.step(steps)
+        assert_identical(sim.get_data(), ref.get_data(), f"{size} {per_bin} after {steps} more steps")
+    sim.get_map()  # (enters every cell anew)
+    sim.step(1)
+    ref.step(1)
+    assert_identical(sim.get_data(), ref.get_data(), f"{size} {per_bin} after introspection")
+    sim.close()

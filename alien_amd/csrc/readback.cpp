@@ -6,7 +6,6 @@
 #include <cstring>
 #include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -109,8 +108,8 @@ void read_records(size_t n, size_t size, void* out, hipStream_t s,
     for (size_t t = 1; t < workers; ++t) {
         try {
             others.emplace_back(work, true);
-        } catch (const std::system_error&) {
-            break;  // no more threads: the ones there are do the rest
+        } catch (...) {
+            break;  // no more threads, or no memory for one: the ones there are do the rest
         }
     }
     work(false);
@@ -139,8 +138,8 @@ void for_ranges(size_t n, const std::function<void(size_t, size_t)>& f) {
     for (; started < pieces; ++started) {
         try {
             others.emplace_back(work, started);
-        } catch (const std::system_error&) {
-            break;  // no more threads: the pieces left are done here
+        } catch (...) {
+            break;  // no more threads, or no memory for one: the pieces left are done here
         }
     }
     work(0);

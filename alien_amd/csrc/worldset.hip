@@ -1796,19 +1796,48 @@ void WorldSet::extract(int wi, WorldImage& img) {
     img.numParticles = int(img.ppos.size());
 }
 
+// The sums in index order, as a whole image of the world would give them; only what they add up is read.
 alien_totals WorldSet::totals(int wi) {
-    WorldImage img;
-    extract(wi, img);
+    const int np = counters(wi).numParticles;
+    const DevWorld& w = worlds_.at(wi);
+    const int n = w.numCells;
+    const HotBuffers& S = buf_[parity_];
+    auto read = [&](auto& out, const auto* from, int count) {
+        out.resize(size_t(count));
+        read_records(out.size(), sizeof(*from), out.data(), stream_, [&](size_t first, size_t c, void* to) {
+            check_hip(hipMemcpyAsync(to, from + first, c * sizeof(*from), hipMemcpyDeviceToHost, stream_), "D2H");
+        });
+    };
+    HostArray<float2> vel;
+    HostArray<float> energy, pen;
+    HostArray<int> slot;
+    HostArray<uint8_t> pflags;
+    HostArray<StagedParticle> halves;
+    read(vel, S.vel + w.cellOff, n);
+    read(slot, S.slot + w.cellOff, n);
+    read(energy, energy_ + w.cellOff, n);
+    read(pen, S.pen + w.partOff, np);
+    read(pflags, S.pflags + w.partOff, np);
+    if (splitStage_ > 0) read(halves, splitStaged_ + w.partOff, np);
     alien_totals t{};
-    for (int i = 0; i < img.host.numCells; ++i) {
-        t.cellEnergy += double(img.energy[img.slot[i]]);
-        t.momentum[0] += double(img.vel[i].x);
-        t.momentum[1] += double(img.vel[i].y);
-        t.kinetic += 0.5 * (double(img.vel[i].x) * double(img.vel[i].x) + double(img.vel[i].y) * double(img.vel[i].y));
+    for (size_t i = 0; i < size_t(n); ++i) {
+        t.cellEnergy += double(energy[size_t(slot[i])]);
+        t.momentum[0] += double(vel[i].x);
+        t.momentum[1] += double(vel[i].y);
+        t.kinetic += 0.5 * (double(vel[i].x) * double(vel[i].x) + double(vel[i].y) * double(vel[i].y));
     }
-    for (int i = 0; i < img.numParticles; ++i) t.particleEnergy += double(img.pen[i]);
-    t.numCells = uint64_t(img.host.numCells);
-    t.numParticles = uint64_t(img.numParticles);
+    // the living particles, then the halves that wait for the next map
+    for (size_t i = 0; i < size_t(np); ++i)
+        if (!(pflags[i] & kParticleDead)) {
+            t.particleEnergy += double(pen[i]);
+            ++t.numParticles;
+        }
+    for (const StagedParticle& r : halves)
+        if (r.color & kStagedPending) {
+            t.particleEnergy += double(r.energy);
+            ++t.numParticles;
+        }
+    t.numCells = uint64_t(n);
     return t;
 }
 

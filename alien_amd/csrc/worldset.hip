@@ -1796,29 +1796,26 @@ void WorldSet::extract(int wi, WorldImage& img) {
     img.numParticles = int(img.ppos.size());
 }
 
+// a device array through the pinned buffers
+template <class T> static HostArray<T> read_array(const T* from, int n, hipStream_t s) {
+    HostArray<T> out(static_cast<size_t>(n));
+    read_records(out.size(), sizeof(T), out.data(), s, [&](size_t first, size_t count, void* to) {
+        check_hip(hipMemcpyAsync(to, from + first, count * sizeof(T), hipMemcpyDeviceToHost, s), "D2H");
+    });
+    return out;
+}
+
 // The sums in index order, as a whole image of the world would give them; only what they add up is read.
 alien_totals WorldSet::totals(int wi) {
     const int np = counters(wi).numParticles;
     const DevWorld& w = worlds_.at(wi);
     const int n = w.numCells;
     const HotBuffers& S = buf_[parity_];
-    auto read = [&](auto& out, const auto* from, int count) {
-        out.resize(size_t(count));
-        read_records(out.size(), sizeof(*from), out.data(), stream_, [&](size_t first, size_t c, void* to) {
-            check_hip(hipMemcpyAsync(to, from + first, c * sizeof(*from), hipMemcpyDeviceToHost, stream_), "D2H");
-        });
-    };
-    HostArray<float2> vel;
-    HostArray<float> energy, pen;
-    HostArray<int> slot;
-    HostArray<uint8_t> pflags;
-    HostArray<StagedParticle> halves;
-    read(vel, S.vel + w.cellOff, n);
-    read(slot, S.slot + w.cellOff, n);
-    read(energy, energy_ + w.cellOff, n);
-    read(pen, S.pen + w.partOff, np);
-    read(pflags, S.pflags + w.partOff, np);
-    if (splitStage_ > 0) read(halves, splitStaged_ + w.partOff, np);
+    const auto vel = read_array(S.vel + w.cellOff, n, stream_);
+    const auto energy = read_array(energy_ + w.cellOff, n, stream_), pen = read_array(S.pen + w.partOff, np, stream_);
+    const auto slot = read_array(S.slot + w.cellOff, n, stream_);
+    const auto pflags = read_array(S.pflags + w.partOff, np, stream_);
+    const auto halves = read_array(splitStaged_ + w.partOff, splitStage_ > 0 ? np : 0, stream_);
     alien_totals t{};
     for (size_t i = 0; i < size_t(n); ++i) {
         t.cellEnergy += double(energy[size_t(slot[i])]);
@@ -1900,17 +1897,14 @@ void WorldSet::cellMap(int wi, std::vector<int>& bins, std::vector<int>& slots) 
     synchronize();
     const DevWorld& w = worlds_.at(wi);
     const int n = w.numCells;
-    std::vector<int> sorted(n), binOfAll(cellCap_), slotAll(cellCap_);
-    if (n) {
-        check_hip(hipMemcpy(sorted.data(), sorted_ + w.cellOff, sizeof(int) * n, hipMemcpyDeviceToHost), "D2H");
-        check_hip(hipMemcpy(binOfAll.data(), binOf_, sizeof(int) * cellCap_, hipMemcpyDeviceToHost), "D2H");
-        check_hip(hipMemcpy(slotAll.data(), buf_[parity_].slot, sizeof(int) * cellCap_, hipMemcpyDeviceToHost), "D2H");
-    }
+    const auto sorted = read_array(sorted_ + w.cellOff, n, stream_), binOf = read_array(binOf_ + w.cellOff, n, stream_);
+    const auto slot = read_array(buf_[parity_].slot + w.cellOff, n, stream_);
     bins.resize(n);
     slots.resize(n);
     for (int k = 0; k < n; ++k) {
-        bins[k] = int(uint32_t(binOfAll[sorted[k]]) & kBinMask);
-        slots[k] = slotAll[sorted[k]];
+        const size_t i = size_t(sorted[k] - w.cellOff);
+        bins[k] = int(uint32_t(binOf[i]) & kBinMask);
+        slots[k] = slot[i];
     }
 }
 

@@ -816,7 +816,7 @@ struct alien_server {
 extern "C" {
 
 uint64_t alien_server_estimate_bytes(uint64_t numCells, uint64_t numParticles, int32_t worldSizeX, int32_t worldSizeY) {
-    return WorldSet::estimateBytes(numCells, numParticles, worldSizeX, worldSizeY, 2);
+    return WorldSet::estimateBytes(numCells, numParticles, worldSizeX, worldSizeY, 2, false, false);
 }
 
 uint64_t alien_server_plan_admission(uint64_t budgetBytes, uint64_t oldSetBytes, uint64_t keptBytes,
@@ -868,7 +868,7 @@ int alien_server_submit(alien_server* s, const alien_world_desc* desc, const ali
         // (a radiating or splitting world is built with room for the particles it will create)
         job->bytes = WorldSet::estimateBytes(
             numCells, uint64_t(alien::particle_room(int64_t(numCells), int64_t(numParticles), *params)),
-            desc->worldSizeX, desc->worldSizeY, alien::bin_size_for(*params));
+            desc->worldSizeX, desc->worldSizeY, alien::bin_size_for(*params), alien::radiates(*params), alien::splits(*params));
         if (job->bytes > s->budget) throw Error(ALIEN_E_BUDGET, "job does not fit the device memory budget");
         job->submitTime = nowSeconds();
         std::lock_guard<std::mutex> lk(s->mu);

@@ -43,7 +43,7 @@ constexpr int kXcdCount = 8;  // XCDs of an MI355X: workgroup b of a launch runs
 // Size limits of one world set.  Cell indices, bin offsets and the bond planes ([kMaxBonds][cap],
 // addressed as b * cap + x) are 32-bit ints in the kernels, so a set holds at most
 // (2^31 - 1) / kMaxBonds cells; particle indices and the uint32 bin scan over cells plus particles
-// stay in range with at most 2^30 particles.  At ~470 B per bonded cell the cell limit is ~168 GB
+// stay in range with at most 2^30 particles.  At ~530 B per cell the cell limit is ~190 GB
 // of the 288 GB of HBM.
 constexpr int64_t kMaxSetCells = (int64_t(0x7fffffff)) / kMaxBonds;  // 357,913,941
 constexpr int64_t kMaxSetParticles = int64_t(1) << 30;

@@ -468,6 +468,8 @@ WorldSet::WorldSet() {
     hostSc_ = reinterpret_cast<StepCounters*>(reinterpret_cast<char*>(liveHost_) + 128);
 }
 
+WorldSet::WorldSet(SizesOnly) {}
+
 WorldSet::~WorldSet() {
     invalidateGraphs();
     if (stream_) (void)hipStreamSynchronize(stream_);
@@ -514,14 +516,45 @@ void WorldSet::invalidateGraphs() {
 
 void WorldSet::synchronize() { check_hip(hipStreamSynchronize(stream_), "hipStreamSynchronize"); }
 
-uint64_t WorldSet::estimateBytes(uint64_t cells, uint64_t particles, int W, int H, int binSize) {
-    const uint64_t perCell = 2 * (8 + 8 + 4 + 4 + 4 + kMaxBonds * 12) + 8 + 4 * 4 + 8 + 3 * 8 + 2 * kMaxBonds * 8 + 4 +
-                             2 + 8 + 4 * 16 + 4 + (8 + 8 + 4 + 4) + 4 + 4;
-    const uint64_t perParticle = 2 * (8 + 8 + 4 + 4 + 4 + 1 + 8) + 6 * 4;
-    const uint64_t bins = uint64_t(std::max(1, W / binSize)) * uint64_t(std::max(1, H / binSize)) +
-                          uint64_t(std::max(1, W / kParticleBin)) * uint64_t(std::max(1, H / kParticleBin));
-    // per bin: two histograms, two offset arrays, two far-list heads and counts (cell bins), sums
-    return cells * perCell + particles * perParticle + bins * 36 + (1u << 20);
+// entries of the fusion candidate list, which is the read-back's scratch as well
+static size_t cand_entries(size_t cells) { return std::max<size_t>(4 * cells, 4096); }
+
+// What a set of one such world takes: its layout, whose arrays grow in step with the cells, the particle slots
+// and the bins, taken at two sizes each; the read-back's sort where the candidate list is too small for it; the
+// launch tables (8 B for 64 elements or more, at most four tables of the cells).  A world that neither radiates
+// nor splits pays staging slots as well in a set with one that does: those are not counted.
+uint64_t WorldSet::estimateBytes(uint64_t cells, uint64_t particles, int W, int H, int binSize, bool radiation,
+                                 bool splitting) {
+    const size_t unit = size_t(1) << 20;
+    auto need = [&](size_t c, size_t p, size_t cellBins, size_t partBins) {
+        WorldSet s{SizesOnly()};
+        Sizes z;
+        z.worlds = 1;
+        z.cells = c;
+        z.cellBins = cellBins;
+        z.bins = cellBins + partBins;
+        z.groupShift = 4;
+        z.extra = true;
+        z.selected = {size_t(p)};
+        z.radStage = radiation;
+        z.splitSlots = splitting ? p : 0;
+        z.particles = p + z.splitSlots + (radiation ? c : 0);
+        Places a, b;
+        s.layout(z, a, b);
+        return uint64_t(a.used + b.used);
+    };
+    const uint64_t base = need(unit, unit, unit, unit);
+    const uint64_t perCell = need(2 * unit, unit, unit, unit) - base, perParticle = need(unit, 2 * unit, unit, unit) - base;
+    const uint64_t perCellBin = need(unit, unit, 2 * unit, unit) - base, perPartBin = need(unit, unit, unit, 2 * unit) - base;
+    auto scaled = [&](uint64_t n, uint64_t perUnit) { return n / unit * perUnit + n % unit * perUnit / unit; };
+    auto bins = [&](int size) { return uint64_t(std::max(1, W / size)) * uint64_t(std::max(1, H / size)); };
+    const uint64_t cellBins = (bins(binSize) + kGroupBins - 1) / kGroupBins * kGroupBins, partBins = bins(kParticleBin);
+    const uint64_t entries = splitting ? 2 * particles : particles;
+    const uint64_t sort = particles ? SortBuffers::bytes(entries) + sizeof(uint32_t) * (entries / kPartTile + 1) : 0;
+    const uint64_t cand = 4 * sizeof(int4) * cells;
+    return base - perCell - perParticle - perCellBin - perPartBin + scaled(cells, perCell) + scaled(particles, perParticle) +
+           scaled(cellBins, perCellBin) + scaled(partBins, perPartBin) + (sort > cand ? sort - cand : 0) +
+           (cells + particles + cellBins + partBins) + (1u << 20);
 }
 
 void WorldSet::clearAll() {
@@ -536,6 +569,92 @@ void WorldSet::clearAll() {
 }
 
 int stageLayout(int64_t caps, int cells, bool radiation, bool splitting, int& splitStage, int& radStage);
+
+// Everything comes from two allocations, one for the particles' arrays (which growParticles replaces) and one
+// for the rest: the layout runs once to add up the sizes and once to hand out the places.
+void WorldSet::layout(const Sizes& z, Places& A, Places& B) {
+    const size_t NC = z.cells, NP = z.particles, NB = z.bins, NCB = std::max<size_t>(z.cellBins, 1);
+    const size_t groups = (NCB >> z.groupShift) + 1, supers = groups / kSuperGroups + 1;
+    dWorlds_ = static_cast<DevWorld*>(A(sizeof(DevWorld) * std::max<size_t>(z.worlds, 1)));
+    dParams_ = static_cast<DevParams*>(A(sizeof(DevParams) * std::max<size_t>(z.worlds, 1)));
+    dCtr_ = static_cast<DevCounters*>(A(sizeof(DevCounters) * std::max<size_t>(z.worlds, 1)));
+    dSc_ = static_cast<StepCounters*>(A(sizeof(StepCounters)));
+    for (int b = 0; b < 2; ++b) {
+        HotBuffers& h = buf_[b];
+        h.pos = static_cast<float2*>(A(sizeof(float2) * NC));
+        h.vel = static_cast<float2*>(A(sizeof(float2) * NC));
+        h.dens = static_cast<float*>(A(sizeof(float) * NC));
+        h.flags = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
+        h.slot = static_cast<int*>(A(sizeof(int) * NC));
+        h.btgt = static_cast<int*>(A(sizeof(int) * kMaxBonds * NC));
+        h.brest = static_cast<float*>(A(sizeof(float) * kMaxBonds * NC));
+        h.bang = static_cast<float*>(A(sizeof(float) * kMaxBonds * NC));
+        h.ppos = static_cast<float2*>(B(sizeof(float2) * NP));
+        h.pvel = static_cast<float2*>(B(sizeof(float2) * NP));
+        h.pen = static_cast<float*>(B(sizeof(float) * NP));
+        h.plast = static_cast<int*>(B(sizeof(int) * NP));
+        h.pslot = static_cast<int*>(B(sizeof(int) * NP));
+        h.pflags = static_cast<uint8_t*>(B(NP));
+        h.pid = static_cast<unsigned long long*>(B(sizeof(unsigned long long) * NP));
+    }
+    energy_ = static_cast<float*>(A(sizeof(float) * NC));
+    stiff_ = static_cast<float*>(A(sizeof(float) * NC));
+    cid_ = static_cast<unsigned long long*>(A(sizeof(unsigned long long) * NC));
+    ageBase_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
+    rankOfSlot_ = static_cast<int*>(A(sizeof(int) * NC));
+    extra_ = z.extra ? static_cast<CellExtra*>(A(sizeof(CellExtra) * NC)) : nullptr;
+    selected_.assign(z.selected.size(), nullptr);
+    for (size_t w = 0; w < z.selected.size(); ++w)
+        if (z.selected[w]) selected_[w] = static_cast<uint8_t*>(A(z.selected[w]));
+    dWords_ = static_cast<unsigned long long*>(A(sizeof(unsigned long long) * 2));
+    staged_ = z.radStage ? static_cast<StagedParticle*>(A(sizeof(StagedParticle) * NC)) : nullptr;
+    splitStaged_ = z.splitSlots > 0 ? static_cast<StagedParticle*>(B(sizeof(StagedParticle) * z.splitSlots)) : nullptr;
+    living_[0] = static_cast<uint8_t*>(A(NC));
+    living_[1] = static_cast<uint8_t*>(A(NC));
+    activation_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
+    creature_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
+    stretched_ = static_cast<uint8_t*>(A(NC));
+    binOf_ = static_cast<int*>(A(sizeof(int) * (NC + kBinOfPad)));
+    pbinOf_ = static_cast<int*>(B(sizeof(int) * NP));
+    count_[0] = static_cast<uint32_t*>(A(sizeof(uint32_t) * NB));
+    count_[1] = static_cast<uint32_t*>(A(sizeof(uint32_t) * NB));
+    farList_ = static_cast<int2*>(A(sizeof(int2) * (NC / 8 + 1)));  // (17 or 64 cells for an entry)
+    for (int b = 0; b < 2; ++b) {
+        start_[b] = static_cast<uint32_t*>(A(sizeof(uint32_t) * (NB + 1)));
+        far_[b].head = static_cast<int*>(A(sizeof(int) * NCB));
+        far_[b].count = static_cast<int*>(A(sizeof(int) * NCB));
+        far_[b].group = static_cast<int*>(A(sizeof(int) * groups));
+        far_[b].total = far_[b].group + groups - 1;
+        far_[b].list = farList_;
+    }
+    farLink_ = static_cast<int*>(A(sizeof(int) * NC));
+    groupWorld_ = static_cast<int*>(A(sizeof(int) * NCB / kGroupBins + sizeof(int)));
+    for (int b = 0; b < 2; ++b) {
+        groupSum_[b] = static_cast<int*>(A(sizeof(int) * groups));
+        superSum_[b] = static_cast<int*>(A(sizeof(int) * supers));
+    }
+    mapStatus_ = static_cast<unsigned long long*>(A(sizeof(unsigned long long) * size_t(map_scan_tiles(int(NB - z.cellBins)) + 1)));
+    mapEpochTicket_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * 2));
+    sorted_ = static_cast<int*>(A(sizeof(int) * NC));
+    bonded_ = static_cast<float4*>(A(sizeof(float4) * NC));
+    psorted_ = static_cast<int*>(B(sizeof(int) * NP));
+    pcode_ = static_cast<uint8_t*>(B(NP));
+    stage_ = static_cast<uint8_t*>(A(NC));
+    own_ = static_cast<float2*>(A(sizeof(float2) * NC));
+    moved_ = static_cast<float4*>(A(sizeof(float4) * NC));
+    lists_ = static_cast<int4*>(A(2 * sizeof(int4) * NC));
+    bstiff_ = static_cast<float*>(A(sizeof(float) * NC));
+    s2_ = static_cast<float2*>(A(sizeof(float2) * NC));
+    out1_ = static_cast<float2*>(A(sizeof(float2) * kMaxBonds * NC));
+    out2_ = static_cast<float2*>(A(sizeof(float2) * kMaxBonds * NC));
+    valid_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
+    claim_ = static_cast<unsigned long long*>(A(sizeof(unsigned long long) * NC));
+    cand_ = static_cast<int4*>(A(sizeof(int4) * cand_entries(NC)));
+    want_ = static_cast<int*>(B(sizeof(int) * NP));
+    fclaim_ = static_cast<int*>(B(sizeof(int) * NP));
+    absorbCell_ = static_cast<int*>(B(sizeof(int) * NP));
+    cclaim_ = static_cast<int*>(A(sizeof(int) * NC));
+}
 
 void WorldSet::build(const std::vector<Source>& sources) {
     // collect the new layout first (sources may live in this very set's old buffers only via a
@@ -652,114 +771,33 @@ void WorldSet::build(const std::vector<Source>& sources) {
     cellCap_ = NC;
     partCap_ = NP;
     numBins_ = NB;
-    candCap_ = std::max(4 * NC, 4096);
-    // Everything comes from two allocations, one for the particles' arrays (which growParticles replaces) and
-    // one for the rest: the layout below runs once to add up the sizes and once to hand out the places.
-    struct Places {
-        char* base = nullptr;
-        size_t used = 0;
-        void* operator()(size_t bytes) {
-            char* p = base ? base + used : nullptr;
-            used += (std::max<size_t>(bytes, 64) + 255) & ~size_t(255);
-            return p;
-        }
-    };
+    candCap_ = int(cand_entries(size_t(NC)));
     const size_t NCB = size_t(std::max(cellBins, 1));
     int64_t usedBins = 1;
     for (const DevWorld& w : worlds) usedBins += int64_t(w.nbx) * w.nby;
     groupShift_ = cellOff <= kDenseBins * usedBins ? 8 : (cellOff <= 2 * kDenseBins * usedBins ? 6 : 4);
     const size_t groups = (NCB >> groupShift_) + 1, supers = groups / kSuperGroups + 1;
-    bool anyExtra = false;
-    for (const auto& h : hosts) anyExtra = anyExtra || h.hasExtra;
-    selected_.assign(hosts.size(), nullptr);
-    auto layout = [&](Places& A, Places& B) {
-        dWorlds_ = static_cast<DevWorld*>(A(sizeof(DevWorld) * std::max<size_t>(worlds.size(), 1)));
-        dParams_ = static_cast<DevParams*>(A(sizeof(DevParams) * std::max<size_t>(worlds.size(), 1)));
-        dCtr_ = static_cast<DevCounters*>(A(sizeof(DevCounters) * std::max<size_t>(worlds.size(), 1)));
-        dSc_ = static_cast<StepCounters*>(A(sizeof(StepCounters)));
-        for (int b = 0; b < 2; ++b) {
-            HotBuffers& h = buf_[b];
-            h.pos = static_cast<float2*>(A(sizeof(float2) * NC));
-            h.vel = static_cast<float2*>(A(sizeof(float2) * NC));
-            h.dens = static_cast<float*>(A(sizeof(float) * NC));
-            h.flags = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
-            h.slot = static_cast<int*>(A(sizeof(int) * NC));
-            h.btgt = static_cast<int*>(A(sizeof(int) * kMaxBonds * size_t(NC)));
-            h.brest = static_cast<float*>(A(sizeof(float) * kMaxBonds * size_t(NC)));
-            h.bang = static_cast<float*>(A(sizeof(float) * kMaxBonds * size_t(NC)));
-            h.ppos = static_cast<float2*>(B(sizeof(float2) * NP));
-            h.pvel = static_cast<float2*>(B(sizeof(float2) * NP));
-            h.pen = static_cast<float*>(B(sizeof(float) * NP));
-            h.plast = static_cast<int*>(B(sizeof(int) * NP));
-            h.pslot = static_cast<int*>(B(sizeof(int) * NP));
-            h.pflags = static_cast<uint8_t*>(B(NP));
-            h.pid = static_cast<unsigned long long*>(B(sizeof(unsigned long long) * NP));
-        }
-        energy_ = static_cast<float*>(A(sizeof(float) * NC));
-        stiff_ = static_cast<float*>(A(sizeof(float) * NC));
-        cid_ = static_cast<unsigned long long*>(A(sizeof(unsigned long long) * NC));
-        ageBase_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
-        extra_ = anyExtra ? static_cast<CellExtra*>(A(sizeof(CellExtra) * NC)) : nullptr;
-        for (size_t w = 0; w < hosts.size(); ++w)
-            if (hosts[w].hasSelected) selected_[w] = static_cast<uint8_t*>(A(hosts[w].cells->particleSelected.size()));
-        dWords_ = static_cast<unsigned long long*>(A(sizeof(unsigned long long) * 2));
-        staged_ = partStage_ > 0 ? static_cast<StagedParticle*>(A(sizeof(StagedParticle) * NC)) : nullptr;
-        splitStaged_ = splitStage_ > 0 ? static_cast<StagedParticle*>(B(sizeof(StagedParticle) * size_t(splitStage_))) : nullptr;
-        living_[0] = static_cast<uint8_t*>(A(NC));
-        living_[1] = static_cast<uint8_t*>(A(NC));
-        activation_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
-        creature_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
-        stretched_ = static_cast<uint8_t*>(A(NC));
-        binOf_ = static_cast<int*>(A(sizeof(int) * (size_t(NC) + kBinOfPad)));
-        pbinOf_ = static_cast<int*>(B(sizeof(int) * NP));
-        count_[0] = static_cast<uint32_t*>(A(sizeof(uint32_t) * NB));
-        count_[1] = static_cast<uint32_t*>(A(sizeof(uint32_t) * NB));
-        numCellBins_ = cellBins;
-        farList_ = static_cast<int2*>(A(sizeof(int2) * (size_t(NC) / 8 + 1)));  // (17 or 64 cells for an entry)
-        for (int b = 0; b < 2; ++b) {
-            start_[b] = static_cast<uint32_t*>(A(sizeof(uint32_t) * (size_t(NB) + 1)));
-            far_[b].head = static_cast<int*>(A(sizeof(int) * NCB));
-            far_[b].count = static_cast<int*>(A(sizeof(int) * NCB));
-            far_[b].group = static_cast<int*>(A(sizeof(int) * groups));
-            far_[b].total = far_[b].group + groups - 1;
-            far_[b].list = farList_;
-        }
-        farLink_ = static_cast<int*>(A(sizeof(int) * NC));
-        groupWorld_ = static_cast<int*>(A(sizeof(int) * NCB / kGroupBins + sizeof(int)));
-        for (int b = 0; b < 2; ++b) {
-            groupSum_[b] = static_cast<int*>(A(sizeof(int) * groups));
-            superSum_[b] = static_cast<int*>(A(sizeof(int) * supers));
-        }
-        mapStatus_ = static_cast<unsigned long long*>(A(sizeof(unsigned long long) * size_t(map_scan_tiles(NB - cellBins) + 1)));
-        mapEpochTicket_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * 2));
-        sorted_ = static_cast<int*>(A(sizeof(int) * NC));
-        bonded_ = static_cast<float4*>(A(sizeof(float4) * NC));
-        psorted_ = static_cast<int*>(B(sizeof(int) * NP));
-        pcode_ = static_cast<uint8_t*>(B(NP));
-        stage_ = static_cast<uint8_t*>(A(NC));
-        own_ = static_cast<float2*>(A(sizeof(float2) * NC));
-        moved_ = static_cast<float4*>(A(sizeof(float4) * NC));
-        lists_ = static_cast<int4*>(A(2 * sizeof(int4) * NC));
-        bstiff_ = static_cast<float*>(A(sizeof(float) * NC));
-        s2_ = static_cast<float2*>(A(sizeof(float2) * NC));
-        out1_ = static_cast<float2*>(A(sizeof(float2) * kMaxBonds * size_t(NC)));
-        out2_ = static_cast<float2*>(A(sizeof(float2) * kMaxBonds * size_t(NC)));
-        valid_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
-        claim_ = static_cast<unsigned long long*>(A(sizeof(unsigned long long) * NC));
-        cand_ = static_cast<int4*>(A(sizeof(int4) * size_t(candCap_)));
-        want_ = static_cast<int*>(B(sizeof(int) * NP));
-        fclaim_ = static_cast<int*>(B(sizeof(int) * NP));
-        absorbCell_ = static_cast<int*>(B(sizeof(int) * NP));
-        cclaim_ = static_cast<int*>(A(sizeof(int) * NC));
-    };
+    Sizes z;
+    z.worlds = worlds.size();
+    z.cells = size_t(NC);
+    z.particles = size_t(NP);
+    z.bins = size_t(NB);
+    z.cellBins = size_t(cellBins);
+    z.groupShift = groupShift_;
+    z.radStage = partStage_ > 0;
+    z.splitSlots = size_t(splitStage_);
+    for (const auto& h : hosts) {
+        z.extra = z.extra || h.hasExtra;
+        z.selected.push_back(h.hasSelected ? h.cells->particleSelected.size() : 0);
+    }
+    numCellBins_ = cellBins;
     {
         Places a, b;
-        layout(a, b);
+        layout(z, a, b);
         Places arena{static_cast<char*>(alloc(a.used))};
         Places parts{static_cast<char*>(partArena_ = alloc(b.used))};
-        layout(arena, parts);
+        layout(z, arena, parts);
     }
-    rankOfSlot_ = nullptr;
     rankState_.assign(hosts.size(), 0);
     idBits_.assign(hosts.size(), 0);
     scratch_ = nullptr;
@@ -1303,7 +1341,6 @@ void WorldSet::ensureRanks(int w) {
     if (rankState_.at(w)) return;
     const DevWorld& dw = worlds_.at(w);
     const int n = dw.numCells;
-    if (!rankOfSlot_) rankOfSlot_ = static_cast<int*>(alloc(sizeof(int) * size_t(cellCap_)));
     const SortBuffers b = SortBuffers::at(scratch(SortBuffers::bytes(size_t(n))), size_t(n));
     launch_fill_u32(reinterpret_cast<uint32_t*>(dWords_), 0u, 4, stream_);
     launch_cell_keys(cid_ + dw.cellOff, nullptr, n, b, dWords_, stream_);

@@ -9,6 +9,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <map>
 #include <memory>
@@ -182,7 +183,9 @@ public:
     };
     std::map<std::string, KernelTime> takeKernelTimes();
     size_t deviceBytes() const { return deviceBytes_; }
-    static uint64_t estimateBytes(uint64_t cells, uint64_t particles, int W, int H, int binSize);
+    // device memory of a set of one world with these cells and particle slots (host arithmetic only)
+    static uint64_t estimateBytes(uint64_t cells, uint64_t particles, int W, int H, int binSize, bool radiation,
+                                  bool splitting);
     void synchronize();
     hipStream_t stream() const { return stream_; }
 
@@ -191,6 +194,28 @@ private:
         void* p = nullptr;
         size_t bytes = 0;
     };
+    // hands out places of an allocation; without one, adds up the bytes
+    struct Places {
+        char* base = nullptr;
+        size_t used = 0;
+        void* operator()(size_t bytes) {
+            char* p = base ? base + used : nullptr;
+            used += (std::max<size_t>(bytes, 64) + 255) & ~size_t(255);
+            return p;
+        }
+    };
+    // what the sizes of a set's arrays follow from
+    struct Sizes {
+        size_t worlds = 0, cells = 0, particles = 0;  // (particles: with the staging slots)
+        size_t bins = 0, cellBins = 0;                // (bins: the particles' ones with them)
+        int groupShift = 8;
+        bool extra = false, radStage = false;
+        size_t splitSlots = 0;
+        std::vector<size_t> selected;  // per world: particles with a selection byte
+    };
+    struct SizesOnly {};
+    explicit WorldSet(SizesOnly);  // no device: for its layout alone
+    void layout(const Sizes& z, Places& A, Places& B);
     void* alloc(size_t bytes);
     void freeAll();
     void buildTables();

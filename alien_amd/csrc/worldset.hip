@@ -557,17 +557,6 @@ uint64_t WorldSet::estimateBytes(uint64_t cells, uint64_t particles, int W, int 
            (cells + particles + cellBins + partBins) + (1u << 20);
 }
 
-void WorldSet::clearAll() {
-    invalidateGraphs();
-    freeAll();
-    hosts_.clear();
-    worlds_.clear();
-    params_.clear();
-    densityPending_.clear();
-    cellCap_ = partCap_ = numBins_ = candCap_ = 0;
-    parity_ = 0;
-}
-
 int stageLayout(int64_t caps, int cells, bool radiation, bool splitting, int& splitStage, int& radStage);
 
 // Everything comes from two allocations, one for the particles' arrays (which growParticles replaces) and one

@@ -127,7 +127,6 @@ public:
         int fromIndex = -1;
     };
     void build(const std::vector<Source>& sources);
-    void clearAll();
 
     int numWorlds() const { return int(hosts_.size()); }
     HostWorld& host(int w) { return hosts_.at(w); }
@@ -221,7 +220,6 @@ private:
     void buildTables();
     void invalidateGraphs();
     Ctx makeCtx(int parity) const;
-    void ensureSorted();
     void checkErrors(StepCounters sc);
     // the same without a host synchronisation: acts on the count read at the previous call (if it
     // has arrived) and starts reading the current one
@@ -326,7 +324,6 @@ private:
     int* numPartBlocks_ = nullptr;  // (device) entries of partBlocks_
     std::vector<uint8_t> bondWork_;  // per world: a bonded or barrier cell exists or can appear by fusion
     std::vector<uint8_t> active_;    // per world: included in the launch tables
-    void adaptGrids();
     std::vector<Arr> tableAllocs_;
 
     hipGraphExec_t graph_[2] = {nullptr, nullptr};  // one step from parity 0 / 1

@@ -286,7 +286,6 @@ __device__ __forceinline__ void part_apply(const Ctx& c, Span at) {
     });
 }
 
-// absorption (:108-165); also bins the surviving particles for the next step
 // RadiationProcessor::splitting (RadiationProcessor.cuh:172-204), after absorption: with
 // probability 0.01 (R9 draw keyed by the particle id) a particle above particleSplitEnergy of its
 // colour halves its energy and splits in two, 1/5 of a random unit vector u either side of its
@@ -323,6 +322,7 @@ __device__ __forceinline__ void split_particle(const Ctx& c, const DevWorld& w, 
     pbin_for_next_step(c, w, c.splitStage + k, other, c.countNext);
 }
 
+// absorption (:108-165); also bins the surviving particles for the next step
 __device__ __forceinline__ void part_absorb(const Ctx& c, Span at) {
     for_live_particles(c, at, [&](int wi, const DevWorld& w, int k) {
         const int cm = c.absorbCell[k];

@@ -914,7 +914,6 @@ void WorldSet::build(const std::vector<Source>& sources) {
     for (int lp : liveParticles) shape_.hasParticles = shape_.hasParticles || lp > 0;
     parity_ = 0;
     shape_.candGrid = 16;
-    // one particle block per workgroup (blocks past a world's live particles exit at once)
 
     std::vector<DevCounters> ctr(worlds_.size());
     for (size_t i = 0; i < worlds_.size(); ++i) {
@@ -1463,9 +1462,8 @@ bool radiates(const alien_params& p) {
     return false;
 }
 
-// Reads the last step's candidate-list size: reports overflow and grows the grid of the fusion
-// kernels when the list outgrew it (the graphs are captured again on the next step).
-// (what the last step left in the counters)
+// From what the last step left in the counters: reports overflow of the candidate list and grows the grid of
+// the fusion kernels when the list outgrew it (the graphs are captured again on the next step).
 void WorldSet::checkErrors(StepCounters sc) {
     if (sc.errors & 1) {
         sc.errors = 0;

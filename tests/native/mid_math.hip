@@ -6,9 +6,21 @@ template <class F> __global__ void apply(const float* in, float* out, int n, F f
     const int i = int(blockIdx.x * blockDim.x + threadIdx.x);
     if (i < n) out[i] = f(in[i]);
 }
+// in, out: n floats of host memory
 template <class F> int run(const float* in, float* out, int n, F f) {
-    if (n > 0) apply<<<(n + 255) / 256, 256>>>(in, out, n, f);
-    return int(hipDeviceSynchronize());
+    if (n <= 0) return 0;
+    const size_t bytes = sizeof(float) * size_t(n);
+    float* d = nullptr;
+    hipError_t e = hipMalloc(reinterpret_cast<void**>(&d), 2 * bytes);
+    if (e != hipSuccess) return int(e);
+    e = hipMemcpy(d, in, bytes, hipMemcpyHostToDevice);
+    if (e == hipSuccess) {
+        apply<<<(n + 255) / 256, 256>>>(d, d + n, n, f);
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipMemcpy(out, d + n, bytes, hipMemcpyDeviceToHost);
+    (void)hipFree(d);
+    return int(e);
 }
 }  // namespace
 

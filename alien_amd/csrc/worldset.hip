@@ -987,7 +987,7 @@ void WorldSet::buildTables() {
             int64_t sum = 0;
             for (size_t wi = 0; wi < worlds_.size(); ++wi)
                 if (active_[wi] && worlds_[wi].numCells > 0 && (params_[wi].motion == 0) == fluid)
-                    sum += int64_t(kEdgeWaves) * (worlds_[wi].nby / n + 1);
+                    sum += int64_t(kEdgeWaves) * (worlds_[wi].nby / n);
             return sum;
         };
         while (n < kEdgeUnitsMost && waves() > kEdgeWavesMost) n *= 2;

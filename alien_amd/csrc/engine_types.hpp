@@ -38,7 +38,7 @@ constexpr int kSuperGroups = 256;  // groups per sum of groups
 constexpr int kFluidShiftMin = 4;
 // waves of the neighbour passes for a group of units of two edge bins (k_neighbor.hip); units per group: as few as
 // keep a set's edge waves at kEdgeWavesMost, two for a SIMD, or less (150k fluid cells of 707 x 1010 units, a step:
-// 24.4 us with 4096 as the limit, 21.7 with 2048, with 1024 the same; 14k cells of 290 x 327: 16.3 us with 2048 and
+// 24.4 us with 4096 as the limit, 21.7 with 2048, with 1024 the same; 17k cells of 214 x 296: 16.1 us with 2048 and
 // 1024, 16.9 with 512, 20.2 with 256)
 constexpr int kEdgeWaves = 8, kEdgeUnitsMost = 8, kEdgeWavesMost = 2048;
 constexpr int kXcdCount = 8;  // XCDs of an MI355X: workgroup b of a launch runs on XCD b % 8
@@ -196,11 +196,30 @@ struct FarCells {
     int2* list;  // (global bin, part); one array for both steps: read before it is written
 };
 
+// Every launch of a forked graph copies the context (launch.hip): a step of a small radiating world, 70 us in nine
+// launches, took 2.5 us more with 128 bytes more in it, so its numbers lie together without gaps.
 struct Ctx {
     int numWorlds;
     int cellCap;  // total cells (= sum of numCells)
     int partCap;  // total particle slots
     int numBins;  // cell bins + particle bins of all worlds
+    int numCellBins;  // cell bins of all worlds, each world's padded to a multiple of kGroupBins
+    int cellCount;    // cells of all worlds
+    int groupShift;   // 1 << groupShift bins per group of the map: 8, 6 or 4
+    int candCap;
+    int timestepAdvanced;  // 1 if the step's map scan advanced the worlds' timesteps
+    // Particles emitted by cell radiation during a step are written at partStage + (cell index),
+    // behind the worlds' particle ranges (partStage = 0: no staging area), and enter the step's
+    // particle map like the live particles.
+    int partStage;
+    // Particles split off at the end of a step: staging slot splitStage + k for the particle at k
+    // (0: no split staging area), record splitStaged[k]; they enter the next step's map behind the
+    // particles that lived and before that step's radiation
+    int splitStage;
+    int blockThreads;        // cells, bins or living cells per entry of cellBlocks .. livingBlocks
+    int partBlockParticles;  // particles per entry of partBlocks
+    int fluidShift, collideShift;     // waves of the fluid / collision pass take 1 << shift cells
+    int edgeUnits, collideEdgeUnits;  // edge units that kEdgeWaves waves share
     const DevWorld* worlds;
     const DevParams* params;
     DevCounters* ctr;
@@ -211,17 +230,8 @@ struct Ctx {
     float* stiff;   // cold [cellCap]
     unsigned long long* cid;  // cold [cellCap]: cell id (key of the cell's random draws)
     uint32_t* ageBase;        // cold [cellCap]: cell age at the world's ageTs
-    // Particles emitted by cell radiation during a step are written at partStage + (cell index),
-    // behind the worlds' particle ranges (partStage = 0: no staging area), and enter the step's
-    // particle map like the live particles.
-    int partStage;
     StagedParticle* staged;  // [cellCap]: the particle of staging slot partStage + i at staged[i]
-    // Particles split off at the end of a step: staging slot splitStage + k for the particle at k
-    // (0: no split staging area), record splitStaged[k]; they enter the next step's map behind the
-    // particles that lived and before that step's radiation
-    int splitStage;
     StagedParticle* splitStaged;
-    int timestepAdvanced;  // 1 if the step's map scan advanced the worlds' timesteps
     // living states of the worlds with livingWork, cold by slot: `living` holds the state at the
     // start of the step, `livingNext` the other buffer (the step's phases alternate between the
     // two and leave the end-of-step state in `livingNext`, the next step's `living`)
@@ -236,10 +246,7 @@ struct Ctx {
     // positions (and by seeding), brought back to zero by the particle scatter.
     uint32_t* count;      // [numBins] start-of-step state
     uint32_t* countNext;  // [numBins] end-of-step state (next step's `count`)
-    int numCellBins;      // cell bins of all worlds, each world's padded to a multiple of kGroupBins
-    int cellCount;        // cells of all worlds
     const int* groupWorld;  // [numCellBins / kGroupBins] the bins' world
-    int groupShift;         // 1 << groupShift bins per group of the map: 8, 6 or 4
     // Cells that the groups of cell bins, and kSuperGroups of those, gained (or lost) since the
     // last map; ...Next: for the next step (built during this step)
     int* groupSum;
@@ -274,7 +281,6 @@ struct Ctx {
     uint32_t* valid;  // [cellCap]
     unsigned long long* claim;  // [cellCap]
     int4* cand;                 // [candCap] (a, b, world, live)
-    int candCap;
     int* want;        // [partCap]
     int* fclaim;      // [partCap]
     int* absorbCell;  // [partCap]
@@ -287,15 +293,10 @@ struct Ctx {
     // particle bin sort for the ranges it publishes (*numPartBlocks entries)
     int2* partBlocks;
     int* numPartBlocks;
-    int partBlockParticles;
     const int2* fluidBlocks;  // per workgroup of the fluid pass: (world, its first wave)
-    int fluidShift;           // its waves take 1 << fluidShift cells
     const int2 *collideBlocks, *collideEdgeBlocks;  // the same of the collision pass
-    int collideShift;
     const int2* edgeBlocks;  // per workgroup: (world, its first edge wave), see k_neighbor.hip
-    int edgeUnits, collideEdgeUnits;  // edge units that kEdgeWaves waves share
     const int2* livingBlocks;  // per block: (world, first global cell index) over livingWork worlds
-    int blockThreads;  // cells, bins or living cells per entry of the block tables above
 };
 
 }  // namespace alien

@@ -37,10 +37,11 @@ constexpr int kSuperGroups = 256;  // groups per sum of groups
 // wave's fixed work counts (134k cells in bodies: 159, 157 and 162 us; 256k free ones: 22, 26 and 32 us).
 constexpr int kFluidShiftMin = 4;
 // waves of the neighbour passes for a group of units of two edge bins (k_neighbor.hip); units per group: as few as
-// keep a set's edge waves at kEdgeWavesMost, two for a SIMD, or less (150k fluid cells of 707 x 1010 units, a step:
-// 24.4 us with 4096 as the limit, 21.7 with 2048, with 1024 the same; 17k cells of 214 x 296: 16.1 us with 2048 and
-// 1024, 16.9 with 512, 20.2 with 256)
-constexpr int kEdgeWaves = 8, kEdgeUnitsMost = 8, kEdgeWavesMost = 2048;
+// keep a set's edge waves at kEdgeWavesMost, two and a half for a SIMD, or less.  A step, us: 150k fluid cells of
+// 707 x 1010 units 24.4 with 4096 as the limit, 21.7 with 2048; cells in bodies of 926 x 1115 units 145.2 with 2048,
+// 141.9 with 2560, 141.4 with 4096, of 1024 x 1024 units 133.2, 133.2 and 136.5; 17k fluid cells of 214 x 296 units
+// 16.1 with 1024, 16.9 with 512, 20.2 with 256.
+constexpr int kEdgeWaves = 8, kEdgeUnitsMost = 8, kEdgeWavesMost = 2560;
 constexpr int kXcdCount = 8;  // XCDs of an MI355X: workgroup b of a launch runs on XCD b % 8
 // Size limits of one world set.  Cell indices, bin offsets and the bond planes ([kMaxBonds][cap],
 // addressed as b * cap + x) are 32-bit ints in the kernels, so a set holds at most

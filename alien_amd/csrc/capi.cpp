@@ -578,6 +578,9 @@ struct Job {
     int state = ALIEN_JOB_QUEUED;
     uint64_t stepsRequested = 0, stepsDone = 0;
     uint64_t numCells = 0, numParticles = 0;
+    // estimated bytes in a set none of whose worlds radiates [0][], splits [][0], or some do; alone: bytes
+    uint64_t inSet[2][2] = {};
+    bool radiates = false, splits = false;
     uint64_t bytes = 0;
     double submitTime = 0, startTime = 0, finishTime = 0;
     std::unique_ptr<WorldImage> image;
@@ -632,15 +635,16 @@ struct alien_server {
                 }
             }
             std::vector<uint64_t> admitted;
-            uint64_t kept = 0, cells = 0, parts = 0;
+            uint64_t cells = 0, parts = 0;
+            bool radiation = false, splitting = false;
             for (auto id : keep) {
-                kept += jobs.at(id)->bytes;
+                radiation = radiation || jobs.at(id)->radiates;
+                splitting = splitting || jobs.at(id)->splits;
                 cells += jobs.at(id)->numCells;
                 parts += jobs.at(id)->numParticles;
             }
             // the old set keeps its memory until the new one is built (the budget bounds the peak)
             const uint64_t oldSet = set ? uint64_t(set->deviceBytes()) : 0;
-            uint64_t used = 0;
             while (!queue.empty()) {
                 uint64_t id = queue.front();
                 auto it = jobs.find(id);
@@ -650,12 +654,18 @@ struct alien_server {
                     continue;
                 }
                 Job& j = *it->second;
-                // the budget, and the size limits of one world set (alien::kMaxSetCells)
-                if (alien_server_plan_admission(budget, oldSet, kept + used, &j.bytes, 1) == 0 ||
+                // the budget, for the set with this job in it (a world that radiates or splits gives every
+                // world of its set staging slots), and the size limits of one world set (alien::kMaxSetCells)
+                const bool rad = radiation || j.radiates, split = splitting || j.splits;
+                uint64_t kept = 0;
+                for (const auto* ids : {&keep, &admitted})
+                    for (auto other : *ids) kept += jobs.at(other)->inSet[rad][split];
+                if (alien_server_plan_admission(budget, oldSet, kept, &j.inSet[rad][split], 1) == 0 ||
                     cells + j.numCells > uint64_t(alien::kMaxSetCells) ||
                     parts + j.numParticles > uint64_t(alien::kMaxSetParticles))
                     break;
-                used += j.bytes;
+                radiation = rad;
+                splitting = split;
                 cells += j.numCells;
                 parts += j.numParticles;
                 admitted.push_back(id);
@@ -866,9 +876,13 @@ int alien_server_submit(alien_server* s, const alien_world_desc* desc, const ali
         job->numCells = numCells;
         job->numParticles = numParticles;
         // (a radiating or splitting world is built with room for the particles it will create)
-        job->bytes = WorldSet::estimateBytes(
-            numCells, uint64_t(alien::particle_room(int64_t(numCells), int64_t(numParticles), *params)),
-            desc->worldSizeX, desc->worldSizeY, alien::bin_size_for(*params), alien::radiates(*params), alien::splits(*params));
+        const uint64_t room = uint64_t(alien::particle_room(int64_t(numCells), int64_t(numParticles), *params));
+        job->radiates = alien::radiates(*params);
+        job->splits = alien::splits(*params);
+        for (int k = 0; k < 4; ++k)
+            job->inSet[k >> 1][k & 1] = WorldSet::estimateBytes(numCells, room, desc->worldSizeX, desc->worldSizeY,
+                                                                alien::bin_size_for(*params), k >> 1, k & 1);
+        job->bytes = job->inSet[job->radiates][job->splits];
         if (job->bytes > s->budget) throw Error(ALIEN_E_BUDGET, "job does not fit the device memory budget");
         job->submitTime = nowSeconds();
         std::lock_guard<std::mutex> lk(s->mu);

@@ -521,8 +521,8 @@ static size_t cand_entries(size_t cells) { return std::max<size_t>(4 * cells, 40
 
 // What a set of one such world takes: its layout, whose arrays grow in step with the cells, the particle slots
 // and the bins, taken at two sizes each; the read-back's sort where the candidate list is too small for it; the
-// launch tables (8 B for 64 elements or more, at most four tables of the cells).  A world that neither radiates
-// nor splits pays staging slots as well in a set with one that does: those are not counted.
+// launch tables (8 B for 64 elements or more, at most four tables of the cells).  radiation, splitting: of some
+// world of its set (every world pays the staging slots).
 uint64_t WorldSet::estimateBytes(uint64_t cells, uint64_t particles, int W, int H, int binSize, bool radiation,
                                  bool splitting) {
     const size_t unit = size_t(1) << 20;

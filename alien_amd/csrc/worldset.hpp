@@ -182,7 +182,8 @@ public:
     };
     std::map<std::string, KernelTime> takeKernelTimes();
     size_t deviceBytes() const { return deviceBytes_; }
-    // device memory of a set of one world with these cells and particle slots (host arithmetic only)
+    // device memory of a world with these cells and particle slots as part of a set with radiating or splitting
+    // worlds (host arithmetic only)
     static uint64_t estimateBytes(uint64_t cells, uint64_t particles, int W, int H, int binSize, bool radiation,
                                   bool splitting);
     void synchronize();

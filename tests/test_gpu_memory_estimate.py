@@ -61,3 +61,34 @@ def test_estimate_covers_a_simulation(n, np_, size, radiation, splitting):
     print("took", took, "estimate", estimate, flush=True)
     assert took <= estimate + SLACK
     assert estimate <= 1.3 * took + SLACK
+
+
+def test_admission_counts_the_staging_of_mixed_sets():
+    """A world without radiation takes staging slots too beside one that radiates: two jobs that fit the budget by
+    their own estimates, but not in one set, run one after the other."""
+    rng = np.random.default_rng(5)
+    size = (800, 800)
+
+    def job(n, radiation):
+        cells = worlds.free_cells(rng, size, n, vel_sigma=0.1)
+        cells["energy"] = 150
+        params = H.params(MOTION_FLUID)
+        for c in range(abi.MAX_COLORS):
+            params.radiationCellAgeStrength[c] = 0.001 if radiation else 0.0
+        return params, cells, np.zeros(0, dtype=abi.PARTICLE_DTYPE)
+
+    big, small = job(300_000, False), job(10_000, True)
+    probe = engine.Server(budget_bytes=1 << 40, chunk_steps=8)
+    need = [probe.poll(probe.submit(size, *j, 0)).deviceBytes for j in (big, small)]
+    probe.close()
+    print("need", need, flush=True)
+    server = engine.Server(budget_bytes=sum(need) + (2 << 20), chunk_steps=50)
+    # (the first job leaves no room until it is done; the other two are queued by then)
+    first = server.submit(size, *big, 20000)
+    later = [server.submit(size, *j, 100) for j in (big, small)]
+    for j in [first] + later:
+        server.wait(j, timeout=100)
+    one, two = (server.poll(j) for j in later)
+    assert one.startTime >= server.poll(first).finishTime  # (both were queued while the first ran)
+    assert two.startTime >= one.finishTime
+    server.close()

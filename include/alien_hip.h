@@ -309,7 +309,8 @@ int alien_server_get_snapshot(alien_server* s, uint64_t jobId, alien_cell_to* ce
                               uint64_t* numParticles);
 /* Drops a finished job's snapshot, or cancels a queued/running job. */
 int alien_server_release(alien_server* s, uint64_t jobId);
-/* Estimated device bytes a job of this size needs (the admission figure). */
+/* Estimated device bytes a job of this size needs, without cell radiation and particle splitting.  (The
+ * admission figure of a job, alien_job_info.deviceBytes, counts their room and staging slots too.) */
 uint64_t alien_server_estimate_bytes(uint64_t numCells, uint64_t numParticles, int32_t worldSizeX,
                                      int32_t worldSizeY);
 /* The admission rule of the server (host arithmetic only): how many of the queued jobs, in order,

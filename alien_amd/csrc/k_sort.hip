@@ -262,7 +262,7 @@ __device__ __forceinline__ void part_scan(const Ctx& c, int tiles) {
 //    with one bin of a round after the other, 26 with turns).
 //  - Far cells: the near cells of a bin with few of them take its first places, and at the end the bin's lane
 //    merges its far cells in (256k cells that move 5 units a step: a step of 158 us with a wave for each far
-//    cell, 62 so; 1M of them 500 and 117).  Bins with more far cells than a lane takes (kFarWalk) get a wave
+//    cell, 58 so; 1M of them 500 and 111).  Bins with more far cells than a lane takes (kFarWalk) get a wave
 //    per 64 of them: it counts the cells of the group before them over the group's reach, and their ranks
 //    along the list; the near cells of such a bin add the list's smaller indices.
 // ---------------------------------------------------------------------------------------------
